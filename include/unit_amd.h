@@ -185,6 +185,13 @@ int unit_gemm_f16_static(const void *a, const void *b, void *c, int32_t M, int32
 int unit_conv2d_nchw16c_f16f32(const unit_conv_desc *d, const void *a, const void *b, void *out,
                                unit_stream_t stream);
 
+/* The same operator on plain operands a f16 (N, C, H, W), b f16 (K, C, KH, KW) (any alignment of an element), which it
+ * re-lays itself as the reference operator does (python/tensorizer/ops/gpu.py:25-33): one launch writes NCHW16c data
+ * and MFMA-ordered weights into the caller's workspace, a second convolves.  C and K multiples of 16, d->cb == 16. */
+int unit_conv2d_nchw_f16f32_ws_bytes(const unit_conv_desc *d, size_t *bytes);
+int unit_conv2d_nchw_f16f32(const unit_conv_desc *d, const void *a, const void *b, void *out, void *workspace,
+                            size_t workspace_bytes, unit_stream_t stream);
+
 /* ------------------------------------------------------------------ layout / pre-pack */
 
 /* layout_transform NCHW -> NCHW{cb}c (apps/cpu/relay/result.log:7,6807-6808; in-op form

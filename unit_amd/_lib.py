@@ -32,6 +32,8 @@ SYMBOLS = (
     "unit_gemm_f16_prepare_b_packed32",
     "unit_gemm_f16_prepared",
     "unit_conv2d_nchw16c_f16f32",
+    "unit_conv2d_nchw_f16f32_ws_bytes",
+    "unit_conv2d_nchw_f16f32",
     "unit_pack_nchwc",
     "unit_unpack_nchwc",
     "unit_prepack_conv_weight_s8",
@@ -100,6 +102,8 @@ def load():
     L.unit_gemm_f16_prepare_b_packed32.argtypes = [vp, vp, i32, i32, vp]
     L.unit_gemm_f16_prepared.argtypes = [vp, vp, vp, i32, i32, i32, i32, vp]
     L.unit_conv2d_nchw16c_f16f32.argtypes = [dp, vp, vp, vp, vp]
+    L.unit_conv2d_nchw_f16f32_ws_bytes.argtypes = [dp, ctypes.POINTER(ctypes.c_size_t)]
+    L.unit_conv2d_nchw_f16f32.argtypes = [dp, vp, vp, vp, vp, ctypes.c_size_t, vp]
     L.unit_pack_nchwc.argtypes = [vp, vp, i32, i32, i32, i32, i32, i32, vp]
     L.unit_unpack_nchwc.argtypes = [vp, vp, i32, i32, i32, i32, i32, i32, vp]
     L.unit_prepack_conv_weight_s8.argtypes = [vp, vp, i32, i32, i32, i32, i32, vp]

@@ -504,9 +504,19 @@ def conv2d_NCHW16c_OHWI16o(a, b, stride_h, stride_w, out_type="float32"):
     if a.dim() == 4 and b.dim() == 4:
         if a.shape[1] % 16 or b.shape[0] % 16 or b.shape[1] != a.shape[1]:
             raise ValueError("a, b: channel counts must match and be multiples of 16")
-        a = pack_nchwc(a, 16)
-        b = prepack_conv_weight_f16(b)
-    elif not (a.dim() == 5 and b.dim() == 6):
+        n, c, h, w = a.shape
+        k, _, kh, kw = b.shape
+        d = ConvDesc(n, c, h, w, k, kh, kw, int(stride_h), int(stride_w), 0, 0, 0, 0, 1, 1, 16)
+        L = _lib.load()
+        oh, ow, need = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_size_t()
+        check(L.unit_conv_out_hw(ctypes.byref(d), ctypes.byref(oh), ctypes.byref(ow)))
+        check(L.unit_conv2d_nchw_f16f32_ws_bytes(ctypes.byref(d), ctypes.byref(need)))
+        ws = torch.empty((need.value,), dtype=torch.uint8, device=a.device)
+        out = torch.empty((n, k // 16, oh.value, ow.value, 16), dtype=torch.float32, device=a.device)
+        check(L.unit_conv2d_nchw_f16f32(ctypes.byref(d), a.data_ptr(), b.data_ptr(), out.data_ptr(), ws.data_ptr(),
+                                        need.value, _stream()))
+        return out
+    if not (a.dim() == 5 and b.dim() == 6):
         raise ValueError("a, b: expected 4-D + 4-D or 5-D + 6-D operands")
     n, cc, h, w, cb = a.shape
     ko, ib, kh, kw, ic, ob = b.shape
