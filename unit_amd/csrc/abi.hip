@@ -13,9 +13,9 @@ char *error_buf() {
   return buf;
 }
 
-char *variant_buf() {
-  static thread_local char buf[96] = "";
-  return buf;
+VariantNote &variant_note() {
+  static thread_local VariantNote note = {nullptr, nullptr, {}};
+  return note;
 }
 
 int tuning_override(const char *name) {
@@ -210,7 +210,12 @@ extern "C" int unit_version(void) { return 106; }  // 1.6: results stored sc1 nt
 
 extern "C" const char *unit_last_error(void) { return unit::error_buf(); }
 
-extern "C" const char *unit_last_variant(void) { return unit::variant_buf(); }
+extern "C" const char *unit_last_variant(void) {
+  static thread_local char name[96] = "";
+  const unit::VariantNote &note = unit::variant_note();
+  if (note.spell) note.spell(note, name, sizeof name);
+  return name;
+}
 
 extern "C" int unit_conv_out_hw(const unit_conv_desc *d, int32_t *OH, int32_t *OW) {
   if (!d || !OH || !OW) return unit::fail(UNIT_E_ARG, "unit_conv_out_hw: null pointer");

@@ -28,10 +28,8 @@ int run_conv_f16(const unit_conv_desc *d, const ConvGeom &g0, const void *a, con
   typename Epi::Params ep{out, d->K, g.OH * g.OW, g.npix, g.by_ohw, nullptr, 1, nullptr, 0};
   const int gx = ceil_div(d->K, T::BX), gy = ceil_div(g.npix, T::BY);
   const int panel = plan.panel > 0 && plan.panel < gx ? plan.panel : 0;
-  char tail[16] = "";
-  if (panel) snprintf(tail, sizeof tail, "_r%d", panel);
   set_variant("f16conv_x%d_y%d_k%d_w%dx%d_p%d%s%s%s", T::BX, T::BY, T::BKB, T::WX, T::WY, PF, T::FF ? "f" : "",
-              T::KG == 1 ? "" : (T::KG == 2 ? "_g2" : "_g4"), tail);
+              T::KG == 1 ? "" : (T::KG == 2 ? "_g2" : "_g4"), Panel{panel});
   return launch_mma<OpF16, T, XL, YL, Epi, WS_NONE>(xp, yp, ep, nk, gx, gy, panel ? panel : gx, 1, out, 0, g.ntab * 8, s,
                                                     "unit_conv2d_nchw16c_f16f32");
 }

@@ -27,10 +27,8 @@ int run_conv_i8(const unit_conv_desc *d, const ConvGeom &g0, const void *data, c
   const int gx = ceil_div(d->K, T::BX), gy = ceil_div(g.npix, T::BY);
   const int splits = plan.splits > nk ? nk : plan.splits;
   const int panel = plan.panel > 0 && plan.panel < gx ? plan.panel : 0;
-  char tail[16] = "";
-  if (panel) snprintf(tail, sizeof tail, "_r%d", panel);
   set_variant("%s_c%d_x%d_y%d_k%d_w%dx%d_p%d%s%s%s_s%d", SIGNED ? "s8conv" : "i8conv", TAPB, T::BX, T::BY, T::BKB, T::WX, T::WY, PF, T::FF ? "f" : "",
-              T::KG == 1 ? "" : (T::KG == 2 ? "_g2" : "_g4"), tail, splits);
+              T::KG == 1 ? "" : (T::KG == 2 ? "_g2" : "_g4"), Panel{panel}, splits);
   return launch_mma<OpI8, T, XL, YL, Epi, SIGNED ? WS_NONE : WS_X>(xp, yp, ep, nk, gx, gy, panel ? panel : gx, splits,
                                                                    out, (size_t)g.npix * d->K * 4, g.ntab * 8, s, what);
 }

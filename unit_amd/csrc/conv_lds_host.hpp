@@ -26,9 +26,7 @@ int run_lds(const char *what, const char *tag, const unit_conv_desc *d, const Co
   const int gx = ceil_div(d->K, S::BX), gy = ceil_div(g.npix, S::BY);
   const int panel = plan.panel > 0 && plan.panel < gx ? plan.panel : 0;
   const GridMap gm = GridMap::make(gx, gy, panel ? panel : gx, 1);
-  char tail[16] = "";
-  if (panel) snprintf(tail, sizeof tail, "_r%d", panel);
-  set_variant("%s_x%d_y%d_w%dx%d_g%d_k%d_r%d%s_s1", tag, S::BX, S::BY, S::WX, S::WY, S::KG, S::KS, S::NST, tail);
+  set_variant("%s_x%d_y%d_w%dx%d_g%d_k%d_r%d%s_s1", tag, S::BX, S::BY, S::WX, S::WY, S::KG, S::KS, S::NST, Panel{panel});
   hipLaunchKernelGGL(kern, dim3(gm.total), dim3(S::NT), lds, s, static_cast<const char *>(data),
                      static_cast<const char *>(w), zero, ep, g, gm, pl.nsteps);
   hipError_t e = hipGetLastError();

@@ -12,6 +12,7 @@ Reference call sites:
 """
 import ctypes
 import re
+from functools import lru_cache
 
 import torch
 
@@ -29,7 +30,8 @@ __all__ = [
 
 # ------------------------------------------------------------------------------- helpers
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    # the handle of torch.cuda.current_stream(), without building the Stream object (0.2 against 2.7 us)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _dev(t, name, dtype=None, ndim=None):
@@ -65,6 +67,7 @@ def _pad4(padding):
     raise ValueError(f"padding: expected an int, (ph, pw) or (pt, pl, pb, pr), got {p}")
 
 
+@lru_cache(maxsize=64)
 def _layout_block(layout, name):
     m = re.fullmatch(r"NCHW(\d+)c", layout)
     if not m:
@@ -78,10 +81,73 @@ def conv_out_hw(h, w, kh, kw, stride, padding=0, dilation=1):
     dh, dw = _pair(dilation, "dilation")
     pt, pl, pb, pr = _pad4(padding)
     d = ConvDesc(1, 16, h, w, 16, kh, kw, sh, sw, pt, pl, pb, pr, dh, dw, 16)
-    import ctypes
     oh, ow = ctypes.c_int32(), ctypes.c_int32()
     check(_lib.load().unit_conv_out_hw(ctypes.byref(d), ctypes.byref(oh), ctypes.byref(ow)))
     return oh.value, ow.value
+
+
+# Shapes, strides and padding of a convolution -> its descriptor and result shape.  A call costs the GPU as little as
+# 4 us, less than checking the operands' shapes against each other and asking the library for the output size on
+# every call did: that is a function of these plain values alone and is kept for the last 1024 combinations.
+class _ConvPlan:
+    __slots__ = ("desc", "ref", "ko", "n", "oh", "ow", "blocked")
+
+    def __init__(self, n, c, h, w, k, kh, kw, stride, padding, dilation, cb):
+        sh, sw = _pair(stride, "stride")
+        dh, dw = _pair(dilation, "dilation")
+        pt, pl, pb, pr = _pad4(padding)
+        self.desc = ConvDesc(n, c, h, w, k, kh, kw, sh, sw, pt, pl, pb, pr, dh, dw, cb)
+        self.ref = ctypes.byref(self.desc)
+        oh, ow = ctypes.c_int32(), ctypes.c_int32()
+        check(_lib.load().unit_conv_out_hw(self.ref, ctypes.byref(oh), ctypes.byref(ow)))
+        self.n, self.ko, self.oh, self.ow = n, k // 16, oh.value, ow.value
+        self.blocked = (n, self.ko, self.oh, self.ow, 16)  # shape of the blocked result
+
+
+@lru_cache(maxsize=1024, typed=True)
+def _plan_int8(dshape, kshape, stride, padding, dilation):
+    """dshape: the data's; kshape: the blocked kernel's, or (K, C, KH, KW, cb) of a prepared one."""
+    n, cc, h, w, cb = dshape
+    if cb not in (4, 16):
+        raise ValueError(f"data: channel block must be 16 or 4, got {cb}")
+    if len(kshape) == 5:
+        k, c, kh, kw, kcb = kshape
+        if kcb != cb or c != cc * cb:
+            raise ValueError(f"kernel: prepared for K={k}, C={c}, {kh} x {kw}, channel blocks of {kcb}: does not match data {tuple(dshape)}")
+    else:
+        ko, cc2, kh, kw, e, kb, i4 = kshape
+        if (cc2, e, kb, i4) != (cc, cb // 4, 16, 4):
+            raise ValueError(f"kernel: shape {tuple(kshape)} does not match data {tuple(dshape)}; "
+                             f"expected (K/16, {cc}, KH, KW, {cb // 4}, 16, 4)")
+        k = ko * 16
+    return _ConvPlan(n, cc * cb, h, w, k, kh, kw, stride, padding, dilation, cb)
+
+
+@lru_cache(maxsize=1024, typed=True)
+def _plan_f16(dshape, kshape, stride_h, stride_w):
+    """dshape (N, C/16, H, W, 16); kshape: the blocked kernel's, or (K, C, KH, KW, 16) of a prepared one."""
+    n, cc, h, w, cb = dshape
+    if len(kshape) == 5:
+        k, c, kh, kw, kcb = kshape
+        if kcb != cb or c != cc * cb:
+            raise ValueError(f"kernel: prepared for K={k}, C={c}, {kh} x {kw}, channel blocks of {kcb}: does not match data {tuple(dshape)}")
+    else:
+        ko, ib, kh, kw, ic, ob = kshape
+        if cb != 16 or ic != 16 or ob != 16 or ib != cc:
+            raise ValueError(f"a {tuple(dshape)} / b {tuple(kshape)}: expected (N, C/16, H, W, 16) and "
+                             f"(K/16, C/16, KH, KW, 16, 16)")
+        k = ko * 16
+    return _ConvPlan(n, cc * 16, h, w, k, kh, kw, (int(stride_h), int(stride_w)), 0, 1, 16)
+
+
+def _hashable(v):
+    """A stride / padding / dilation argument as a key: ints and tuples as they are, other sequences as tuples of ints."""
+    return v if type(v) is int else v if isinstance(v, int) else tuple(int(x) for x in v)
+
+
+def _plan(data, kernel, stride, padding, dilation):
+    kshape = kernel.key if isinstance(kernel, PreparedConvWeight) else kernel.shape
+    return _plan_int8(data.shape, kshape, _hashable(stride), _hashable(padding), _hashable(dilation))
 
 
 def last_variant():
@@ -99,6 +165,10 @@ class PreparedConvWeight:
     def __init__(self, buf, K, C, KH, KW, cb, dtype):
         self.buf, self.K, self.C, self.KH, self.KW, self.cb, self.dtype = buf, K, C, KH, KW, cb, dtype
 
+    @property
+    def key(self):
+        return self.K, self.C, self.KH, self.KW, self.cb
+
     def __repr__(self):
         return (f"PreparedConvWeight(K={self.K}, C={self.C}, KH={self.KH}, KW={self.KW}, cb={self.cb}, "
                 f"dtype={self.dtype})")
@@ -113,7 +183,6 @@ def prepare_conv2d_weight(kernel):
            4-channel blocks), or fp16 (K/16, C/16, KH, KW, 16 in, 16 out)
     returns a PreparedConvWeight; convolutions on it give the same results as on `kernel`.
     """
-    import ctypes
     if isinstance(kernel, torch.Tensor) and kernel.dtype == torch.float16:
         kernel = _dev(kernel, "kernel", torch.float16, 6)
         ko, cc, kh, kw, ic, ob = kernel.shape
@@ -134,16 +203,17 @@ def prepare_conv2d_weight(kernel):
     return PreparedConvWeight(buf, ko * 16, cc * cb, kh, kw, cb, kernel.dtype)
 
 
-def _prepared_dims(kernel, data, want_dtype):
-    """(K/16, C/16, KH, KW) of a PreparedConvWeight after checking it against the data tensor."""
-    n, cc, h, w, cb = data.shape
+def _check_prepared(kernel, data, want_dtype):
     if kernel.dtype != want_dtype:
         raise TypeError(f"kernel: prepared from {kernel.dtype}, this operator takes {want_dtype}")
-    if cb != kernel.cb or kernel.C != cc * cb:
-        raise ValueError(f"kernel: {kernel!r} does not match data {tuple(data.shape)}")
     if kernel.buf.device != data.device:
         raise ValueError("kernel: prepared on another device")
-    return kernel.K // 16, cc, kernel.KH, kernel.KW
+
+
+def _check_bias(bias, k, data):
+    if bias.dtype != torch.int32 or bias.numel() != k or bias.device != data.device:
+        raise ValueError(f"bias: expected {k} int32 values on {data.device}")
+    return bias.contiguous()
 
 
 # ------------------------------------------------------------------------------- int8
@@ -158,7 +228,6 @@ def conv2d_NCHWc_int8(data, kernel, stride, padding, dilation=1, out_dtype="int3
     As in TVM the channel block is taken from the tensor shapes; `layout` / `out_layout` are
     checked for form only (the reference's driver passes 'NCHW4c' for 16-channel blocks too).
     """
-    import ctypes
     data = _dev(data, "data", torch.uint8, 5)
     prepared = isinstance(kernel, PreparedConvWeight)
     if not prepared:
@@ -168,30 +237,15 @@ def conv2d_NCHWc_int8(data, kernel, stride, padding, dilation=1, out_dtype="int3
     _layout_block(layout, "layout")
     if _layout_block(out_layout, "out_layout") != 16:
         raise ValueError("out_layout: the output channel block is 16 (NCHW16c)")
-    n, cc, h, w, cb = data.shape
-    if cb not in (4, 16):
-        raise ValueError(f"data: channel block must be 16 or 4, got {cb}")
     if prepared:
-        ko, cc2, kh, kw = _prepared_dims(kernel, data, torch.int8)
-    else:
-        ko, cc2, kh, kw, e, kb, i4 = kernel.shape
-        if (cc2, e, kb, i4) != (cc, cb // 4, 16, 4):
-            raise ValueError(f"kernel: shape {tuple(kernel.shape)} does not match data {tuple(data.shape)}; "
-                             f"expected (K/16, {cc}, KH, KW, {cb // 4}, 16, 4)")
-    sh, sw = _pair(stride, "stride")
-    dh, dw = _pair(dilation, "dilation")
-    pt, pl, pb, pr = _pad4(padding)
-    d = ConvDesc(n, cc * cb, h, w, ko * 16, kh, kw, sh, sw, pt, pl, pb, pr, dh, dw, cb)
+        _check_prepared(kernel, data, torch.int8)
+    p = _plan(data, kernel, stride, padding, dilation)
     L = _lib.load()
-    oh, ow = ctypes.c_int32(), ctypes.c_int32()
-    check(L.unit_conv_out_hw(ctypes.byref(d), ctypes.byref(oh), ctypes.byref(ow)))
-    out = torch.empty((n, ko, oh.value, ow.value, 16), dtype=torch.int32, device=data.device)
+    out = data.new_empty(p.blocked, dtype=torch.int32)
     if prepared:
-        check(L.unit_conv2d_nchwc_u8s8s32_prepared(ctypes.byref(d), data.data_ptr(), kernel.buf.data_ptr(),
-                                                   out.data_ptr(), _stream()))
+        check(L.unit_conv2d_nchwc_u8s8s32_prepared(p.ref, data.data_ptr(), kernel.buf.data_ptr(), out.data_ptr(), _stream()))
     else:
-        check(L.unit_conv2d_nchwc_u8s8s32(ctypes.byref(d), data.data_ptr(), kernel.data_ptr(), out.data_ptr(),
-                                          _stream()))
+        check(L.unit_conv2d_nchwc_u8s8s32(p.ref, data.data_ptr(), kernel.data_ptr(), out.data_ptr(), _stream()))
     return out
 
 
@@ -214,7 +268,6 @@ def conv2d_NCHWc_int8_fused(data, kernel, bias, scale, stride, padding, dilation
     (result.log:25) into the store: returns int32 (N, out_channels, OH, OW), out_channels
     (default K) being the channel count before the caller padded it up to a multiple of 16.
     """
-    import ctypes
     data = _dev(data, "data", torch.int8, 5)
     prepared = isinstance(kernel, PreparedConvWeight)
     if not prepared:
@@ -229,43 +282,32 @@ def conv2d_NCHWc_int8_fused(data, kernel, bias, scale, stride, padding, dilation
         raise ValueError("out_channels: only with out_layout='NCHW'")
     if not planar and _layout_block(out_layout, "out_layout") != 16:
         raise ValueError("out_layout: the output channel block is 16 (NCHW16c), or 'NCHW'")
-    n, cc, h, w, cb = data.shape
-    if cb not in (4, 16):
-        raise ValueError(f"data: channel block must be 16 or 4, got {cb}")
     if prepared:
-        ko, cc2, kh, kw = _prepared_dims(kernel, data, torch.int8)
-    else:
-        ko, cc2, kh, kw, e, kb, i4 = kernel.shape
-        if (cc2, e, kb, i4) != (cc, cb // 4, 16, 4):
-            raise ValueError(f"kernel: shape {tuple(kernel.shape)} does not match data {tuple(data.shape)}; "
-                             f"expected (K/16, {cc}, KH, KW, {cb // 4}, 16, 4)")
+        _check_prepared(kernel, data, torch.int8)
+    p = _plan(data, kernel, stride, padding, dilation)
+    bias_ptr = None
     if bias is not None:
-        if bias.dtype != torch.int32 or bias.numel() != ko * 16 or bias.device != data.device:
-            raise ValueError(f"bias: expected {ko * 16} int32 values on {data.device}")
-        bias = bias.contiguous()
+        bias = _check_bias(bias, p.ko * 16, data)
+        bias_ptr = bias.data_ptr()
     scale = int(scale)
     if not -2 ** 31 <= scale < 2 ** 31:
         raise ValueError("scale: must fit int32")
-    sh, sw = _pair(stride, "stride")
-    dh, dw = _pair(dilation, "dilation")
-    pt, pl, pb, pr = _pad4(padding)
-    d = ConvDesc(n, cc * cb, h, w, ko * 16, kh, kw, sh, sw, pt, pl, pb, pr, dh, dw, cb)
     L = _lib.load()
-    oh, ow = ctypes.c_int32(), ctypes.c_int32()
-    check(L.unit_conv_out_hw(ctypes.byref(d), ctypes.byref(oh), ctypes.byref(ow)))
     if planar:
-        oc = ko * 16 if out_channels is None else int(out_channels)
-        if not ko * 16 - 16 < oc <= ko * 16:
-            raise ValueError(f"out_channels: {oc} does not round up to K = {ko * 16}")
-        out = torch.empty((n, oc, oh.value, ow.value), dtype=torch.int32, device=data.device)
-        check(L.unit_conv2d_nchwc_s8s8s32_fused_prepared_nchw(
-            ctypes.byref(d), data.data_ptr(), kernel.buf.data_ptr(), bias.data_ptr() if bias is not None else None,
-            scale, out.data_ptr(), oc, _stream()))
+        oc = p.ko * 16 if out_channels is None else int(out_channels)
+        if not p.ko * 16 - 16 < oc <= p.ko * 16:
+            raise ValueError(f"out_channels: {oc} does not round up to K = {p.ko * 16}")
+        out = data.new_empty((p.n, oc, p.oh, p.ow), dtype=torch.int32)
+        check(L.unit_conv2d_nchwc_s8s8s32_fused_prepared_nchw(p.ref, data.data_ptr(), kernel.buf.data_ptr(), bias_ptr, scale,
+                                                              out.data_ptr(), oc, _stream()))
         return out
-    out = torch.empty((n, ko, oh.value, ow.value, 16), dtype=torch.int32, device=data.device)
-    fn = L.unit_conv2d_nchwc_s8s8s32_fused_prepared if prepared else L.unit_conv2d_nchwc_s8s8s32_fused
-    check(fn(ctypes.byref(d), data.data_ptr(), kernel.buf.data_ptr() if prepared else kernel.data_ptr(),
-             bias.data_ptr() if bias is not None else None, scale, out.data_ptr(), _stream()))
+    out = data.new_empty(p.blocked, dtype=torch.int32)
+    if prepared:
+        check(L.unit_conv2d_nchwc_s8s8s32_fused_prepared(p.ref, data.data_ptr(), kernel.buf.data_ptr(), bias_ptr, scale,
+                                                         out.data_ptr(), _stream()))
+    else:
+        check(L.unit_conv2d_nchwc_s8s8s32_fused(p.ref, data.data_ptr(), kernel.data_ptr(), bias_ptr, scale, out.data_ptr(),
+                                                _stream()))
     return out
 
 
@@ -284,31 +326,37 @@ def conv2d_NCHWc_int8_requant(data, kernel, bias, scale, shift, stride, padding,
     (apps/cpu/relay/result.log:15-24); this is the integer requantisation that follows it in a
     quantised network.
     """
-    import ctypes
     data = _dev(data, "data", torch.uint8, 5)
     if not isinstance(kernel, PreparedConvWeight):
         kernel = prepare_conv2d_weight(kernel)
-    n, cc, h, w, cb = data.shape
-    ko, _, kh, kw = _prepared_dims(kernel, data, torch.int8)
+    _check_prepared(kernel, data, torch.int8)
+    p = _plan(data, kernel, stride, padding, dilation)
+    bias_ptr = None
     if bias is not None:
-        if bias.dtype != torch.int32 or bias.numel() != ko * 16 or bias.device != data.device:
-            raise ValueError(f"bias: expected {ko * 16} int32 values on {data.device}")
-        bias = bias.contiguous()
+        bias = _check_bias(bias, p.ko * 16, data)
+        bias_ptr = bias.data_ptr()
     scale, shift = int(scale), int(shift)
     if not -2 ** 31 <= scale < 2 ** 31:
         raise ValueError("scale: must fit int32")
-    sh, sw = _pair(stride, "stride")
-    dh, dw = _pair(dilation, "dilation")
-    pt, pl, pb, pr = _pad4(padding)
-    d = ConvDesc(n, cc * cb, h, w, ko * 16, kh, kw, sh, sw, pt, pl, pb, pr, dh, dw, cb)
-    L = _lib.load()
-    oh, ow = ctypes.c_int32(), ctypes.c_int32()
-    check(L.unit_conv_out_hw(ctypes.byref(d), ctypes.byref(oh), ctypes.byref(ow)))
-    out = torch.empty((n, ko, oh.value, ow.value, 16), dtype=torch.uint8, device=data.device)
-    check(L.unit_conv2d_nchwc_u8s8u8_requant_prepared(ctypes.byref(d), data.data_ptr(), kernel.buf.data_ptr(),
-                                                      bias.data_ptr() if bias is not None else None, scale, shift,
-                                                      out.data_ptr(), _stream()))
+    out = data.new_empty(p.blocked)
+    check(_lib.load().unit_conv2d_nchwc_u8s8u8_requant_prepared(p.ref, data.data_ptr(), kernel.buf.data_ptr(), bias_ptr, scale,
+                                                                shift, out.data_ptr(), _stream()))
     return out
+
+
+@lru_cache(maxsize=1024, typed=True)
+def _plan_3d(dshape, kshape, stride):
+    n, cc, dd, h, w, cb = dshape
+    ko, cc2, kd, kh, kw, e, kb, i4 = kshape
+    if cb not in (4, 16) or (cb == 4 and (cc * cb) % 16 == 0):
+        raise ValueError(f"data: channel block must be 16, or 4 when C is not a multiple of 16 (got {cb}, C = {cc * cb})")
+    if (cc2, e, kb, i4) != (cc, cb // 4, 16, 4):
+        raise ValueError(f"kernel: shape {tuple(kshape)} does not match data {tuple(dshape)}; "
+                         f"expected (K/16, {cc}, KD, KH, KW, {cb // 4}, 16, 4)")
+    if stride <= 0 or kd > dd or kh > h or kw > w:
+        raise ValueError("stride must be positive and the kernel window must fit the input")
+    d = _lib.Conv3dDesc(n, cc * cb, dd, h, w, ko * 16, kd, kh, kw, stride)
+    return d, ctypes.byref(d), (n, ko, (dd - kd) // stride + 1, (h - kh) // stride + 1, (w - kw) // stride + 1, 16)
 
 
 def conv3d_NCDHWc_int8(data, kernel, stride=1):
@@ -319,24 +367,11 @@ def conv3d_NCDHWc_int8(data, kernel, stride=1):
     kernel int8  (K/16, C/cb, KD, KH, KW, cb/4, 16, 4)
     returns int32 (N, K/16, OD, OH, OW, 16)
     """
-    import ctypes
     data = _dev(data, "data", torch.int8, 6)
     kernel = _dev(kernel, "kernel", torch.int8, 8)
-    n, cc, dd, h, w, cb = data.shape
-    ko, cc2, kd, kh, kw, e, kb, i4 = kernel.shape
-    if cb not in (4, 16) or (cb == 4 and (cc * cb) % 16 == 0):
-        raise ValueError(f"data: channel block must be 16, or 4 when C is not a multiple of 16 (got {cb}, C = {cc * cb})")
-    if (cc2, e, kb, i4) != (cc, cb // 4, 16, 4):
-        raise ValueError(f"kernel: shape {tuple(kernel.shape)} does not match data {tuple(data.shape)}; "
-                         f"expected (K/16, {cc}, KD, KH, KW, {cb // 4}, 16, 4)")
-    stride = int(stride)
-    if stride <= 0 or kd > dd or kh > h or kw > w:
-        raise ValueError("stride must be positive and the kernel window must fit the input")
-    d = _lib.Conv3dDesc(n, cc * cb, dd, h, w, ko * 16, kd, kh, kw, stride)
-    od, oh, ow = (dd - kd) // stride + 1, (h - kh) // stride + 1, (w - kw) // stride + 1
-    out = torch.empty((n, ko, od, oh, ow, 16), dtype=torch.int32, device=data.device)
-    check(_lib.load().unit_conv3d_ncdhwc_s8s8s32(ctypes.byref(d), data.data_ptr(), kernel.data_ptr(), out.data_ptr(),
-                                                  _stream()))
+    _, ref, shape = _plan_3d(data.shape, kernel.shape, int(stride))
+    out = data.new_empty(shape, dtype=torch.int32)
+    check(_lib.load().unit_conv3d_ncdhwc_s8s8s32(ref, data.data_ptr(), kernel.data_ptr(), out.data_ptr(), _stream()))
     return out
 
 
@@ -354,13 +389,13 @@ def dense_dotprod(data, weight, bias=None, out_dtype="int32"):
         if (t, four) != (128, 4) or kg * 4 != k:
             raise ValueError(f"weight: expected (N/128, {k // 4}, 128, 4), got {tuple(weight.shape)}")
         n = nb * 128
-        out = torch.empty((m, n), dtype=torch.int32, device=data.device)
+        out = data.new_empty((m, n), dtype=torch.int32)
         check(L.unit_dense_dotprod_u8s8s32(data.data_ptr(), weight.data_ptr(), out.data_ptr(), m, n, k, _stream()))
     else:
         n, k2 = weight.shape
         if k2 != k:
             raise ValueError(f"weight: expected (N, {k}), got {tuple(weight.shape)}")
-        out = torch.empty((m, n), dtype=torch.int32, device=data.device)
+        out = data.new_empty((m, n), dtype=torch.int32)
         check(L.unit_dense_u8s8s32(data.data_ptr(), weight.data_ptr(), out.data_ptr(), m, n, k, _stream()))
     if bias is not None:
         out += _dev(bias, "bias", torch.int32)
@@ -395,7 +430,7 @@ def dense(data, weight, out_dtype="int32"):
         n, k2 = weight.shape
         if k2 != k:
             raise ValueError(f"weight: expected (N, {k}), got {weight.shape}")
-        out = torch.empty((m, n), dtype=torch.int32, device=data.device)
+        out = data.new_empty((m, n), dtype=torch.int32)
         check(_lib.load().unit_dense_u8s8s32_prepared(data.data_ptr(), weight.w.data_ptr(), weight.wsum.data_ptr(),
                                                       out.data_ptr(), m, n, k, _stream()))
         return out
@@ -449,7 +484,7 @@ def gemm_fp16(a, b, out_dtype="float32", workspace=None):
     if isinstance(b, PreparedGemmB):
         if b.K != k or b.bt.device != a.device:
             raise ValueError(f"b: {b!r} does not match a {tuple(a.shape)} on {a.device}")
-        out = torch.empty((m, b.N), dtype=torch.float16 if half else torch.float32, device=a.device)
+        out = a.new_empty((m, b.N), dtype=torch.float16 if half else torch.float32)
         check(_lib.load().unit_gemm_f16_prepared(a.data_ptr(), b.bt.data_ptr(), out.data_ptr(), m, b.N, k, int(half),
                                                  _stream()))
         return out
@@ -457,7 +492,7 @@ def gemm_fp16(a, b, out_dtype="float32", workspace=None):
     k2, n = b.shape
     if k2 != k:
         raise ValueError(f"b: expected ({k}, N), got {tuple(b.shape)}")
-    out = torch.empty((m, n), dtype=torch.float16 if half else torch.float32, device=a.device)
+    out = a.new_empty((m, n), dtype=torch.float16 if half else torch.float32)
     if workspace is not None and workspace is not False:
         need = gemm_fp16_workspace_bytes(m, n, k)
         if workspace is True:
@@ -483,53 +518,43 @@ def conv2d_NCHW16c_OHWI16o(a, b, stride_h, stride_w, out_type="float32"):
     Either a (N, C, H, W) + b (K, C, KH, KW), packed here exactly as the reference operator packs
     them in-op, or a (N, C/16, H, W, 16) + b (K/16, C/16, KH, KW, 16 in, 16 out).
     Returns float32 (N, K/16, OH, OW, 16)."""
-    import ctypes
     if out_type != "float32":
         raise ValueError(f"out_type: only 'float32' is supported, got {out_type!r}")
     a = _dev(a, "a", torch.float16, (4, 5))
+    L = _lib.load()
     if isinstance(b, PreparedConvWeight):
         if a.dim() != 5:
             raise ValueError("a: prepared weights take the blocked (N, C/16, H, W, 16) operand")
-        ko, cc, kh, kw = _prepared_dims(b, a, torch.float16)
-        n, _, h, w, _ = a.shape
-        d = ConvDesc(n, cc * 16, h, w, ko * 16, kh, kw, int(stride_h), int(stride_w), 0, 0, 0, 0, 1, 1, 16)
-        L = _lib.load()
-        oh, ow = ctypes.c_int32(), ctypes.c_int32()
-        check(L.unit_conv_out_hw(ctypes.byref(d), ctypes.byref(oh), ctypes.byref(ow)))
-        out = torch.empty((n, ko, oh.value, ow.value, 16), dtype=torch.float32, device=a.device)
-        check(L.unit_conv2d_nchw16c_f16f32_prepared(ctypes.byref(d), a.data_ptr(), b.buf.data_ptr(), out.data_ptr(),
-                                                    _stream()))
+        _check_prepared(b, a, torch.float16)
+        p = _plan_f16(a.shape, b.key, stride_h, stride_w)
+        out = a.new_empty(p.blocked, dtype=torch.float32)
+        check(L.unit_conv2d_nchw16c_f16f32_prepared(p.ref, a.data_ptr(), b.buf.data_ptr(), out.data_ptr(), _stream()))
         return out
     b = _dev(b, "b", torch.float16, (4, 6))
     if a.dim() == 4 and b.dim() == 4:
-        if a.shape[1] % 16 or b.shape[0] % 16 or b.shape[1] != a.shape[1]:
-            raise ValueError("a, b: channel counts must match and be multiples of 16")
-        n, c, h, w = a.shape
-        k, _, kh, kw = b.shape
-        d = ConvDesc(n, c, h, w, k, kh, kw, int(stride_h), int(stride_w), 0, 0, 0, 0, 1, 1, 16)
-        L = _lib.load()
-        oh, ow, need = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_size_t()
-        check(L.unit_conv_out_hw(ctypes.byref(d), ctypes.byref(oh), ctypes.byref(ow)))
-        check(L.unit_conv2d_nchw_f16f32_ws_bytes(ctypes.byref(d), ctypes.byref(need)))
-        ws = torch.empty((need.value,), dtype=torch.uint8, device=a.device)
-        out = torch.empty((n, k // 16, oh.value, ow.value, 16), dtype=torch.float32, device=a.device)
-        check(L.unit_conv2d_nchw_f16f32(ctypes.byref(d), a.data_ptr(), b.data_ptr(), out.data_ptr(), ws.data_ptr(),
-                                        need.value, _stream()))
+        p, need = _plan_f16_plain(a.shape, b.shape, stride_h, stride_w)
+        ws = a.new_empty((need,), dtype=torch.uint8)
+        out = a.new_empty(p.blocked, dtype=torch.float32)
+        check(L.unit_conv2d_nchw_f16f32(p.ref, a.data_ptr(), b.data_ptr(), out.data_ptr(), ws.data_ptr(), need, _stream()))
         return out
     if not (a.dim() == 5 and b.dim() == 6):
         raise ValueError("a, b: expected 4-D + 4-D or 5-D + 6-D operands")
-    n, cc, h, w, cb = a.shape
-    ko, ib, kh, kw, ic, ob = b.shape
-    if cb != 16 or ic != 16 or ob != 16 or ib != cc:
-        raise ValueError(f"a {tuple(a.shape)} / b {tuple(b.shape)}: expected (N, C/16, H, W, 16) and "
-                         f"(K/16, C/16, KH, KW, 16, 16)")
-    d = ConvDesc(n, cc * 16, h, w, ko * 16, kh, kw, int(stride_h), int(stride_w), 0, 0, 0, 0, 1, 1, 16)
-    L = _lib.load()
-    oh, ow = ctypes.c_int32(), ctypes.c_int32()
-    check(L.unit_conv_out_hw(ctypes.byref(d), ctypes.byref(oh), ctypes.byref(ow)))
-    out = torch.empty((n, ko, oh.value, ow.value, 16), dtype=torch.float32, device=a.device)
-    check(L.unit_conv2d_nchw16c_f16f32(ctypes.byref(d), a.data_ptr(), b.data_ptr(), out.data_ptr(), _stream()))
+    p = _plan_f16(a.shape, b.shape, stride_h, stride_w)
+    out = a.new_empty(p.blocked, dtype=torch.float32)
+    check(L.unit_conv2d_nchw16c_f16f32(p.ref, a.data_ptr(), b.data_ptr(), out.data_ptr(), _stream()))
     return out
+
+
+@lru_cache(maxsize=1024, typed=True)
+def _plan_f16_plain(ashape, bshape, stride_h, stride_w):
+    n, c, h, w = ashape
+    k, c2, kh, kw = bshape
+    if c % 16 or k % 16 or c2 != c:
+        raise ValueError("a, b: channel counts must match and be multiples of 16")
+    p = _ConvPlan(n, c, h, w, k, kh, kw, (int(stride_h), int(stride_w)), 0, 1, 16)
+    need = ctypes.c_size_t()
+    check(_lib.load().unit_conv2d_nchw_f16f32_ws_bytes(p.ref, ctypes.byref(need)))
+    return p, need.value
 
 
 # ------------------------------------------------------------------------------- layouts
