@@ -294,6 +294,20 @@ int unit_conv2d_nchwc_u8s8u8_requant_prepared(const unit_conv_desc *d, const voi
                                               const int32_t *bias, int32_t scale, int32_t shift, void *out,
                                               unit_stream_t stream);
 
+/* A network's requantising convolutions one after the other (unit_amd/chain.py): layer i is
+ * unit_conv2d_nchwc_u8s8u8_requant_prepared(&desc, data, prepared, bias, scale, shift, out), with data == NULL standing
+ * for x; the name of the kernel it ran goes to `variant` (96 bytes) when that is not NULL.  Stops at the first error. */
+typedef struct unit_chain_layer {
+  unit_conv_desc desc;
+  const void *data;
+  const void *prepared;
+  const int32_t *bias;
+  void *out;
+  char *variant;
+  int32_t scale, shift;
+} unit_chain_layer;
+int unit_conv_chain_u8(const unit_chain_layer *layers, int32_t count, const void *x, unit_stream_t stream);
+
 /* ------------------------------------------------------------------ diagnostics */
 
 /* One v_mfma_i32_32x32x32_i8 / v_mfma_f32_32x32x16_f16 on a single wavefront, operands and

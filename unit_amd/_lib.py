@@ -46,6 +46,7 @@ SYMBOLS = (
     "unit_conv2d_nchwc_s8s8s32_fused_prepared_nchw",
     "unit_conv2d_nchw16c_f16f32_prepared",
     "unit_conv2d_nchwc_u8s8u8_requant_prepared",
+    "unit_conv_chain_u8",
     "unit_mfma_tile_i8",
     "unit_mfma_tile_f16",
     "unit_mfma_peak",
@@ -61,6 +62,12 @@ class ConvDesc(ctypes.Structure):
 class Conv3dDesc(ctypes.Structure):
     """struct unit_conv3d_desc"""
     _fields_ = [(k, ctypes.c_int32) for k in ("N", "C", "D", "H", "W", "K", "KD", "KH", "KW", "stride")]
+
+
+class ChainLayerDesc(ctypes.Structure):
+    """struct unit_chain_layer"""
+    _fields_ = [("desc", ConvDesc)] + [(k, ctypes.c_void_p) for k in ("data", "prepared", "bias", "out", "variant")] + [
+        (k, ctypes.c_int32) for k in ("scale", "shift")]
 
 
 class UnitError(RuntimeError):
@@ -116,6 +123,7 @@ def load():
     L.unit_conv2d_nchwc_s8s8s32_fused_prepared_nchw.argtypes = [dp, vp, vp, vp, i32, vp, i32, vp]
     L.unit_conv2d_nchw16c_f16f32_prepared.argtypes = [dp, vp, vp, vp, vp]
     L.unit_conv2d_nchwc_u8s8u8_requant_prepared.argtypes = [dp, vp, vp, vp, i32, i32, vp, vp]
+    L.unit_conv_chain_u8.argtypes = [ctypes.POINTER(ChainLayerDesc), i32, vp, vp]
     L.unit_mfma_tile_i8.argtypes = [vp, vp, vp, vp]
     L.unit_mfma_tile_f16.argtypes = [vp, vp, vp, vp]
     L.unit_mfma_peak.argtypes = [i32, i32, i32, vp, vp]

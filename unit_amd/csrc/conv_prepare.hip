@@ -254,6 +254,19 @@ extern "C" int unit_conv2d_nchwc_u8s8u8_requant_prepared(const unit_conv_desc *d
                           static_cast<hipStream_t>(stream));
 }
 
+extern "C" int unit_conv_chain_u8(const unit_chain_layer *layers, int32_t count, const void *x, unit_stream_t stream) {
+  using namespace unit;
+  if (!layers || !x || count < 0) return fail(UNIT_E_ARG, "unit_conv_chain_u8: null pointer or negative count");
+  for (int32_t i = 0; i < count; ++i) {
+    const unit_chain_layer &l = layers[i];
+    if (int rc = unit_conv2d_nchwc_u8s8u8_requant_prepared(&l.desc, l.data ? l.data : x, l.prepared, l.bias, l.scale, l.shift,
+                                                           l.out, stream))
+      return rc;
+    if (l.variant) snprintf(l.variant, 96, "%s", unit_last_variant());
+  }
+  return UNIT_OK;
+}
+
 namespace unit {
 namespace {
 
