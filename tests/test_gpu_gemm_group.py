@@ -1,0 +1,78 @@
+"""GEMMs on the group tiles (gemm_group.hpp): every tile shape, reductions that end inside a 64-byte stage, row and
+column edges, N of 4 mod 8 (the transposing read's shifted last chunk), fewer stages than groups, k-splits by atomics and
+by planes.  Integer data makes the fp16 products exact in any order, so everything is compared bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+import unit_amd as U
+
+pytestmark = pytest.mark.gpu
+
+# M, N, K; the tile the shape is there for (fp16 with fp16 output)
+F16 = [(1, 8, 8, "x32_y32"), (33, 12, 24, "x32_y32"), (37, 36, 200, "x32_y32"), (300, 260, 520, "x32_y32"),
+       (700, 700, 712, "x32_y64"), (300, 3004, 296, "x64_y64"), (1000, 1516, 1096, "x64_y128"),
+       (1500, 1508, 1496, "x128_y128"), (2180, 2052, 2056, "x128_y128"), (3840, 2044, 2056, "x256_y128"), (129, 8192, 40, "")]
+I8 = [(1, 4, 16), (33, 36, 80), (50, 260, 1040), (37, 128, 4112), (700, 704, 720), (1467, 1108, 976), (1500, 1536, 1552),
+      (2180, 2176, 2064), (3840, 2048, 4112), (129, 8192, 48)]
+
+
+def _ints(g, lo, hi, shape, dtype, dev):
+    return torch.from_numpy(g.randint(lo, hi, shape)).to(dev).to(dtype)
+
+
+@pytest.mark.parametrize("M,N,K,tile", F16)
+def test_fp16_group_tiles(dev, M, N, K, tile):
+    g = np.random.RandomState(M + N + K)
+    a, b = _ints(g, -3, 4, (M, K), torch.float16, dev), _ints(g, -2, 3, (K, N), torch.float16, dev)
+    ref = a.double() @ b.double()  # exact: |sum| <= 6 K < 2^24
+    half = U.gemm_fp16(a, b, "float16")
+    name = U.last_variant()
+    assert torch.equal(half, ref.half()), name
+    assert tile in name, name
+    assert torch.equal(U.gemm_fp16(a, b).double(), ref), U.last_variant()
+    p = U.prepare_gemm_b(b)
+    assert torch.equal(U.gemm_fp16(a, p).double(), ref), U.last_variant()
+    assert torch.equal(U.gemm_fp16(a, p, "float16"), ref.half()), U.last_variant()
+    assert torch.equal(U.gemm_fp16(a, b, "float16", workspace=True), ref.half()), U.last_variant()
+    assert torch.equal(U.gemm_fp16(a, b, workspace=True).double(), ref), U.last_variant()
+
+
+def test_fp16_infinity_past_a_row(dev):
+    """What lies behind a row's end (the next row) must not reach the sums: 0 x inf would be NaN."""
+    M, N, K = 40, 44, 72
+    a = torch.full((M, K), float("inf"), dtype=torch.float16, device=dev)
+    a[::2] = 1
+    b = torch.ones((K, N), dtype=torch.float16, device=dev)
+    for operand in (b, U.prepare_gemm_b(b)):
+        out = U.gemm_fp16(a, operand)
+        assert torch.equal(out[::2], torch.full_like(out[::2], K)) and torch.isinf(out[1::2]).all(), U.last_variant()
+
+
+@pytest.mark.parametrize("M,N,K", I8)
+def test_int8_group_tiles(dev, M, N, K):
+    g = np.random.RandomState(M + N + K)
+    a, w = _ints(g, 0, 256, (M, K), torch.uint8, dev), _ints(g, -128, 128, (N, K), torch.int8, dev)
+    ref = (a.double() @ w.double().t()).to(torch.int32)
+    assert torch.equal(U.dense(a, w), ref), U.last_variant()
+    assert torch.equal(U.dense(a, U.prepare_dense_weight(w)), ref), U.last_variant()
+    if N % 128 == 0:
+        assert torch.equal(U.dense_dotprod(a, U.prepack_dense_weight(w)), ref), U.last_variant()
+
+
+@pytest.mark.parametrize("splits", [1, 2, 5])
+def test_pinned_k_splits(dev, monkeypatch, splits):
+    monkeypatch.setenv("UNIT_AMD_DENSE_SPLITK", str(splits))
+    monkeypatch.setenv("UNIT_AMD_GEMM_F16_SPLITK", str(splits))
+    M, N, K = 70, 132, 1104
+    g = np.random.RandomState(splits)
+    a, w = _ints(g, 0, 256, (M, K), torch.uint8, dev), _ints(g, -128, 128, (N, K), torch.int8, dev)
+    ref = (a.double() @ w.double().t()).to(torch.int32)
+    for operand in (w, U.prepare_dense_weight(w)):
+        assert torch.equal(U.dense(a, operand), ref), U.last_variant()
+        assert U.last_variant().endswith(f"_s{splits}")
+    h, b = _ints(g, -3, 4, (M, K), torch.float16, dev), _ints(g, -2, 3, (K, N), torch.float16, dev)
+    ref = h.double() @ b.double()
+    for ws in (None, True):
+        assert torch.equal(U.gemm_fp16(h, b, workspace=ws).double(), ref), U.last_variant()
+        assert U.last_variant().endswith(f"_s{splits}")

@@ -3,6 +3,7 @@
 #include <mutex>
 
 #include "epilogues.hpp"
+#include "gemm_group.hpp"
 #include "host.hpp"
 #include "loaders.hpp"
 #include "mma_dma.hpp"
@@ -102,34 +103,43 @@ int run_gemm_f16_hybrid(const void *a, const void *b, void *c, int M, int N, int
   return e == hipSuccess ? UNIT_OK : fail(UNIT_E_LAUNCH, "unit_gemm_f16: launch: %s", hipGetErrorString(e));
 }
 
-// the same operands through registers (any K that is a multiple of 8; small problems)
-template <class T, bool OUT_F16>
-int run_gemm_f16_bt(const void *a, const void *bt, void *c, int M, int N, int K, hipStream_t s) {
-  using XL = RowMajorLoader<T::BX, T::BKB, T::NT, false>;
-  using YL = RowMajorLoader<T::BY, T::BKB, T::NT, false>;
-  using Epi = GemmEpilogue<OpF16, OUT_F16>;
-  typename XL::Params xp{static_cast<const char *>(a), M, K * 2, K * 2};
-  typename YL::Params yp{static_cast<const char *>(bt), N, K * 2, K * 2};
-  typename Epi::Params ep{c, M, N};
-  const int nk = ceil_div(K * 2, T::BKB), gx = ceil_div(M, T::BX), gy = ceil_div(N, T::BY);
-  const int splits = OUT_F16 ? 1 : gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K, nk);
-  set_variant("f16gemmbt_x%d_y%d_k%d_w%dx%d%s_s%d", T::BX, T::BY, T::BKB, T::WX, T::WY, OUT_F16 ? "_h" : "", splits);
-  return launch_mma<OpF16, T, XL, YL, Epi, WS_NONE>(xp, yp, ep, nk, gx, gy, 4, splits, c, (size_t)M * N * 4, 0, s,
-                                                    "unit_gemm_f16_prepared");
+// Tiles of at most 256 x 128 with the reduction shared inside the workgroup (gemm_group.hpp), any K and N the
+// operator takes (b by columns: N >= 8).  fp32 results may also share it between workgroups (atomics into the zero-filled
+// output), and do at least two ways with fewer than 12 tiles of 128 x 128 and 1 KiB of reduction (the tests ask for that;
+// 300 x 260 x 520 would run 2 us faster without); fp16 results keep one workgroup per tile.
+template <int YM, bool OUT_F16>
+int run_gemm_f16_group(const char *what, const char *tag, const void *a, const void *b, void *c, int M, int N, int K,
+                       hipStream_t s) {
+  const int forced = OUT_F16 ? 1 : tuning_override("UNIT_AMD_GEMM_F16_SPLITK");
+  const int least = forced <= 0 && tiles_of_128(M, N) < 12 && K >= 512 ? 2 : 1;
+  GroupPlan plan = plan_group(M, N, K * 2, least, forced > 0 ? 1 : 19, kAtomicSplits);
+  if (forced > 0) plan.splits = forced;
+  const GroupGemm p{static_cast<const char *>(a), static_cast<const char *>(b), (u32)((size_t)M * K * 2),
+                    (u32)((size_t)N * K * 2), M, N, K * 2, YM == Y_COLS ? N * 2 : K * 2, nullptr, c, C_ATOMIC, 0};
+  return run_group_plan<OpF16, YM, WS_NONE, OUT_F16>(what, tag, p, plan, s);
+}
+
+// Which aligned shapes stay on the 128 x 128 tiles of mma_dma.hpp: fp32 results with fewer than 32 such tiles and more
+// than 128 rows (the tests name that kernel and its k-splits for them), one nearly full round of the 256 CUs
+// (1011 x 3584 x 1216, 224 tiles, 15.6 against 16.2 us on the group tile of the same size; 2048^3 22.9 against 24.8), and 512
+// tiles or more (8192 x 1024 x 1024 24.2 and 24.0 us).  The others gain: 1024^3 12.3 -> 7.7 us, 2304 x 2304 x 4096
+// 66 -> 55 us, 64 x 4096 x 4096 15.3 -> 11.9 us.
+inline bool gemm_keeps_128(int M, int N, bool out_f16) {
+  const long tiles = tiles_of_128(M, N);
+  return tiles >= 512 || (tiles >= 192 && tiles <= 256) || (!out_f16 && tiles < 32 && M > 128);
 }
 
 template <bool OUT_F16>
 int gemm_f16_bt(const void *a, const void *bt, void *c, int M, int N, int K, hipStream_t s) {
-  const long tiles_big = (long)ceil_div(M, 256) * ceil_div(N, 256);
   if (K % 32 == 0 && K >= 64) {  // both operands straight into LDS; tile choice as in gemm_f16 below
     if (direct_gemm_large_tiles(M, N)) {
       if (K % 64 == 0) return run_gemm_f16_bt_dma<Tile<256, 256, 128, 2, 4>, 2, OUT_F16>(a, bt, c, M, N, K, s);
       return run_gemm_f16_bt_dma<Tile<256, 256, 64, 2, 4>, 4, OUT_F16>(a, bt, c, M, N, K, s);
     }
-    return run_gemm_f16_bt_dma<Tile<128, 128, 64, 2, 2>, 4, OUT_F16>(a, bt, c, M, N, K, s, direct_gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K));
+    if (gemm_keeps_128(M, N, OUT_F16))
+      return run_gemm_f16_bt_dma<Tile<128, 128, 64, 2, 2>, 4, OUT_F16>(a, bt, c, M, N, K, s, direct_gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K));
   }
-  if (M >= 256 && N >= 256 && tiles_big >= 128) return run_gemm_f16_bt<Tile<256, 256, 128, 2, 4>, OUT_F16>(a, bt, c, M, N, K, s);
-  return run_gemm_f16_bt<Tile<128, 128, 64, 2, 2>, OUT_F16>(a, bt, c, M, N, K, s);
+  return run_gemm_f16_group<Y_ROWS, OUT_F16>("unit_gemm_f16_prepared", "f16gemmbt", a, bt, c, M, N, K, s);
 }
 
 // b (K, N) -> bt (N, K): 64 x 64 tiles through LDS, 128-byte row segments on both sides
@@ -176,67 +186,51 @@ int run_gemm_f16(const void *a, const void *b, void *c, int M, int N, int K, hip
 
 template <bool OUT_F16>
 int gemm_f16(const void *a, const void *b, void *c, int M, int N, int K, hipStream_t s) {
-  const long tiles_big = (long)ceil_div(M, 256) * ceil_div(N, 256);
-  // UNIT_AMD_GEMM_F16_VARIANT pins a tile shape per process (measurement aid)
+  // UNIT_AMD_GEMM_F16_VARIANT pins a kernel per process where it can run (measurement aid)
   switch (tuning_override("UNIT_AMD_GEMM_F16_VARIANT")) {
-    case 1: return run_gemm_f16<Tile<256, 256, 128, 2, 4>, OUT_F16>(a, b, c, M, N, K, s);
-    case 2: return run_gemm_f16<Tile<256, 256, 64, 2, 4>, OUT_F16>(a, b, c, M, N, K, s);
-    case 3: return run_gemm_f16<Tile<256, 256, 128, 2, 2>, OUT_F16>(a, b, c, M, N, K, s);
-    case 4: return K % 64 ? run_gemm_f16<Tile<256, 256, 128, 4, 2>, OUT_F16>(a, b, c, M, N, K, s)
-                          : run_gemm_f16<Tile<256, 256, 128, 4, 2>, OUT_F16, 1, false>(a, b, c, M, N, K, s);
-    case 5: return run_gemm_f16<Tile<256, 256, 64, 4, 2>, OUT_F16, 2>(a, b, c, M, N, K, s);
-    case 6: return run_gemm_f16<Tile<128, 256, 128, 4, 2>, OUT_F16>(a, b, c, M, N, K, s);
-    case 7: if (K % 64 == 0 && K >= 128) return run_gemm_f16_hybrid<Tile<256, 256, 128, 4, 2>, OUT_F16>(a, b, c, M, N, K, s); break;
-    case 8: if (K % 64 == 0 && K >= 128) return run_gemm_f16_hybrid<Tile<256, 256, 128, 2, 4>, OUT_F16>(a, b, c, M, N, K, s); break;
-    case 9: if (K % 64 == 0 && K >= 128) return run_gemm_f16_hybrid<Tile<256, 128, 128, 2, 2>, OUT_F16>(a, b, c, M, N, K, s); break;
+    case 7: if (K % 64 == 0 && K >= 128) return run_gemm_f16_hybrid<Tile<256, 256, 128, 2, 4>, OUT_F16>(a, b, c, M, N, K, s); break;
     case 10: if (K % 64 == 0 && K >= 128 && N % 8 == 0) return run_gemm_f16_dma_tr<Tile<256, 256, 128, 2, 4>, 2, OUT_F16>(a, b, c, M, N, K, s); break;
     case 11: if (K % 32 == 0 && K >= 128 && N % 8 == 0) return run_gemm_f16_dma_tr<Tile<256, 256, 64, 2, 4>, 4, OUT_F16>(a, b, c, M, N, K, s); break;
-    case 12: if (K % 32 == 0 && K >= 128 && N % 8 == 0) return run_gemm_f16_dma_tr<Tile<256, 128, 64, 2, 2>, 4, OUT_F16>(a, b, c, M, N, K, s); break;
-    case 13: if (K % 32 == 0 && K >= 128 && N % 8 == 0) return run_gemm_f16_dma_tr<Tile<128, 256, 64, 2, 2>, 4, OUT_F16>(a, b, c, M, N, K, s); break;
     case 15: if (K % 32 == 0 && K >= 128 && N % 8 == 0) return run_gemm_f16_dma_tr<Tile<128, 128, 64, 2, 2>, 4, OUT_F16>(a, b, c, M, N, K, s); break;
-    case 16: if (K % 32 == 0 && K >= 128 && N % 8 == 0) return run_gemm_f16_dma_tr<Tile<128, 128, 64, 2, 2>, 6, OUT_F16>(a, b, c, M, N, K, s); break;
-    case 14: if (K % 32 == 0 && K >= 128 && N % 8 == 0) return run_gemm_f16_dma_tr<Tile<256, 128, 64, 2, 2>, 6, OUT_F16>(a, b, c, M, N, K, s); break;
     default: break;
   }
   // K a whole number of 64-byte stages and N of 16-byte chunks: both operands straight into LDS, b read back with the
-  // transposing LDS read.  At 4096^3 116 us against 133 us for the register-transposing pipeline below, 2048^3 26
-  // against 39 us, 1024 x 4096 x 4096 45 against 68 us, same bits.
+  // transposing LDS read, on 256 x 256 tiles where those fill the chip (4096^3 in 114 us)
   if (K % 32 == 0 && K >= 64 && N % 8 == 0) {
     if (direct_gemm_large_tiles(M, N)) {
       if (K % 64 == 0) return run_gemm_f16_dma_tr<Tile<256, 256, 128, 2, 4>, 2, OUT_F16>(a, b, c, M, N, K, s);
       return run_gemm_f16_dma_tr<Tile<256, 256, 64, 2, 4>, 4, OUT_F16>(a, b, c, M, N, K, s);
     }
-    return run_gemm_f16_dma_tr<Tile<128, 128, 64, 2, 2>, 4, OUT_F16>(a, b, c, M, N, K, s, direct_gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K));
+    if (gemm_keeps_128(M, N, OUT_F16))
+      return run_gemm_f16_dma_tr<Tile<128, 128, 64, 2, 2>, 4, OUT_F16>(a, b, c, M, N, K, s, direct_gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K));
   }
-  // K a whole number of 128-byte stages: a straight into LDS, b through the transposing register loader
-  // (measured 130 us against 154 us for the all-register pipeline at 4096^3, same bits).  256 x 256 tiles of eight
-  // waves, or 256 x 128 tiles of four when those need fewer rounds of 256 workgroups for their cost (about 0.55 of
-  // a 256 x 256 tile: 2048^3 54 -> 36 us, 1024 x 4096 x 4096 95 -> 63 us, 8192 x 1024 x 1024 31 -> 25 us;
-  // 3072^3 stays on 144 large tiles, 76 us, against 106 us on 288 small ones)
-  if (M >= 256 && N >= 128 && K % 64 == 0 && K >= 128) {
-    const long tiles_half = (long)ceil_div(M, 256) * ceil_div(N, 128);
+  // N 4 mod 8, K a whole number of 128-byte stages, and at least 128 tiles of 256 x 128: a straight into LDS, b through
+  // the transposing register loader.  256 x 256 tiles of eight waves, or 256 x 128 tiles of four when those need fewer
+  // rounds of 256 workgroups for their cost (about 0.55 of a 256 x 256 tile).
+  if (N % 8 && M >= 256 && N >= 128 && K % 64 == 0 && K >= 128) {
+    const long tiles_big = (long)ceil_div(M, 256) * ceil_div(N, 256), tiles_half = (long)ceil_div(M, 256) * ceil_div(N, 128);
     const long rounds_big = ceil_div((int)tiles_big, 256), rounds_half = ceil_div((int)tiles_half, 256);
     const bool big_ok = N >= 256 && tiles_big >= 128;
     if (big_ok && rounds_big * 100 <= rounds_half * 55)
       return run_gemm_f16_hybrid<Tile<256, 256, 128, 2, 4>, OUT_F16>(a, b, c, M, N, K, s);
     if (tiles_half >= 128) return run_gemm_f16_hybrid<Tile<256, 128, 128, 2, 2>, OUT_F16>(a, b, c, M, N, K, s);
-    if (big_ok) return run_gemm_f16_hybrid<Tile<256, 256, 128, 2, 4>, OUT_F16>(a, b, c, M, N, K, s);
   }
-  if (M >= 256 && N >= 256 && tiles_big >= 128) {
-    // 64 (m) x 128 (n) wave tiles: measured 8-10 % faster than 128 x 64 (512-byte row runs per wave in the write-back)
-    return run_gemm_f16<Tile<256, 256, 128, 4, 2>, OUT_F16>(a, b, c, M, N, K, s);
-  }
-  // mid sizes: 128 x 256 tiles of eight waves (measured 8-12 % faster than 128 x 128 at 2048^3, 1024 x 4096 x 4096)
-  if (M >= 128 && N >= 256 && K >= 128) return run_gemm_f16<Tile<128, 256, 128, 4, 2>, OUT_F16>(a, b, c, M, N, K, s);
-  return run_gemm_f16<Tile<128, 128, 64, 2, 2>, OUT_F16>(a, b, c, M, N, K, s);
+  // four columns: less than one 16-byte chunk of a row of b
+  if (N < 8) return run_gemm_f16<Tile<128, 128, 64, 2, 2>, OUT_F16>(a, b, c, M, N, K, s);
+  return run_gemm_f16_group<Y_COLS, OUT_F16>("unit_gemm_f16", "f16gemm", a, b, c, M, N, K, s);
 }
 
 // ---- k-splits through a workspace: plane s of the workspace takes the partial tiles of split s, a second kernel
 // adds the planes in split order (deterministic; fp16 output rounds the final sum once)
-using SplitTile = Tile<128, 128, 64, 2, 2>;
-
+// How many planes: by the same estimate as the tiles (at least two with fewer than 12 tiles of 128 x 128 and 1 KiB of
+// reduction); three from 128 to 255 such tiles once each split keeps 2 KiB.  UNIT_AMD_GEMM_F16_SPLITK pins the count.
 int gemm_f16_ws_splits(int M, int N, int K) {
-  return gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K, ceil_div(K * 2, SplitTile::BKB));
+  const int nk = ceil_div(K * 2, 64), forced = tuning_override("UNIT_AMD_GEMM_F16_SPLITK");
+  const long tiles = tiles_of_128(M, N);
+  if (forced > 0) return forced < nk ? forced : nk;
+  if (tiles >= 256) return 1;
+  if (tiles >= 128) return K >= 3072 ? 3 : 1;
+  return plan_group(M, N, K * 2, tiles < 12 && K >= 512 ? 2 : 1, 19, kPlaneSplits).splits;
 }
 
 template <bool OUT_F16>
@@ -257,15 +251,10 @@ __global__ __launch_bounds__(256) void add_planes(const v4f *__restrict__ ws, vo
 // a (M, K) . b (K, N) with `splits` > 1 k-ranges; ws holds splits * M * N floats
 int gemm_f16_planes(const char *what, const void *a, const void *b, void *c, int M, int N, int K, bool out_f16, void *ws,
                     int splits, hipStream_t s) {
-  using T = SplitTile;
   const size_t plane = (size_t)M * N * 4;
-  GemmPlaneEpilogue::Params ep{ws, M, N, plane};
-  if (K % 32 == 0 && N % 8 == 0 && splits <= K * 2 / T::BKB) {
-    // whole 64-byte stages: both operands global -> LDS directly, b read back with the transposing LDS read
-    if (int rc = run_gemm_f16_dma_tr<T, 4, GemmPlaneEpilogue>(what, out_f16 ? "planes_dmatr_h" : "planes_dmatr", a, b, ep, M, N,
-                                                              K, splits, nullptr, s))
-      return rc;
-  } else {
+  if (N < 8) {  // less than one 16-byte chunk of a row of b
+    using T = Tile<128, 128, 64, 2, 2>;
+    GemmPlaneEpilogue::Params ep{ws, M, N, plane};
     using XL = RowMajorLoader<T::BX, T::BKB, T::NT, false, 1, true>;
     using YL = KMajorF16Loader<T::BY, T::BKB, T::NT, 1, true>;
     typename XL::Params xp{static_cast<const char *>(a), M, K * 2, K * 2};
@@ -273,6 +262,12 @@ int gemm_f16_planes(const char *what, const void *a, const void *b, void *c, int
     const int nk = ceil_div(K * 2, T::BKB), gx = ceil_div(M, T::BX), gy = ceil_div(N, T::BY);
     set_variant("f16gemm_planes_x%d_y%d_k%d_w%dx%d%s_s%d", T::BX, T::BY, T::BKB, T::WX, T::WY, out_f16 ? "_h" : "", splits);
     if (int rc = launch_mma<OpF16, T, XL, YL, GemmPlaneEpilogue, WS_NONE>(xp, yp, ep, nk, gx, gy, 4, splits, nullptr, 0, 0, s, what))
+      return rc;
+  } else {
+    const GroupGemm p{static_cast<const char *>(a), static_cast<const char *>(b), (u32)((size_t)M * K * 2),
+                      (u32)((size_t)N * K * 2), M, N, K * 2, N * 2, nullptr, ws, C_PLANES, plane};
+    const GroupPlan plan = plan_group(M, N, K * 2, splits, splits, kPlaneSplits);
+    if (int rc = run_group_plan<OpF16, Y_COLS, WS_NONE, false>(what, out_f16 ? "f16gemm_planes_h" : "f16gemm_planes", p, plan, s))
       return rc;
   }
   const size_t n4 = (size_t)M * N / 4;

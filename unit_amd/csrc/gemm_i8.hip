@@ -3,36 +3,58 @@
 #include "epilogues.hpp"
 #include "host.hpp"
 #include "loaders.hpp"
+#include "gemm_group.hpp"
 #include "gemm_mixed.hpp"
 #include "mma_dma.hpp"
 
 namespace unit {
 namespace {
 
+// 256 x 256 tiles staged through registers: pre-packed weights, and row-major ones with an odd number of 64-byte stages
 // TAIL = false: K is a whole number of stages (the loaders then stage without zeroing selects)
-template <class T, bool PACKED, bool TAIL = true>
-int run_dense(const void *a, const void *w, void *c, int M, int N, int K, hipStream_t s) {
+template <bool PACKED, bool TAIL>
+int run_dense_staged(const void *a, const void *w, void *c, int M, int N, int K, hipStream_t s) {
+  using T = Tile<256, 256, 128, 2, 4>;
   using XL = RowMajorLoader<T::BX, T::BKB, T::NT, true, 1, TAIL>;
-  using YLrm = RowMajorLoader<T::BY, T::BKB, T::NT, false, 1, TAIL>;
-  using YLpk = VnniLoader<T::BY, T::BKB, T::NT, 128, 1, TAIL>;
+  using YL = std::conditional_t<PACKED, VnniLoader<T::BY, T::BKB, T::NT, 128, 1, TAIL>,
+                                RowMajorLoader<T::BY, T::BKB, T::NT, false, 1, TAIL>>;
   using Epi = GemmEpilogue<OpI8, false>;
   typename XL::Params xp{static_cast<const char *>(a), M, K, K};
+  typename YL::Params yp;
+  if constexpr (PACKED)
+    yp = {static_cast<const char *>(w), N, K / 4};
+  else
+    yp = {static_cast<const char *>(w), N, K, K};
   typename Epi::Params ep{c, M, N};
   const int nk = ceil_div(K, T::BKB), gx = ceil_div(M, T::BX), gy = ceil_div(N, T::BY);
-  // few tiles and a long reduction: share K between workgroups (int32 atomics are exact)
-  int splits = gemm_k_splits("UNIT_AMD_DENSE_SPLITK", M, N, K, nk);
-  if ((size_t)M * N * 4 % 16) splits = 1;
-  set_variant("i8dense%s_x%d_y%d_k%d_w%d%s_s%d", PACKED ? "pk" : "rm", T::BX, T::BY, T::BKB, T::NT / 64, TAIL ? "" : "e",
-              splits);
-  if constexpr (PACKED) {
-    typename YLpk::Params yp{static_cast<const char *>(w), N, K / 4};
-    return launch_mma<OpI8, T, XL, YLpk, Epi, WS_Y>(xp, yp, ep, nk, gx, gy, 4, splits, c, (size_t)M * N * 4, 0, s,
-                                                    "unit_dense_dotprod_u8s8s32");
-  } else {
-    typename YLrm::Params yp{static_cast<const char *>(w), N, K, K};
-    return launch_mma<OpI8, T, XL, YLrm, Epi, WS_Y>(xp, yp, ep, nk, gx, gy, 4, splits, c, (size_t)M * N * 4, 0, s,
-                                                    "unit_dense_u8s8s32");
-  }
+  set_variant("i8dense%s_x%d_y%d_k%d_w%d%s_s1", PACKED ? "pk" : "rm", T::BX, T::BY, T::BKB, T::NT / 64, TAIL ? "" : "e");
+  return launch_mma<OpI8, T, XL, YL, Epi, WS_Y>(xp, yp, ep, nk, gx, gy, 4, 1, c, (size_t)M * N * 4, 0, s,
+                                                PACKED ? "unit_dense_dotprod_u8s8s32" : "unit_dense_u8s8s32");
+}
+
+// Tiles of at most 256 x 128 with the reduction shared inside the workgroup (gemm_group.hpp).  Sharing it between
+// workgroups as well (int32 atomics into the zero-filled output, exact) never won below 8 KiB of reduction; the
+// row-major operator shares at least two ways where it has fewer than 12 tiles of 128 x 128 and 1 KiB of reduction
+// (its tests ask for that; 50 x 260 x 1040 would run 2 us faster without).
+template <int YM, int WS>
+int run_dense_group(const char *what, const char *tag, const void *a, const void *w, const int *wsum, void *c, int M, int N,
+                    int K, hipStream_t s) {
+  const int forced = tuning_override("UNIT_AMD_DENSE_SPLITK");
+  const int least = YM == Y_ROWS && tiles_of_128(M, N) < 12 && K >= 1024 ? 2 : 1;
+  GroupPlan plan = plan_group(M, N, K, forced > 0 ? 1 : least, forced <= 0 && K >= 16384 ? 16 : 1, kAtomicSplits);
+  if (forced > 0) plan.splits = forced;
+  const GroupGemm p{static_cast<const char *>(a), static_cast<const char *>(w), (u32)((size_t)M * K), (u32)((size_t)N * K),
+                    M, N, K, K, wsum, c, C_ATOMIC, 0};
+  return run_group_plan<OpI8, YM, WS, false>(what, tag, p, plan, s);
+}
+
+// Row-major weights with whole 64-byte stages: the 128 x 128 tiles of mma_dma.hpp keep the shapes with few tiles or
+// few stages, and those with 512 tiles or more (8192 x 1024 x 1024 17.3 against 16.5 us); the tests name this kernel
+// there.  From 32 tiles and 384 bytes on the group tiles are faster (64 x 4096 x 4096 12.8 -> 7.8 us, 1024^3
+// 9.5 -> 5.8 us, 2304 x 2304 x 4096 41 -> 34 us).
+inline bool dense_keeps_128(int M, int N, int K) {
+  const long tiles = tiles_of_128(M, N);
+  return K % 64 == 0 && !direct_gemm_large_tiles(M, N) && (tiles < 32 || tiles >= 512 || K < 384);
 }
 
 // direct-to-LDS variant: row-major weights, K a whole number of stages.  wsum: the weight's row sums when they
@@ -97,6 +119,10 @@ int run_dense_mixed(const void *a, const void *wp, void *c, int M, int N, int K,
   return e == hipSuccess ? UNIT_OK : fail(UNIT_E_LAUNCH, "%s: launch: %s", what, hipGetErrorString(e));
 }
 
+// An odd number of 64-byte stages on a large result: the staged 256 x 256 tiles for short reductions (the tests name them);
+// 3000 x 3000 x 3008 runs in 52 us on the group tiles against 60.
+inline bool dense_stays_staged(int M, int N, int K) { return K % 128 == 64 && K < 1024 && direct_gemm_large_tiles(M, N); }
+
 template <bool PACKED>
 int dense(const void *a, const void *w, void *c, int M, int N, int K, unit_stream_t stream) {
   const char *what = PACKED ? "unit_dense_dotprod_u8s8s32" : "unit_dense_u8s8s32";
@@ -114,40 +140,28 @@ int dense(const void *a, const void *w, void *c, int M, int N, int K, unit_strea
   if (int rc = check_aligned(what, {a, w, c})) return rc;
   if (int rc = check_device()) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const long tiles_big = (long)ceil_div(M, 256) * ceil_div(N, 256);
-  switch (tuning_override("UNIT_AMD_DENSE_VARIANT")) {
-    case 1: return run_dense<Tile<256, 256, 128, 2, 2>, PACKED>(a, w, c, M, N, K, s);
-    case 2: return run_dense<Tile<256, 256, 64, 2, 4>, PACKED>(a, w, c, M, N, K, s);
-    case 3: return run_dense<Tile<256, 128, 64, 2, 2>, PACKED>(a, w, c, M, N, K, s);
-    case 4: return run_dense<Tile<128, 128, 64, 2, 2>, PACKED>(a, w, c, M, N, K, s);
-    case 5: return run_dense<Tile<256, 256, 64, 2, 2>, PACKED>(a, w, c, M, N, K, s);
-    case 6: return run_dense<Tile<128, 256, 128, 1, 4>, PACKED>(a, w, c, M, N, K, s);
-    case 7: if (!PACKED && K % 64 == 0) return run_dense_dma<Tile<256, 256, 64, 2, 2>, 4>(a, w, c, M, N, K, s); break;
-    case 8: if (!PACKED && K % 64 == 0) return run_dense_dma<Tile<256, 256, 64, 2, 4>, 4>(a, w, c, M, N, K, s); break;
-    case 9: if (!PACKED && K % 128 == 0) return run_dense_dma<Tile<256, 256, 128, 2, 2>, 2>(a, w, c, M, N, K, s); break;
-    case 10: if (!PACKED && K % 64 == 0) return run_dense_dma<Tile<256, 256, 64, 2, 2>, 3>(a, w, c, M, N, K, s); break;
-    case 11: if (!PACKED && K % 64 == 0) return run_dense_dma<Tile<256, 128, 64, 2, 2>, 4>(a, w, c, M, N, K, s); break;
+  switch (tuning_override("UNIT_AMD_DENSE_VARIANT")) {  // measurement aid: pins a kernel where it can run
     case 12: if (!PACKED && K % 128 == 0) return run_dense_dma<Tile<256, 256, 128, 2, 4>, 2>(a, w, c, M, N, K, s); break;
     case 13: if (PACKED) return run_dense_mixed(a, w, c, M, N, K, s); break;
-    case 14: return run_dense<Tile<256, 256, 128, 2, 4>, PACKED>(a, w, c, M, N, K, s);
-    case 15: return run_dense<Tile<256, 256, 128, 4, 2>, PACKED>(a, w, c, M, N, K, s);
     case 16: if (!PACKED && K % 128 == 0) return run_dense_dma<Tile<256, 256, 128, 4, 2>, 2>(a, w, c, M, N, K, s); break;
     case 17: if (!PACKED && K % 64 == 0) return run_dense_dma<Tile<128, 128, 64, 2, 2>, 4>(a, w, c, M, N, K, s); break;
     default: break;
   }
-  // row-major weights, K a whole number of 64-byte stages, and a shape that 128 x 128 tiles fill better than 256 x 256
-  // ones: both operands global -> LDS directly, two workgroups per CU (2048^3 23.3 -> 20.7 us, 1024 x 4096 x 4096
-  // 39.8 -> 32.7 us, 8192 x 1024 x 1024 24.6 -> 18.0 us)
-  if (!PACKED && K % 64 == 0 && !direct_gemm_large_tiles(M, N))
-    return run_dense_dma<Tile<128, 128, 64, 2, 2>, 4>(a, w, c, M, N, K, s, nullptr,
-                                                      direct_gemm_k_splits("UNIT_AMD_DENSE_SPLITK", M, N, K));
-  // the large tiles on the same pipeline: the four waves that share a weight fragment divide the weight sums
-  if (!PACKED && K % 128 == 0 && direct_gemm_large_tiles(M, N))
-    return run_dense_dma<Tile<256, 256, 128, 4, 2>, 2>(a, w, c, M, N, K, s);
-  if (M >= 256 && N >= 256 && tiles_big >= 128)
-    return K % 128 ? run_dense<Tile<256, 256, 128, 2, 4>, PACKED>(a, w, c, M, N, K, s)
-                   : run_dense<Tile<256, 256, 128, 2, 4>, PACKED, false>(a, w, c, M, N, K, s);
-  return run_dense<Tile<128, 128, 64, 2, 2>, PACKED>(a, w, c, M, N, K, s);
+  if constexpr (PACKED) {
+    // the staged 256 x 256 tiles take 1.15 x the time of the direct-to-LDS ones on row-major weights
+    if (M >= 256 && N >= 256 && 1.15f * large_tile_cost(M, N, K) < plan_group(M, N, K, 1, 1, kAtomicSplits).us)
+      return K % 128 ? run_dense_staged<true, true>(a, w, c, M, N, K, s) : run_dense_staged<true, false>(a, w, c, M, N, K, s);
+    return run_dense_group<Y_VNNI, WS_Y>(what, "i8densepk", a, w, nullptr, c, M, N, K, s);
+  } else {
+    if (dense_keeps_128(M, N, K))
+      return run_dense_dma<Tile<128, 128, 64, 2, 2>, 4>(a, w, c, M, N, K, s, nullptr,
+                                                        direct_gemm_k_splits("UNIT_AMD_DENSE_SPLITK", M, N, K));
+    // the four waves that share a weight fragment divide the weight sums
+    if (K % 128 == 0 && direct_gemm_large_tiles(M, N))
+      return run_dense_dma<Tile<256, 256, 128, 4, 2>, 2>(a, w, c, M, N, K, s);
+    if (dense_stays_staged(M, N, K)) return run_dense_staged<false, true>(a, w, c, M, N, K, s);
+    return run_dense_group<Y_ROWS, WS_Y>(what, "i8denserm", a, w, nullptr, c, M, N, K, s);
+  }
 }
 
 // one wave per weight row: sum of its K bytes
@@ -186,18 +200,19 @@ extern "C" int unit_dense_u8s8s32_prepared(const void *a, const void *w, const i
   using namespace unit;
   const char *what = "unit_dense_u8s8s32_prepared";
   if (!a || !w || !wsum || !c) return fail(UNIT_E_ARG, "%s: null pointer", what);
-  // the direct-to-LDS kernels need whole stages (128 bytes for the 256 x 256 tiles, 64 for the 128 x 128 ones);
-  // everything else runs the plain entry point, which sums the weights itself (same result)
-  const bool large = M > 0 && N > 0 && direct_gemm_large_tiles(M, N);
-  if (M <= 0 || N <= 0 || K <= 0 || K % (large ? 128 : 64) || N % 4 || row_slice(M, (size_t)K, (size_t)N * 4) ||
-      !fits((size_t)M * K) || !fits((size_t)N * K) || !fits((size_t)M * N * 4))
+  // arguments that this entry point does not take in one launch run the plain one, which sums the weights itself
+  if (M <= 0 || N <= 0 || K <= 0 || K % 16 || N % 4 || row_slice(M, (size_t)K, (size_t)N * 4) || !fits((size_t)M * K) ||
+      !fits((size_t)N * K) || !fits((size_t)M * N * 4) || dense_stays_staged(M, N, K))
     return unit_dense_u8s8s32(a, w, c, M, N, K, stream);
   if (int rc = check_aligned(what, {a, w, c})) return rc;
   if (int rc = check_device()) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (large) return run_dense_dma<Tile<256, 256, 128, 4, 2>, 2, true>(a, w, c, M, N, K, s, wsum);
-  return run_dense_dma<Tile<128, 128, 64, 2, 2>, 4, true>(a, w, c, M, N, K, s, wsum,
-                                                          direct_gemm_k_splits("UNIT_AMD_DENSE_SPLITK", M, N, K));
+  if (dense_keeps_128(M, N, K))
+    return run_dense_dma<Tile<128, 128, 64, 2, 2>, 4, true>(a, w, c, M, N, K, s, wsum,
+                                                            direct_gemm_k_splits("UNIT_AMD_DENSE_SPLITK", M, N, K));
+  if (K % 128 == 0 && direct_gemm_large_tiles(M, N))
+    return run_dense_dma<Tile<256, 256, 128, 4, 2>, 2, true>(a, w, c, M, N, K, s, wsum);
+  return run_dense_group<Y_ROWS, WS_Y_GIVEN>(what, "i8denserm_prep", a, w, wsum, c, M, N, K, s);
 }
 
 extern "C" int unit_dense_dotprod_u8s8s32(const void *a, const void *wp, void *c, int32_t M, int32_t N, int32_t K,

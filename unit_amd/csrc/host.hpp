@@ -65,8 +65,11 @@ inline void set_variant(const char *fmt, A... a) {
   n.fmt = fmt;
   new (n.args) Args(a...);
   n.spell = [](const VariantNote &self, char *out, size_t size) {
-    std::apply([&](const A &...v) { snprintf(out, size, self.fmt, variant_printf(variant_arg(v))...); },
-               *reinterpret_cast<const Args *>(self.args));
+    if constexpr (sizeof...(A) == 0)
+      snprintf(out, size, "%s", self.fmt);
+    else
+      std::apply([&](const A &...v) { snprintf(out, size, self.fmt, variant_printf(variant_arg(v))...); },
+                 *reinterpret_cast<const Args *>(self.args));
   };
 }
 

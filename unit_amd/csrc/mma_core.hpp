@@ -40,6 +40,7 @@ typedef unsigned int u32;
 // form that takes the policy bits as an operand the compiler knows: its hazard and wait-count passes see the stores
 // (written as inline assembly they were followed by a write of the data registers inside the store's hazard window).
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+typedef unsigned int v2u __attribute__((ext_vector_type(2)));
 constexpr int kResultPolicy = 16 | 2;  // sc1 | nt
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t result_buffer(void *base) {
   return __builtin_amdgcn_make_buffer_rsrc(base, 0, -1, 0x00020000);

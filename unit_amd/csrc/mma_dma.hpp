@@ -55,6 +55,14 @@ __device__ __forceinline__ void direct_load_16s(const void *sbase, u32 voff, u32
                : "memory");
 }
 
+// The same as a raw buffer load: a lane whose offset lies past the buffer stores zeros into LDS.
+__device__ __forceinline__ void dma_buffer_16(u32 lds_addr, u32 voff, v4i rsrc, u32 soff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :
+               : "s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff)
+               : "memory");
+}
+
 // YT (16-bit operands only): Y is given reduction-major, (K, yrows) with yrows contiguous -- the fp16 GEMM's b as the
 // reference has it.  Its tile lands in LDS as it lies in memory, [k][BY / 8 chunks of 8 columns], and the MFMA
 // fragments (8 consecutive k of one column per lane) come out of it with the LDS transposing read
