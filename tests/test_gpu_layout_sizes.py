@@ -1,0 +1,28 @@
+"""Layout kernels on both sides of their dispatch lines: planes smaller than a four-byte word of pixels, planes of odd
+size (words at any byte address, the last one moved back), and tensors on either side of the line from which packing
+takes sixteen pixels per thread."""
+import numpy as np
+import pytest
+import torch
+
+import unit_amd as U
+from unit_amd import rng
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape,cb,dtype", [
+    ((2, 3, 1, 3), 4, np.uint8), ((2, 5, 1, 5), 4, np.uint8), ((3, 3, 61, 43), 4, np.int8),
+    ((2, 33, 1, 2), 16, np.uint8), ((2, 33, 2, 2), 16, np.uint8), ((7, 320, 9, 11), 16, np.int8),
+    ((5625, 250, 3, 5), 16, np.uint8),    # 90000 planes of 15 pixels: partial groups of the sixteen-pixel kernel
+    ((22499, 16, 4, 4), 16, np.uint8),    # 89996 four-pixel groups
+    ((22500, 16, 4, 4), 16, np.uint8),    # 90000
+    ((2, 20, 3, 7), 16, np.float16), ((2, 20, 1, 1), 16, np.float16), ((1, 20, 3, 3), 16, np.int32),
+])
+def test_pack_and_back(dev, oracle, shape, cb, dtype):
+    x = rng.random_bytes(int(np.prod(shape)) * np.dtype(dtype).itemsize, 7).view(dtype).reshape(shape)
+    if dtype == np.float16:
+        x = np.nan_to_num(x, nan=1.0)
+    p = U.pack_nchwc(torch.from_numpy(x).to(dev), cb)
+    assert np.array_equal(p.cpu().numpy().view(np.uint8), oracle.pack_nchwc(x, cb).view(np.uint8))
+    assert np.array_equal(U.unpack_nchwc(p, shape[1]).cpu().numpy().view(np.uint8), x.view(np.uint8))

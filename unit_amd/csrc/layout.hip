@@ -6,73 +6,6 @@ namespace unit {
 namespace {
 
 // ---- NCHW <-> NCHW{CB}c -------------------------------------------------------------------
-// A thread moves PP = 4 / ES consecutive pixels of one channel block: CB 4-byte words (one per
-// channel plane, coalesced across lanes) <-> PP contiguous rows of CB elements.
-template <int ES, int CB, bool PACK>
-__global__ __launch_bounds__(256) void nchwc_words(const char *src, char *dst, int C, int HW, int cc,
-                                                   int groups /* HW / PP */) {
-  constexpr int PP = 4 / ES, ROWW = CB * ES / 4;  // words per output row
-  const int g = blockIdx.x * 256 + threadIdx.x;
-  if (g >= groups) return;
-  const int plane = blockIdx.y;  // n * cc + ci
-  const int n = plane / cc, ci = plane - n * cc;
-  const size_t p0 = (size_t)g * PP;
-  const char *nchw = PACK ? src : dst;
-  u32 w[CB];
-  u32 rows[PP][ROWW];
-  if (PACK) {
-#pragma unroll
-    for (int c = 0; c < CB; ++c) {
-      const int ch = ci * CB + c;
-      w[c] = ch < C ? *reinterpret_cast<const u32 *>(nchw + (((size_t)n * C + ch) * HW + p0) * ES) : 0u;
-    }
-#pragma unroll
-    for (int pp = 0; pp < PP; ++pp)
-#pragma unroll
-      for (int j = 0; j < ROWW; ++j) {
-        u32 v = 0;
-#pragma unroll
-        for (int e = 0; e < 4 / ES; ++e) {
-          const u32 el = ES == 4 ? w[j] : (w[j * (4 / ES) + e] >> (8 * ES * pp)) & (ES == 1 ? 0xffu : 0xffffu);
-          v |= el << (8 * ES * e);
-        }
-        rows[pp][j] = v;
-      }
-    char *o = dst + ((size_t)plane * HW + p0) * CB * ES;
-#pragma unroll
-    for (int pp = 0; pp < PP; ++pp)
-#pragma unroll
-      for (int j = 0; j < ROWW; ++j) reinterpret_cast<u32 *>(o)[pp * ROWW + j] = rows[pp][j];
-  } else {
-    const char *in = src + ((size_t)plane * HW + p0) * CB * ES;
-#pragma unroll
-    for (int pp = 0; pp < PP; ++pp)
-#pragma unroll
-      for (int j = 0; j < ROWW; ++j) rows[pp][j] = reinterpret_cast<const u32 *>(in)[pp * ROWW + j];
-#pragma unroll
-    for (int c = 0; c < CB; ++c) {
-      u32 v = 0;
-#pragma unroll
-      for (int pp = 0; pp < PP; ++pp) {
-        const u32 word = rows[pp][c * ES / 4];
-        const u32 el = ES == 4 ? word : (word >> (8 * ES * (c % (4 / ES)))) & (ES == 1 ? 0xffu : 0xffffu);
-        v |= el << (8 * ES * pp);
-      }
-      const int ch = ci * CB + c;
-      if (ch < C) *reinterpret_cast<u32 *>(dst + (((size_t)n * C + ch) * HW + p0) * ES) = v;
-    }
-  }
-}
-
-// u8 / s8 with 16-channel blocks: a thread moves 16 pixels x 16 channels of one (image, channel block)
-// plane, 16-byte loads and stores on both sides (16 consecutive pixels of one channel plane <-> one
-// pixel's 16 channels) and a 16 x 16 byte transpose in registers: sixteen 4 x 4 transposes of
-// two v_perm_b32 stages each.  Packing then passes the rows through a wave-private LDS area so that
-// a store instruction writes 64 consecutive pixels (1 KiB) instead of 16-byte pieces 256 bytes
-// apart; LDS operations of one wave execute in order, so the area needs no barrier.
-// The work items are the 16-pixel groups of all planes in one flat index (small planes still fill
-// the blocks); a plane of fewer than 16 pixels is one partial group that goes byte by byte on the
-// NCHW side.
 // 4 x 4 byte transpose: rows a, b, c, d (byte k of a row = column k) -> t[k] = {a.k, b.k, c.k, d.k}
 __device__ __forceinline__ void transpose4x4(u32 a, u32 b, u32 c, u32 d, u32 (&t)[4]) {
   const u32 x0 = __builtin_amdgcn_perm(b, a, 0x05010400u), x1 = __builtin_amdgcn_perm(b, a, 0x07030602u);
@@ -83,15 +16,90 @@ __device__ __forceinline__ void transpose4x4(u32 a, u32 b, u32 c, u32 d, u32 (&t
   t[3] = __builtin_amdgcn_perm(y1, x1, 0x07060302u);
 }
 
+// A thread moves PP = 4 / ES consecutive pixels of one channel block: CB 4-byte words (one per channel plane, coalesced
+// across lanes) <-> PP contiguous rows of CB elements.  The pixel groups of all planes lie in one flat index, so that
+// small planes still fill the blocks; the last group of a plane whose size PP does not divide is moved back to end with
+// the plane (it overlaps its neighbour, and both write the same bytes there), so words start at any element: planes of
+// fewer than PP pixels go to nchwc_elems.  (Planes of odd size went there too: 30 x 3 x 189 x 171 bytes in 12.6 us.)
+typedef u32 word_at_t __attribute__((aligned(1)));
+
+template <int ES, int CB, bool PACK>
+__global__ __launch_bounds__(256) void nchwc_words(const char *src, char *dst, int C, int HW, int cc, FastDiv by_groups,
+                                                   int total_groups) {
+  constexpr int PP = 4 / ES, ROWW = CB * ES / 4;  // words per blocked row
+  const int gid = blockIdx.x * 256 + threadIdx.x;
+  if (gid >= total_groups) return;
+  int plane, g;  // plane = n * cc + ci
+  by_groups.divmod(gid, plane, g);
+  const int n = plane / cc, ci = plane - n * cc;
+  const int p0 = min(g * PP, HW - PP);
+  const char *nchw = PACK ? src : dst;
+  const size_t chan0 = (((size_t)n * C + ci * CB) * HW + p0) * ES, blocked0 = ((size_t)plane * HW + p0) * CB * ES;
+  u32 w[CB];
+  u32 rows[PP][ROWW];
+  if (PACK) {
+#pragma unroll
+    for (int c = 0; c < CB; ++c)
+      w[c] = ci * CB + c < C ? *reinterpret_cast<const word_at_t *>(nchw + chan0 + (size_t)c * HW * ES) : 0u;
+#pragma unroll
+    for (int j = 0; j < ROWW; ++j) {
+      if constexpr (ES == 1) {
+        u32 t[4];
+        transpose4x4(w[4 * j], w[4 * j + 1], w[4 * j + 2], w[4 * j + 3], t);
+#pragma unroll
+        for (int pp = 0; pp < 4; ++pp) rows[pp][j] = t[pp];
+      } else if constexpr (ES == 2) {
+        rows[0][j] = __builtin_amdgcn_perm(w[2 * j + 1], w[2 * j], 0x05040100u);
+        rows[1][j] = __builtin_amdgcn_perm(w[2 * j + 1], w[2 * j], 0x07060302u);
+      } else {
+        rows[0][j] = w[j];
+      }
+    }
+    char *o = dst + blocked0;
+#pragma unroll
+    for (int pp = 0; pp < PP; ++pp)
+#pragma unroll
+      for (int j = 0; j < ROWW; ++j) reinterpret_cast<u32 *>(o)[pp * ROWW + j] = rows[pp][j];
+  } else {
+    const char *in = src + blocked0;
+#pragma unroll
+    for (int pp = 0; pp < PP; ++pp)
+#pragma unroll
+      for (int j = 0; j < ROWW; ++j) rows[pp][j] = reinterpret_cast<const u32 *>(in)[pp * ROWW + j];
+#pragma unroll
+    for (int j = 0; j < ROWW; ++j) {
+      if constexpr (ES == 1) {
+        u32 t[4];
+        transpose4x4(rows[0][j], rows[1][j], rows[2][j], rows[3][j], t);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[4 * j + k] = t[k];
+      } else if constexpr (ES == 2) {
+        w[2 * j] = __builtin_amdgcn_perm(rows[1][j], rows[0][j], 0x05040100u);
+        w[2 * j + 1] = __builtin_amdgcn_perm(rows[1][j], rows[0][j], 0x07060302u);
+      } else {
+        w[j] = rows[0][j];
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < CB; ++c)
+      if (ci * CB + c < C) *reinterpret_cast<word_at_t *>(dst + chan0 + (size_t)c * HW * ES) = w[c];
+  }
+}
+
+// u8 / s8 into 16-channel blocks, large tensors: a thread moves 16 pixels x 16 channels of one (image, channel block)
+// plane, 16-byte loads (16 consecutive pixels of one channel plane) and a 16 x 16 byte transpose in registers: sixteen
+// 4 x 4 transposes of two v_perm_b32 stages each.  The rows (one pixel's 16 channels) then pass through a wave-private LDS
+// area so that a store instruction writes 64 consecutive pixels (1 KiB) instead of 16-byte pieces 256 bytes apart;
+// LDS operations of one wave execute in order, so the area needs no barrier.
+// The work items are the 16-pixel groups of all planes in one flat index (small planes still fill the blocks); a plane
+// of fewer than 16 pixels is one partial group that goes byte by byte on the NCHW side.
 // 16 bytes at any byte address (a group's first byte in a plane of H * W bytes)
 typedef int bytes16_t __attribute__((ext_vector_type(4), aligned(1)));
 
-template <bool PACK>
-__global__ __launch_bounds__(256) void nchw16c_bytes(const char *src, char *dst, int C, int HW, int cc,
+__global__ __launch_bounds__(256) void pack16c_bytes(const char *src, char *dst, int C, int HW, int cc,
                                                      FastDiv by_groups /* ceil(HW / 16) */, int total_groups) {
   const int gid = blockIdx.x * 256 + threadIdx.x;
-  if (!PACK && gid >= total_groups) return;
-  const bool live = gid < total_groups;  // packing: lanes past the end still take part in the wave's write-back
+  const bool live = gid < total_groups;  // lanes past the end still take part in the wave's write-back
   int plane, g;                          // plane = n * cc + ci
   by_groups.divmod(live ? gid : 0, plane, g);
   const int n = plane / cc, ci = plane - n * cc;
@@ -99,73 +107,47 @@ __global__ __launch_bounds__(256) void nchw16c_bytes(const char *src, char *dst,
   // write the same bytes there); only planes of fewer than 16 pixels have a partial group
   const int p0 = g * 16 + 16 <= HW || HW < 16 ? g * 16 : HW - 16;
   const int cnt = live ? min(16, HW - p0) : 0;  // pixels of this group
-  const char *nchw = PACK ? src : dst;
   const size_t chan0 = ((size_t)n * C + ci * 16) * HW + p0;  // byte offset of channel ci * 16, pixel p0
   const size_t flat0 = (size_t)plane * HW + p0;              // pixel index in the blocked tensor
   v4i planes[16];  // [channel]: 16 pixels
   v4i rows[16];    // [pixel]: 16 channels
-  if (PACK) {
-    if (cnt == 16) {
+  if (cnt == 16) {
 #pragma unroll
-      for (int c = 0; c < 16; ++c)
-        planes[c] = ci * 16 + c < C ? (v4i) * reinterpret_cast<const bytes16_t *>(nchw + chan0 + (size_t)c * HW) : v4i{0, 0, 0, 0};
-    } else {
-#pragma unroll
-      for (int c = 0; c < 16; ++c) {
-        u32 w[4] = {0, 0, 0, 0};
-        if (ci * 16 + c < C)
-          for (int e = 0; e < cnt; ++e) w[e >> 2] |= (u32)(unsigned char)nchw[chan0 + (size_t)c * HW + e] << (8 * (e & 3));
-        planes[c] = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        u32 t[4];
-        transpose4x4(planes[4 * j][q], planes[4 * j + 1][q], planes[4 * j + 2][q], planes[4 * j + 3][q], t);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) rows[4 * q + k][j] = (int)t[k];
-      }
-    // lane l parks its 16 rows at pitch 272 bytes (conflict-free both ways) with the group's first pixel and
-    // pixel count behind them; the wave then stores row after row, 64 rows per instruction
-    __shared__ __attribute__((aligned(16))) char stage[4][64 * 272];
-    const int lane = threadIdx.x & 63;
-    char *st = stage[threadIdx.x >> 6];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) *reinterpret_cast<v4i *>(st + lane * 272 + r * 16) = rows[r];
-    *reinterpret_cast<v2i *>(st + lane * 272 + 256) = v2i{(int)flat0, cnt};
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const int pix = k * 64 + lane;
-      const char *slot = st + (pix >> 4) * 272;
-      const v4i v = *reinterpret_cast<const v4i *>(slot + (pix & 15) * 16);
-      const v2i where = *reinterpret_cast<const v2i *>(slot + 256);
-      if ((pix & 15) < where[1]) reinterpret_cast<v4i *>(dst)[(size_t)where[0] + (pix & 15)] = v;
-    }
+    for (int c = 0; c < 16; ++c)
+      planes[c] = ci * 16 + c < C ? (v4i) * reinterpret_cast<const bytes16_t *>(src + chan0 + (size_t)c * HW) : v4i{0, 0, 0, 0};
   } else {
-    const v4i *blocked = reinterpret_cast<const v4i *>(src) + flat0;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) rows[r] = r < cnt ? blocked[r] : v4i{0, 0, 0, 0};
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        u32 t[4];
-        transpose4x4(rows[4 * q][j], rows[4 * q + 1][j], rows[4 * q + 2][j], rows[4 * q + 3][j], t);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) planes[4 * j + k][q] = (int)t[k];
-      }
-    if (cnt == 16) {
-#pragma unroll
-      for (int c = 0; c < 16; ++c)
-        if (ci * 16 + c < C) *reinterpret_cast<bytes16_t *>(dst + chan0 + (size_t)c * HW) = (bytes16_t)planes[c];
-    } else {
-#pragma unroll
-      for (int c = 0; c < 16; ++c)
-        if (ci * 16 + c < C)
-          for (int e = 0; e < cnt; ++e) dst[chan0 + (size_t)c * HW + e] = (char)((u32)planes[c][e >> 2] >> (8 * (e & 3)));
+    for (int c = 0; c < 16; ++c) {
+      u32 w[4] = {0, 0, 0, 0};
+      if (ci * 16 + c < C)
+        for (int e = 0; e < cnt; ++e) w[e >> 2] |= (u32)(unsigned char)src[chan0 + (size_t)c * HW + e] << (8 * (e & 3));
+      planes[c] = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
     }
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      u32 t[4];
+      transpose4x4(planes[4 * j][q], planes[4 * j + 1][q], planes[4 * j + 2][q], planes[4 * j + 3][q], t);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) rows[4 * q + k][j] = (int)t[k];
+    }
+  // lane l parks its 16 rows at pitch 272 bytes (conflict-free both ways) with the group's first pixel and
+  // pixel count behind them; the wave then stores row after row, 64 rows per instruction
+  __shared__ __attribute__((aligned(16))) char stage[4][64 * 272];
+  const int lane = threadIdx.x & 63;
+  char *st = stage[threadIdx.x >> 6];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) *reinterpret_cast<v4i *>(st + lane * 272 + r * 16) = rows[r];
+  *reinterpret_cast<v2i *>(st + lane * 272 + 256) = v2i{(int)flat0, cnt};
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    const int pix = k * 64 + lane;
+    const char *slot = st + (pix >> 4) * 272;
+    const v4i v = *reinterpret_cast<const v4i *>(slot + (pix & 15) * 16);
+    const v2i where = *reinterpret_cast<const v2i *>(slot + 256);
+    if ((pix & 15) < where[1]) reinterpret_cast<v4i *>(dst)[(size_t)where[0] + (pix & 15)] = v;
   }
 }
 
@@ -190,6 +172,12 @@ __global__ __launch_bounds__(256) void nchwc_elems(const char *src, char *dst, i
   }
 }
 
+// u8 / s8 NCHW -> NCHW16c: from this many four-pixel groups on, sixteen pixels per thread (nchw16c_bytes) win.  Below, the
+// tensor gives such threads too few waves and each a long chain: 7 x 320 x 9 x 11 5.3 us against 2.9 us with four pixels
+// per thread, 32 x 64 x 56 x 56 5.5 against 5.7, 32 x 256 x 56 x 56 10.4 against 15.7 us.  The way back is faster with
+// four pixels per thread at every size (14.5 -> 10.5 us for the last).
+constexpr long kManyGroups = 90000;
+
 template <bool PACK>
 int nchwc(const void *src, void *dst, int N, int C, int H, int W, int cb, int es, hipStream_t s, const char *what) {
   if (!src || !dst) return fail(UNIT_E_ARG, "%s: null pointer", what);
@@ -213,19 +201,20 @@ int nchwc(const void *src, void *dst, int N, int C, int H, int W, int cb, int es
   const char *in = static_cast<const char *>(src);
   char *out = static_cast<char *>(dst);
   const int HW = (int)hw, pp = 4 / es;
-  const bool words = HW % pp == 0 && (cb == 16 || (cb == 4 && es == 1)) && (size_t)N * cc <= 65535;
-  if (es == 1 && cb == 16) {
-    const int groups = ceil_div(HW, 16), total_groups = N * cc * groups;  // < 2^27: the tensor fits 2^31 bytes
-    const dim3 grid(ceil_div(total_groups, 256));
-    const FastDiv by_groups = FastDiv::make(groups);
-    hipLaunchKernelGGL(nchw16c_bytes<PACK>, grid, dim3(256), 0, s, in, out, C, HW, cc, by_groups, total_groups);
+  const int groups = ceil_div(HW, pp);
+  const long total_groups = (long)N * cc * groups;  // < 2^29: the tensor fits 2^31 bytes
+  const bool words = HW >= pp && (cb == 16 || (cb == 4 && es == 1));
+  if (PACK && es == 1 && cb == 16 && (total_groups >= kManyGroups || !words)) {
+    const int groups16 = ceil_div(HW, 16), total16 = N * cc * groups16;
+    hipLaunchKernelGGL(pack16c_bytes, dim3(ceil_div(total16, 256)), dim3(256), 0, s, in, out, C, HW, cc,
+                       FastDiv::make(groups16), total16);
   } else if (words) {
-    const int groups = HW / pp;
-    dim3 grid(ceil_div(groups, 256), N * cc);
-#define UNIT_NCHWC(ES, CB)                                                                                   \
-  hipLaunchKernelGGL((nchwc_words<ES, CB, PACK>), grid, dim3(256), 0, s, in, out, C, HW, cc, groups)
+    const dim3 grid((unsigned)((total_groups + 255) / 256));
+    const FastDiv by_groups = FastDiv::make(groups);
+#define UNIT_NCHWC(ES, CB)                                                                                          \
+  hipLaunchKernelGGL((nchwc_words<ES, CB, PACK>), grid, dim3(256), 0, s, in, out, C, HW, cc, by_groups, (int)total_groups)
     if (es == 1 && cb == 16) UNIT_NCHWC(1, 16);
-    else if (es == 1 && cb == 4) UNIT_NCHWC(1, 4);
+    else if (es == 1) UNIT_NCHWC(1, 4);
     else if (es == 2) UNIT_NCHWC(2, 16);
     else UNIT_NCHWC(4, 16);
 #undef UNIT_NCHWC
