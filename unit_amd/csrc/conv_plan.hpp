@@ -58,6 +58,18 @@ inline ConvPlan heuristic_plan(int npix, int K, int kbytes, bool allow_split, bo
     // thousand waves on the chip; the smallest problems use 64 x 32 (fp16: 32 x 64) tiles.
     const long t64 = tiles(64, 64);
     int v, panel = 0;
+    // Long reductions on few output pixels: eight waves share a tile of one 32-channel block, which gives such a layer
+    // twice the workgroups of 64 x 32 tiles and each wave half the k-steps in a row (its time is a chain of load
+    // latencies, not a rate).  While 32 x 32 tiles are at most one per CU: u8 1536 -> 720, 3 x 3 on 17 x 14, 19.7 -> 10.6 us;
+    // fp16 1168 -> 32, 5 x 5 on 27 x 17, 85 -> 43; the 137 such rows of the tables 901 -> 751 in all.  Below 20 k-steps the
+    // sum of eight partial tiles costs what it gains (18: 4.36 against 4.34 us), above 256 tiles the second round does
+    // (342 of them: 10.6 -> 8.0, 555: 22.0 -> 21.0, 720: 49.2 -> 51.1).  Up to 32 channels a 64-channel tile is half
+    // padding: 32 x 64 tiles there (480 -> 32 on 76 x 72: 10.6 -> 7.0).  The tap table of 4096 k-steps still fits the LDS.
+    const int ksteps = kbytes / 32;
+    if (ksteps >= 20 && ksteps <= 4096 && tiles(32, 32) <= 256)
+      return ConvPlan{82, 1, 4};
+    if (ksteps >= 20 && ksteps <= 4096 && K <= 32 && tiles(32, 64) <= 384)
+      return ConvPlan{83, 1, 0};
     if (allow_split) {  // the int8 operator; distilled from the tuner's choices on cold operands (batch 1 .. 256)
       const int nsteps = kbytes / 32;
       const bool wide = K % 128 == 0;  // 128-channel tiles
