@@ -138,6 +138,17 @@ def test_out_hw_and_error_paths_without_gpu():
         _lib.check(-1)
 
 
+def test_gemm_planes_fit_the_library_scratch():
+    """Below 128 tiles of 128 x 128 the k-split planes fit the 16 MiB scratch of unit_gemm_f16_static, which rejects more."""
+    from unit_amd import _lib
+    lib = _lib.load()
+    nbytes = ctypes.c_size_t()
+    for m, n, k in ((435, 2376, 18640), (231, 5780, 12824), (212, 2736, 13864), (848, 1168, 30072), (899, 468, 20792),
+                    (1920, 1024, 32768), (1, 16256, 65536)):
+        assert lib.unit_gemm_f16_ws_bytes(m, n, k, ctypes.byref(nbytes)) == 0
+        assert nbytes.value <= 16 << 20, (m, n, k, nbytes.value)
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     from unit_amd import _lib
     monkeypatch.setattr(_lib, "_lib", None)

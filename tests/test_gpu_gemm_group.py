@@ -76,3 +76,14 @@ def test_pinned_k_splits(dev, monkeypatch, splits):
     for ws in (None, True):
         assert torch.equal(U.gemm_fp16(h, b, workspace=ws).double(), ref), U.last_variant()
         assert U.last_variant().endswith(f"_s{splits}")
+
+
+@pytest.mark.parametrize("M,N,K", [(512, 512, 512), (640, 640, 992), (256, 256, 256), (128, 4096, 480)])
+def test_fp16_without_planes_runs_whole(dev, M, N, K):
+    """A shape for which no planes are planned keeps one workgroup per tile when it comes through the workspace entry
+    point: k-splits by atomics, which the plain entry point may choose there, would not give the same bits each time."""
+    assert U.gemm_fp16_workspace_bytes(M, N, K) == 0
+    g = np.random.RandomState(M + K)
+    a, b = _ints(g, -3, 4, (M, K), torch.float16, dev), _ints(g, -2, 3, (K, N), torch.float16, dev)
+    assert torch.equal(U.gemm_fp16(a, b, workspace=True).double(), a.double() @ b.double())
+    assert U.last_variant().endswith("_s1") or "_s" not in U.last_variant(), U.last_variant()

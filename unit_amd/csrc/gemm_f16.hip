@@ -109,8 +109,8 @@ int run_gemm_f16_hybrid(const void *a, const void *b, void *c, int M, int N, int
 // 300 x 260 x 520 would run 2 us faster without); fp16 results keep one workgroup per tile.
 template <int YM, bool OUT_F16>
 int run_gemm_f16_group(const char *what, const char *tag, const void *a, const void *b, void *c, int M, int N, int K,
-                       hipStream_t s) {
-  const int forced = OUT_F16 ? 1 : tuning_override("UNIT_AMD_GEMM_F16_SPLITK");
+                       hipStream_t s, bool whole = false) {
+  const int forced = OUT_F16 || whole ? 1 : tuning_override("UNIT_AMD_GEMM_F16_SPLITK");
   const int least = forced <= 0 && tiles_of_128(M, N) < 12 && K >= 512 ? 2 : 1;
   GroupPlan plan = plan_group(M, N, K * 2, least, forced > 0 ? 1 : 19, kAtomicSplits);
   if (forced > 0) plan.splits = forced;
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(256) void unpack32_f16(const _Float16 *__restrict__
 
 // TAIL = false: K is a whole number of stages (the loaders then stage without zeroing selects)
 template <class T, bool OUT_F16, int PF = 1, bool TAIL = true>
-int run_gemm_f16(const void *a, const void *b, void *c, int M, int N, int K, hipStream_t s) {
+int run_gemm_f16(const void *a, const void *b, void *c, int M, int N, int K, hipStream_t s, bool whole) {
   using XL = RowMajorLoader<T::BX, T::BKB, T::NT, false, PF, TAIL>;
   using YL = KMajorF16Loader<T::BY, T::BKB, T::NT, PF, TAIL>;
   using Epi = GemmEpilogue<OpF16, OUT_F16>;
@@ -177,15 +177,17 @@ int run_gemm_f16(const void *a, const void *b, void *c, int M, int N, int K, hip
   typename YL::Params yp{static_cast<const char *>(b), N, K, N + 4, 0, N * 2};
   typename Epi::Params ep{c, M, N};
   const int nk = ceil_div(K * 2, T::BKB), gx = ceil_div(M, T::BX), gy = ceil_div(N, T::BY);
-  const int splits = OUT_F16 ? 1 : gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K, nk);
+  const int splits = OUT_F16 || whole ? 1 : gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K, nk);
   set_variant("f16gemm_x%d_y%d_k%d_w%dx%d_p%d%s%s_s%d", T::BX, T::BY, T::BKB, T::WX, T::WY, PF, TAIL ? "" : "e",
               OUT_F16 ? "_h" : "", splits);
   return launch_mma<OpF16, T, XL, YL, Epi, WS_NONE>(xp, yp, ep, nk, gx, gy, 4, splits, c, (size_t)M * N * 4, 0, s,
                                                     "unit_gemm_f16");
 }
 
+// whole: one workgroup per tile, whatever the shape (the entry points that promise the same bits from run to run
+// come here when they plan no planes; k-splits added by atomics would end in another order each time)
 template <bool OUT_F16>
-int gemm_f16(const void *a, const void *b, void *c, int M, int N, int K, hipStream_t s) {
+int gemm_f16(const void *a, const void *b, void *c, int M, int N, int K, hipStream_t s, bool whole = false) {
   // UNIT_AMD_GEMM_F16_VARIANT pins a kernel per process where it can run (measurement aid)
   switch (tuning_override("UNIT_AMD_GEMM_F16_VARIANT")) {
     case 7: if (K % 64 == 0 && K >= 128) return run_gemm_f16_hybrid<Tile<256, 256, 128, 2, 4>, OUT_F16>(a, b, c, M, N, K, s); break;
@@ -201,8 +203,9 @@ int gemm_f16(const void *a, const void *b, void *c, int M, int N, int K, hipStre
       if (K % 64 == 0) return run_gemm_f16_dma_tr<Tile<256, 256, 128, 2, 4>, 2, OUT_F16>(a, b, c, M, N, K, s);
       return run_gemm_f16_dma_tr<Tile<256, 256, 64, 2, 4>, 4, OUT_F16>(a, b, c, M, N, K, s);
     }
-    if (gemm_keeps_128(M, N, OUT_F16))
-      return run_gemm_f16_dma_tr<Tile<128, 128, 64, 2, 2>, 4, OUT_F16>(a, b, c, M, N, K, s, direct_gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K));
+    const int splits = direct_gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K);
+    if (gemm_keeps_128(M, N, OUT_F16) && !(whole && splits > 1))
+      return run_gemm_f16_dma_tr<Tile<128, 128, 64, 2, 2>, 4, OUT_F16>(a, b, c, M, N, K, s, splits);
   }
   // N 4 mod 8, K a whole number of 128-byte stages, and at least 128 tiles of 256 x 128: a straight into LDS, b through
   // the transposing register loader.  256 x 256 tiles of eight waves, or 256 x 128 tiles of four when those need fewer
@@ -216,21 +219,24 @@ int gemm_f16(const void *a, const void *b, void *c, int M, int N, int K, hipStre
     if (tiles_half >= 128) return run_gemm_f16_hybrid<Tile<256, 128, 128, 2, 2>, OUT_F16>(a, b, c, M, N, K, s);
   }
   // four columns: less than one 16-byte chunk of a row of b
-  if (N < 8) return run_gemm_f16<Tile<128, 128, 64, 2, 2>, OUT_F16>(a, b, c, M, N, K, s);
-  return run_gemm_f16_group<Y_COLS, OUT_F16>("unit_gemm_f16", "f16gemm", a, b, c, M, N, K, s);
+  if (N < 8) return run_gemm_f16<Tile<128, 128, 64, 2, 2>, OUT_F16>(a, b, c, M, N, K, s, whole);
+  return run_gemm_f16_group<Y_COLS, OUT_F16>("unit_gemm_f16", "f16gemm", a, b, c, M, N, K, s, whole);
 }
 
 // ---- k-splits through a workspace: plane s of the workspace takes the partial tiles of split s, a second kernel
 // adds the planes in split order (deterministic; fp16 output rounds the final sum once)
 // How many planes: by the same estimate as the tiles (at least two with fewer than 12 tiles of 128 x 128 and 1 KiB of
-// reduction); three from 128 to 255 such tiles once each split keeps 2 KiB.  UNIT_AMD_GEMM_F16_SPLITK pins the count.
+// reduction), and no more than the library's own scratch holds (two always fit below 128 tiles); three from 128 to 255 such
+// tiles once each split keeps 2 KiB.  UNIT_AMD_GEMM_F16_SPLITK pins the count.
+constexpr size_t kStaticScratchBytes = 16u << 20;
 int gemm_f16_ws_splits(int M, int N, int K) {
   const int nk = ceil_div(K * 2, 64), forced = tuning_override("UNIT_AMD_GEMM_F16_SPLITK");
   const long tiles = tiles_of_128(M, N);
   if (forced > 0) return forced < nk ? forced : nk;
   if (tiles >= 256) return 1;
   if (tiles >= 128) return K >= 3072 ? 3 : 1;
-  return plan_group(M, N, K * 2, tiles < 12 && K >= 512 ? 2 : 1, 19, kPlaneSplits).splits;
+  const size_t fit = kStaticScratchBytes / ((size_t)M * N * 4);
+  return plan_group(M, N, K * 2, tiles < 12 && K >= 512 ? 2 : 1, fit < 19 ? (int)fit : 19, kPlaneSplits).splits;
 }
 
 template <bool OUT_F16>
@@ -302,7 +308,6 @@ int gemm_f16_ws_check(const char *what, const void *a, const void *b, const void
 // per device on the first call there (with that device current); host code uses that pointer, never the array's name.
 namespace unit {
 namespace {
-constexpr size_t kStaticScratchBytes = 16u << 20;
 static __device__ __align__(256) char scratch[kStaticScratchBytes];
 constexpr int kMaxDevices = 64;
 void *g_scratch_ptr[kMaxDevices];
@@ -337,7 +342,7 @@ extern "C" int unit_gemm_f16_static(const void *a, const void *b, void *c, int32
   if (int rc = check_device()) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (splits <= 1)  // nothing to split: no scratch is touched
-    return out_f16 ? gemm_f16<true>(a, b, c, M, N, K, s) : gemm_f16<false>(a, b, c, M, N, K, s);
+    return out_f16 ? gemm_f16<true>(a, b, c, M, N, K, s, true) : gemm_f16<false>(a, b, c, M, N, K, s, true);
   const size_t need = (size_t)splits * M * N * 4;
   if (need > kStaticScratchBytes)
     return fail(UNIT_E_ARG, "%s: %d k-splits of %d x %d need %zu bytes of scratch, the static buffer holds %zu; "
@@ -365,11 +370,11 @@ extern "C" int unit_gemm_f16_ws(const void *a, const void *b, void *c, int32_t M
   const char *what = "unit_gemm_f16_ws";
   int splits = 1;
   if (int rc = gemm_f16_ws_check(what, a, b, c, M, N, K, &splits)) return rc;
-  if (splits <= 1) {  // enough tiles, or a short reduction: nothing to split (the plain path makes the same choice)
+  if (splits <= 1) {  // enough tiles, or a short reduction: nothing to split 
     if (int rc = check_aligned(what, {a, b, c})) return rc;
     if (int rc = check_device()) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    return out_f16 ? gemm_f16<true>(a, b, c, M, N, K, s) : gemm_f16<false>(a, b, c, M, N, K, s);
+    return out_f16 ? gemm_f16<true>(a, b, c, M, N, K, s, true) : gemm_f16<false>(a, b, c, M, N, K, s, true);
   }
   const size_t need = (size_t)splits * M * N * 4;
   if (!workspace || workspace_bytes < need)
