@@ -59,6 +59,22 @@ def test_chain_with_side_branch_bit_exact(dev, oracle):
     assert last is c.outputs[-1]
 
 
+def test_chain_follows_replaced_buffers(dev, oracle):
+    layers_np = _small_layers()
+    x = rng.uniform_u8((3, 1, 13, 11, 16), 8)
+    c = chain.ConvChain(_to_chain(layers_np, dev), x.shape)
+    c(_t(x, dev))
+    old = [o.clone() for o in c.outputs]
+    oc, ic, k = layers_np[2][0].shape[:3]
+    layers_np[2] = (rng.uniform_s8((oc, ic, k, k), 300),) + layers_np[2][1:]
+    c.weights[2] = U.prepare_conv2d_weight(U.prepack_conv_weight(_t(layers_np[2][0], dev), 16))
+    kept, c.outputs[1] = c.outputs[1], torch.empty_like(c.outputs[1])
+    c(_t(x, dev))
+    for got, want in zip(c.outputs, _oracle_chain(oracle, layers_np, x)):
+        assert np.array_equal(got.cpu().numpy(), want)
+    assert torch.equal(kept, old[1]) and not torch.equal(c.outputs[2], old[2])
+
+
 def test_chain_graph_replay_follows_the_input(dev, oracle):
     layers_np = _small_layers()[:3]
     x1 = rng.uniform_u8((2, 1, 9, 9, 16), 8)

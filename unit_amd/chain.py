@@ -78,18 +78,24 @@ class ConvChain:
         self._names = ctypes.create_string_buffer(96 * count)  # kernel names, written by the first run
         self._native = (ChainLayerDesc * count)()
         for i, d in enumerate(self._native):
-            bias = self.biases[i]
             d.desc = self.descs[i]
-            d.data = None if self.sources[i] < 0 else self.outputs[self.sources[i]].data_ptr()
-            d.prepared, d.out = self.weights[i].buf.data_ptr(), self.outputs[i].data_ptr()
-            d.bias = None if bias is None else bias.data_ptr()
             d.variant = ctypes.addressof(self._names) + 96 * i
-            d.scale, d.shift = self.consts[i]
+        self._bound = None
+
+    def _bind(self):
+        """Buffers and constants as they are now: a caller may have put other ones into the lists."""
+        bound = [(w.buf.data_ptr(), o.data_ptr(), None if b is None else b.data_ptr(), *c, src)
+                 for w, o, b, c, src in zip(self.weights, self.outputs, self.biases, self.consts, self.sources)]
+        if bound != self._bound:
+            for d, (d.prepared, d.out, d.bias, d.scale, d.shift, src) in zip(self._native, bound):
+                d.data = None if src < 0 else bound[src][1]
+            self._bound = bound
 
     def run(self, x):
         x = ops._dev(x, "x", torch.uint8, 5)
         if tuple(x.shape) != self.input_shape:
             raise ValueError(f"x: expected {self.input_shape}, got {tuple(x.shape)}")
+        self._bind()
         check(self._L.unit_conv_chain_u8(self._native, len(self._native), x.data_ptr(), ops._stream()))
         if None in self.variants:
             self.variants = [self._names[96 * i:96 * i + 96].split(b"\0")[0].decode() for i in range(len(self._native))]

@@ -137,7 +137,7 @@ def _plan_f16(dshape, kshape, stride_h, stride_w):
             raise ValueError(f"a {tuple(dshape)} / b {tuple(kshape)}: expected (N, C/16, H, W, 16) and "
                              f"(K/16, C/16, KH, KW, 16, 16)")
         k = ko * 16
-    return _ConvPlan(n, cc * 16, h, w, k, kh, kw, (int(stride_h), int(stride_w)), 0, 1, 16)
+    return _ConvPlan(n, cc * 16, h, w, k, kh, kw, (stride_h, stride_w), 0, 1, 16)
 
 
 def _hashable(v):
@@ -526,20 +526,20 @@ def conv2d_NCHW16c_OHWI16o(a, b, stride_h, stride_w, out_type="float32"):
         if a.dim() != 5:
             raise ValueError("a: prepared weights take the blocked (N, C/16, H, W, 16) operand")
         _check_prepared(b, a, torch.float16)
-        p = _plan_f16(a.shape, b.key, stride_h, stride_w)
+        p = _plan_f16(a.shape, b.key, int(stride_h), int(stride_w))
         out = a.new_empty(p.blocked, dtype=torch.float32)
         check(L.unit_conv2d_nchw16c_f16f32_prepared(p.ref, a.data_ptr(), b.buf.data_ptr(), out.data_ptr(), _stream()))
         return out
     b = _dev(b, "b", torch.float16, (4, 6))
     if a.dim() == 4 and b.dim() == 4:
-        p, need = _plan_f16_plain(a.shape, b.shape, stride_h, stride_w)
+        p, need = _plan_f16_plain(a.shape, b.shape, int(stride_h), int(stride_w))
         ws = a.new_empty((need,), dtype=torch.uint8)
         out = a.new_empty(p.blocked, dtype=torch.float32)
         check(L.unit_conv2d_nchw_f16f32(p.ref, a.data_ptr(), b.data_ptr(), out.data_ptr(), ws.data_ptr(), need, _stream()))
         return out
     if not (a.dim() == 5 and b.dim() == 6):
         raise ValueError("a, b: expected 4-D + 4-D or 5-D + 6-D operands")
-    p = _plan_f16(a.shape, b.shape, stride_h, stride_w)
+    p = _plan_f16(a.shape, b.shape, int(stride_h), int(stride_w))
     out = a.new_empty(p.blocked, dtype=torch.float32)
     check(L.unit_conv2d_nchw16c_f16f32(p.ref, a.data_ptr(), b.data_ptr(), out.data_ptr(), _stream()))
     return out
@@ -551,7 +551,7 @@ def _plan_f16_plain(ashape, bshape, stride_h, stride_w):
     k, c2, kh, kw = bshape
     if c % 16 or k % 16 or c2 != c:
         raise ValueError("a, b: channel counts must match and be multiples of 16")
-    p = _ConvPlan(n, c, h, w, k, kh, kw, (int(stride_h), int(stride_w)), 0, 1, 16)
+    p = _ConvPlan(n, c, h, w, k, kh, kw, (stride_h, stride_w), 0, 1, 16)
     need = ctypes.c_size_t()
     check(_lib.load().unit_conv2d_nchw_f16f32_ws_bytes(p.ref, ctypes.byref(need)))
     return p, need.value
