@@ -282,6 +282,13 @@ int unit_conv2d_nchwc_s8s8s32_fused_prepared_nchw(const unit_conv_desc *d, const
                                                   const int32_t *bias, int32_t scale, void *out,
                                                   int32_t out_channels, unit_stream_t stream);
 
+/* The same with the opening layout_transform NCHW -> NCHW{cb}c (result.log:7,6807-6808) inside as well: x is
+ * (N, in_channels, H, W) s8, d->C - d->cb < in_channels <= d->C.  `packed` (N * d->C * H * W bytes, 16-byte aligned) takes the
+ * blocked copy where one is made; convolutions of at most four input channels usually run without. */
+int unit_conv2d_nchw_s8s8s32_fused_prepared(const unit_conv_desc *d, int32_t in_channels, const void *x,
+                                            const void *prepared, const int32_t *bias, int32_t scale, void *out,
+                                            int32_t out_channels, void *packed, unit_stream_t stream);
+
 /* u8 x s8 convolution on prepared weights with the output requantised to u8 in the blocked
  * layout the next convolution reads, (N, K/16, OH, OW, 16) u8:
  *   q = clamp(((conv_u8(data, w)[k] + bias[k]) * scale + 2^(shift-1)) >> shift, 0, 255)

@@ -144,3 +144,26 @@ def test_graph_replay_follows_the_input(dev):
         xd.copy_(torch.from_numpy(x).to(dev))
         torch.cuda.synchronize()
         assert np.array_equal(replay().cpu().numpy(), _plain_graph(x, wt, None, 5, 1, 1))
+
+
+@pytest.mark.parametrize("n,ic,h,w,oc,kh,kw,stride,padding,dilation", [
+    (1, 3, 7, 4, 5, 7, 4, 1, 0, 1),                # one output pixel, the narrowest rows
+    (1, 1, 9, 5, 16, 1, 1, 1, 0, 1),               # one channel, one tap
+    (3, 2, 40, 17, 30, 3, 3, 2, 1, 1),             # narrow: many output rows per workgroup, images end inside one
+    (1, 4, 19, 33, 130, 5, 8, 1, (3, 5, 2, 4), 1),  # all eight taps of a row, five channel blocks, four different pads
+    (2, 3, 23, 131, 96, 7, 7, 2, 3, 1),            # three channel blocks, rows that end inside a word
+    (2, 3, 30, 29, 64, 3, 3, (3, 2), 9, (4, 1)),   # padding wider than the window, dilated rows
+    (6, 3, 193, 187, 81, 7, 7, 2, 3, 1),           # 256 pixels per workgroup
+])
+def test_image_stem_in_one_launch(dev, n, ic, h, w, oc, kh, kw, stride, padding, dilation):
+    x, wt, b = rng.uniform_s8((n, ic, h, w), h), rng.uniform_s8((oc, ic, kh, kw), w), _i32((oc,), 13, -5000, 5000)
+    pads = (padding,) * 4 if isinstance(padding, int) else padding
+    xp = np.pad(x, ((0, 0), (0, 0), (pads[0], pads[2]), (pads[1], pads[3])))
+    want = _plain_graph(xp, wt, b, -11, stride, 0, dilation)
+    g = relay.Conv2dBiasMultiply(torch.from_numpy(wt).to(dev), torch.from_numpy(b).to(dev), -11, stride, padding, dilation)
+    room = torch.zeros(x.size + 1, dtype=torch.int8, device=dev)  # the input may start at any byte
+    room[1:] = torch.from_numpy(x.reshape(-1)).to(dev)
+    got = g(room[1:].view(x.shape))
+    assert "stem" in U.last_variant(), U.last_variant()
+    assert np.array_equal(got.cpu().numpy(), want), U.last_variant()
+    assert torch.equal(g(room[1:].view(x.shape), fold_output_transform=False), got)

@@ -44,6 +44,7 @@ SYMBOLS = (
     "unit_conv2d_nchwc_u8s8s32_prepared",
     "unit_conv2d_nchwc_s8s8s32_fused_prepared",
     "unit_conv2d_nchwc_s8s8s32_fused_prepared_nchw",
+    "unit_conv2d_nchw_s8s8s32_fused_prepared",
     "unit_conv2d_nchw16c_f16f32_prepared",
     "unit_conv2d_nchwc_u8s8u8_requant_prepared",
     "unit_conv_chain_u8",
@@ -121,6 +122,7 @@ def load():
     L.unit_conv2d_nchwc_u8s8s32_prepared.argtypes = [dp, vp, vp, vp, vp]
     L.unit_conv2d_nchwc_s8s8s32_fused_prepared.argtypes = [dp, vp, vp, vp, i32, vp, vp]
     L.unit_conv2d_nchwc_s8s8s32_fused_prepared_nchw.argtypes = [dp, vp, vp, vp, i32, vp, i32, vp]
+    L.unit_conv2d_nchw_s8s8s32_fused_prepared.argtypes = [dp, i32, vp, vp, vp, i32, vp, i32, vp, vp]
     L.unit_conv2d_nchw16c_f16f32_prepared.argtypes = [dp, vp, vp, vp, vp]
     L.unit_conv2d_nchwc_u8s8u8_requant_prepared.argtypes = [dp, vp, vp, vp, i32, i32, vp, vp]
     L.unit_conv_chain_u8.argtypes = [ctypes.POINTER(ChainLayerDesc), i32, vp, vp]

@@ -26,6 +26,9 @@ int conv_s8_prepared(const ConvPlan &plan, const unit_conv_desc *d, const ConvGe
                      const int *bias, int scale, void *out, int planar, hipStream_t s);  // conv_prepared_s8.hip
 int conv_c4_prepared(const ConvPlan &plan, const unit_conv_desc *d, const ConvGeom &g, const void *data, const void *w,
                      const int *addend, int scale, bool shift, void *out, int planar, hipStream_t s);  // conv_prepared_c4.hip
+bool planar_c4_takes(const ConvGeom &g, int K);
+int conv_planar_c4(const unit_conv_desc *d, const ConvGeom &g, int in_channels, const void *x, const void *w, const int *bias,
+                   int scale, void *out, int oc, hipStream_t s);  // conv_planar_c4.hip
 int conv_q8_prepared(const ConvPlan &plan, const unit_conv_desc *d, const ConvGeom &g, const void *data, const void *w,
                      const int *addend, const int *bias, int scale, int shift, void *out, hipStream_t s);  // conv_prepared_q8.hip
 int conv_f16_prepared(const ConvPlan &plan, const unit_conv_desc *d, const ConvGeom &g, const void *a, const void *w,
@@ -312,6 +315,29 @@ extern "C" int unit_conv2d_nchwc_s8s8s32_fused_prepared_nchw(const unit_conv_des
   if (d && (out_channels <= d->K - 16 || out_channels > d->K))
     return fail(UNIT_E_ARG, "%s: out_channels %d does not round up to K = %d", what, out_channels, d->K);
   return fused_prepared(what, d, data, prepared, bias, scale, out, out_channels, stream);
+}
+
+extern "C" int unit_conv2d_nchw_s8s8s32_fused_prepared(const unit_conv_desc *d, int32_t in_channels, const void *x,
+                                                       const void *prepared, const int32_t *bias, int32_t scale, void *out,
+                                                       int32_t out_channels, void *packed, unit_stream_t stream) {
+  using namespace unit;
+  const char *what = "unit_conv2d_nchw_s8s8s32_fused_prepared";
+  if (!d || !x || !prepared || !out || !packed) return fail(UNIT_E_ARG, "%s: null pointer", what);
+  if (d->cb <= 0 || in_channels <= d->C - d->cb || in_channels > d->C)
+    return fail(UNIT_E_ARG, "%s: in_channels %d does not round up to C = %d", what, in_channels, d->C);
+  if (out_channels <= d->K - 16 || out_channels > d->K)
+    return fail(UNIT_E_ARG, "%s: out_channels %d does not round up to K = %d", what, out_channels, d->K);
+  // image stems in one launch, unless the batch needs slices or a variant of the general kernels is pinned
+  size_t in_img, out_img;
+  if (d->cb == 4 && d->C == 4 && !batch_slice(d, (size_t)d->C, (size_t)d->K * 4, &in_img, &out_img) &&
+      tuning_override("UNIT_AMD_CONV_VARIANT") <= 0) {
+    ConvGeom g;
+    if (int rc = check_prepared_conv(what, d, 16, &g, packed, prepared, out)) return rc;
+    if (planar_c4_takes(g, d->K))
+      return conv_planar_c4(d, g, in_channels, x, prepared, bias, scale, out, out_channels, static_cast<hipStream_t>(stream));
+  }
+  if (int rc = unit_pack_nchwc(x, packed, d->N, in_channels, d->H, d->W, d->cb, 1, stream)) return rc;
+  return fused_prepared(what, d, packed, prepared, bias, scale, out, out_channels, stream);
 }
 
 extern "C" int unit_conv2d_nchw16c_f16f32_prepared(const unit_conv_desc *d, const void *a, const void *prepared,

@@ -80,12 +80,9 @@ class Conv2dBiasMultiply:
             out = torch.empty((n, self.oc, oh.value, ow.value), dtype=torch.int32, device=x.device)
             plan = self._plans[tuple(x.shape)] = (desc, ctypes.byref(desc), data, out)
         desc, desc_ref, data, out = plan
-        stream = ops._stream()
-        n, c, h, w = x.shape
-        ops.check(self._L.unit_pack_nchwc(x.data_ptr(), data.data_ptr(), n, c, h, w, self.cb, 1, stream))     # Op #0
-        ops.check(self._L.unit_conv2d_nchwc_s8s8s32_fused_prepared_nchw(                                       # Ops #5 + #6
-            desc_ref, data.data_ptr(), self.weight.buf.data_ptr(), self.bias.data_ptr() if self.bias is not None else None,
-            self.multiplier, out.data_ptr(), self.oc, stream))
+        ops.check(self._L.unit_conv2d_nchw_s8s8s32_fused_prepared(                                             # Ops #0, #5, #6
+            desc_ref, self.ic, x.data_ptr(), self.weight.buf.data_ptr(), self.bias.data_ptr() if self.bias is not None else None,
+            self.multiplier, out.data_ptr(), self.oc, data.data_ptr(), ops._stream()))
         return out
 
 
