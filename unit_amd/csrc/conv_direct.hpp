@@ -114,7 +114,7 @@ __device__ __forceinline__ void store_block(const typename ConvEpilogue<Op>::Par
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         if (c0 + 8 * q + 4 * half + e < p.planar && m < p.npix)
-          store_result<kPlanarPolicy>(obuf, (dst + (u32)(8 * q + e) * (u32)p.ohw) * (u32)sizeof(out_t), v[e]);
+          store_result<kRowPolicy>(obuf, (dst + (u32)(8 * q + e) * (u32)p.ohw) * (u32)sizeof(out_t), v[e]);
     }
     return;
   }

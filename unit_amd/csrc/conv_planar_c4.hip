@@ -140,7 +140,7 @@ __global__ __launch_bounds__(256) void conv_planar_c4_kernel(PlanarC4 p) {
 #pragma unroll
         for (int j = 0; j < TY; ++j)
           if (c < p.oc && (int)m0 + j * 32 <= last)
-            store_result<kPlanarPolicy>(obuf, (dst + (u32)(j * 32)) * 4u, (acc[i][j][4 * q + e] + b[e]) * p.scale);
+            store_result<kRowPolicy>(obuf, (dst + (u32)(j * 32)) * 4u, (acc[i][j][4 * q + e] + b[e]) * p.scale);
       }
     }
 }

@@ -328,9 +328,9 @@ __global__ __launch_bounds__(T::NT) void gemm_group(GroupGemm p, GridMap gm) {
     } else if (OUT_F16 && p.mode == C_STORE) {
       typedef _Float16 v4h __attribute__((ext_vector_type(4)));
       const v4h h = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
-      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, h), cbuf, (int)(idx * 2u), 0, kResultPolicy);
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, h), cbuf, (int)(idx * 2u), 0, kRowPolicy);
     } else {
-      store_result(cbuf, idx * 4u, v);
+      store_result<kRowPolicy>(cbuf, idx * 4u, v);
     }
   }
 }

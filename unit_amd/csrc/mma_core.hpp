@@ -42,11 +42,12 @@ typedef unsigned int u32;
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 typedef unsigned int v2u __attribute__((ext_vector_type(2)));
 constexpr int kResultPolicy = 16 | 2;  // sc1 | nt
-// Planar results (a store instruction writes 128 bytes of each of two channel planes) without nt: where a plane is no
-// multiple of 128 bytes these pieces start and end inside lines, and nt sends every such part of a line to memory by itself.
-// 32 x 64 x 55 x 55 -> 256 planar: 83 us with sc1 nt, 76 with nt, 33 with sc1, 30 with neither; planes of whole
-// lines, 32 x 64 x 56 x 56: 30.3, 31.0, 27.3, 28.0.
-constexpr int kPlanarPolicy = 16;  // sc1
+// Planar and row-major results without nt: their store instructions write 128- to 512-byte pieces of planes or rows, and where
+// those are no multiple of 128 bytes the pieces start and end inside lines; nt sends every such part of a line to memory
+// by itself.  us with sc1 nt / nt / sc1 / neither: 32 x 64 x 55 x 55 -> 256 planar 83 / 76 / 33 / 30; fp16 GEMM
+// 8000 x 3004 x 200 43.5 / 35.5 / 29.0 / 27.3; int8 8000 x 3004 x 208 41.9 / 31.2 / 27.0 / 26.9.  Whole lines: planar
+// 32 x 64 x 56 x 56 -> 256 30.3 / 31.0 / 27.3 / 28.0; int8 4096^3 65.9 / 66.9 / 64.2 / 67.1.
+constexpr int kRowPolicy = 16;  // sc1
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t result_buffer(void *base) {
   return __builtin_amdgcn_make_buffer_rsrc(base, 0, -1, 0x00020000);
 }
