@@ -153,7 +153,7 @@ def test_graph_replay_follows_the_input(dev):
     (1, 4, 19, 33, 130, 5, 8, 1, (3, 5, 2, 4), 1),  # all eight taps of a row, five channel blocks, four different pads
     (2, 3, 23, 131, 96, 7, 7, 2, 3, 1),            # three channel blocks, rows that end inside a word
     (2, 3, 30, 29, 64, 3, 3, (3, 2), 9, (4, 1)),   # padding wider than the window, dilated rows
-    (6, 3, 193, 187, 81, 7, 7, 2, 3, 1),           # 256 pixels per workgroup
+    (6, 3, 193, 187, 81, 7, 7, 2, 3, 1),           # results end inside a 16-byte store
 ])
 def test_image_stem_in_one_launch(dev, n, ic, h, w, oc, kh, kw, stride, padding, dilation):
     x, wt, b = rng.uniform_s8((n, ic, h, w), h), rng.uniform_s8((oc, ic, kh, kw), w), _i32((oc,), 13, -5000, 5000)

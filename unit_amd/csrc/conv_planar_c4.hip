@@ -3,17 +3,22 @@
 // layout_transform, convolution, layout_transform (apps/cpu/relay/result.log:6803-6838); here it is one launch.
 //
 // What bounds it is the result (51 MB at 16 x 3 x 224 x 224, 64 channels, 7 x 7, stride 2: 8 us at the rate of a fill),
-// so everything in front of the stores has to be short.  A workgroup takes 32 TY x 4 consecutive output pixels of one
-// image and all or a third / half of the channels: it lays the input rows under its window out in LDS, once, as 4-byte pixels with the
+// so everything in front of the stores has to be short.  A workgroup takes 128 consecutive output pixels of one
+// image and all, a third or half of the channels: it lays the input rows under its window out in LDS, once, as 4-byte pixels with the
 // zero padding in place, beside the weight fragments.  A k-step (one window row) is then one 16-byte LDS read per
 // 32 pixels -- the direct kernel on a packed copy spends four masked 4-byte gathers from memory there, and a
-// launch and a round trip through memory on the copy.
+// launch and a round trip through memory on the copy.  That size: 21.5 us with the packed copy, 13.0 here.
+// 128 pixels and not 256: more workgroups than the chip holds at once, so that some load while others store (13.0 against
+// 15.4; 32 x 3 x 229 x 92 -> 96, 3 x 3 stride 2, 15.2 against 16.9; one shape of five was 6 % faster on 256).  Results through LDS
+// and not 128 bytes per store and channel straight from the accumulators: the latter 18.8 against 15.2, equal on whole lines.
 #include "conv_plan.hpp"
 #include "conv_prepare.hpp"
 #include "mma_dma.hpp"
 
 namespace unit {
 namespace {
+
+constexpr int PT = 128;  // output pixels per workgroup
 
 struct PlanarC4 {
   const char *x, *w;
@@ -28,10 +33,9 @@ struct PlanarC4 {
 typedef u32 word_at_t __attribute__((aligned(1)));
 
 // NC: input channels read (3, or 4 with those past C masked)
-template <int TX, int TY, int NC>
+template <int TX, int NC>
 __global__ __launch_bounds__(256) void conv_planar_c4_kernel(PlanarC4 p) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  constexpr int PT = 128 * TY;
   const int lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   int rest, kg, n, tile, oh0, oh1, rem;
@@ -94,77 +98,80 @@ __global__ __launch_bounds__(256) void conv_planar_c4_kernel(PlanarC4 p) {
     }
   }
 
-  int yoff[TY];  // of this lane's pixel: its window's first row, taps 4 half .. + 3
-#pragma unroll
-  for (int j = 0; j < TY; ++j) {
-    int oh, ow;
-    p.by_ow.divmod(min(p0 + (wave * TY + j) * 32 + l32, last), oh, ow);
-    yoff[j] = (oh - oh0) * p.sh * pitch + ow * p.sw * 4 + half * 16;
-  }
-  v16i acc[TX][TY];
+  int oh, ow;
+  p.by_ow.divmod(min(p0 + wave * 32 + l32, last), oh, ow);
+  const char *window = patch + (oh - oh0) * p.sh * pitch + ow * p.sw * 4 + half * 16;  // its first row, taps 4 half .. + 3
+  v16i acc[TX];
 #pragma unroll
   for (int i = 0; i < TX; ++i)
 #pragma unroll
-    for (int j = 0; j < TY; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+    for (int r = 0; r < 16; ++r) acc[i][r] = 0;
   UNIT_WAIT_VMCNT(0);  // the weight fragments have landed
   __syncthreads();
 
   const int rstep = p.dh * pitch;
   for (int kh = 0; kh < p.KH; ++kh) {
-    v4i x[TX], y[TY];
-#pragma unroll
-    for (int j = 0; j < TY; ++j) y[j] = *reinterpret_cast<const v4i_a4 *>(patch + yoff[j] + kh * rstep);
+    const v4i y = *reinterpret_cast<const v4i_a4 *>(window + kh * rstep);
+    v4i x[TX];
 #pragma unroll
     for (int i = 0; i < TX; ++i) x[i] = *reinterpret_cast<const v4i *>(lds + ((i * p.KH + kh) * 64 + lane) * 16);
 #pragma unroll
-    for (int i = 0; i < TX; ++i)
-#pragma unroll
-      for (int j = 0; j < TY; ++j) acc[i][j] = OpI8::mma(x[i], y[j], acc[i][j]);
+    for (int i = 0; i < TX; ++i) acc[i] = OpI8::mma(x[i], y, acc[i]);
   }
 
-  // register r of a lane is channel 8 (r / 4) + 4 half + r % 4 of its pixel: 128 consecutive bytes per 32 lanes
-  const __amdgpu_buffer_rsrc_t obuf = result_buffer(p.out);
-  const u32 m0 = (u32)(p0 + wave * TY * 32 + l32);
+  // Results, 32 channels at a time, through LDS: register r of a lane is channel 8 (r / 4) + 4 half + r % 4 of its pixel;
+  // a store instruction then writes 512 consecutive bytes of each of two channel planes.
+  v4i add[TX][4];
 #pragma unroll
   for (int i = 0; i < TX; ++i)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int c4 = i * 32 + 8 * q + 4 * half;
-      const v4i b = *reinterpret_cast<const v4i *>(bias + c4);
+    for (int q = 0; q < 4; ++q) add[i][q] = *reinterpret_cast<const v4i *>(bias + i * 32 + 8 * q + 4 * half);
+  constexpr int kPitch = PT + 4;
+  int *tile_out = reinterpret_cast<int *>(lds);
+  const __amdgpu_buffer_rsrc_t obuf = result_buffer(p.out);
+  const int px = (int)(threadIdx.x * 4) % PT, row0 = (int)(threadIdx.x * 4) / PT;  // eight channels at a time
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int c = kg * (TX * 32) + c4 + e;
-        const u32 dst = (u32)(n * p.oc + c) * (u32)p.OHW + m0;
+  for (int i = 0; i < TX; ++i) {
+    __syncthreads();  // the patch, or the block before, has been read
 #pragma unroll
-        for (int j = 0; j < TY; ++j)
-          if (c < p.oc && (int)m0 + j * 32 <= last)
-            store_result<kRowPolicy>(obuf, (dst + (u32)(j * 32)) * 4u, (acc[i][j][4 * q + e] + b[e]) * p.scale);
+    for (int r = 0; r < 16; ++r)
+      tile_out[(8 * (r >> 2) + 4 * half + (r & 3)) * kPitch + wave * 32 + l32] = (acc[i][r] + add[i][r >> 2][r & 3]) * p.scale;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int row = row0 + k * 8, c = (kg * TX + i) * 32 + row;
+      const v4i v = *reinterpret_cast<const v4i *>(tile_out + row * kPitch + px);
+      const u32 dst = ((u32)(n * p.oc + c) * (u32)p.OHW + (u32)(p0 + px)) * 4u;
+      if (c < p.oc) {
+        if (p0 + px + 3 <= last) {
+          store_result<kRowPolicy>(obuf, dst, v);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 3; ++e)
+            if (p0 + px + e <= last) store_result<kRowPolicy>(obuf, dst + 4u * e, v[e]);
+        }
       }
     }
+  }
 }
 
-// Bytes of LDS of a workgroup of 128 ty pixels and tx channel blocks: the rows that many consecutive pixels can touch.
-size_t planar_c4_lds(const ConvGeom &g, int tx, int ty) {
-  const int span = (128 * ty + g.OW - 2) / g.OW + 1, rows = (span < g.OH ? span : g.OH) - 1;
+// Bytes of LDS of a workgroup of tx channel blocks: the rows that PT consecutive pixels can touch, or a block of results.
+size_t planar_c4_lds(const ConvGeom &g, int tx) {
+  const int span = (PT + g.OW - 2) / g.OW + 1, rows = (span < g.OH ? span : g.OH) - 1;
   const size_t quads = ((size_t)(g.OW - 1) * g.sw + 8 + 3) / 4;
-  return (size_t)tx * (g.KH * 1024 + 128) + ((size_t)rows * g.sh + (size_t)(g.KH - 1) * g.dh + 1) * quads * 16;
-}
-
-template <int TX, int TY, int NC>
-int launch(const PlanarC4 &p, unsigned grid, size_t lds, hipStream_t s) {
-  set_variant("s8stem_nchw_x%d_y%d_c%d", TX * 32, TY * 128, NC);
-  hipLaunchKernelGGL((conv_planar_c4_kernel<TX, TY, NC>), dim3(grid), dim3(256), lds, s, p);
-  hipError_t e = hipGetLastError();
-  return e == hipSuccess ? UNIT_OK
-                         : fail(UNIT_E_LAUNCH, "unit_conv2d_nchw_s8s8s32_fused_prepared: launch: %s", hipGetErrorString(e));
+  const size_t front = (size_t)tx * (g.KH * 1024 + 128) + ((size_t)rows * g.sh + (size_t)(g.KH - 1) * g.dh + 1) * quads * 16;
+  const size_t back = (size_t)32 * (PT + 4) * 4;
+  return front > back ? front : back;
 }
 
 template <int TX>
-int launch_tx(const PlanarC4 &p, int ty, unsigned grid, size_t lds, hipStream_t s) {
-  if (p.C == 3) return ty == 2 ? launch<TX, 2, 3>(p, grid, lds, s) : launch<TX, 1, 3>(p, grid, lds, s);
-  return ty == 2 ? launch<TX, 2, 4>(p, grid, lds, s) : launch<TX, 1, 4>(p, grid, lds, s);
+int launch(const PlanarC4 &p, unsigned grid, size_t lds, hipStream_t s) {
+  const int nc = p.C == 3 ? 3 : 4;
+  set_variant("s8stem_nchw_x%d_y%d_c%d", TX * 32, PT, nc);
+  hipLaunchKernelGGL((nc == 3 ? conv_planar_c4_kernel<TX, 3> : conv_planar_c4_kernel<TX, 4>), dim3(grid), dim3(256), lds, s, p);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? UNIT_OK
+                         : fail(UNIT_E_LAUNCH, "unit_conv2d_nchw_s8s8s32_fused_prepared: launch: %s", hipGetErrorString(e));
 }
 
 }  // namespace
@@ -174,15 +181,13 @@ static int planar_c4_tx(int kblocks) { return kblocks % 3 == 0 ? 3 : kblocks % 2
 
 // Whether the one-launch kernel takes the convolution: rows of at least a word, and a workgroup's patch and weights in 64 KiB.
 bool planar_c4_takes(const ConvGeom &g, int K) {
-  return g.W >= 4 && g.c4_steps == g.KH && planar_c4_lds(g, planar_c4_tx((K + 31) / 32), 1) <= 64 * 1024;
+  return g.W >= 4 && g.c4_steps == g.KH && planar_c4_lds(g, planar_c4_tx((K + 31) / 32)) <= 64 * 1024;
 }
 
 int conv_planar_c4(const unit_conv_desc *d, const ConvGeom &g, int in_channels, const void *x, const void *w, const int *bias,
                    int scale, void *out, int oc, hipStream_t s) {
   const int kblocks = (d->K + 31) / 32, tx = planar_c4_tx(kblocks), groups = kblocks / tx, ohw = g.OH * g.OW;
-  // 256 pixels per workgroup while that leaves two workgroups per CU, else 128
-  const int ty = (long)g.N * ceil_div(ohw, 256) * groups >= 512 && planar_c4_lds(g, tx, 2) <= 64 * 1024 ? 2 : 1;
-  const int tiles = ceil_div(ohw, 128 * ty);
+  const int tiles = ceil_div(ohw, PT);
   PlanarC4 p;
   p.x = static_cast<const char *>(x);
   p.w = static_cast<const char *>(w);
@@ -207,11 +212,11 @@ int conv_planar_c4(const unit_conv_desc *d, const ConvGeom &g, int in_channels, 
   p.by_tiles = FastDiv::make(tiles);
   p.by_kg = FastDiv::make(groups);
   const unsigned grid = (unsigned)((size_t)g.N * tiles * groups);
-  const size_t lds = planar_c4_lds(g, tx, ty);
+  const size_t lds = planar_c4_lds(g, tx);
   switch (tx) {
-    case 3: return launch_tx<3>(p, ty, grid, lds, s);
-    case 2: return launch_tx<2>(p, ty, grid, lds, s);
-    default: return launch_tx<1>(p, ty, grid, lds, s);
+    case 3: return launch<3>(p, grid, lds, s);
+    case 2: return launch<2>(p, grid, lds, s);
+    default: return launch<1>(p, grid, lds, s);
   }
 }
 
