@@ -119,9 +119,14 @@ int run_dense_mixed(const void *a, const void *wp, void *c, int M, int N, int K,
   return e == hipSuccess ? UNIT_OK : fail(UNIT_E_LAUNCH, "%s: launch: %s", what, hipGetErrorString(e));
 }
 
-// An odd number of 64-byte stages on a large result: the staged 256 x 256 tiles for short reductions (the tests name them);
-// 3000 x 3000 x 3008 runs in 52 us on the group tiles against 60.
-inline bool dense_stays_staged(int M, int N, int K) { return K % 128 == 64 && K < 1024 && direct_gemm_large_tiles(M, N); }
+// Row-major weights and a K that the direct tiles do not take, on a large result: the staged 256 x 256 tiles for short
+// reductions of an odd number of 64-byte stages (the tests name them), and where their estimate, 1.15 x that of the direct
+// tiles, is the lower one (8000 x 2048 x 2000, one round of 256 tiles, 48 us against 56; 5000 x 4096 x 2000, two, 84 against 80).
+inline bool dense_stays_staged(int M, int N, int K) {
+  if (K % 128 == 0 || M < 256 || N < 256) return false;
+  if (K % 128 == 64 && K < 1024 && direct_gemm_large_tiles(M, N)) return true;
+  return 1.15f * large_tile_cost(M, N, K) < plan_group(M, N, K, 1, 1, kAtomicSplits).us;
+}
 
 template <bool PACKED>
 int dense(const void *a, const void *w, void *c, int M, int N, int K, unit_stream_t stream) {
@@ -148,8 +153,12 @@ int dense(const void *a, const void *w, void *c, int M, int N, int K, unit_strea
     default: break;
   }
   if constexpr (PACKED) {
-    // the staged 256 x 256 tiles take 1.15 x the time of the direct-to-LDS ones on row-major weights
-    if (M >= 256 && N >= 256 && 1.15f * large_tile_cost(M, N, K) < plan_group(M, N, K, 1, 1, kAtomicSplits).us)
+    // The staged 256 x 256 tiles take 1.1 x the time of the direct-to-LDS ones on row-major weights (1.15 x with a part of a
+    // stage at the end); the 256 x 128 group tile takes 1.3 x its estimate here, whose fragments are four dword reads
+    // each (8192 x 4096 x 1024: 70 us, staged 59; 5000 x 4096 x 2000: 75, staged 81).
+    const GroupPlan group = plan_group(M, N, K, 1, 1, kAtomicSplits);
+    if (M >= 256 && N >= 256 &&
+        (K % 128 ? 1.15f : 1.1f) * large_tile_cost(M, N, K) < group.us * (group.tile == kGroupTiles - 1 ? 1.3f : 1.f))
       return K % 128 ? run_dense_staged<true, true>(a, w, c, M, N, K, s) : run_dense_staged<true, false>(a, w, c, M, N, K, s);
     return run_dense_group<Y_VNNI, WS_Y>(what, "i8densepk", a, w, nullptr, c, M, N, K, s);
   } else {
