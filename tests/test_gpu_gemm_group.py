@@ -38,6 +38,28 @@ def test_fp16_group_tiles(dev, M, N, K, tile):
     assert torch.equal(U.gemm_fp16(a, b, workspace=True).double(), ref), U.last_variant()
 
 
+@pytest.mark.parametrize("M,N,K", [(2900, 2900, 2904), (4096, 4092, 1000), (3000, 3004, 3000)])
+def test_fp16_large_ragged_products_stay_staged(dev, M, N, K):
+    """Large results whose K no direct tile takes: 256 x 256 tiles, with b by columns and prepared."""
+    g = np.random.RandomState(M + N + K)
+    a, b = _ints(g, -3, 4, (M, K), torch.float16, dev), _ints(g, -2, 3, (K, N), torch.float16, dev)
+    ref = a.double() @ b.double()
+    for operand in (b, U.prepare_gemm_b(b)):
+        assert torch.equal(U.gemm_fp16(a, operand).double(), ref)
+        assert "x256_y256" in U.last_variant(), U.last_variant()
+        assert torch.equal(U.gemm_fp16(a, operand, "float16"), ref.half())
+
+
+@pytest.mark.parametrize("M,N,K,packed", [(2048, 8192, 1024, True), (8000, 2048, 2000, True), (8000, 2048, 2000, False)])
+def test_int8_large_products_stay_staged(dev, M, N, K, packed):
+    g = np.random.RandomState(M + N + K)
+    a, w = _ints(g, 0, 256, (M, K), torch.uint8, dev), _ints(g, -128, 128, (N, K), torch.int8, dev)
+    ref = (a.double() @ w.double().t()).to(torch.int32)
+    assert torch.equal(U.dense_dotprod(a, U.prepack_dense_weight(w)) if packed else U.dense(a, w), ref)
+    assert "x256_y256" in U.last_variant(), U.last_variant()
+    assert torch.equal(U.dense(a, U.prepare_dense_weight(w)), ref), U.last_variant()
+
+
 def test_fp16_infinity_past_a_row(dev):
     """What lies behind a row's end (the next row) must not reach the sums: 0 x inf would be NaN."""
     M, N, K = 40, 44, 72

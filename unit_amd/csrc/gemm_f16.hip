@@ -129,6 +129,32 @@ inline bool gemm_keeps_128(int M, int N, bool out_f16) {
   return tiles >= 512 || (tiles >= 192 && tiles <= 256) || (!out_f16 && tiles < 32 && M > 128);
 }
 
+// (N, K) b and a through registers on 256 x 256 tiles: large results with a K that the direct tiles do not take
+template <class T, bool OUT_F16>
+int run_gemm_f16_bt(const void *a, const void *bt, void *c, int M, int N, int K, hipStream_t s) {
+  using XL = RowMajorLoader<T::BX, T::BKB, T::NT, false>;
+  using YL = RowMajorLoader<T::BY, T::BKB, T::NT, false>;
+  using Epi = GemmEpilogue<OpF16, OUT_F16>;
+  typename XL::Params xp{static_cast<const char *>(a), M, K * 2, K * 2};
+  typename YL::Params yp{static_cast<const char *>(bt), N, K * 2, K * 2};
+  typename Epi::Params ep{c, M, N};
+  const int nk = ceil_div(K * 2, T::BKB), gx = ceil_div(M, T::BX), gy = ceil_div(N, T::BY);
+  set_variant("f16gemmbt_x%d_y%d_k%d_w%dx%d%s_s1", T::BX, T::BY, T::BKB, T::WX, T::WY, OUT_F16 ? "_h" : "");
+  return launch_mma<OpF16, T, XL, YL, Epi, WS_NONE>(xp, yp, ep, nk, gx, gy, 4, 1, c, (size_t)M * N * 4, 0, s,
+                                                    "unit_gemm_f16_prepared");
+}
+
+// Large results whose K or N the direct tiles do not take: the 256 x 256 tiles staged through registers take about 9 us
+// + 29 us per 1000 of K for each round of 256 tiles, and `scale` is what the group tiles' estimate falls short by there
+// (power: 1.2 with b by columns, 1.35 with b in rows).  Staged against group, fp32 results: 3000 x 3004 x 3000 94.7 / 100.6 us
+// (b in rows 88.3 / 119.6), 4000 x 4000 x 4008 138 / 156 (135 / 182), 3500 x 3500 x 3000 93 / 114 (95 / 124); the other way
+// 4500 x 4500 x 1496, 324 tiles in two rounds, 108 / 97 (105 / 105).
+inline bool gemm_staged_pays(int M, int N, int K, float scale) {
+  if (M < 256 || N < 256) return false;
+  const long tiles = (long)ceil_div(M, 256) * ceil_div(N, 256);
+  return 2.f + (float)((tiles + 255) / 256) * (9.f + 0.029f * K) < scale * plan_group(M, N, K * 2, 1, 1, kAtomicSplits).us;
+}
+
 template <bool OUT_F16>
 int gemm_f16_bt(const void *a, const void *bt, void *c, int M, int N, int K, hipStream_t s) {
   if (K % 32 == 0 && K >= 64) {  // both operands straight into LDS; tile choice as in gemm_f16 below
@@ -139,6 +165,7 @@ int gemm_f16_bt(const void *a, const void *bt, void *c, int M, int N, int K, hip
     if (gemm_keeps_128(M, N, OUT_F16))
       return run_gemm_f16_bt_dma<Tile<128, 128, 64, 2, 2>, 4, OUT_F16>(a, bt, c, M, N, K, s, direct_gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K));
   }
+  if (gemm_staged_pays(M, N, K, 1.35f)) return run_gemm_f16_bt<Tile<256, 256, 128, 2, 4>, OUT_F16>(a, bt, c, M, N, K, s);
   return run_gemm_f16_group<Y_ROWS, OUT_F16>("unit_gemm_f16_prepared", "f16gemmbt", a, bt, c, M, N, K, s);
 }
 
@@ -220,6 +247,7 @@ int gemm_f16(const void *a, const void *b, void *c, int M, int N, int K, hipStre
   }
   // four columns: less than one 16-byte chunk of a row of b
   if (N < 8) return run_gemm_f16<Tile<128, 128, 64, 2, 2>, OUT_F16>(a, b, c, M, N, K, s, whole);
+  if (gemm_staged_pays(M, N, K, 1.2f)) return run_gemm_f16<Tile<256, 256, 128, 4, 2>, OUT_F16>(a, b, c, M, N, K, s, whole);
   return run_gemm_f16_group<Y_COLS, OUT_F16>("unit_gemm_f16", "f16gemm", a, b, c, M, N, K, s, whole);
 }
 
