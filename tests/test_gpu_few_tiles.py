@@ -47,3 +47,22 @@ def test_fp16(dev, oracle, N, C, H, W, K, ks, stride):
     for weight in (t(b), U.prepare_conv2d_weight(t(b))):
         out = U.conv2d_NCHW16c_OHWI16o(t(a), weight, stride, stride).cpu().numpy()
         assert np.array_equal(out.astype(np.float64), ref) and "_g8_" in U.last_variant(), U.last_variant()
+
+
+@pytest.mark.parametrize("C,H,W,K,KH,KW,tile", [
+    (60, 9, 8, 48, 5, 5, "x32_y32_g8"),    # 75 window rows
+    (1056, 38, 8, 32, 31, 1, "x64_y32_g4"),  # 8184 rows: their table leaves no room for the eight waves' tiles
+    (524, 38, 8, 32, 31, 1, "x32_y32_g8"),   # 4061 rows
+])
+def test_four_channel_blocks(dev, oracle, C, H, W, K, KH, KW, tile):
+    g = np.random.RandomState(C + K)
+    x = g.randint(0, 256, (1, C // 4, H, W, 4)).astype(np.uint8)
+    w = g.randint(-128, 128, (K // 16, C // 4, KH, KW, 1, 16, 4)).astype(np.int8)
+    ref = oracle.c_conv2d_nchwc(x, w, 1, 0, 1)
+    signed = oracle.conv2d_nchwc_int8_fused(x.view(np.int8), w, np.zeros(K, np.int32), 1, 1, 0, 1, conv=oracle.c_conv2d_nchwc)
+    t = lambda a: torch.from_numpy(a).to(dev)
+    for weight in (t(w), U.prepare_conv2d_weight(t(w))):
+        out = U.conv2d_NCHWc_int8(t(x), weight, 1, 0)
+        assert np.array_equal(out.cpu().numpy(), ref) and tile in U.last_variant(), U.last_variant()
+        fused = U.conv2d_NCHWc_int8_fused(t(x.view(np.int8)), weight, None, 1, 1, 0)
+        assert np.array_equal(fused.cpu().numpy(), signed) and tile in U.last_variant(), U.last_variant()

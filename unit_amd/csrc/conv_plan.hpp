@@ -48,8 +48,10 @@ struct TunedConv {
 // layers (few input channels, many pixels) want 64..128-pixel tiles of 64 channels with many
 // workgroups in flight; long reductions want the 128-channel tiles with two stages of loads in
 // flight; the 256 x 256 tiles only pay when they still give every CU several workgroups.
-inline ConvPlan heuristic_plan(int npix, int K, int kbytes, bool allow_split, bool direct_ok, bool strided = false,
+inline ConvPlan heuristic_plan(const unit_conv_desc *d, int npix, int kbytes, bool allow_split, bool direct_ok,
                                bool staged_too = false) {
+  const int K = d->K;
+  const bool strided = d->sh * d->sw > 1;
   const bool k128 = kbytes % 128 == 0;
   const auto tiles = [&](int bx, int by) { return (long)ceil_div(K, bx) * ceil_div(npix, by); };
   if (direct_ok) {
@@ -64,11 +66,13 @@ inline ConvPlan heuristic_plan(int npix, int K, int kbytes, bool allow_split, bo
     // fp16 1168 -> 32, 5 x 5 on 27 x 17, 85 -> 43; the 137 such rows of the tables 901 -> 751 in all.  Below 20 k-steps the
     // sum of eight partial tiles costs what it gains (18: 4.36 against 4.34 us), above 256 tiles the second round does
     // (342 of them: 10.6 -> 8.0, 555: 22.0 -> 21.0, 720: 49.2 -> 51.1).  Up to 32 channels a 64-channel tile is half
-    // padding: 32 x 64 tiles there (480 -> 32 on 76 x 72: 10.6 -> 7.0).  The tap table of 4096 k-steps still fits the LDS.
-    const int ksteps = kbytes / 32;
-    if (ksteps >= 20 && ksteps <= 4096 && tiles(32, 32) <= 256)
+    // padding: 32 x 64 tiles there (480 -> 32 on 76 x 72: 10.6 -> 7.0).  The eight waves' scratch and tile leave the tap
+    // table less of the LDS than the four-wave tiles below do (with 4-channel blocks, a k-step per window row, 7352 rows
+    // against 8528): up to 4096 steps, 64 KiB of table, all of them fit.
+    const int ksteps = kbytes / 32, table_steps = d->cb == 4 ? kbytes / (4 * d->KW) : ksteps;
+    if (ksteps >= 20 && table_steps <= 4096 && tiles(32, 32) <= 256)
       return ConvPlan{82, 1, 4};
-    if (ksteps >= 20 && ksteps <= 4096 && K <= 32 && tiles(32, 64) <= 384)
+    if (ksteps >= 20 && table_steps <= 4096 && K <= 32 && tiles(32, 64) <= 384)
       return ConvPlan{83, 1, 0};
     if (allow_split) {  // the int8 operator; distilled from the tuner's choices on cold operands (batch 1 .. 256)
       const int nsteps = kbytes / 32;
@@ -138,7 +142,7 @@ inline ConvPlan heuristic_plan(int npix, int K, int kbytes, bool allow_split, bo
 
 inline ConvPlan plan_conv(const unit_conv_desc *d, int npix, int kbytes, const TunedConv *table, int ntable,
                           bool allow_split, bool direct_ok, bool staged_too = false, bool lds_ok = false) {
-  ConvPlan p = heuristic_plan(npix, d->K, kbytes, allow_split, direct_ok, d->sh * d->sw > 1, staged_too);
+  ConvPlan p = heuristic_plan(d, npix, kbytes, allow_split, direct_ok, staged_too);
   // UNIT_AMD_CONV_NOTABLE=1: heuristic only (the tuner measures it as the baseline)
   if (tuning_override("UNIT_AMD_CONV_NOTABLE") > 0) ntable = 0;
   for (int i = 0; i < ntable; ++i) {
@@ -167,7 +171,7 @@ inline ConvPlan plan_conv(const unit_conv_desc *d, int npix, int kbytes, const T
   if (!allow_split) p.splits = 1;
   // the LDS-shared variants exist for prepared weights with 16-channel blocks only: elsewhere their ids run the heuristic's choice
   if (kConvTiles[p.variant].lds && !lds_ok) {
-    const ConvPlan h = heuristic_plan(npix, d->K, kbytes, allow_split, direct_ok, d->sh * d->sw > 1, staged_too);
+    const ConvPlan h = heuristic_plan(d, npix, kbytes, allow_split, direct_ok, staged_too);
     p.variant = h.variant;
     if (!allow_split) p.splits = 1;
   }

@@ -138,7 +138,7 @@ ConvPlan plan_prepared(const unit_conv_desc *d, const ConvGeom &g, int kbytes, c
   lds_ok = lds_ok && d->cb == 16 && d->KH * d->KW <= 31;
   ConvPlan p = plan_conv(d, g.npix, kbytes, table, ntable, int8, true, false, lds_ok);
   const TileShape &t = kConvTiles[p.variant];
-  if (!(t.direct || (t.lds && lds_ok))) p = heuristic_plan(g.npix, d->K, kbytes, int8, true, d->sh * d->sw > 1);
+  if (!(t.direct || (t.lds && lds_ok))) p = heuristic_plan(d, g.npix, kbytes, int8, true);
   p.splits = 1;
   return p;
 }
