@@ -75,6 +75,28 @@ def test_chain_follows_replaced_buffers(dev, oracle):
     assert torch.equal(kept, old[1]) and not torch.equal(c.outputs[2], old[2])
 
 
+def test_chain_follows_replaced_descriptors(dev, oracle, monkeypatch):
+    layers_np = _small_layers()
+    x = rng.uniform_u8((3, 1, 13, 11, 16), 9)
+    c = chain.ConvChain(_to_chain(layers_np, dev), x.shape)
+    c(_t(x, dev))
+    first = list(c.variants)
+    w, b, scale, shift, stride, _, source = layers_np[2]
+    for pads in ((2, 2, 0, 0), (0, 2, 2, 0)):  # as many output pixels from another place: a new descriptor, then a changed one
+        layers_np[2] = (w, b, scale, shift, stride, pads, source)
+        if pads[0]:
+            c.descs[2] = type(c.descs[2]).from_buffer_copy(c.descs[2])
+        c.descs[2].pt, c.descs[2].pl, c.descs[2].pb, c.descs[2].pr = pads
+        c(_t(x, dev))
+        for i, (got, want) in enumerate(zip(c.outputs, _oracle_chain(oracle, layers_np, x))):
+            assert np.array_equal(got.cpu().numpy(), want), (pads, i)
+    assert c.variants == first
+    monkeypatch.setenv("UNIT_AMD_CONV_VARIANT", "51")
+    c.variants[2] = None  # asks for the kernel's name again
+    c(_t(x, dev))
+    assert "x64_y64_g1_d4" in c.variants[2] and c.variants[:2] + c.variants[3:] == first[:2] + first[3:]
+
+
 def test_chain_graph_replay_follows_the_input(dev, oracle):
     layers_np = _small_layers()[:3]
     x1 = rng.uniform_u8((2, 1, 9, 9, 16), 8)

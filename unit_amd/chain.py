@@ -73,21 +73,20 @@ class ConvChain:
         if not self.outputs:
             raise ValueError("layers: empty chain")
         self.variants = [None] * len(self.outputs)
-        # the whole chain as one call of the library: the host then spends a launch's 2.5 us per layer, not 8
-        count = len(self.outputs)
-        self._names = ctypes.create_string_buffer(96 * count)  # kernel names, written by the first run
-        self._native = (ChainLayerDesc * count)()
-        for i, d in enumerate(self._native):
-            d.desc = self.descs[i]
-            d.variant = ctypes.addressof(self._names) + 96 * i
-        self._bound = None
+        self._native, self._bound = (), None
 
     def _bind(self):
-        """Buffers and constants as they are now: a caller may have put other ones into the lists."""
+        """The layers for the library, which runs them all in one call (the host then spends a launch's 2.5 us per layer,
+        not 8): descriptors, buffers and constants as they are now, since a caller may have put other ones into the lists."""
+        count = len(self.outputs)
+        if len(self._native) != count:
+            self._native, self._bound = (ChainLayerDesc * count)(), None
+            self._names = ctypes.create_string_buffer(96 * count)  # kernel names, where self.variants has none yet
         bound = [(w.buf.data_ptr(), o.data_ptr(), None if b is None else b.data_ptr(), *c, src)
                  for w, o, b, c, src in zip(self.weights, self.outputs, self.biases, self.consts, self.sources)]
+        bound.append(b"".join(self.descs))
         if bound != self._bound:
-            for d, (d.prepared, d.out, d.bias, d.scale, d.shift, src) in zip(self._native, bound):
+            for d, d.desc, (d.prepared, d.out, d.bias, d.scale, d.shift, src) in zip(self._native, self.descs, bound):
                 d.data = None if src < 0 else bound[src][1]
             self._bound = bound
 
@@ -96,11 +95,13 @@ class ConvChain:
         if tuple(x.shape) != self.input_shape:
             raise ValueError(f"x: expected {self.input_shape}, got {tuple(x.shape)}")
         self._bind()
+        unnamed = [i for i, v in enumerate(self.variants) if v is None]
+        for i in unnamed:
+            self._native[i].variant = ctypes.addressof(self._names) + 96 * i
         check(self._L.unit_conv_chain_u8(self._native, len(self._native), x.data_ptr(), ops._stream()))
-        if None in self.variants:
-            self.variants = [self._names[96 * i:96 * i + 96].split(b"\0")[0].decode() for i in range(len(self._native))]
-            for d in self._native:
-                d.variant = None
+        for i in unnamed:
+            self.variants[i] = self._names[96 * i:96 * i + 96].split(b"\0")[0].decode()
+            self._native[i].variant = None
         return self.outputs[-1]
 
     def source_of(self, i, x):
