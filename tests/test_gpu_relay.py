@@ -167,3 +167,25 @@ def test_image_stem_in_one_launch(dev, n, ic, h, w, oc, kh, kw, stride, padding,
     assert "stem" in U.last_variant(), U.last_variant()
     assert np.array_equal(got.cpu().numpy(), want), U.last_variant()
     assert torch.equal(g(room[1:].view(x.shape), fold_output_transform=False), got)
+
+
+@pytest.mark.parametrize("n,ic,h,w,oc,k,stride,padding,dilation,stem", [
+    (1024, 3, 4, 4, 40, 3, 1, 1, 1, True),    # 16 pixels per image, as many workgroups as always win
+    (1025, 3, 4, 4, 40, 3, 1, 1, 1, False),   # one more
+    (520, 3, 12, 12, 40, 3, 1, 1, 1, False),  # 144 pixels in two workgroups
+    (520, 3, 13, 13, 40, 3, 1, 1, 1, True),   # 169: planes that 64-byte stores do not fit
+    (520, 3, 12, 12, 40, 5, 1, 2, 1, True),   # five window rows
+    (1025, 1, 8, 6, 20, 3, 1, 1, 1, True),    # 48 pixels, one block of channels
+    (1025, 1, 6, 6, 20, 3, 1, 1, 1, False),   # 36
+    (24, 3, 64, 762, 32, 7, 2, 3, 1, True),   # rows of 381 results: a patch of 27 KiB
+    (24, 3, 64, 763, 32, 7, 2, 3, 1, False),  # 382
+])
+def test_image_stem_rule(dev, n, ic, h, w, oc, k, stride, padding, dilation, stem):
+    x, wt, b = rng.uniform_s8((n, ic, h, w), h), rng.uniform_s8((oc, ic, k, k), w), _i32((oc,), 13, -5000, 5000)
+    g = relay.Conv2dBiasMultiply(torch.from_numpy(wt).to(dev), torch.from_numpy(b).to(dev), 7, stride, padding, dilation)
+    got = g(torch.from_numpy(x).to(dev)).clone()
+    assert ("stem" in U.last_variant()) == stem, U.last_variant()
+    ends = np.concatenate([x[:2], x[-2:]])  # the first and last images; all of them against the layout-by-layout graph
+    want = _plain_graph(np.pad(ends, ((0, 0), (0, 0), (padding,) * 2, (padding,) * 2)), wt, b, 7, stride, 0, dilation)
+    assert np.array_equal(got[[0, 1, -2, -1]].cpu().numpy(), want), U.last_variant()
+    assert torch.equal(g(torch.from_numpy(x).to(dev), fold_output_transform=False), got)

@@ -155,12 +155,16 @@ __global__ __launch_bounds__(256) void conv_planar_c4_kernel(PlanarC4 p) {
   }
 }
 
-// Bytes of LDS of a workgroup of tx channel blocks: the rows that PT consecutive pixels can touch, or a block of results.
-size_t planar_c4_lds(const ConvGeom &g, int tx) {
+// Bytes of the patch: the input rows that PT consecutive pixels can touch.
+size_t planar_c4_patch(const ConvGeom &g) {
   const int span = (PT + g.OW - 2) / g.OW + 1, rows = (span < g.OH ? span : g.OH) - 1;
   const size_t quads = ((size_t)(g.OW - 1) * g.sw + 8 + 3) / 4;
-  const size_t front = (size_t)tx * (g.KH * 1024 + 128) + ((size_t)rows * g.sh + (size_t)(g.KH - 1) * g.dh + 1) * quads * 16;
-  const size_t back = (size_t)32 * (PT + 4) * 4;
+  return ((size_t)rows * g.sh + (size_t)(g.KH - 1) * g.dh + 1) * quads * 16;
+}
+
+// Bytes of LDS of a workgroup of tx channel blocks: weights, biases and patch, or a block of results.
+size_t planar_c4_lds(const ConvGeom &g, int tx) {
+  const size_t front = (size_t)tx * (g.KH * 1024 + 128) + planar_c4_patch(g), back = (size_t)32 * (PT + 4) * 4;
   return front > back ? front : back;
 }
 
@@ -180,8 +184,21 @@ int launch(const PlanarC4 &p, unsigned grid, size_t lds, hipStream_t s) {
 static int planar_c4_tx(int kblocks) { return kblocks % 3 == 0 ? 3 : kblocks % 2 == 0 ? 2 : 1; }
 
 // Whether the one-launch kernel takes the convolution: rows of at least a word, and a workgroup's patch and weights in 64 KiB.
+// Up to 1024 workgroups, four per CU, it always wins, by the launch it saves.  Past that a workgroup costs about the same
+// however many of its 128 pixels exist and however wide the rows are that it lays out for them.  How many pixels may be
+// missing goes by what the kernel on a packed copy loses there (us here / there): 1.3 for 1 in general (64 channels, 3 x 3,
+// 39062 images of 16 pixels 135 / 32, 9765 of 64 41.6 / 32.8, 4340 of 144 44.3 / 31.2, 1562 of 400 35.3 / 30.8), 1.55 where its
+// 64-byte stores do not fit the planes (3698 of 169 45.0 / 53.2), 2 with five or more window rows, a masked gather each there
+// (7 x 7, 9765 of 64 49.8 / 55.9, 17361 of 36 81.2 / 60.6), 2.7 where half of its 64-channel tile is padding (32 channels, 25510
+// of 49 58.5 / 70.9, 34722 of 36 71.5 / 66.3).  The patch may have 27 KiB (7 x 7 stride 2 on rows of 320 results, 23 KB,
+// 44.7 / 47.5, on 384, 28 KB, 48.8 / 47.1, on 640 60.6 / 47.1; 3 x 3 stride 2 on 640, 26 KB, 33.4 / 37.3, on 1024, 41 KB,
+// 46.3 / 38.3).
 bool planar_c4_takes(const ConvGeom &g, int K) {
-  return g.W >= 4 && g.c4_steps == g.KH && planar_c4_lds(g, planar_c4_tx((K + 31) / 32)) <= 64 * 1024;
+  const int kblocks = (K + 31) / 32, tx = planar_c4_tx(kblocks);
+  if (g.W < 4 || g.c4_steps != g.KH || planar_c4_lds(g, tx) > 64 * 1024) return false;
+  const long pixels = (long)g.OH * g.OW, tiles = (pixels + PT - 1) / PT;
+  const int slack = kblocks == 1 ? 270 : g.KH >= 5 ? 200 : pixels % 16 ? 155 : 130;
+  return tiles * g.N * (kblocks / tx) <= 1024 || (tiles * PT * 100 <= pixels * slack && planar_c4_patch(g) <= 27 * 1024);
 }
 
 int conv_planar_c4(const unit_conv_desc *d, const ConvGeom &g, int in_channels, const void *x, const void *w, const int *bias,
