@@ -93,6 +93,9 @@ def test_pinned_k_splits(dev, monkeypatch, splits):
     for operand in (w, U.prepare_dense_weight(w)):
         assert torch.equal(U.dense(a, operand), ref), U.last_variant()
         assert U.last_variant().endswith(f"_s{splits}")
+    w = _ints(g, -128, 128, (256, K), torch.int8, dev)  # packed: K ends inside a stage, the next block's weights follow
+    assert torch.equal(U.dense_dotprod(a, U.prepack_dense_weight(w)), (a.double() @ w.double().t()).to(torch.int32))
+    assert U.last_variant().endswith(f"_s{splits}")
     h, b = _ints(g, -3, 4, (M, K), torch.float16, dev), _ints(g, -2, 3, (K, N), torch.float16, dev)
     ref = h.double() @ b.double()
     for ws in (None, True):
