@@ -6,6 +6,7 @@ import pytest
 import torch
 
 import unit_amd as U
+from unit_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -112,3 +113,27 @@ def test_fp16_without_planes_runs_whole(dev, M, N, K):
     a, b = _ints(g, -3, 4, (M, K), torch.float16, dev), _ints(g, -2, 3, (K, N), torch.float16, dev)
     assert torch.equal(U.gemm_fp16(a, b, workspace=True).double(), a.double() @ b.double())
     assert U.last_variant().endswith("_s1") or "_s" not in U.last_variant(), U.last_variant()
+
+
+@pytest.mark.parametrize("M,N,K,layout,splits", [
+    (512, 516, 12304, "row_major", 3), (512, 516, 12304, "prepared", 3), (2, 3968, 8800, "packed", 1),
+    (2, 3968, 8800, "row_major", 1), (700, 128, 12304, "packed", 9), (1, 128, 16384, "packed", 13),
+    (1, 128, 16400, "packed", 13), (130, 384, 16400, "packed", 6),
+])
+def test_int8_automatic_splits(dev, M, N, K, layout, splits):
+    """Where int8 products share a long reduction between workgroups by themselves.  The result starts as garbage: the
+    splits add into what their launch has cleared."""
+    g = np.random.RandomState(M + N + K)
+    a, w = _ints(g, 0, 256, (M, K), torch.uint8, dev), _ints(g, -128, 128, (N, K), torch.int8, dev)
+    out = torch.full((M, N), 0x5a5a5a5a, dtype=torch.int32, device=dev)
+    L, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    if layout == "packed":
+        wp = U.prepack_dense_weight(w)
+        _lib.check(L.unit_dense_dotprod_u8s8s32(a.data_ptr(), wp.data_ptr(), out.data_ptr(), M, N, K, stream))
+    elif layout == "prepared":
+        p = U.prepare_dense_weight(w)
+        _lib.check(L.unit_dense_u8s8s32_prepared(a.data_ptr(), p.w.data_ptr(), p.wsum.data_ptr(), out.data_ptr(), M, N, K, stream))
+    else:
+        _lib.check(L.unit_dense_u8s8s32(a.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, stream))
+    assert torch.equal(out, (a.double() @ w.double().t()).to(torch.int32)), U.last_variant()
+    assert U.last_variant().endswith(f"_s{splits}"), U.last_variant()

@@ -33,16 +33,21 @@ int run_dense_staged(const void *a, const void *w, void *c, int M, int N, int K,
 }
 
 // Tiles of at most 256 x 128 with the reduction shared inside the workgroup (gemm_group.hpp).  Sharing it between
-// workgroups as well (int32 atomics into the zero-filled output, exact) never won below 8 KiB of reduction; the
-// row-major operator shares at least two ways where it has fewer than 12 tiles of 128 x 128 and 1 KiB of reduction
-// (its tests ask for that; 50 x 260 x 1040 would run 2 us faster without).
+// workgroups as well (int32 atomics into the zero-filled output, exact) costs a launch: it pays from 8 KiB of reduction on
+// where the estimate without it is 15 us or more (512 x 516 x 12304 30.8 us whole, 20.0 in three ranges; 2081 x 128 x 10208
+// 25.7 and 16.4; 2 x 3968 x 8800, estimate 12.6, 9.4 whole and 11.8 in three).  The row-major operator shares at least two
+// ways where it has fewer than 12 tiles of 128 x 128 and 1 KiB of reduction (its tests ask for that; 50 x 260 x 1040 would
+// run 2 us faster without).
 template <int YM, int WS>
 int run_dense_group(const char *what, const char *tag, const void *a, const void *w, const int *wsum, void *c, int M, int N,
                     int K, hipStream_t s) {
   const int forced = tuning_override("UNIT_AMD_DENSE_SPLITK");
-  const int least = YM == Y_ROWS && tiles_of_128(M, N) < 12 && K >= 1024 ? 2 : 1;
-  GroupPlan plan = plan_group(M, N, K, forced > 0 ? 1 : least, forced <= 0 && K >= 16384 ? 16 : 1, kAtomicSplits);
-  if (forced > 0) plan.splits = forced;
+  const int least = forced <= 0 && YM == Y_ROWS && tiles_of_128(M, N) < 12 && K >= 1024 ? 2 : 1;
+  GroupPlan plan = plan_group(M, N, K, least, 1, kAtomicSplits);
+  if (forced > 0)
+    plan.splits = forced;
+  else if (K >= 8192 && plan.us >= 15.f)
+    plan = plan_group(M, N, K, least, 16, kAtomicSplits);
   const GroupGemm p{static_cast<const char *>(a), static_cast<const char *>(w), (u32)((size_t)M * K), (u32)((size_t)N * K),
                     M, N, K, K, wsum, c, C_ATOMIC, 0};
   return run_group_plan<OpI8, YM, WS, false>(what, tag, p, plan, s);
