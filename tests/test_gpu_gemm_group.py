@@ -137,3 +137,13 @@ def test_int8_automatic_splits(dev, M, N, K, layout, splits):
         _lib.check(L.unit_dense_u8s8s32(a.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, stream))
     assert torch.equal(out, (a.double() @ w.double().t()).to(torch.int32)), U.last_variant()
     assert U.last_variant().endswith(f"_s{splits}"), U.last_variant()
+
+
+@pytest.mark.parametrize("M,N,K", [(733, 1600, 7616), (69, 8964, 5472), (1030, 1024, 6016)])
+def test_fp32_results_of_more_than_64_tiles_are_reproducible(dev, M, N, K):
+    g = torch.Generator(device=dev).manual_seed(M)
+    a, b = torch.randn((M, K), device=dev, generator=g).half(), torch.randn((K, N), device=dev, generator=g).half()
+    for operand in (b, U.prepare_gemm_b(b)):
+        first = U.gemm_fp16(a, operand)
+        assert U.last_variant().endswith("_s1"), U.last_variant()
+        assert torch.equal(U.gemm_fp16(a, operand), first)

@@ -104,15 +104,18 @@ int run_gemm_f16_hybrid(const void *a, const void *b, void *c, int M, int N, int
 }
 
 // Tiles of at most 256 x 128 with the reduction shared inside the workgroup (gemm_group.hpp), any K and N the
-// operator takes (b by columns: N >= 8).  fp32 results may also share it between workgroups (atomics into the zero-filled
-// output), and do at least two ways with fewer than 12 tiles of 128 x 128 and 1 KiB of reduction (the tests ask for that;
-// 300 x 260 x 520 would run 2 us faster without); fp16 results keep one workgroup per tile.
+// operator takes (b by columns: N >= 8).  fp32 results of up to 64 tiles of 128 x 128 may also share it between workgroups
+// (atomics into the zero-filled output); with more tiles they are the same bits from run to run, although up to 127 a long
+// reduction would gain (900 x 1096 x 7536, 72 tiles, by 19 % in the estimate): unit_gemm_f16_ws has planes for those.  With
+// fewer than 12 such tiles and 1 KiB of reduction at least two ways (the tests ask for that; 300 x 260 x 520 would run 2 us
+// faster without).  fp16 results keep one workgroup per tile.
 template <int YM, bool OUT_F16>
 int run_gemm_f16_group(const char *what, const char *tag, const void *a, const void *b, void *c, int M, int N, int K,
                        hipStream_t s, bool whole = false) {
   const int forced = OUT_F16 || whole ? 1 : tuning_override("UNIT_AMD_GEMM_F16_SPLITK");
-  const int least = forced <= 0 && tiles_of_128(M, N) < 12 && K >= 512 ? 2 : 1;
-  GroupPlan plan = plan_group(M, N, K * 2, least, forced > 0 ? 1 : 19, kAtomicSplits);
+  const long tiles = tiles_of_128(M, N);
+  const int least = forced <= 0 && tiles < 12 && K >= 512 ? 2 : 1;
+  GroupPlan plan = plan_group(M, N, K * 2, least, forced > 0 || tiles > 64 ? 1 : 19, kAtomicSplits);
   if (forced > 0) plan.splits = forced;
   const GroupGemm p{static_cast<const char *>(a), static_cast<const char *>(b), (u32)((size_t)M * K * 2),
                     (u32)((size_t)N * K * 2), M, N, K * 2, YM == Y_COLS ? N * 2 : K * 2, nullptr, c, C_ATOMIC, 0};
