@@ -147,3 +147,27 @@ def test_fp32_results_of_more_than_64_tiles_are_reproducible(dev, M, N, K):
         first = U.gemm_fp16(a, operand)
         assert U.last_variant().endswith("_s1"), U.last_variant()
         assert torch.equal(U.gemm_fp16(a, operand), first)
+
+
+def test_pins_reach_the_large_staged_tiles(dev, monkeypatch):
+    M, N, K = 520, 640, 656
+    g = np.random.RandomState(5)
+    a, w = _ints(g, 0, 256, (M, K), torch.uint8, dev), _ints(g, -128, 128, (N, K), torch.int8, dev)
+    h, b = _ints(g, -3, 4, (M, K), torch.float16, dev), _ints(g, -2, 3, (K, N), torch.float16, dev)
+    ref = (a.double() @ w.double().t()).to(torch.int32)
+    monkeypatch.setenv("UNIT_AMD_DENSE_SPLITK", "2")
+    monkeypatch.setenv("UNIT_AMD_GEMM_F16_SPLITK", "2")
+    monkeypatch.setenv("UNIT_AMD_DENSE_VARIANT", "14")
+    for call in (lambda: U.dense(a, w), lambda: U.dense_dotprod(a, U.prepack_dense_weight(w))):
+        assert torch.equal(call(), ref)
+        assert "x256_y256" in U.last_variant() and U.last_variant().endswith("_s2"), U.last_variant()
+    for pin, name in (("4", "x256_y256_k128_w4x2"), ("7", ""), ("8", "hybrid_x256_y256_k128_w2x4"), ("9", "hybrid_x256_y128_k128_w2x2")):
+        monkeypatch.setenv("UNIT_AMD_GEMM_F16_VARIANT", pin)
+        k = K if pin == "4" else 640  # the hybrid tiles take whole stages
+        assert torch.equal(U.gemm_fp16(h[:, :k].contiguous(), b[:k].contiguous()).double(), h[:, :k].double() @ b[:k].double())
+        assert name in U.last_variant() and (pin != "7" or "hybrid" not in U.last_variant()), U.last_variant()
+    monkeypatch.delenv("UNIT_AMD_GEMM_F16_VARIANT")
+    m, n, k = 2900, 2900, 2904  # stays on staged tiles
+    x, y = _ints(g, -3, 4, (m, k), torch.float16, dev), _ints(g, -2, 3, (k, n), torch.float16, dev)
+    assert torch.equal(U.gemm_fp16(x, U.prepare_gemm_b(y)).double(), x.double() @ y.double())
+    assert "x256_y256" in U.last_variant() and U.last_variant().endswith("_s2"), U.last_variant()

@@ -142,8 +142,9 @@ int run_gemm_f16_bt(const void *a, const void *bt, void *c, int M, int N, int K,
   typename YL::Params yp{static_cast<const char *>(bt), N, K * 2, K * 2};
   typename Epi::Params ep{c, M, N};
   const int nk = ceil_div(K * 2, T::BKB), gx = ceil_div(M, T::BX), gy = ceil_div(N, T::BY);
-  set_variant("f16gemmbt_x%d_y%d_k%d_w%dx%d%s_s1", T::BX, T::BY, T::BKB, T::WX, T::WY, OUT_F16 ? "_h" : "");
-  return launch_mma<OpF16, T, XL, YL, Epi, WS_NONE>(xp, yp, ep, nk, gx, gy, 4, 1, c, (size_t)M * N * 4, 0, s,
+  const int splits = OUT_F16 ? 1 : pinned_k_splits("UNIT_AMD_GEMM_F16_SPLITK", nk);
+  set_variant("f16gemmbt_x%d_y%d_k%d_w%dx%d%s_s%d", T::BX, T::BY, T::BKB, T::WX, T::WY, OUT_F16 ? "_h" : "", splits);
+  return launch_mma<OpF16, T, XL, YL, Epi, WS_NONE>(xp, yp, ep, nk, gx, gy, 4, splits, c, (size_t)M * N * 4, 0, s,
                                                     "unit_gemm_f16_prepared");
 }
 
@@ -218,9 +219,12 @@ int run_gemm_f16(const void *a, const void *b, void *c, int M, int N, int K, hip
 // come here when they plan no planes; k-splits added by atomics would end in another order each time)
 template <bool OUT_F16>
 int gemm_f16(const void *a, const void *b, void *c, int M, int N, int K, hipStream_t s, bool whole = false) {
-  // UNIT_AMD_GEMM_F16_VARIANT pins a kernel per process where it can run (measurement aid)
+  // UNIT_AMD_GEMM_F16_VARIANT pins a kernel per process where it can run (measurement aid); a number without a kernel (any
+  // more) leaves the choice to the rules
   switch (tuning_override("UNIT_AMD_GEMM_F16_VARIANT")) {
-    case 7: if (K % 64 == 0 && K >= 128) return run_gemm_f16_hybrid<Tile<256, 256, 128, 2, 4>, OUT_F16>(a, b, c, M, N, K, s); break;
+    case 4: return run_gemm_f16<Tile<256, 256, 128, 4, 2>, OUT_F16>(a, b, c, M, N, K, s, whole);
+    case 8: if (K % 64 == 0 && K >= 128) return run_gemm_f16_hybrid<Tile<256, 256, 128, 2, 4>, OUT_F16>(a, b, c, M, N, K, s); break;
+    case 9: if (K % 64 == 0 && K >= 128) return run_gemm_f16_hybrid<Tile<256, 128, 128, 2, 2>, OUT_F16>(a, b, c, M, N, K, s); break;
     case 10: if (K % 64 == 0 && K >= 128 && N % 8 == 0) return run_gemm_f16_dma_tr<Tile<256, 256, 128, 2, 4>, 2, OUT_F16>(a, b, c, M, N, K, s); break;
     case 11: if (K % 32 == 0 && K >= 128 && N % 8 == 0) return run_gemm_f16_dma_tr<Tile<256, 256, 64, 2, 4>, 4, OUT_F16>(a, b, c, M, N, K, s); break;
     case 15: if (K % 32 == 0 && K >= 128 && N % 8 == 0) return run_gemm_f16_dma_tr<Tile<128, 128, 64, 2, 2>, 4, OUT_F16>(a, b, c, M, N, K, s); break;

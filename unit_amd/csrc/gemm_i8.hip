@@ -27,8 +27,10 @@ int run_dense_staged(const void *a, const void *w, void *c, int M, int N, int K,
     yp = {static_cast<const char *>(w), N, K, K};
   typename Epi::Params ep{c, M, N};
   const int nk = ceil_div(K, T::BKB), gx = ceil_div(M, T::BX), gy = ceil_div(N, T::BY);
-  set_variant("i8dense%s_x%d_y%d_k%d_w%d%s_s1", PACKED ? "pk" : "rm", T::BX, T::BY, T::BKB, T::NT / 64, TAIL ? "" : "e");
-  return launch_mma<OpI8, T, XL, YL, Epi, WS_Y>(xp, yp, ep, nk, gx, gy, 4, 1, c, (size_t)M * N * 4, 0, s,
+  const int splits = pinned_k_splits("UNIT_AMD_DENSE_SPLITK", nk);
+  set_variant("i8dense%s_x%d_y%d_k%d_w%d%s_s%d", PACKED ? "pk" : "rm", T::BX, T::BY, T::BKB, T::NT / 64, TAIL ? "" : "e",
+              splits);
+  return launch_mma<OpI8, T, XL, YL, Epi, WS_Y>(xp, yp, ep, nk, gx, gy, 4, splits, c, (size_t)M * N * 4, 0, s,
                                                 PACKED ? "unit_dense_dotprod_u8s8s32" : "unit_dense_u8s8s32");
 }
 
@@ -150,9 +152,11 @@ int dense(const void *a, const void *w, void *c, int M, int N, int K, unit_strea
   if (int rc = check_aligned(what, {a, w, c})) return rc;
   if (int rc = check_device()) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  switch (tuning_override("UNIT_AMD_DENSE_VARIANT")) {  // measurement aid: pins a kernel where it can run
+  // measurement aid: pins a kernel where it can run; a number without a kernel (any more) leaves the choice to the rules
+  switch (tuning_override("UNIT_AMD_DENSE_VARIANT")) {
     case 12: if (!PACKED && K % 128 == 0) return run_dense_dma<Tile<256, 256, 128, 2, 4>, 2>(a, w, c, M, N, K, s); break;
     case 13: if (PACKED) return run_dense_mixed(a, w, c, M, N, K, s); break;
+    case 14: return run_dense_staged<PACKED, true>(a, w, c, M, N, K, s);
     case 16: if (!PACKED && K % 128 == 0) return run_dense_dma<Tile<256, 256, 128, 4, 2>, 2>(a, w, c, M, N, K, s); break;
     case 17: if (!PACKED && K % 64 == 0) return run_dense_dma<Tile<128, 128, 64, 2, 2>, 4>(a, w, c, M, N, K, s); break;
     default: break;

@@ -165,6 +165,12 @@ inline int gemm_k_splits(const char *env, int M, int N, long kbytes, int nk) {
   return splits < 1 ? 1 : (splits > nk ? nk : splits);
 }
 
+// The pinned count alone (1 when unset), for tiles that fill the chip by themselves.
+inline int pinned_k_splits(const char *env, int nk) {
+  const int splits = tuning_override(env);
+  return splits < 1 ? 1 : (splits > nk ? nk : splits);
+}
+
 // Which all-direct GEMM tile (both operands global -> LDS): 256 x 256 (eight waves, one workgroup per CU, the least LDS
 // traffic per MFMA) or 128 x 128 (four waves, two workgroups per CU).  Measured time per 2048 reduction bytes (fp16):
 // a round of large tiles 30 us (24 when under 200 CUs are busy), a round of 512 small tiles 21.5 us, 13 us when at
