@@ -149,6 +149,22 @@ def test_gemm_planes_fit_the_library_scratch():
         assert nbytes.value <= 16 << 20, (m, n, k, nbytes.value)
 
 
+def test_plain_fp16_convolution_is_checked_before_anything_runs():
+    """Descriptors that the convolution rejects are rejected before the launch that re-lays the operands: an image whose
+    pixel count passes 31 bits, an image past 2^31 bytes, padding, dilation, a result past 2^31 bytes."""
+    from unit_amd import _lib
+    lib = _lib.load()
+    p = ctypes.c_void_p(4096)  # never read
+    ok = dict(N=1, C=16, H=8, W=8, K=16, KH=3, KW=3, sh=1, sw=1, pt=0, pl=0, pb=0, pr=0, dh=1, dw=1, cb=16)
+    for bad in (dict(H=50000, W=50000), dict(H=16000, W=16000), dict(pt=1), dict(dw=2), dict(H=5000, W=5000, K=32),
+                dict(H=2), dict(sh=0), dict(C=24), dict(N=1 << 24, H=64, W=64, sh=8, sw=8)):
+        d = _lib.ConvDesc(**{**ok, **bad})
+        assert lib.unit_conv2d_nchw_f16f32(ctypes.byref(d), p, p, p, p, 1 << 50, None) == -1, bad
+        nbytes = ctypes.c_size_t()
+        if d.N == 1:
+            assert lib.unit_conv2d_nchw_f16f32_ws_bytes(ctypes.byref(d), ctypes.byref(nbytes)) == -1, bad
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     from unit_amd import _lib
     monkeypatch.setattr(_lib, "_lib", None)

@@ -11,6 +11,9 @@
 #include "mma_core.hpp"
 
 namespace unit {
+
+int conv_geom(const unit_conv_desc *d, int tapb, ConvGeom *g, const char *what);  // abi.hip
+
 namespace {
 
 typedef int halves8_t __attribute__((ext_vector_type(4), aligned(2)));  // plain operands may start at any element
@@ -86,12 +89,20 @@ struct NchwF16Sizes {
   size_t packed, prepared, total;  // bytes; the prepared weights follow the packed data
 };
 
+// Checks the descriptor for everything that the convolution rejects -- the operands are re-laid before it runs -- and
+// gives the sizes.  The batch may need slices, an image not.
 int nchw_f16_sizes(const char *what, const unit_conv_desc *d, NchwF16Sizes *z) {
   if (d->N <= 0 || d->C <= 0 || d->H <= 0 || d->W <= 0 || d->K <= 0 || d->KH <= 0 || d->KW <= 0)
     return fail(UNIT_E_ARG, "%s: N, C, H, W, K, KH, KW must be positive", what);
   if (d->cb != 16 || d->C % 16 || d->K % 16)
     return fail(UNIT_E_ARG, "%s: C and K must be multiples of 16 and cb 16 (got %d, %d, %d)", what, d->C, d->K, d->cb);
-  if (!fits((size_t)d->K * d->C * d->KH * d->KW * 2)) return fail(UNIT_E_ARG, "%s: tensor exceeds 2^31-1 bytes", what);
+  if (d->pt || d->pl || d->pb || d->pr) return fail(UNIT_E_ARG, "%s: the operator has no padding argument; pre-pad the data", what);
+  if (d->dh != 1 || d->dw != 1) return fail(UNIT_E_ARG, "%s: dilation must be 1", what);
+  unit_conv_desc image = *d;
+  image.N = 1;
+  ConvGeom g;
+  if (int rc = conv_geom(&image, 32, &g, what)) return rc;
+  if (!fits((size_t)g.npix * d->K * 4)) return fail(UNIT_E_ARG, "%s: tensor exceeds 2^31-1 bytes", what);
   z->packed = ((size_t)d->N * d->C * d->H * d->W * 2 + 255) / 256 * 256;
   z->prepared = prepared_layout(d->K, d->C, d->KH, d->KW, 16, 2).total_bytes;
   if (!fits(z->prepared)) return fail(UNIT_E_ARG, "%s: tensor exceeds 2^31-1 bytes", what);
@@ -119,17 +130,15 @@ extern "C" int unit_conv2d_nchw_f16f32(const unit_conv_desc *d, const void *a, c
   if (!d || !a || !b || !out || !workspace) return fail(UNIT_E_ARG, "%s: null pointer", what);
   NchwF16Sizes z;
   if (int rc = nchw_f16_sizes(what, d, &z)) return rc;
-  int32_t OH, OW;
-  if (int rc = unit_conv_out_hw(d, &OH, &OW)) return rc;
   if (workspace_bytes < z.total)
     return fail(UNIT_E_ARG, "%s: workspace of %zu bytes needed (got %zu)", what, z.total, workspace_bytes);
   if (int rc = check_aligned(what, {out, workspace})) return rc;
-  if (int rc = check_device()) return rc;
   const int cc = d->C / 16, HW = d->H * d->W, npos = d->KH * d->KW;
   const size_t npix = (size_t)d->N * cc * HW;
   const int wblocks = ceil_div(d->K, 32) * cc;
   const size_t blocks = wblocks + (npix + 255) / 256;
-  if (blocks > 0x7fffffffull) return fail(UNIT_E_ARG, "%s: tensor too large", what);
+  if (blocks >= 1u << 24) return fail(UNIT_E_ARG, "%s: tensor too large", what);  // a grid has fewer than 2^32 threads
+  if (int rc = check_device()) return rc;
   char *packed = static_cast<char *>(workspace), *prepared = packed + z.packed;
   const int lds = npos <= kMaxWindow ? 32 * (npos * 32 + 4) : 0;
   hipLaunchKernelGGL(pack_f16_operands, dim3((unsigned)blocks), dim3(256), lds, static_cast<hipStream_t>(stream),
