@@ -31,3 +31,14 @@ def test_plain_operands(dev, oracle, N, C, H, W, K, KH, KW, stride, offset):
     out = U.conv2d_NCHW16c_OHWI16o(shifted(a), shifted(b), stride, stride).cpu().numpy()
     ref = oracle.conv2d_nchw16c_f16(oracle.pack_nchwc(a, 16), oracle.prepack_conv_weight_f16(b), stride, stride)
     assert np.array_equal(out.astype(np.float64), ref), U.last_variant()
+
+
+def test_weights_at_the_size_limit(dev):
+    """2 147 200 000 bytes of weights whose 32-channel form would pass 2^31 - 1."""
+    K, C = 10000, 16 * 6710
+    g = torch.Generator(device=dev).manual_seed(1)
+    a = torch.randint(-1, 2, (1, C, 1, 1), dtype=torch.int8, device=dev, generator=g).half()
+    b = torch.randint(-1, 2, (K, C, 1, 1), dtype=torch.int8, device=dev, generator=g).half()
+    out = U.conv2d_NCHW16c_OHWI16o(a, b, 1, 1)
+    ref = torch.cat([part.reshape(-1, C).float() @ a.reshape(C).float() for part in b.split(2000)])  # exact: sums below 2^24
+    assert torch.equal(out.reshape(K), ref), U.last_variant()

@@ -533,10 +533,12 @@ def conv2d_NCHW16c_OHWI16o(a, b, stride_h, stride_w, out_type="float32"):
     b = _dev(b, "b", torch.float16, (4, 6))
     if a.dim() == 4 and b.dim() == 4:
         p, need = _plan_f16_plain(a.shape, b.shape, int(stride_h), int(stride_w))
-        ws = a.new_empty((need,), dtype=torch.uint8)
-        out = a.new_empty(p.blocked, dtype=torch.float32)
-        check(L.unit_conv2d_nchw_f16f32(p.ref, a.data_ptr(), b.data_ptr(), out.data_ptr(), ws.data_ptr(), need, _stream()))
-        return out
+        if need:
+            ws = a.new_empty((need,), dtype=torch.uint8)
+            out = a.new_empty(p.blocked, dtype=torch.float32)
+            check(L.unit_conv2d_nchw_f16f32(p.ref, a.data_ptr(), b.data_ptr(), out.data_ptr(), ws.data_ptr(), need, _stream()))
+            return out
+        a, b = pack_nchwc(a, 16), prepack_conv_weight_f16(b)
     if not (a.dim() == 5 and b.dim() == 6):
         raise ValueError("a, b: expected 4-D + 4-D or 5-D + 6-D operands")
     p = _plan_f16(a.shape, b.shape, int(stride_h), int(stride_w))
@@ -553,6 +555,8 @@ def _plan_f16_plain(ashape, bshape, stride_h, stride_w):
         raise ValueError("a, b: channel counts must match and be multiples of 16")
     p = _ConvPlan(n, c, h, w, k, kh, kw, (stride_h, stride_w), 0, 1, 16)
     need = ctypes.c_size_t()
+    if -(-k // 32) * 64 * c * kh * kw > 2 ** 31 - 1:  # the prepared form fills 32-channel blocks: past the size limit
+        return p, 0
     check(_lib.load().unit_conv2d_nchw_f16f32_ws_bytes(p.ref, ctypes.byref(need)))
     return p, need.value
 
