@@ -17,6 +17,8 @@ pytestmark = pytest.mark.gpu
     ((5625, 250, 3, 5), 16, np.uint8),    # 90000 planes of 15 pixels: partial groups of the sixteen-pixel kernel
     ((22499, 16, 4, 4), 16, np.uint8),    # 89996 four-pixel groups
     ((22500, 16, 4, 4), 16, np.uint8),    # 90000
+    ((70001, 16, 1, 1), 16, np.uint8), ((70001, 17, 1, 3), 16, np.int8), ((70001, 16, 1, 1), 16, np.int32),
+    ((70001, 16, 1, 2), 16, np.float16), ((70001, 3, 1, 4), 4, np.uint8), ((11, 7, 3, 5), 6, np.float16),
     ((2, 20, 3, 7), 16, np.float16), ((2, 20, 1, 1), 16, np.float16), ((1, 20, 3, 3), 16, np.int32),
 ])
 def test_pack_and_back(dev, oracle, shape, cb, dtype):

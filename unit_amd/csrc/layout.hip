@@ -151,28 +151,29 @@ __global__ __launch_bounds__(256) void pack16c_bytes(const char *src, char *dst,
   }
 }
 
-// any shape / element size: one thread per blocked element
-template <bool PACK>
-__global__ __launch_bounds__(256) void nchwc_elems(const char *src, char *dst, int C, int HW, int cc, int cb,
-                                                   int es, size_t total) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+// any shape / element size: one thread per blocked element, at any address (E: an unsigned type of alignment 1)
+typedef unsigned short half_at_t __attribute__((aligned(1)));
+
+template <bool PACK, class E>
+__global__ __launch_bounds__(256) void nchwc_elems(const char *src, char *dst, int C, int HW, int cc, FastDiv by_cb, FastDiv by_hw,
+                                                   FastDiv by_cc, int total) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= total) return;
-  const int c = (int)(i % cb);
-  const size_t r = i / cb;
-  const size_t p = r % HW, plane = r / HW;
-  const int ci = (int)(plane % cc);
-  const size_t n = plane / cc;
-  const int ch = ci * cb + c;
-  const size_t flat = ((n * C + ch) * HW + p) * es;
-  for (int b = 0; b < es; ++b) {
-    if (PACK)
-      dst[i * es + b] = ch < C ? src[flat + b] : 0;
-    else if (ch < C)
-      dst[flat + b] = src[i * es + b];
-  }
+  int r, c, plane, p, n, ci;
+  by_cb.divmod(i, r, c);
+  by_hw.divmod(r, plane, p);
+  by_cc.divmod(plane, n, ci);
+  const int ch = ci * by_cb.d + c;
+  const size_t flat = ((size_t)n * C + ch) * HW + p;
+  const E *from = reinterpret_cast<const E *>(src);
+  E *to = reinterpret_cast<E *>(dst);
+  if (PACK)
+    to[i] = ch < C ? from[flat] : E(0);
+  else if (ch < C)
+    to[flat] = from[i];
 }
 
-// u8 / s8 NCHW -> NCHW16c: from this many four-pixel groups on, sixteen pixels per thread (nchw16c_bytes) win.  Below, the
+// u8 / s8 NCHW -> NCHW16c: from this many four-pixel groups on, sixteen pixels per thread (pack16c_bytes) win.  Below, the
 // tensor gives such threads too few waves and each a long chain: 7 x 320 x 9 x 11 5.3 us against 2.9 us with four pixels
 // per thread, 32 x 64 x 56 x 56 5.5 against 5.7, 32 x 256 x 56 x 56 10.4 against 15.7 us.  The way back is faster with
 // four pixels per thread at every size (14.5 -> 10.5 us for the last).
@@ -203,7 +204,11 @@ int nchwc(const void *src, void *dst, int N, int C, int H, int W, int cb, int es
   const int HW = (int)hw, pp = 4 / es;
   const int groups = ceil_div(HW, pp);
   const long total_groups = (long)N * cc * groups;  // < 2^29: the tensor fits 2^31 bytes
-  const bool words = HW >= pp && (cb == 16 || (cb == 4 && es == 1));
+  // Planes of one group leave a thread's words of all channels side by side, and a wave's words of one channel a row apart:
+  // element by element is then faster on the way back (400000 x 16 x 2 fp16 47.8 -> 21.9 us, 1000000 x 16 x 1 int32 77 -> 29) and
+  // for single pixels (44 -> 29 us), while fp16 and bytes pack a little faster as words (21.8 against 23.2).
+  const bool one_group = PACK && es < 4 ? HW < pp : HW <= pp;
+  const bool words = !one_group && (cb == 16 || (cb == 4 && es == 1));
   if (PACK && es == 1 && cb == 16 && (total_groups >= kManyGroups || !words)) {
     const int groups16 = ceil_div(HW, 16), total16 = N * cc * groups16;
     hipLaunchKernelGGL(pack16c_bytes, dim3(ceil_div(total16, 256)), dim3(256), 0, s, in, out, C, HW, cc,
@@ -219,8 +224,10 @@ int nchwc(const void *src, void *dst, int N, int C, int H, int W, int cb, int es
     else UNIT_NCHWC(4, 16);
 #undef UNIT_NCHWC
   } else {
-    hipLaunchKernelGGL(nchwc_elems<PACK>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, in, out, C, HW,
-                       cc, cb, es, total);
+    const dim3 grid((unsigned)((total + 255) / 256));
+    const FastDiv by_cb = FastDiv::make(cb), by_hw = FastDiv::make(HW), by_cc = FastDiv::make(cc);
+    auto kern = es == 1 ? nchwc_elems<PACK, unsigned char> : es == 2 ? nchwc_elems<PACK, half_at_t> : nchwc_elems<PACK, word_at_t>;
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, in, out, C, HW, cc, by_cb, by_hw, by_cc, (int)total);
   }
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? UNIT_OK : fail(UNIT_E_LAUNCH, "%s: %s", what, hipGetErrorString(e));
