@@ -28,3 +28,14 @@ def test_pack_and_back(dev, oracle, shape, cb, dtype):
     p = U.pack_nchwc(torch.from_numpy(x).to(dev), cb)
     assert np.array_equal(p.cpu().numpy().view(np.uint8), oracle.pack_nchwc(x, cb).view(np.uint8))
     assert np.array_equal(U.unpack_nchwc(p, shape[1]).cpu().numpy().view(np.uint8), x.view(np.uint8))
+
+
+@pytest.mark.parametrize("shape,cb,dtype", [((2, 20, 3, 5), 16, np.float16), ((3, 3, 5, 7), 4, np.uint8), ((2, 18, 5, 5), 16, np.int8)])
+def test_blocked_tensor_at_an_odd_element(dev, oracle, shape, cb, dtype):
+    """The blocked side of the word kernels is read and written in aligned words: other addresses go element by element."""
+    x = rng.random_bytes(int(np.prod(shape)) * np.dtype(dtype).itemsize, 8).view(dtype).reshape(shape)
+    want = oracle.pack_nchwc(x, cb)
+    room = torch.zeros(want.size + 1, dtype=torch.from_numpy(x).dtype, device=dev)
+    room[1:] = torch.from_numpy(want.reshape(-1)).to(dev)
+    back = U.unpack_nchwc(room[1:].view(want.shape), shape[1])
+    assert np.array_equal(back.cpu().numpy().view(np.uint8), x.view(np.uint8))

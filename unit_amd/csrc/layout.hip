@@ -204,11 +204,12 @@ int nchwc(const void *src, void *dst, int N, int C, int H, int W, int cb, int es
   const int HW = (int)hw, pp = 4 / es;
   const int groups = ceil_div(HW, pp);
   const long total_groups = (long)N * cc * groups;  // < 2^29: the tensor fits 2^31 bytes
+  // Words of the blocked side are aligned ones, so a tensor that starts elsewhere goes element by element.
   // Planes of one group leave a thread's words of all channels side by side, and a wave's words of one channel a row apart:
   // element by element is then faster on the way back (400000 x 16 x 2 fp16 47.8 -> 21.9 us, 1000000 x 16 x 1 int32 77 -> 29) and
   // for single pixels (44 -> 29 us), while fp16 and bytes pack a little faster as words (21.8 against 23.2).
   const bool one_group = PACK && es < 4 ? HW < pp : HW <= pp;
-  const bool words = !one_group && (cb == 16 || (cb == 4 && es == 1));
+  const bool words = !one_group && (cb == 16 || (cb == 4 && es == 1)) && reinterpret_cast<uintptr_t>(PACK ? dst : src) % 4 == 0;
   if (PACK && es == 1 && cb == 16 && (total_groups >= kManyGroups || !words)) {
     const int groups16 = ceil_div(HW, 16), total16 = N * cc * groups16;
     hipLaunchKernelGGL(pack16c_bytes, dim3(ceil_div(total16, 256)), dim3(256), 0, s, in, out, C, HW, cc,
