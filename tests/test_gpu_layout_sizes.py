@@ -6,7 +6,7 @@ import pytest
 import torch
 
 import unit_amd as U
-from unit_amd import rng
+from unit_amd import _lib, rng
 
 pytestmark = pytest.mark.gpu
 
@@ -30,7 +30,8 @@ def test_pack_and_back(dev, oracle, shape, cb, dtype):
     assert np.array_equal(U.unpack_nchwc(p, shape[1]).cpu().numpy().view(np.uint8), x.view(np.uint8))
 
 
-@pytest.mark.parametrize("shape,cb,dtype", [((2, 20, 3, 5), 16, np.float16), ((3, 3, 5, 7), 4, np.uint8), ((2, 18, 5, 5), 16, np.int8)])
+@pytest.mark.parametrize("shape,cb,dtype", [((2, 20, 3, 5), 16, np.float16), ((3, 3, 5, 7), 4, np.uint8), ((2, 18, 5, 5), 16, np.int8),
+                                            ((3, 18, 1, 3), 16, np.int8)])
 def test_blocked_tensor_at_an_odd_element(dev, oracle, shape, cb, dtype):
     """The blocked side of the word kernels is read and written in aligned words: other addresses go element by element."""
     x = rng.random_bytes(int(np.prod(shape)) * np.dtype(dtype).itemsize, 8).view(dtype).reshape(shape)
@@ -39,3 +40,8 @@ def test_blocked_tensor_at_an_odd_element(dev, oracle, shape, cb, dtype):
     room[1:] = torch.from_numpy(want.reshape(-1)).to(dev)
     back = U.unpack_nchwc(room[1:].view(want.shape), shape[1])
     assert np.array_equal(back.cpu().numpy().view(np.uint8), x.view(np.uint8))
+    room.zero_()
+    xd = torch.from_numpy(x).to(dev)
+    code = _lib.load().unit_pack_nchwc(xd.data_ptr(), room[1:].data_ptr(), *shape, cb, x.itemsize,
+                                       torch.cuda.current_stream().cuda_stream)
+    assert code == 0 and np.array_equal(room[1:].cpu().numpy().view(np.uint8), want.reshape(-1).view(np.uint8)) and room[0] == 0

@@ -157,8 +157,9 @@ typedef unsigned short half_at_t __attribute__((aligned(1)));
 template <bool PACK, class E>
 __global__ __launch_bounds__(256) void nchwc_elems(const char *src, char *dst, int C, int HW, int cc, FastDiv by_cb, FastDiv by_hw,
                                                    FastDiv by_cc, int total) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= total) return;
+  const u32 at = blockIdx.x * 256u + threadIdx.x;  // total may be 2^31 - 1
+  if (at >= (u32)total) return;
+  const int i = (int)at;
   int r, c, plane, p, n, ci;
   by_cb.divmod(i, r, c);
   by_hw.divmod(r, plane, p);
@@ -209,8 +210,9 @@ int nchwc(const void *src, void *dst, int N, int C, int H, int W, int cb, int es
   // element by element is then faster on the way back (400000 x 16 x 2 fp16 47.8 -> 21.9 us, 1000000 x 16 x 1 int32 77 -> 29) and
   // for single pixels (44 -> 29 us), while fp16 and bytes pack a little faster as words (21.8 against 23.2).
   const bool one_group = PACK && es < 4 ? HW < pp : HW <= pp;
-  const bool words = !one_group && (cb == 16 || (cb == 4 && es == 1)) && reinterpret_cast<uintptr_t>(PACK ? dst : src) % 4 == 0;
-  if (PACK && es == 1 && cb == 16 && (total_groups >= kManyGroups || !words)) {
+  const uintptr_t blocked = reinterpret_cast<uintptr_t>(PACK ? dst : src);
+  const bool words = !one_group && (cb == 16 || (cb == 4 && es == 1)) && blocked % 4 == 0;
+  if (PACK && es == 1 && cb == 16 && blocked % 16 == 0 && (total_groups >= kManyGroups || !words)) {
     const int groups16 = ceil_div(HW, 16), total16 = N * cc * groups16;
     hipLaunchKernelGGL(pack16c_bytes, dim3(ceil_div(total16, 256)), dim3(256), 0, s, in, out, C, HW, cc,
                        FastDiv::make(groups16), total16);
