@@ -29,9 +29,14 @@ __all__ = [
 
 
 # ------------------------------------------------------------------------------- helpers
+_raw_stream, _device = (getattr(torch._C, name, None) for name in ("_cuda_getCurrentRawStream", "_cuda_getDevice"))
+
+
 def _stream():
-    # the handle of torch.cuda.current_stream(), without building the Stream object (0.2 against 2.7 us)
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    # the handle of torch.cuda.current_stream(); without building the Stream object where torch allows (0.2 against 2.7 us)
+    if _raw_stream is None or _device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_device())
 
 
 def _dev(t, name, dtype=None, ndim=None):
