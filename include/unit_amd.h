@@ -132,8 +132,9 @@ int unit_dense_u8s8s32(const void *a, const void *w, void *c, int32_t M, int32_t
  * compiled graphs fold sum(w) next to their u8 x s8 operators (apps/cpu/relay/result.log:15-16 for the
  * convolution; the dense weight of apps/cpu/relay/int8-gemm.py:15 is a constant the same way):
  *   unit_dense_prepare_weight  wsum[n] = sum_k w[n][k]  (int32[N], caller-owned)
- *   unit_dense_u8s8s32_prepared  c = a . w^T with both operand tiles moved global -> LDS directly (K % 128 == 0
- *   and at least 128 tiles of 256 x 256; other shapes run unit_dense_u8s8s32).  Results are identical. */
+ *   unit_dense_u8s8s32_prepared  c = a . w^T with both operand tiles moved global -> LDS directly, any K % 16 == 0
+ *   (large results with an odd number of 64-byte stages or a part of one, where tiles staged through registers are
+ *   faster, and operands past 2^31 - 1 bytes run unit_dense_u8s8s32).  Results are identical. */
 int unit_dense_prepare_weight(const void *w, int32_t *wsum, int32_t N, int32_t K, unit_stream_t stream);
 int unit_dense_u8s8s32_prepared(const void *a, const void *w, const int32_t *wsum, void *c, int32_t M,
                                 int32_t N, int32_t K, unit_stream_t stream);
@@ -144,8 +145,8 @@ int unit_dense_u8s8s32_prepared(const void *a, const void *w, const int32_t *wsu
  *   c[x][y] = sum_k f32(a[x][k]) * f32(b[k][y]),  a f16 (M, K), b f16 (K, N), row-major;
  * c is f32 when out_f16 == 0, else f16 (round-to-nearest-even of the fp32 sum).
  * K % 8 == 0, N % 4 == 0.  Replaces wmma.m16n16k16 (python/tensorizer/intrinsics/gpu.py:104-216)
- * with v_mfma_f32_32x32x16_f16.  With few output tiles and a long reduction (the script's own
- * 128 x 768 x 3072) and f32 output, the reduction is split between workgroups as the reference's
+ * with v_mfma_f32_32x32x16_f16.  With few output tiles (up to 64 of 128 x 128, or a single column of them), a long
+ * reduction (the script's own 128 x 768 x 3072) and f32 output, the reduction is split between workgroups as the reference's
  * rfactor schedule does (apps/gpu/gemm.py:22-40): partial tiles are added into the zero-filled c,
  * so the summation order, and with it the last bits of c, can differ from run to run
  * (UNIT_AMD_GEMM_F16_SPLITK=1 keeps one workgroup per tile). */

@@ -15,9 +15,9 @@ and :6803-6828 (the 3-channel stem: channels padded to 4, NCHW4c), which runs as
     #6 fused_layout_transform                          NCHW16c -> NCHW
 
 Here #1-#4 depend on constants only and run once, when the graph object is built (weights end up
-in the kernels' prepared form, which carries 128 * sum(w)); a call runs #0 as the layout kernel on
-the signed data (the +128 shift is the convolution kernel's sign flip of the operand), #5 as the
-fused convolution and, by default, #6 inside its store.
+in the kernels' prepared form, which carries 128 * sum(w)); a call is one library call: #0 as the layout
+kernel on the signed data (the +128 shift is the convolution kernel's sign flip of the operand), #5 as the
+fused convolution with #6 inside its store -- or, for image stems, all three in one kernel.
 """
 import sys
 
@@ -85,7 +85,6 @@ class Conv2dBiasMultiply:
             self.multiplier, out.data_ptr(), self.oc, data.data_ptr(), ops._stream()))
         return out
 
-
     def graph(self, x):
         """Capture a run on x into a HIP graph; returns a callable that replays it and returns the result tensor
         (x's storage is the graph's input)."""
@@ -123,8 +122,8 @@ def time_evaluator(fn, number=3, repeat=10):
 def main(argv=None):
     """python -m unit_amd.relay N C H W OC IC KH KW SH SW   (or the ten integers on stdin, as the
     reference's driver reads them): builds the graph on random operands drawn as the reference
-    draws them (randn * 128 cast to int8 / int32) and prints the mean time of a run in us (two kernel
-    launches from Python per run; replaying so short a sequence as a HIP graph measured slower, 35 against 17 us)."""
+    draws them (randn * 128 cast to int8 / int32) and prints the mean time of a run in us (one or two kernel
+    launches per run; replaying so short a sequence as a HIP graph measured slower, 35 against 17 us)."""
     import numpy as np
     argv = sys.argv[1:] if argv is None else argv
     fields = argv if argv else sys.stdin.readline().split()
