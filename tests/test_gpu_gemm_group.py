@@ -1,6 +1,6 @@
-"""GEMMs on the group tiles (gemm_group.hpp): every tile shape, reductions that end inside a 64-byte stage, row and
-column edges, N of 4 mod 8 (the transposing read's shifted last chunk), fewer stages than groups, k-splits by atomics and
-by planes.  Integer data makes the fp16 products exact in any order, so everything is compared bit for bit."""
+"""GEMMs on the group tiles (gemm_group.hpp): every tile shape with every layout of the second operand, reductions that
+end inside a 64-byte stage, row and column edges, N of 4 mod 8 (the transposing read's shifted last chunk), fewer stages
+than groups, k-splits by atomics (pinned, and where int8 takes them by itself) and by planes.  Integer data makes the fp16 products exact in any order, so everything is compared bit for bit."""
 import numpy as np
 import pytest
 import torch
@@ -11,11 +11,17 @@ from unit_amd import _lib
 pytestmark = pytest.mark.gpu
 
 # M, N, K; the tile the shape is there for (fp16 with fp16 output)
-F16 = [(1, 8, 8, "x32_y32"), (33, 12, 24, "x32_y32"), (37, 36, 200, "x32_y32"), (300, 260, 520, "x32_y32"),
+F16 = [(1, 8, 8, "x32_y32_k64_w1x1_g4"), (33, 12, 24, "x32_y32"), (37, 36, 200, "x32_y32_k64_w1x1_g8"), (300, 260, 520, "x32_y32"),
        (700, 700, 712, "x32_y64"), (300, 3004, 296, "x64_y64"), (1000, 1516, 1096, "x64_y128"),
        (1500, 1508, 1496, "x128_y128"), (2180, 2052, 2056, "x128_y128"), (3840, 2044, 2056, "x256_y128"), (129, 8192, 40, "")]
-I8 = [(1, 4, 16), (33, 36, 80), (50, 260, 1040), (37, 128, 4112), (700, 704, 720), (1467, 1108, 976), (1500, 1536, 1552),
-      (2180, 2176, 2064), (3840, 2048, 4112), (129, 8192, 48)]
+# M, N, K; the tile with row-major or prepared weights, and with packed ones (None: N is no multiple of 128)
+G4, G8 = "x32_y32_k64_w1x1_g4", "x32_y32_k64_w1x1_g8"
+I8 = [(1, 4, 16, G4, None), (33, 36, 80, G4, None), (1, 256, 480, G8, G8), (50, 260, 1040, G4, None), (37, 128, 4112, G4, G4),
+      (64, 4096, 4096, G8, G8), (700, 704, 720, "x32_y64", None), (128, 3072, 784, "x32_y64", "x32_y64"),
+      (129, 8192, 48, "x64_y64", "x64_y64"), (300, 3072, 304, "x64_y64", "x64_y64"), (1467, 1108, 976, "x64_y128", None),
+      (1000, 1536, 1104, "x64_y128", "x64_y128"), (1500, 1536, 1552, "x128_y128", "x128_y128"),
+      (2180, 2176, 2064, "x128_y128", "x128_y128"), (1175, 4864, 1632, "x256_y128", "x256_y128"),
+      (3840, 2048, 4112, "x256_y128", "x256_y256")]
 
 
 def _ints(g, lo, hi, shape, dtype, dev):
@@ -72,15 +78,17 @@ def test_fp16_infinity_past_a_row(dev):
         assert torch.equal(out[::2], torch.full_like(out[::2], K)) and torch.isinf(out[1::2]).all(), U.last_variant()
 
 
-@pytest.mark.parametrize("M,N,K", I8)
-def test_int8_group_tiles(dev, M, N, K):
+@pytest.mark.parametrize("M,N,K,tile,packed_tile", I8)
+def test_int8_group_tiles(dev, M, N, K, tile, packed_tile):
     g = np.random.RandomState(M + N + K)
     a, w = _ints(g, 0, 256, (M, K), torch.uint8, dev), _ints(g, -128, 128, (N, K), torch.int8, dev)
     ref = (a.double() @ w.double().t()).to(torch.int32)
-    assert torch.equal(U.dense(a, w), ref), U.last_variant()
-    assert torch.equal(U.dense(a, U.prepare_dense_weight(w)), ref), U.last_variant()
-    if N % 128 == 0:
+    for operand in (w, U.prepare_dense_weight(w)):
+        assert torch.equal(U.dense(a, operand), ref), U.last_variant()
+        assert tile in U.last_variant() and "dma" not in U.last_variant(), U.last_variant()
+    if packed_tile:
         assert torch.equal(U.dense_dotprod(a, U.prepack_dense_weight(w)), ref), U.last_variant()
+        assert packed_tile in U.last_variant(), U.last_variant()
 
 
 @pytest.mark.parametrize("splits", [1, 2, 5])
