@@ -44,11 +44,12 @@ int run_gemm_f16_bt_dma(const void *a, const void *bt, void *c, int M, int N, in
 
 // b (K, N) as the reference gives it, both operands global -> LDS directly: b's tile lands as it lies in memory and
 // the fragments come out of it with the LDS transposing read (K a whole number of stages, N a multiple of 8).
-// splits > 1: k-ranges, added with atomics into the zero-filled c (Epi = GemmEpilogue, f32) or written as planes.
-template <class T, int NSTAGE, class Epi>
-int run_gemm_f16_dma_tr(const char *what, const char *tag, const void *a, const void *b, const typename Epi::Params &ep,
-                        int M, int N, int K, int splits, void *zero, hipStream_t s) {
+// splits > 1: k-ranges, added with atomics into the zero-filled c (fp32 results only).
+template <class T, int NSTAGE, bool OUT_F16>
+int run_gemm_f16_dma_tr(const void *a, const void *b, void *c, int M, int N, int K, hipStream_t s, int splits = 1) {
+  using Epi = GemmEpilogue<OpF16, OUT_F16>;
   DmaParams p{static_cast<const char *>(a), static_cast<const char *>(b), M, N, K * 2, nullptr, N * 2};
+  typename Epi::Params ep{c, M, N};
   const int nk = K * 2 / T::BKB, gx = ceil_div(M, T::BX), gy = ceil_div(N, T::BY);
   constexpr int lds = NSTAGE * T::STAGE;
   static_assert(lds <= kMaxLds, "ring does not fit the LDS");
@@ -56,27 +57,20 @@ int run_gemm_f16_dma_tr(const char *what, const char *tag, const void *a, const 
   static thread_local bool allowed = false;
   if (!allowed) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
-    if (e != hipSuccess) return fail(UNIT_E_LAUNCH, "%s: hipFuncSetAttribute: %s", what, hipGetErrorString(e));
+    if (e != hipSuccess) return fail(UNIT_E_LAUNCH, "unit_gemm_f16: hipFuncSetAttribute: %s", hipGetErrorString(e));
     allowed = true;
   }
-  splits = splits < 1 ? 1 : (splits > nk ? nk : splits);
-  if (splits > 1 && zero) {
+  splits = OUT_F16 || splits < 1 ? 1 : (splits > nk ? nk : splits);
+  if (splits > 1) {
     const size_t n16 = (size_t)M * N * 4 / 16;
-    hipLaunchKernelGGL(zero_fill, dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, s, static_cast<v4i *>(zero), n16);
+    hipLaunchKernelGGL(zero_fill, dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, s, static_cast<v4i *>(c), n16);
   }
   const GridMap gm = GridMap::make(gx, gy, gx < 4 ? gx : 4, splits);
-  set_variant("f16gemm_%s_x%d_y%d_k%d_w%dx%d_r%d_s%d", tag, T::BX, T::BY, T::BKB, T::WX, T::WY, NSTAGE, splits);
+  set_variant("f16gemm_%s_x%d_y%d_k%d_w%dx%d_r%d_s%d", OUT_F16 ? "dmatr_h" : "dmatr", T::BX, T::BY, T::BKB, T::WX, T::WY, NSTAGE,
+              splits);
   hipLaunchKernelGGL(kern, dim3(gm.total), dim3(T::NT), lds, s, p, ep, nk, gm UNIT_TRACE(, trace_buffer()));
   hipError_t e = hipGetLastError();
-  return e == hipSuccess ? UNIT_OK : fail(UNIT_E_LAUNCH, "%s: launch: %s", what, hipGetErrorString(e));
-}
-
-template <class T, int NSTAGE, bool OUT_F16>
-int run_gemm_f16_dma_tr(const void *a, const void *b, void *c, int M, int N, int K, hipStream_t s, int splits = 1) {
-  using Epi = GemmEpilogue<OpF16, OUT_F16>;
-  typename Epi::Params ep{c, M, N};
-  return run_gemm_f16_dma_tr<T, NSTAGE, Epi>("unit_gemm_f16", OUT_F16 ? "dmatr_h" : "dmatr", a, b, ep, M, N, K,
-                                             OUT_F16 ? 1 : splits, c, s);
+  return e == hipSuccess ? UNIT_OK : fail(UNIT_E_LAUNCH, "unit_gemm_f16: launch: %s", hipGetErrorString(e));
 }
 
 // b (K, N): a goes global -> LDS directly, b through the transposing register loader (K a whole number of stages)
@@ -198,19 +192,18 @@ __global__ __launch_bounds__(256) void unpack32_f16(const _Float16 *__restrict__
   for (int r = ty; r < 32; r += 8) bt[(size_t)(nb * 32 + r) * K + kb * 32 + tx] = tile[tx][r];
 }
 
-// TAIL = false: K is a whole number of stages (the loaders then stage without zeroing selects)
-template <class T, bool OUT_F16, int PF = 1, bool TAIL = true>
+// both operands through registers: a by rows, b by columns
+template <class T, bool OUT_F16>
 int run_gemm_f16(const void *a, const void *b, void *c, int M, int N, int K, hipStream_t s, bool whole) {
-  using XL = RowMajorLoader<T::BX, T::BKB, T::NT, false, PF, TAIL>;
-  using YL = KMajorF16Loader<T::BY, T::BKB, T::NT, PF, TAIL>;
+  using XL = RowMajorLoader<T::BX, T::BKB, T::NT, false>;
+  using YL = KMajorF16Loader<T::BY, T::BKB, T::NT>;
   using Epi = GemmEpilogue<OpF16, OUT_F16>;
   typename XL::Params xp{static_cast<const char *>(a), M, K * 2, K * 2};
   typename YL::Params yp{static_cast<const char *>(b), N, K, N + 4, 0, N * 2};
   typename Epi::Params ep{c, M, N};
   const int nk = ceil_div(K * 2, T::BKB), gx = ceil_div(M, T::BX), gy = ceil_div(N, T::BY);
   const int splits = OUT_F16 || whole ? 1 : gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K, nk);
-  set_variant("f16gemm_x%d_y%d_k%d_w%dx%d_p%d%s%s_s%d", T::BX, T::BY, T::BKB, T::WX, T::WY, PF, TAIL ? "" : "e",
-              OUT_F16 ? "_h" : "", splits);
+  set_variant("f16gemm_x%d_y%d_k%d_w%dx%d_p1%s_s%d", T::BX, T::BY, T::BKB, T::WX, T::WY, OUT_F16 ? "_h" : "", splits);
   return launch_mma<OpF16, T, XL, YL, Epi, WS_NONE>(xp, yp, ep, nk, gx, gy, 4, splits, c, (size_t)M * N * 4, 0, s,
                                                     "unit_gemm_f16");
 }
@@ -296,8 +289,8 @@ int gemm_f16_planes(const char *what, const void *a, const void *b, void *c, int
   if (N < 8) {  // less than one 16-byte chunk of a row of b
     using T = Tile<128, 128, 64, 2, 2>;
     GemmPlaneEpilogue::Params ep{ws, M, N, plane};
-    using XL = RowMajorLoader<T::BX, T::BKB, T::NT, false, 1, true>;
-    using YL = KMajorF16Loader<T::BY, T::BKB, T::NT, 1, true>;
+    using XL = RowMajorLoader<T::BX, T::BKB, T::NT, false>;
+    using YL = KMajorF16Loader<T::BY, T::BKB, T::NT>;
     typename XL::Params xp{static_cast<const char *>(a), M, K * 2, K * 2};
     typename YL::Params yp{static_cast<const char *>(b), N, K, N + 4, 0, N * 2};
     const int nk = ceil_div(K * 2, T::BKB), gx = ceil_div(M, T::BX), gy = ceil_div(N, T::BY);
@@ -405,7 +398,7 @@ extern "C" int unit_gemm_f16_ws(const void *a, const void *b, void *c, int32_t M
   const char *what = "unit_gemm_f16_ws";
   int splits = 1;
   if (int rc = gemm_f16_ws_check(what, a, b, c, M, N, K, &splits)) return rc;
-  if (splits <= 1) {  // enough tiles, or a short reduction: nothing to split 
+  if (splits <= 1) {  // enough tiles, or a short reduction: nothing to split
     if (int rc = check_aligned(what, {a, b, c})) return rc;
     if (int rc = check_device()) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
