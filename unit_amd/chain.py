@@ -74,6 +74,7 @@ class ConvChain:
             raise ValueError("layers: empty chain")
         self.variants = [None] * len(self.outputs)
         self._native, self._bound = (), None
+        self._bind()
 
     def _bind(self):
         """The layers for the library, which runs them all in one call (the host then spends a launch's 2.5 us per layer,
@@ -82,6 +83,8 @@ class ConvChain:
         if len(self._native) != count:
             self._native, self._bound = (ChainLayerDesc * count)(), None
             self._names = ctypes.create_string_buffer(96 * count)  # kernel names, where self.variants has none yet
+            for i, d in enumerate(self._native):
+                d.variant = ctypes.addressof(self._names) + 96 * i
         bound = [(w.buf.data_ptr(), o.data_ptr(), None if b is None else b.data_ptr(), *c, src)
                  for w, o, b, c, src in zip(self.weights, self.outputs, self.biases, self.consts, self.sources)]
         bound.append(b"".join(self.descs))
@@ -97,7 +100,8 @@ class ConvChain:
         self._bind()
         unnamed = [i for i, v in enumerate(self.variants) if v is None]
         for i in unnamed:
-            self._native[i].variant = ctypes.addressof(self._names) + 96 * i
+            if not self._native[i].variant:
+                self._native[i].variant = ctypes.addressof(self._names) + 96 * i
         check(self._L.unit_conv_chain_u8(self._native, len(self._native), x.data_ptr(), ops._stream()))
         for i in unnamed:
             self.variants[i] = self._names[96 * i:96 * i + 96].split(b"\0")[0].decode()
