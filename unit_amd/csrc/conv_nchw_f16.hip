@@ -11,9 +11,6 @@
 #include "mma_core.hpp"
 
 namespace unit {
-
-int conv_geom(const unit_conv_desc *d, int tapb, ConvGeom *g, const char *what);  // abi.hip
-
 namespace {
 
 typedef int halves8_t __attribute__((ext_vector_type(4), aligned(2)));  // plain operands may start at any element
@@ -92,17 +89,15 @@ struct NchwF16Sizes {
 // Checks the descriptor for everything that the convolution rejects -- the operands are re-laid before it runs -- and
 // gives the sizes.  The batch may need slices, an image not.
 int nchw_f16_sizes(const char *what, const unit_conv_desc *d, NchwF16Sizes *z) {
-  if (d->N <= 0 || d->C <= 0 || d->H <= 0 || d->W <= 0 || d->K <= 0 || d->KH <= 0 || d->KW <= 0)
-    return fail(UNIT_E_ARG, "%s: N, C, H, W, K, KH, KW must be positive", what);
+  int32_t OH, OW;
+  if (int rc = unit_conv_out_hw(d, &OH, &OW)) return rc;
   if (d->cb != 16 || d->C % 16 || d->K % 16)
     return fail(UNIT_E_ARG, "%s: C and K must be multiples of 16 and cb 16 (got %d, %d, %d)", what, d->C, d->K, d->cb);
   if (d->pt || d->pl || d->pb || d->pr) return fail(UNIT_E_ARG, "%s: the operator has no padding argument; pre-pad the data", what);
   if (d->dh != 1 || d->dw != 1) return fail(UNIT_E_ARG, "%s: dilation must be 1", what);
-  unit_conv_desc image = *d;
-  image.N = 1;
-  ConvGeom g;
-  if (int rc = conv_geom(&image, 32, &g, what)) return rc;
-  if (!fits((size_t)g.npix * d->K * 4)) return fail(UNIT_E_ARG, "%s: tensor exceeds 2^31-1 bytes", what);
+  if (d->H >= 16384 || d->W >= 16384) return fail(UNIT_E_ARG, "%s: spatial extent too large", what);  // the window fits the image
+  if (!fits((size_t)d->C * d->H * d->W * 2) || !fits((size_t)d->K * d->C * d->KH * d->KW * 2) || !fits((size_t)OH * OW * d->K * 4))
+    return fail(UNIT_E_ARG, "%s: tensor exceeds 2^31-1 bytes", what);
   z->packed = ((size_t)d->N * d->C * d->H * d->W * 2 + 255) / 256 * 256;
   z->prepared = prepared_layout(d->K, d->C, d->KH, d->KW, 16, 2).total_bytes;
   if (!fits(z->prepared)) return fail(UNIT_E_ARG, "%s: tensor exceeds 2^31-1 bytes", what);
