@@ -5,7 +5,8 @@
 // The re-laying launch is bound by latency at one image and by memory traffic at large batches (it reads and
 // writes each operand once).  Packing the weights into the reference's blocked layout first, one thread per element, took
 // 4.8 us at 256 x 256 x 3 x 3 and 27 us at 1984 x 496 x 3 x 3 (strided two-byte reads), the data pack another launch of
-// 3.4 us, and left the convolution on the per-element weight loads of that layout (10.8 us at 1 x 256 x 30 x 30, stride 2).  That call: 27.9 us then, 16.0 us in this form.
+// 3.4 us, and left the convolution on the per-element weight loads of that layout (10.8 us at 1 x 256 x 30 x 30, stride 2).  That call: 28.1 us then,
+// 11.2 us in this form and on the eight-wave tiles that the convolution takes since.
 #include "conv_plan.hpp"
 #include "conv_prepare.hpp"
 #include "mma_core.hpp"

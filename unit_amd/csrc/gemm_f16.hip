@@ -99,8 +99,8 @@ int run_gemm_f16_hybrid(const void *a, const void *b, void *c, int M, int N, int
 
 // Tiles of at most 256 x 128 with the reduction shared inside the workgroup (gemm_group.hpp), any K and N the
 // operator takes (b by columns: N >= 8).  fp32 results of up to 64 tiles of 128 x 128 may also share it between workgroups
-// (atomics into the zero-filled output); with more tiles they are the same bits from run to run, although up to 127 a long
-// reduction would gain (900 x 1096 x 7536, 72 tiles, by 19 % in the estimate): unit_gemm_f16_ws has planes for those.  With
+// (atomics into the zero-filled output); with more tiles they are the same bits from run to run, and the estimate's splits
+// lost there (900 x 1096 x 7536, 72 tiles, two ranges 64.9 us, whole 49.4; 733 x 1600 x 7616, 78 tiles, 61.8 and 46.2).  With
 // fewer than 12 such tiles and 1 KiB of reduction at least two ways (the tests ask for that; 300 x 260 x 520 would run 2 us
 // faster without).  fp16 results keep one workgroup per tile.
 template <int YM, bool OUT_F16>
@@ -119,8 +119,8 @@ int run_gemm_f16_group(const char *what, const char *tag, const void *a, const v
 // Which aligned shapes stay on the 128 x 128 tiles of mma_dma.hpp: fp32 results with fewer than 32 such tiles and more
 // than 128 rows (the tests name that kernel and its k-splits for them), one nearly full round of the 256 CUs
 // (1011 x 3584 x 1216, 224 tiles, 15.6 against 16.2 us on the group tile of the same size; 2048^3 22.9 against 24.8), and 512
-// tiles or more (8192 x 1024 x 1024 24.2 and 24.0 us).  The others gain: 1024^3 12.3 -> 7.7 us, 2304 x 2304 x 4096
-// 66 -> 55 us, 64 x 4096 x 4096 15.3 -> 11.9 us.
+// tiles or more (8192 x 1024 x 1024 24.2 and 24.0 us).  The others gain: 1024^3 11.1 -> 7.1 us, 2304 x 2304 x 4096
+// 65.5 -> 57.2, 64 x 4096 x 4096 15.6 -> 14.0.
 inline bool gemm_keeps_128(int M, int N, bool out_f16) {
   const long tiles = tiles_of_128(M, N);
   return tiles >= 512 || (tiles >= 192 && tiles <= 256) || (!out_f16 && tiles < 32 && M > 128);

@@ -384,8 +384,9 @@ int run_gemm_group(const char *what, const char *tag, GroupGemm p, int splits, h
 // busy the clock gives).  The constants are least-squares fits to 4200 timings (70 fp16 and 60 int8 shapes per weight
 // layout, 1 x 836 x 2736 to 8192 x 8192 x 2048, every tile and up to 16 splits): the pick is on average 3 % above the
 // best measured tile.  Against the 128 x 128 tiles with k-splits by atomics and the register pipelines that served these
-// shapes: fp16 1000 x 1516 x 1096 27.1 -> 13.4 us, 64 x 4096 x 4096 15.3 -> 11.9, int8 packed 128 x 768 x 3072
-// 10.1 -> 5.0, 1 x 4096 x 4096 15.4 -> 6.3, 1467 x 1152 x 976 16.2 -> 9.3, geometric mean over the shapes 1.6 - 1.7 x.
+// shapes, us a call in a row of them: fp16 1000 x 1516 x 1096 24.8 -> 10.3, 64 x 4096 x 4096 15.6 -> 14.0 (b prepared
+// 15.9 -> 11.5), int8 packed 128 x 768 x 3072 12.4 -> 6.4, 1 x 4096 x 4096 15.9 -> 6.8, 1467 x 1152 x 976 16.2 -> 9.3;
+// geometric mean over random shapes 1.5 x.
 struct GroupCost {
   int bx, by, kg, per_cu;
   float launch, tile, stage, share, hbm, rate;

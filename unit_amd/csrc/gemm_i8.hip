@@ -57,8 +57,8 @@ int run_dense_group(const char *what, const char *tag, const void *a, const void
 
 // Row-major weights with whole 64-byte stages: the 128 x 128 tiles of mma_dma.hpp keep the shapes with few tiles or
 // few stages, and those with 512 tiles or more (8192 x 1024 x 1024 17.3 against 16.5 us); the tests name this kernel
-// there.  From 32 tiles and 384 bytes on the group tiles are faster (64 x 4096 x 4096 12.8 -> 7.8 us, 1024^3
-// 9.5 -> 5.8 us, 2304 x 2304 x 4096 41 -> 34 us).
+// there.  From 32 tiles and 384 bytes on the group tiles are faster (64 x 4096 x 4096 13.3 -> 7.9 us, 1024^3
+// 11.2 -> 7.0, 1024 x 4096 x 4096 29.4 -> 25.3).
 inline bool dense_keeps_128(int M, int N, int K) {
   const long tiles = tiles_of_128(M, N);
   return K % 64 == 0 && !direct_gemm_large_tiles(M, N) && (tiles < 32 || tiles >= 512 || K < 384);
@@ -128,7 +128,7 @@ int run_dense_mixed(const void *a, const void *wp, void *c, int M, int N, int K,
 
 // Row-major weights and a K that the direct tiles do not take, on a large result: the staged 256 x 256 tiles for short
 // reductions of an odd number of 64-byte stages (the tests name them), and where their estimate, 1.15 x that of the direct
-// tiles, is the lower one (8000 x 2048 x 2000, one round of 256 tiles, 48 us against 56; 5000 x 4096 x 2000, two, 84 against 80).
+// tiles, is the lower one (8000 x 2048 x 2000, one round of 256 tiles, 45 us against 56; 5000 x 4096 x 2000, two, 82 against 77).
 inline bool dense_stays_staged(int M, int N, int K) {
   if (K % 128 == 0 || M < 256 || N < 256) return false;
   if (K % 128 == 64 && K < 1024 && direct_gemm_large_tiles(M, N)) return true;
@@ -164,7 +164,7 @@ int dense(const void *a, const void *w, void *c, int M, int N, int K, unit_strea
   if constexpr (PACKED) {
     // The staged 256 x 256 tiles take 1.1 x the time of the direct-to-LDS ones on row-major weights (1.15 x with a part of a
     // stage at the end); the 256 x 128 group tile takes 1.3 x its estimate here, whose fragments are four dword reads
-    // each (8192 x 4096 x 1024: 70 us, staged 59; 5000 x 4096 x 2000: 75, staged 81).
+    // each (8192 x 4096 x 1024: 70 us, staged 55; 5000 x 4096 x 2000: 73, staged 81).
     const GroupPlan group = plan_group(M, N, K, 1, 1, kAtomicSplits);
     if (M >= 256 && N >= 256 &&
         (K % 128 ? 1.15f : 1.1f) * large_tile_cost(M, N, K) < group.us * (group.tile == kGroupTiles - 1 ? 1.3f : 1.f))
