@@ -19,6 +19,9 @@ pytestmark = pytest.mark.gpu
     ((22500, 16, 4, 4), 16, np.uint8),    # 90000
     ((70001, 16, 1, 1), 16, np.uint8), ((70001, 17, 1, 3), 16, np.int8), ((70001, 16, 1, 1), 16, np.int32),
     ((70001, 16, 1, 2), 16, np.float16), ((70001, 3, 1, 4), 4, np.uint8), ((11, 7, 3, 5), 6, np.float16),
+    ((110, 24, 1, 220), 16, np.float16), ((400, 32, 7, 7), 16, np.int32),   # both sides of 600000 elements: 774400 and
+    ((300, 32, 7, 7), 16, np.float16), ((38000, 16, 1, 1), 16, np.int32),   # 627200, 470400 and 608000
+    ((1700, 32, 7, 7), 16, np.int32), ((1500, 64, 1, 26), 16, np.int32),    # 2.67 million by plane, 2.50 million flat
     ((2, 20, 3, 7), 16, np.float16), ((2, 20, 1, 1), 16, np.float16), ((1, 20, 3, 3), 16, np.int32),
 ])
 def test_pack_and_back(dev, oracle, shape, cb, dtype):

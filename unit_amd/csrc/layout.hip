@@ -28,9 +28,15 @@ __global__ __launch_bounds__(256) void nchwc_words(const char *src, char *dst, i
                                                    int total_groups) {
   constexpr int PP = 4 / ES, ROWW = CB * ES / 4;  // words per blocked row
   const int gid = blockIdx.x * 256 + threadIdx.x;
-  if (gid >= total_groups) return;
   int plane, g;  // plane = n * cc + ci
-  by_groups.divmod(gid, plane, g);
+  if (ES == 4 && PACK && gridDim.y > 1) {  // one workgroup per plane (the host's kPlaneElems)
+    if (gid >= by_groups.d) return;
+    plane = blockIdx.y;
+    g = gid;
+  } else {
+    if (gid >= total_groups) return;
+    by_groups.divmod(gid, plane, g);
+  }
   const int n = plane / cc, ci = plane - n * cc;
   const int p0 = min(g * PP, HW - PP);
   const char *nchw = PACK ? src : dst;
@@ -180,6 +186,14 @@ __global__ __launch_bounds__(256) void nchwc_elems(const char *src, char *dst, i
 // four pixels per thread at every size (14.5 -> 10.5 us for the last).
 constexpr long kManyGroups = 90000;
 
+// 16-channel blocks: up to this many elements one thread per element is faster, both ways and for every element size
+// (threads of sixteen or more elements are too few to hide their chain of latencies): 64 x 64 x 9 fp16 3.1 -> 2.3 us packing,
+// 3.5 -> 2.3 back; 4096 x 16 x 9, 590 thousand, 3.4 -> 2.8 and 3.7 -> 2.9; 512 x 128 x 16, a million, 3.3 -> 4.1.
+constexpr size_t kFewElems = 600000;
+// Packing 4-byte elements, planes of 25 to 255 pixels: from this many elements on, a workgroup per plane writes to memory
+// in better order than the flat index (956 x 256 x 49 22.4 -> 20.3 us, 1992 x 256 x 49 38.1 -> 36.4; the same at 1.5 million).
+constexpr size_t kPlaneElems = 2500000;
+
 template <bool PACK>
 int nchwc(const void *src, void *dst, int N, int C, int H, int W, int cb, int es, hipStream_t s, const char *what) {
   if (!src || !dst) return fail(UNIT_E_ARG, "%s: null pointer", what);
@@ -211,13 +225,15 @@ int nchwc(const void *src, void *dst, int N, int C, int H, int W, int cb, int es
   // for single pixels (44 -> 29 us), while fp16 and bytes pack a little faster as words (21.8 against 23.2).
   const bool one_group = PACK && es < 4 ? HW < pp : HW <= pp;
   const uintptr_t blocked = reinterpret_cast<uintptr_t>(PACK ? dst : src);
-  const bool words = !one_group && (cb == 16 || (cb == 4 && es == 1)) && blocked % 4 == 0;
-  if (PACK && es == 1 && cb == 16 && blocked % 16 == 0 && (total_groups >= kManyGroups || !words)) {
+  const bool few = cb == 16 && total < kFewElems;
+  const bool words = !one_group && !few && (cb == 16 || (cb == 4 && es == 1)) && blocked % 4 == 0;
+  if (PACK && es == 1 && cb == 16 && !few && blocked % 16 == 0 && (total_groups >= kManyGroups || !words)) {
     const int groups16 = ceil_div(HW, 16), total16 = N * cc * groups16;
     hipLaunchKernelGGL(pack16c_bytes, dim3(ceil_div(total16, 256)), dim3(256), 0, s, in, out, C, HW, cc,
                        FastDiv::make(groups16), total16);
   } else if (words) {
-    const dim3 grid((unsigned)((total_groups + 255) / 256));
+    const bool by_plane = PACK && es == 4 && HW >= 25 && HW < 256 && total >= kPlaneElems && N * cc <= 65535;
+    const dim3 grid = by_plane ? dim3(1, N * cc) : dim3((unsigned)((total_groups + 255) / 256));
     const FastDiv by_groups = FastDiv::make(groups);
 #define UNIT_NCHWC(ES, CB)                                                                                          \
   hipLaunchKernelGGL((nchwc_words<ES, CB, PACK>), grid, dim3(256), 0, s, in, out, C, HW, cc, by_groups, (int)total_groups)
