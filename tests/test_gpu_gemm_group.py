@@ -179,3 +179,14 @@ def test_pins_reach_the_large_staged_tiles(dev, monkeypatch):
     x, y = _ints(g, -3, 4, (m, k), torch.float16, dev), _ints(g, -2, 3, (k, n), torch.float16, dev)
     assert torch.equal(U.gemm_fp16(x, U.prepare_gemm_b(y)).double(), x.double() @ y.double())
     assert "x256_y256" in U.last_variant() and U.last_variant().endswith("_s2"), U.last_variant()
+
+
+@pytest.mark.parametrize("M,K", [(300, 600), (1, 640), (129, 8200)])
+def test_fp16_four_columns_through_planes(dev, M, K):
+    g = np.random.RandomState(M + K)
+    a, b = _ints(g, -3, 4, (M, K), torch.float16, dev), _ints(g, -2, 3, (K, 4), torch.float16, dev)
+    ref = a.double() @ b.double()
+    assert U.gemm_fp16_workspace_bytes(M, 4, K) > 0
+    assert torch.equal(U.gemm_fp16(a, b, workspace=True).double(), ref)
+    assert "planes" in U.last_variant(), U.last_variant()
+    assert torch.equal(U.gemm_fp16(a, b, "float16", workspace=True), ref.half())

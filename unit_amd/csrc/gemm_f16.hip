@@ -261,6 +261,7 @@ int gemm_f16_ws_splits(int M, int N, int K) {
   const int nk = ceil_div(K * 2, 64), forced = tuning_override("UNIT_AMD_GEMM_F16_SPLITK");
   const long tiles = tiles_of_128(M, N);
   if (forced > 0) return forced < nk ? forced : nk;
+  if (N < 8) return gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K, nk);  // its kernel has 128 x 128 tiles alone
   if (tiles >= 256) return 1;
   if (tiles >= 128) return K >= 3072 ? 3 : 1;
   const size_t fit = kStaticScratchBytes / ((size_t)M * N * 4);
