@@ -190,3 +190,15 @@ def test_fp16_four_columns_through_planes(dev, M, K):
     assert torch.equal(U.gemm_fp16(a, b, workspace=True).double(), ref)
     assert "planes" in U.last_variant(), U.last_variant()
     assert torch.equal(U.gemm_fp16(a, b, "float16", workspace=True), ref.half())
+
+
+@pytest.mark.parametrize("M,N,K,out,kept", [(4405, 1536, 160, "float16", True), (6000, 704, 640, "float16", True),
+                                            (6000, 704, 128, "float16", False), (6000, 704, 672, "float16", False),
+                                            (6000, 720, 256, "float16", False), (6000, 704, 256, "float32", False)])
+def test_fp16_results_on_128_tiles(dev, M, N, K, out, kept):
+    g = np.random.RandomState(M + N + K)
+    a, b = _ints(g, -3, 4, (M, K), torch.float16, dev), _ints(g, -2, 3, (K, N), torch.float16, dev)
+    ref = (a.double() @ b.double()).to(getattr(torch, out))
+    for operand in (b, U.prepare_gemm_b(b)):
+        assert torch.equal(U.gemm_fp16(a, operand, out), ref), U.last_variant()
+        assert ("dma" in U.last_variant()) == kept, U.last_variant()

@@ -109,7 +109,7 @@ int run_gemm_f16_group(const char *what, const char *tag, const void *a, const v
   const int forced = OUT_F16 || whole ? 1 : tuning_override("UNIT_AMD_GEMM_F16_SPLITK");
   const long tiles = tiles_of_128(M, N);
   const int least = forced <= 0 && tiles < 12 && K >= 512 ? 2 : 1;
-  GroupPlan plan = plan_group(M, N, K * 2, least, forced > 0 || tiles > 64 ? 1 : 19, kAtomicSplits);
+  GroupPlan plan = plan_group(M, N, K * 2, least, forced > 0 || tiles > 64 ? 1 : 19, kAtomicSplits, OUT_F16 ? 2 : 4);
   if (forced > 0) plan.splits = forced;
   const GroupGemm p{static_cast<const char *>(a), static_cast<const char *>(b), (u32)((size_t)M * K * 2),
                     (u32)((size_t)N * K * 2), M, N, K * 2, YM == Y_COLS ? N * 2 : K * 2, nullptr, c, C_ATOMIC, 0};
@@ -121,9 +121,12 @@ int run_gemm_f16_group(const char *what, const char *tag, const void *a, const v
 // (1011 x 3584 x 1216, 224 tiles, 15.6 against 16.2 us on the group tile of the same size; 2048^3 22.9 against 24.8), and 512
 // tiles or more (8192 x 1024 x 1024 24.2 and 24.0 us).  The others gain: 1024^3 11.1 -> 7.1 us, 2304 x 2304 x 4096
 // 65.5 -> 57.2, 64 x 4096 x 4096 15.6 -> 14.0.
-inline bool gemm_keeps_128(int M, int N, bool out_f16) {
+// fp16 results of whole 128-byte rows keep them up to 511 tiles for K of 160 to 640 (6000 x 704 x 256 7.3 us of kernel
+// against 8.1, 5000 x 1024 x 512 11.1 and 12.0; K = 128 6.1 and 5.8).
+inline bool gemm_keeps_128(int M, int N, int K, bool out_f16) {
   const long tiles = tiles_of_128(M, N);
-  return tiles >= 512 || (tiles >= 192 && tiles <= 256) || (!out_f16 && tiles < 32 && M > 128);
+  return tiles >= 512 || (tiles >= 192 && tiles <= 256) || (!out_f16 && tiles < 32 && M > 128) ||
+         (out_f16 && tiles > 256 && N % 64 == 0 && K >= 160 && K <= 640);
 }
 
 // (N, K) b and a through registers on 256 x 256 tiles: large results with a K that the direct tiles do not take
@@ -160,7 +163,7 @@ int gemm_f16_bt(const void *a, const void *bt, void *c, int M, int N, int K, hip
       if (K % 64 == 0) return run_gemm_f16_bt_dma<Tile<256, 256, 128, 2, 4>, 2, OUT_F16>(a, bt, c, M, N, K, s);
       return run_gemm_f16_bt_dma<Tile<256, 256, 64, 2, 4>, 4, OUT_F16>(a, bt, c, M, N, K, s);
     }
-    if (gemm_keeps_128(M, N, OUT_F16))
+    if (gemm_keeps_128(M, N, K, OUT_F16))
       return run_gemm_f16_bt_dma<Tile<128, 128, 64, 2, 2>, 4, OUT_F16>(a, bt, c, M, N, K, s, direct_gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K));
   }
   if (gemm_staged_pays(M, N, K, 1.35f)) return run_gemm_f16_bt<Tile<256, 256, 128, 2, 4>, OUT_F16>(a, bt, c, M, N, K, s);
@@ -231,7 +234,7 @@ int gemm_f16(const void *a, const void *b, void *c, int M, int N, int K, hipStre
       return run_gemm_f16_dma_tr<Tile<256, 256, 64, 2, 4>, 4, OUT_F16>(a, b, c, M, N, K, s);
     }
     const int splits = direct_gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K);
-    if (gemm_keeps_128(M, N, OUT_F16) && !(whole && splits > 1))
+    if (gemm_keeps_128(M, N, K, OUT_F16) && !(whole && splits > 1))
       return run_gemm_f16_dma_tr<Tile<128, 128, 64, 2, 2>, 4, OUT_F16>(a, b, c, M, N, K, s, splits);
   }
   // N 4 mod 8, K a whole number of 128-byte stages, and at least 128 tiles of 256 x 128: a straight into LDS, b through
@@ -261,7 +264,10 @@ int gemm_f16_ws_splits(int M, int N, int K) {
   const int nk = ceil_div(K * 2, 64), forced = tuning_override("UNIT_AMD_GEMM_F16_SPLITK");
   const long tiles = tiles_of_128(M, N);
   if (forced > 0) return forced < nk ? forced : nk;
-  if (N < 8) return gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K, nk);  // its kernel has 128 x 128 tiles alone
+  if (N < 8) {  // its kernel has 128 x 128 tiles alone (8 x 4 x 10712: 25.4 us in 83 planes, 18.3 in 19)
+    const int most = gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K, nk);
+    return most < 19 ? most : 19;
+  }
   if (tiles >= 256) return 1;
   if (tiles >= 128) return K >= 3072 ? 3 : 1;
   const size_t fit = kStaticScratchBytes / ((size_t)M * N * 4);

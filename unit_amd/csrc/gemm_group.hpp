@@ -380,8 +380,9 @@ int run_gemm_group(const char *what, const char *tag, GroupGemm p, int splits, h
 // Estimated time (us) of a launch of `tiles` output tiles in `splits` k-ranges: the busiest of the 256 CUs runs
 // w = ceil(tiles * splits / 256) workgroups, per_cu of them at a time (LDS), each t_tile plus t_stage per stage of its
 // reduction share -- or, side by side, share per stage and workgroup (operand delivery into the CU).  Not below the
-// operand + result traffic at `hbm` TB/s, nor below the padded work at `rate` (kilobyte-products per us: with most CUs
-// busy the clock gives).  The constants are least-squares fits to 4200 timings (70 fp16 and 60 int8 shapes per weight
+// padded work at `rate` (kilobyte-products per us: with most CUs busy the clock gives).  Where the operand + result
+// traffic at `hbm` TB/s is the longer of the two, a third of the difference hides behind it (4405 x 1536 x 64 fp16: 64 x 128
+// tiles, 60 of them in a second round, 7.1 us, 128 x 128 in one 5.7).  The constants are least-squares fits to 4200 timings (70 fp16 and 60 int8 shapes per weight
 // layout, 1 x 836 x 2736 to 8192 x 8192 x 2048, every tile and up to 16 splits): the pick is on average 3 % above the
 // best measured tile.  Against the 128 x 128 tiles with k-splits by atomics and the register pipelines that served these
 // shapes, us a call in a row of them: fp16 1000 x 1516 x 1096 24.8 -> 10.3, 64 x 4096 x 4096 15.6 -> 14.0 (b prepared
@@ -416,7 +417,7 @@ inline float group_cost(const GroupCost &g, long M, long N, long kb, int splits,
   const float work = g.launch + g.tile + (float)tiles * g.bx * g.by * kb / (g.rate * 1e6f);
   const float mem = 2.f + (operand_bytes + (float)out_bytes * splits) / (g.hbm * 1e6f);
   t = t > work ? t : work;
-  return t > mem ? t : mem;
+  return ((t > mem ? t : mem) + 0.5f * t) / 1.5f;
 }
 
 inline long tiles_of_128(int M, int N) { return (long)ceil_div(M, 128) * ceil_div(N, 128); }
@@ -428,9 +429,9 @@ struct SplitCost {
 };
 constexpr SplitCost kAtomicSplits{2.4f, 1.2f}, kPlaneSplits{2.8f, 4.5f};
 
-inline GroupPlan plan_group(int M, int N, int kb, int min_splits, int max_splits, SplitCost split) {
+inline GroupPlan plan_group(int M, int N, int kb, int min_splits, int max_splits, SplitCost split, int out_elem = 4) {
   GroupPlan best{0, 1, 1e30f};
-  const long nk = ceil_div(kb, 64), operands = (long)M * kb + (long)N * kb, out = (long)M * N * 4;
+  const long nk = ceil_div(kb, 64), operands = (long)M * kb + (long)N * kb, out = (long)M * N * out_elem;
   if (min_splits > nk) min_splits = (int)nk;
   if (max_splits < min_splits) max_splits = min_splits;
   for (int i = 0; i < kGroupTiles; ++i) {
