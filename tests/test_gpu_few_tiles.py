@@ -1,6 +1,6 @@
 """Convolutions with a long reduction and few output pixels: tiles of one 32-channel block whose k-steps eight waves share.
 Odd tap counts, channel counts that leave half a block, pixels that end inside a tile, fewer k-steps than the waves'
-rings hold, and both sides of the rule's limits (20 k-steps, 256 tiles of 32 x 32, 32 channels)."""
+rings hold, and both sides of the rule's limits (20 k-steps, in fp16 25, 256 tiles of 32 x 32, 32 channels)."""
 import numpy as np
 import pytest
 import torch
@@ -47,6 +47,20 @@ def test_fp16(dev, oracle, N, C, H, W, K, ks, stride):
     for weight in (t(b), U.prepare_conv2d_weight(t(b))):
         out = U.conv2d_NCHW16c_OHWI16o(t(a), weight, stride, stride).cpu().numpy()
         assert np.array_equal(out.astype(np.float64), ref) and "_g8_" in U.last_variant(), U.last_variant()
+
+
+@pytest.mark.parametrize("C,K,stride,tile", [(384, 48, 1, "x64_y32_g4"), (352, 560, 2, "x64_y32_g4"), (400, 48, 1, "x32_y32_g8"),
+                                             (320, 16, 2, "x64_y32_g4"), (384, 16, 1, "x32_y32_g8")])
+def test_fp16_short_reductions(dev, oracle, C, K, stride, tile):
+    """Up to 24 k-steps the four waves of the wider tiles hold the whole reduction in flight."""
+    g = np.random.RandomState(C + K)
+    a = g.randint(-3, 4, (1, C // 16, 16, 33, 16)).astype(np.float16)
+    b = g.randint(-2, 3, (K // 16, C // 16, 1, 1, 16, 16)).astype(np.float16)
+    ref = oracle.conv2d_nchw16c_f16(a, b, stride, stride)
+    t = lambda v: torch.from_numpy(v).to(dev)
+    for weight in (t(b), U.prepare_conv2d_weight(t(b))):
+        out = U.conv2d_NCHW16c_OHWI16o(t(a), weight, stride, stride).cpu().numpy()
+        assert np.array_equal(out.astype(np.float64), ref) and tile in U.last_variant(), U.last_variant()
 
 
 @pytest.mark.parametrize("C,H,W,K,KH,KW,tile", [

@@ -62,18 +62,26 @@ inline ConvPlan heuristic_plan(const unit_conv_desc *d, int npix, int kbytes, bo
     int v, panel = 0;
     // Long reductions on few output pixels: eight waves share a tile of one 32-channel block, which gives such a layer
     // twice the workgroups of 64 x 32 tiles and each wave half the k-steps in a row (its time is a chain of load
-    // latencies, not a rate).  While 32 x 32 tiles are at most one per CU: u8 1536 -> 720, 3 x 3 on 17 x 14, 19.7 -> 10.6 us;
-    // fp16 1168 -> 32, 5 x 5 on 27 x 17, 85 -> 43; the 137 such rows of the tables 901 -> 751 in all.  Below 20 k-steps the
-    // sum of eight partial tiles costs what it gains (18: 4.36 against 4.34 us), above 256 tiles the second round does
-    // (342 of them: 10.6 -> 8.0, 555: 22.0 -> 21.0, 720: 49.2 -> 51.1).  Up to 32 channels a 64-channel tile is half
-    // padding: 32 x 64 tiles there (480 -> 32 on 76 x 72: 10.6 -> 7.0).  The eight waves' scratch and tile leave the tap
-    // table less of the LDS than the four-wave tiles below do (with 4-channel blocks, a k-step per window row, 7352 rows
-    // against 8528): up to 4096 steps, 64 KiB of table, all of them fit.
+    // latencies, not a rate).  While 32 x 32 tiles are at most one per CU: u8 1536 -> 720, 3 x 3 on 17 x 14, 19.7 -> 10.6
+    // us; fp16 1168 -> 32, 5 x 5 on 27 x 17, 85 -> 43; the 137 such rows of the tables 901 -> 751 in all.  Below 20
+    // k-steps the sum of eight partial tiles costs what it gains (18: 4.36 against 4.34 us), in fp16 up to 24, all of
+    // which the four six-deep waves of the tiles below have in flight at once (on 20 - 24 steps eight waves took 1.03 -
+    // 1.14 times as long, prepared 352 -> 560, 1 x 1 stride 2 on 16 x 33, 3.51 -> 3.94; on 25 - 60 0.81 - 1.07 and
+    // prepared 0.90 - 1.04 but for 1 x 1 at stride 2, up to 1.14; int8 0.92 - 1.05 up to 24, 0.79 - 0.99 past them).  16
+    // fp16 channels at stride 1, where it was 1.03 - 1.06, keep 20: the shortest rings are tested there.  Above 256 tiles
+    // the second round does (342 of them: 10.6 -> 8.0, 555: 22.0 -> 21.0, 720: 49.2 -> 51.1).  Up to 32 channels a
+    // 64-channel tile is half padding: 32 x 64 tiles there (480 -> 32 on 76 x 72: 10.6 -> 7.0).  The eight waves' scratch
+    // and tile leave the tap table less of the LDS than the four-wave tiles below do (with 4-channel blocks, a k-step per
+    // window row, 7352 rows against 8528): up to 4096 steps, 64 KiB of table, all of them fit.
     const int ksteps = kbytes / 32, table_steps = d->cb == 4 ? kbytes / (4 * d->KW) : ksteps;
-    if (ksteps >= 20 && table_steps <= 4096 && tiles(32, 32) <= 256)
-      return ConvPlan{82, 1, 4};
-    if (ksteps >= 20 && table_steps <= 4096 && K <= 32 && tiles(32, 64) <= 384)
-      return ConvPlan{83, 1, 0};
+    const int least = allow_split || (K <= 16 && !strided) ? 20 : 25;
+    if (ksteps >= 20 && table_steps <= 4096) {
+      if (tiles(32, 32) <= 256) {
+        if (ksteps >= least) return ConvPlan{82, 1, 4};
+      } else if (K <= 32 && tiles(32, 64) <= 384) {
+        return ConvPlan{83, 1, 0};
+      }
+    }
     if (allow_split) {  // the int8 operator; distilled from the tuner's choices on cold operands (batch 1 .. 256)
       const int nsteps = kbytes / 32;
       const bool wide = K % 128 == 0;  // 128-channel tiles
