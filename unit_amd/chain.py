@@ -6,8 +6,9 @@ cpu-shapes.log:388-420.
 
 Every layer is the requantising convolution (ops.conv2d_NCHWc_int8_requant): u8 in, u8 out, so a layer's
 output is the next layer's input as it lies in memory.  The runner owns all activation buffers and
-prepared weights, issues nothing but kernel launches through the C ABI (no allocation per call), and
-can therefore be captured into a HIP graph.
+prepared weights and issues nothing but kernel launches through the C ABI (a chain that pays for it as one
+persistent kernel, with a few KiB of the caching allocator's memory per run), and can therefore be captured into
+a HIP graph.
 """
 import ctypes
 from collections import namedtuple
@@ -26,7 +27,7 @@ class ConvChain:
     PreparedConvWeight, `bias` int32 (OC,) or None, integer `scale`, `shift` in 1..62, `stride`, `padding`.
     input_shape: (N, C/16, H, W, 16) of the u8 chain input.
 
-    run(x) launches every layer on the current stream and returns the last layer's output buffer (owned by
+    run(x) runs every layer on the current stream and returns the last layer's output buffer (owned by
     the chain and overwritten by the next run); outputs[i] is layer i's.  graph(x) captures run(x) once and
     returns a callable that replays it (x's storage is the graph's input)."""
 
@@ -91,7 +92,9 @@ class ConvChain:
         if bound != self._bound:
             for d, d.desc, (d.prepared, d.out, d.bias, d.scale, d.shift, src) in zip(self._native, self.descs, bound):
                 d.data = None if src < 0 else bound[src][1]
-            self._bound = bound
+            size = ctypes.c_size_t()  # 0: a chain that runs launch by launch
+            check(self._L.unit_conv_chain_u8_ws_bytes(self._native, count, ctypes.byref(size)))
+            self._bound, self._ws_bytes = bound, size.value
 
     def run(self, x):
         x = ops._dev(x, "x", torch.uint8, 5)
@@ -102,7 +105,10 @@ class ConvChain:
         for i in unnamed:
             if not self._native[i].variant:
                 self._native[i].variant = ctypes.addressof(self._names) + 96 * i
-        check(self._L.unit_conv_chain_u8(self._native, len(self._native), x.data_ptr(), ops._stream()))
+        # a run's own: runs of one chain on several streams share nothing but the activation buffers
+        ws = torch.empty(self._ws_bytes, dtype=torch.uint8, device=x.device)
+        check(self._L.unit_conv_chain_u8_ws(self._native, len(self._native), x.data_ptr(), ws.data_ptr(), self._ws_bytes,
+                                            ops._stream()))
         for i in unnamed:
             self.variants[i] = self._names[96 * i:96 * i + 96].split(b"\0")[0].decode()
             self._native[i].variant = None

@@ -1,0 +1,593 @@
+// A chain of requantising convolutions (unit_conv_chain_u8) inside one persistent kernel.
+//
+// What bounds a chain of launches: a layer of a residual network at batch 32 is 6.5 - 14 us of which the launch gap, the
+// argument fetch, the decode, the first loads from cold L2s and the last write-back are 4 - 5 us, fifty-two times over
+// (ResNet-50 behind its stem: 489 us; at batch 1, where nothing else is left, 237 us).  Here
+//   * the images are dealt to the XCDs in groups (batch / 8 each), and an XCD takes its group through all layers: what a
+//     layer writes, the next one reads from the same L2, with no write-back and no cold cache in between;
+//   * a layer's tile waits for the tiles of its source layer that it reads, not for the layer: a flag per tile, set when
+//     the tile's results have reached the L2 (a message from one workgroup to another through the L2 takes 0.2 us; a
+//     kernel boundary 1.2 - 1.5 us and the caches);
+//   * the weights of a tile, which depend on no other tile, are under way while it waits.
+// Measured against the launches, us: ResNet-50 batch 1 213 / 237, 8 223 / 310, 16 252 / 361, 32 389 / 489, 128 1057 /
+// 1294; ResNet-18 95 / 100 at 4, 106 / 139 at 16, 133 / 168 at 32.
+//
+// Tiles are handed out by a ticket counter per XCD, in the order of the layers.  A workgroup that holds a ticket runs, and
+// everything its tile waits for has an earlier ticket, so the earliest unfinished tile never waits: the kernel ends
+// whatever part of the grid the device keeps resident.  Groups are claimed, not assigned: an XCD that runs out of
+// tickets takes the next group, so the work is done also where some XCD has no workgroup at all.
+//
+// A wave reads the results of other CUs of its XCD with agent-scope (sc1) loads, which pass the CU's vector cache by and
+// hit in the L2 (188 clocks against 108 for a hit in the vector cache); plain loads could return a line that the CU
+// fetched before its neighbour wrote it, and dropping the vector cache with buffer_inv sc1 holds up the CU's other loads (1190 us
+// for the ResNet-50 above).  Stores and flags are plain: they stay in the L2 (an sc1 store goes to memory, and a load
+// after it with it).
+//
+// The tile: four waves of 64 channels x 64 pixels each, operands straight into registers as in conv_direct.hpp, either
+// side by side (over channels first, then pixels) or in two or four k-groups that share a tile.
+#include "conv_direct.hpp"
+#include "conv_prepare.hpp"
+#include "host.hpp"
+
+#include <algorithm>
+
+namespace unit {
+
+int conv_geom(const unit_conv_desc *d, int tapb, ConvGeom *g, const char *what);  // abi.hip
+
+namespace {
+
+constexpr int kWaves = 4, kThreads = 64 * kWaves;
+constexpr int kPerCu = 2;         // workgroups per CU: 222 VGPRs (three of 168 with three k-steps in flight: 392 us at batch 32, 234 at 8)
+constexpr int kDepth = 5;         // k-steps of fragments in flight per wave
+constexpr int kMaxXcd = 16, kMaxChain = 256;
+constexpr int kAgent = 16;        // sc1
+// Polls a wave may spend in all before it stops waiting (seconds; a whole chain takes some thousand): every wave ends, also
+// after a fault in another one.
+constexpr int kPolls = 1 << 24;
+
+// q = n / d for n * d < 2^31
+inline u32 small_div(int d) { return (u32)(0x80000000ull / (unsigned)d) + (d != 1); }
+__device__ __forceinline__ int quot(int n, u32 mul) { return (int)__umulhi((u32)n << 1, mul); }
+
+// A layer as the kernel reads it.  Sizes are those of a group of images.
+struct alignas(128) ChainStep {
+  const char *data, *w;
+  char *out;
+  const int *bias;
+  int first, next;  // its tickets in a group's program; a tile's flag has the ticket's number
+  int scale, K, nsteps, ntaps, ohw, img_bytes;
+  u32 by_ohw, by_ow, by_win, by_kw, by_nct;  // small_div
+  int nct;                                   // channel tiles; a pixel tile's are neighbours
+  int src_first, src_nct;                    // the source layer's first ticket and channel tiles
+  u32 row_ones;                              // ConvGeom
+  unsigned short H, W, OW;
+  unsigned char pt, pl, KH, KW, sh, sw;
+  unsigned char shift, win, mode;  // KH * KW; chain_reduce's MODE
+  unsigned char flat;              // 1 x 1 at stride 1: output pixels are input pixels
+  unsigned char reads, src_shift;  // the source is a layer of the chain, its pixel tiles are 1 << src_shift
+  unsigned char kg_log, wx_log, wy_log, unused;
+};
+static_assert(sizeof(ChainStep) == 128, "ChainStep");
+using StepPtr = const __attribute__((address_space(4))) ChainStep *;
+// a layer's 128 bytes as two scalar loads of a cache line each
+__device__ __forceinline__ ChainStep load_step(StepPtr p) {
+  const auto *q = (const __attribute__((address_space(4))) v16i *)p;
+  struct alignas(128) Raw {
+    v16i a, b;
+  } r{q[0], q[1]};
+  return __builtin_bit_cast(ChainStep, r);
+}
+
+// The workspace: control words (zeroed by chain_setup), then the layers.  Words: groups claimed; a line per XCD with its
+// ticket counter; per XCD the groups it has claimed (+ 1), in its order; per group the tiles' flags.  No line of it is
+// written by two XCDs but the first.
+constexpr int kCtlGroups = 0, kCtlTickets = 32, kCtlSlots = kCtlTickets + 32 * kMaxXcd;
+
+struct ChainArgs {
+  const ChainStep *steps;
+  int *ctl;
+  int count, images, per, groups;
+  int slot_pitch, flags0, flag_pitch;
+  FastDiv by_tickets;
+};
+
+// The layers travel as kernel arguments (at most 4 KiB of them), so that a captured chain keeps the ones it was captured
+// with, and nothing is copied from host memory.
+constexpr int kSetupSteps = 31;
+struct ChainSetup {
+  ChainStep s[kSetupSteps];
+};
+
+__global__ __launch_bounds__(256) void chain_setup(const ChainSetup a, ChainStep *steps, int count, v4i *clear, int nclear) {
+  if (blockIdx.x == 0 && threadIdx.x < count * 8)
+    reinterpret_cast<v4i *>(steps)[threadIdx.x] = reinterpret_cast<const v4i *>(a.s)[threadIdx.x];
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < nclear; i += gridDim.x * 256) clear[i] = v4i{0, 0, 0, 0};
+}
+
+struct alignas(16) ChainLds {
+  v4i part[kWaves][3][4][64];  // [wave][block, its own left out][quad][lane]: partial blocks for their owners
+  int addend[kWaves][64];
+  int ticket[2], group;
+};
+
+__device__ __forceinline__ int load_l2(const int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// a step's pointers come out of scalar registers: told to be global memory, or every load through them is a flat one
+template <class T>
+using Global = const __attribute__((address_space(1))) T *;
+
+// MODE 0: one tap per channel block, an even number of them, no padding; 1: any window without padding; 2: any window
+struct TapWalk {
+  int ntaps, KW, win, row_skip, ch_skip, hw16, w16;
+  u32 by_win, by_kw;
+};
+
+template <int MODE>
+__device__ __forceinline__ void chain_reduce(v16i (&acc)[2][2], __amdgpu_buffer_rsrc_t wbuf, const u32 (&wp)[2], __amdgpu_buffer_rsrc_t data, const u32 lane16,
+                                             int (&pixoff)[2], const u32 (&inside)[2], v4i (&xf)[kDepth][2], int half, int s0, int s1,
+                                             int slast, const TapWalk &tw) {
+  constexpr int D = kDepth;
+  v4i yf[D][2];
+  auto for_slots = [&](auto f) __attribute__((always_inline)) {
+    f(std::integral_constant<int, 0>{});
+    f(std::integral_constant<int, 1>{});
+    f(std::integral_constant<int, 2>{});
+    if constexpr (D > 3) f(std::integral_constant<int, 3>{});
+    if constexpr (D > 4) f(std::integral_constant<int, 4>{});
+    if constexpr (D > 5) f(std::integral_constant<int, 5>{});
+  };
+  // The state of the running tap; it advances by a k-step per fetch and stops at the wave's last one.  Uniform and
+  // without branches, so that the loads keep one order on all paths.
+  int sf = s0;
+  int kw = 0, pos = 0, off = 0;
+  if constexpr (MODE != 0) {
+    const int t = 2 * s0, ci = quot(t, tw.by_win);
+    pos = t - ci * tw.win;
+    const int kh = quot(pos, tw.by_kw);
+    kw = pos - kh * tw.KW;
+    off = ci * tw.hw16 + kh * tw.w16 + kw * 16;
+  } else {
+    off = 2 * s0 * tw.hw16;
+    if (half) pixoff[0] += tw.hw16, pixoff[1] += tw.hw16;
+  }
+  auto fetch_d = [&](auto slot) __attribute__((always_inline)) {
+    constexpr int U = decltype(slot)::value;
+    if constexpr (MODE == 0) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        yf[U][j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(data, pixoff[j], off, kAgent));
+      const bool more = sf < slast;
+      sf += more;
+      off += more ? 2 * tw.hw16 : 0;
+    } else {
+      int k2 = kw, p2 = pos, o2 = off;
+      auto step = [&]() __attribute__((always_inline)) {
+        ++k2, ++p2, o2 += 16;
+        const bool cr = k2 == tw.KW;
+        k2 = cr ? 0 : k2;
+        o2 += cr ? tw.row_skip : 0;
+        const bool cc = p2 == tw.win;
+        p2 = cc ? 0 : p2;
+        o2 += cc ? tw.ch_skip : 0;
+      };
+      step();
+      const bool odd = 2 * sf + 1 < tw.ntaps;
+      const int o = half ? (odd ? o2 : off) : off, ps = half ? (odd ? p2 : 31) : pos;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        u32 v = (u32)(pixoff[j] + o);
+        if constexpr (MODE == 2) v |= ~(u32)__builtin_amdgcn_sbfe((int)inside[j], (u32)ps, 1u);
+        yf[U][j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(data, (int)v, 0, kAgent));
+      }
+      step();
+      const bool more = sf < slast;
+      sf += more;
+      kw = more ? k2 : kw, pos = more ? p2 : pos, off = more ? o2 : off;
+    }
+  };
+  auto consume = [&](auto slot) __attribute__((always_inline)) {
+    constexpr int U = decltype(slot)::value;
+    v4i y[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int d = 0; d < 4; ++d) y[j][d] = yf[U][j][d] ^ (int)0x80808080;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] = OpI8::mma(xf[U][i], y[j], acc[i][j]);
+  };
+  for_slots([&](auto u) __attribute__((always_inline)) { fetch_d(u); });
+  __builtin_amdgcn_sched_barrier(0);
+  u32 sw = (u32)min(s0 + D, slast) * 1024u;
+  const u32 swlast = (u32)slast * 1024u;
+  auto round = [&]() __attribute__((always_inline)) {
+    for_slots([&](auto u) __attribute__((always_inline)) {
+      consume(u);
+      __builtin_amdgcn_sched_barrier(0);
+      constexpr int U = decltype(u)::value;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) xf[U][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wbuf, (int)lane16, (int)(wp[i] + sw), 0));
+      sw = min(sw + 1024u, swlast);
+      fetch_d(u);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  int s = s0;
+  if (s + D < s1) {
+    round();
+    for (s += D; s + D < s1; s += D) round();
+  }
+  for_slots([&](auto u) __attribute__((always_inline)) {
+    if (s + decltype(u)::value < s1) consume(u);
+    __builtin_amdgcn_sched_barrier(0);
+  });
+}
+
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kPerCu, kPerCu))) void chain_run(const ChainArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char lds_raw[];
+  ChainLds &sh = *reinterpret_cast<ChainLds *>(lds_raw);
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int xcd = __builtin_amdgcn_s_getreg((31 << 11) | 20) & (kMaxXcd - 1);
+  const StepPtr steps = (StepPtr)(unsigned long long)a.steps;
+  int *const tickets = a.ctl + kCtlTickets + 32 * xcd;
+  int *const slots = a.ctl + kCtlSlots + xcd * a.slot_pitch;
+  if (tid == 0) sh.ticket[0] = __hip_atomic_fetch_add(tickets, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  int turn = 0, q_now = -1, group = 0, l = 0, budget = kPolls;
+  for (;;) {
+    const int ticket = __builtin_amdgcn_readfirstlane(sh.ticket[turn]);
+    turn ^= 1;
+    int q, idx;
+    a.by_tickets.divmod(ticket, q, idx);
+    if (q != q_now) {
+      if (q >= a.groups) break;
+      if (tid == 0) {
+        int v;
+        if (idx == 0) {
+          v = __hip_atomic_fetch_add(a.ctl + kCtlGroups, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+          store_result<0>(result_buffer(slots), (u32)q * 4u, v);
+        } else {
+          while ((v = load_l2(slots + q)) == 0 && --budget > 0) __builtin_amdgcn_s_sleep(1);
+          if (v == 0) v = a.groups + 1;
+        }
+        sh.group = v - 1;
+      }
+      __syncthreads();
+      group = __builtin_amdgcn_readfirstlane(sh.group);
+      q_now = q;
+      l = 0;
+    }
+    if (group >= a.groups) break;
+    ChainStep L = load_step(steps + l);
+    while (idx >= L.next) L = load_step(steps + ++l);
+    const int nct = L.nct, ohw = L.ohw, K = L.K, nsteps = L.nsteps, kl = L.kg_log, wl = L.wx_log;
+    const int local = idx - L.first;
+    const int pt = quot(local, L.by_nct), ct = local - pt * nct;
+    const int image0 = group * a.per, npix = min(a.per, a.images - image0) * ohw;
+    const int m0 = pt << (6 + L.wy_log), me = min(m0 + (64 << L.wy_log), npix) - 1;
+    if (m0 > me) {  // the last group may hold fewer images
+      if (tid == 0) sh.ticket[turn] = __hip_atomic_fetch_add(tickets, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __syncthreads();
+      continue;
+    }
+    const int set = wave >> kl, kidx = wave & ((1 << kl) - 1);
+    const int x0 = ((ct << wl) + (set & ((1 << wl) - 1))) * 64, y0 = m0 + (set >> wl) * 64;
+    const bool idle = x0 >= K || y0 >= npix;
+    const int s0 = idle ? 0 : (nsteps * kidx) >> kl, s1 = idle ? 0 : (nsteps * (kidx + 1)) >> kl;
+    const int slast = max(s1 - 1, s0);
+
+    // the source layer's tiles that this one reads: their flags are asked for first and looked at when the loads of
+    // the weights are out
+    const int H = L.H, W = L.W;
+    int lo = m0, hi = me;
+    if (!L.flat) {
+      const int n0 = quot(m0, L.by_ohw), n1 = quot(me, L.by_ohw), hw = H * W;
+      const int r0 = quot(m0 - n0 * ohw, L.by_ow) * L.sh - L.pt;
+      const int r1 = quot(me - n1 * ohw, L.by_ow) * L.sh - L.pt + L.KH - 1;
+      lo = n0 * hw + min(max(r0, 0), H - 1) * W;
+      hi = n1 * hw + max(min(r1, H - 1), 0) * W + W - 1;
+    }
+    int *const flags = a.ctl + (size_t)(u32)(a.flags0 + group * a.flag_pitch);
+    const int *const wanted = flags + L.src_first;
+    const int fa = (lo >> L.src_shift) * L.src_nct, fb = ((hi >> L.src_shift) + 1) * L.src_nct;
+    const int flag = load_l2(wanted + (u32)min(fa + lane, max(fb - 1, 0)));
+    __builtin_amdgcn_sched_barrier(0);
+
+    // weights: the ring's fragments depend on the tile alone
+    const u32 lane16 = (u32)lane * 16u;
+    const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc((void *)L.w, 0, -1, 0x00020000);
+    const int kblocks = (K + 31) >> 5;
+    u32 wp[2];  // byte offsets of the two 32-channel blocks; blocks past the last one re-read it
+#pragma unroll
+    for (int i = 0; i < 2; ++i) wp[i] = (u32)(min((x0 >> 5) + i, kblocks - 1) * nsteps) * 1024u;
+    v4i xf[kDepth][2];
+#pragma unroll
+    for (int u = 0; u < kDepth; ++u)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        xf[u][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wbuf, (int)lane16, (int)(wp[i] + (u32)min(s0 + u, slast) * 1024u), 0));
+    const u32 cc = (u32)min(x0 + lane, K - 1) * 4u;
+    const int add0 = __builtin_amdgcn_raw_buffer_load_b32(wbuf, (int)cc, kblocks * nsteps * 1024, 0);
+    const int add1 = L.bias ? ((Global<int>)L.bias)[cc >> 2] : 0;
+    __builtin_amdgcn_sched_barrier(0);
+
+    const __amdgpu_buffer_rsrc_t data = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(L.data + (size_t)image0 * (size_t)(u32)L.img_bytes), 0, min(a.per, a.images - image0) * L.img_bytes, 0x00020000);
+    int pixoff[2];
+    u32 inside[2], dst[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int m = y0 + j * 32 + l32;
+      const int mm = m < npix ? m : 0;
+      const int n = quot(mm, L.by_ohw), pix = mm - n * ohw;
+      dst[j] = ((u32)(n * (K >> 4) * ohw) + (u32)pix) * 16u;
+      inside[j] = 0;
+      if (L.flat) {
+        pixoff[j] = n * L.img_bytes + pix * 16;
+      } else {
+        const int oh = quot(pix, L.by_ow), ow = pix - __mul24(oh, (int)L.OW);
+        const int ih0 = __mul24(oh, (int)L.sh) - L.pt, iw0 = __mul24(ow, (int)L.sw) - L.pl;
+        pixoff[j] = n * L.img_bytes + (__mul24(ih0, W) + iw0) * 16;
+        if (L.mode == 2) {
+          const int KH = L.KH, KW = L.KW;
+          const int ka = min(max(-iw0, 0), KW), kb = min(max(W - iw0, ka), KW);
+          const int ra = min(max(-ih0, 0), KH), rb = min(max(H - ih0, ra), KH);
+          const u32 rows = L.row_ones & ((1u << __mul24(rb, KW)) - (1u << __mul24(ra, KW)));
+          inside[j] = m < npix ? ((1u << kb) - (1u << ka)) * rows : 0u;
+        }
+      }
+    }
+    if (L.reads) {
+      if (!__all(flag != 0)) {
+        while (!__all(load_l2(wanted + (u32)min(fa + lane, fb - 1)) != 0) && --budget > 0) __builtin_amdgcn_s_sleep(1);
+      }
+      for (int b = fa + 64; b < fb; b += 64) {
+        while (!__all(load_l2(wanted + (u32)min(b + lane, fb - 1)) != 0) && --budget > 0) __builtin_amdgcn_s_sleep(1);
+      }
+    }
+
+    v16i acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+    const TapWalk tw{L.ntaps, L.KW, L.win, (W - L.KW) * 16, (H - L.KH) * W * 16, H * W * 16, W * 16, L.by_win, L.by_kw};
+    if (L.mode == 0)
+      chain_reduce<0>(acc, wbuf, wp, data, lane16, pixoff, inside, xf, half, s0, s1, slast, tw);
+    else if (L.mode == 1)
+      chain_reduce<1>(acc, wbuf, wp, data, lane16, pixoff, inside, xf, half, s0, s1, slast, tw);
+    else
+      chain_reduce<2>(acc, wbuf, wp, data, lane16, pixoff, inside, xf, half, s0, s1, slast, tw);
+    int next = 0;
+    if (tid == 0) next = __hip_atomic_fetch_add(tickets, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+
+    sh.addend[wave][lane] = add0 + add1;
+    const __amdgpu_buffer_rsrc_t obuf = result_buffer(L.out + (size_t)image0 * (size_t)(u32)(K * ohw));
+    auto store = [&](int i, int j, const v16i &v) __attribute__((always_inline)) {
+      const v4i row = requant_row(v, &sh.addend[wave][i * 32], L.scale, L.shift, half);
+      const int c = x0 + i * 32 + half * 16;
+      if (c < K && y0 + j * 32 + l32 < npix) store_result<0>(obuf, dst[j] + (u32)((c >> 4) * ohw) * 16u, row);
+    };
+    // KG k-groups: each parks the blocks that others own and adds up its own
+    auto finish = [&](auto kg_) __attribute__((always_inline)) {
+      constexpr int KG = decltype(kg_)::value, OWN = 4 / KG;
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        if (b / OWN != kidx) {
+#pragma unroll
+          for (int q4 = 0; q4 < 4; ++q4)
+            sh.part[wave][KG == 2 ? b & 1 : b - (b > kidx)][q4][lane] =
+                v4i{acc[b >> 1][b & 1][4 * q4], acc[b >> 1][b & 1][4 * q4 + 1], acc[b >> 1][b & 1][4 * q4 + 2],
+                    acc[b >> 1][b & 1][4 * q4 + 3]};
+        }
+      __syncthreads();
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        if (b / OWN == kidx) {
+          v16i v = acc[b >> 1][b & 1];
+#pragma unroll
+          for (int o = 1; o < KG; ++o) {
+            const int other = (kidx + o) & (KG - 1);
+#pragma unroll
+            for (int q4 = 0; q4 < 4; ++q4) {
+              const v4i x = sh.part[set * KG + other][KG == 2 ? b & 1 : b - (b > other)][q4][lane];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) v[4 * q4 + e] += x[e];
+            }
+          }
+          store(b >> 1, b & 1, v);
+        }
+    };
+    if (kl == 2) {
+      finish(std::integral_constant<int, 4>{});
+    } else if (kl == 1) {
+      finish(std::integral_constant<int, 2>{});
+    } else {
+#pragma unroll
+      for (int b = 0; b < 4; ++b) store(b >> 1, b & 1, acc[b >> 1][b & 1]);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // results are in this XCD's L2
+    if (tid == 0) sh.ticket[turn] = next;
+    __syncthreads();
+    if (tid == 0) store_result<0>(result_buffer(flags), (u32)idx * 4u, 1);
+  }
+}
+
+struct ChainPlan {
+  int per, groups, tickets, slot_pitch, flags0, flag_pitch, clear_words;
+  size_t steps_off, bytes;
+};
+
+struct Range {
+  const char *a, *b;
+};
+
+// false: the layers run one launch each
+bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainStep *st, ChainPlan *p) {
+  if (count < 2 || count > kMaxChain) return false;
+  const int N = layers[0].desc.N;
+  if (N < 1) return false;
+  // one group per XCD (smaller ones, two in a row: batch 64 773 against 621 us; larger ones leave XCDs idle)
+  const int per = (N + 7) / 8;
+  p->per = per;
+  p->groups = (N + per - 1) / per;
+  long first = 0;
+  double here = 7, launches = 0;  // us, below
+  Range outs[kMaxChain];
+  for (int i = 0; i < count; ++i) {
+    const unit_chain_layer &l = layers[i];
+    const unit_conv_desc &d = l.desc;
+    if (!l.prepared || !l.out || l.shift < 1 || l.shift > 62 || check_aligned("chain", {l.data, l.prepared, l.out})) return false;
+    if (d.N != N || d.cb != 16 || d.dh != 1 || d.dw != 1 || d.C <= 0 || d.K <= 0 || d.KH <= 0 || d.KW <= 0) return false;
+    ConvGeom g;
+    if (conv_geom(&d, 16, &g, "chain") != UNIT_OK) return false;
+    if (d.KH * d.KW > 31 || d.sh > 255 || d.sw > 255 || d.pt > 255 || d.pl > 255) return false;
+    const long out_bytes = (long)g.npix * d.K;
+    if (out_bytes > 0x7fffffffl) return false;
+    outs[i] = Range{static_cast<const char *>(l.out), static_cast<const char *>(l.out) + out_bytes};
+    ChainStep &s = st[i];
+    s.data = static_cast<const char *>(l.data ? l.data : x);
+    s.w = static_cast<const char *>(l.prepared);
+    s.out = static_cast<char *>(l.out);
+    s.bias = l.bias;
+    int scale = l.scale, shift = l.shift;
+    while (shift < 33 && scale >= -(1 << 30) && scale < (1 << 30)) scale *= 2, ++shift;
+    s.scale = scale;
+    s.shift = (unsigned char)shift;
+    s.K = d.K;
+    s.ntaps = g.ntaps;
+    s.nsteps = (g.ntaps + 1) / 2;
+    s.ohw = g.OH * g.OW;
+    s.win = (unsigned char)(d.KH * d.KW);
+    s.img_bytes = (int)g.img_bytes;
+    s.by_ohw = small_div(s.ohw);
+    s.by_ow = small_div(g.OW);
+    s.by_win = small_div(s.win);
+    s.by_kw = small_div(d.KW);
+    s.H = (unsigned short)d.H, s.W = (unsigned short)d.W, s.OW = (unsigned short)g.OW;
+    s.pt = (unsigned char)d.pt, s.pl = (unsigned char)d.pl;
+    s.row_ones = g.row_ones;
+    s.KH = (unsigned char)d.KH, s.KW = (unsigned char)d.KW, s.sh = (unsigned char)d.sh, s.sw = (unsigned char)d.sw;
+    const bool masked = d.pt || d.pl || d.pb || d.pr;
+    s.mode = masked ? 2 : (s.win == 1 && s.ntaps % 2 == 0 ? 0 : 1);
+    s.flat = !masked && d.KH == 1 && d.KW == 1 && d.sh == 1 && d.sw == 1;
+    const double gmac = 1e-9 * s.ohw * d.K * s.ntaps * 16;  // of an image
+    here += 2.5 + gmac * per / 0.1, launches += 3.9 + gmac * N / 0.65;
+    const long npix = (long)per * s.ohw;
+    if (npix * s.ohw > 0x7fffffffl) return false;
+    // k-groups: a tile costs 2.6 us beside its reduction (decode, first loads, requantisation, stores, flag), 0.4 more with
+    // k-groups, and 0.25 us per k-step of a wave; an XCD runs 64 at a time
+    const long wt = (long)ceil_div(d.K, 64) * ((npix + 63) / 64);
+    int kg = 1;
+    double best = 1e30;
+    for (int k = 1; k <= 4 && k <= s.nsteps; k *= 2) {
+      const double rounds = std::max(1.0, (double)wt * k / 4 / 64);
+      const double t = rounds * (2.6 + (k > 1 ? 0.4 : 0.0) + 0.25 * ceil_div(s.nsteps, k));
+      if (t < best) best = t, kg = k;
+    }
+    const int sets = 4 / kg;
+    int wx = 1;
+    while (wx < sets && d.K >= 128 * wx) wx *= 2;
+    const int wy = sets / wx;
+    s.kg_log = (unsigned char)(kg >> 1), s.wx_log = (unsigned char)(wx >> 1), s.wy_log = (unsigned char)(wy >> 1);
+    s.nct = ceil_div(d.K, 64 * wx);
+    s.by_nct = small_div(s.nct);
+    const long npt = (npix + 64 * wy - 1) / (64 * wy);
+    if (npt * s.nct * s.nct > 0x7fffffffl) return false;
+    s.first = (int)first;
+    first += npt * s.nct;
+    s.next = (int)first;
+    if (first * (p->groups + 2) + 4096 > 0x7fffffffl) return false;
+    s.reads = 0, s.src_first = 0, s.src_nct = 0, s.src_shift = 0, s.unused = 0;
+    for (int j = i - 1; j >= 0; --j)
+      if (layers[j].out == s.data) {
+        if (layers[j].desc.K != d.C || st[j].OW != d.W || st[j].ohw != d.H * d.W) return false;
+        s.reads = 1;
+        s.src_first = st[j].first, s.src_nct = st[j].nct, s.src_shift = (unsigned char)(6 + st[j].wy_log);
+        break;
+      }
+  }
+  // Short chains, and few images through large layers, stay launches: the kernel costs 7 us before its first tile, 2.5 us a
+  // layer and 10 us per GMAC of an XCD's group, a launch 3.9 us and 1.5 us per GMAC of the batch.  us here / as launches:
+  // 3 x 3 64 -> 64 on 56 x 56, batch 1, 2 layers 13.7 / 7.9, 12 layers 48.9 / 48.0; batch 8, 3 layers 17.6 / 20.1, 8 layers
+  // 36.9 / 53.6; 1 x 1 256 -> 256 on 14 x 14, batch 1, 2 layers 10.0 / 7.5, 8 layers 24.3 / 30.3; seven 3 x 3 layers of 128 to 512
+  // channels from 56 x 56 on, batch 1 54.8 / 34.6, 8 56.4 / 57.3, 128 398 / 432.
+  if (here > 0.95 * launches) return false;
+  // The layers no longer run one after the other: none may write what another one reads or writes, but for a source's
+  // whole result.
+  std::sort(outs, outs + count, [](const Range &u, const Range &v) { return u.a < v.a; });
+  for (int i = 1; i < count; ++i)
+    if (outs[i].a < outs[i - 1].b) return false;
+  const auto clear_of_outs = [&](const void *q, size_t n) {
+    const char *a = static_cast<const char *>(q), *b = a + n;
+    const Range *r = std::upper_bound(outs, outs + count, a, [](const char *v, const Range &u) { return v < u.b; });
+    return r == outs + count || r->a >= b;
+  };
+  for (int i = 0; i < count; ++i) {
+    const unit_conv_desc &d = layers[i].desc;
+    if (!clear_of_outs(st[i].w, prepared_layout(d.K, d.C, d.KH, d.KW, 16, 1).total_bytes)) return false;
+    if (st[i].bias && !clear_of_outs(st[i].bias, (size_t)d.K * 4)) return false;
+    if (!st[i].reads && !clear_of_outs(st[i].data, (size_t)N * d.C * d.H * d.W)) return false;
+  }
+  p->tickets = (int)first;
+  p->slot_pitch = (p->groups + 31) / 32 * 32;
+  p->flags0 = kCtlSlots + kMaxXcd * p->slot_pitch;
+  p->flag_pitch = (p->tickets + 31) / 32 * 32;
+  p->clear_words = p->flags0 + p->groups * p->flag_pitch;
+  p->steps_off = ((size_t)p->clear_words * 4 + 255) / 256 * 256;
+  p->bytes = p->steps_off + (size_t)count * sizeof(ChainStep);
+  return true;
+}
+
+}  // namespace
+}  // namespace unit
+
+extern "C" int unit_conv_chain_u8_ws_bytes(const unit_chain_layer *layers, int32_t count, size_t *bytes) {
+  using namespace unit;
+  if (!layers || !bytes || count < 0) return fail(UNIT_E_ARG, "unit_conv_chain_u8_ws_bytes: null pointer or negative count");
+  ChainStep st[kMaxChain];
+  ChainPlan p;
+  *bytes = plan_chain(layers, count, nullptr, st, &p) ? p.bytes : 0;
+  return UNIT_OK;
+}
+
+extern "C" int unit_conv_chain_u8_ws(const unit_chain_layer *layers, int32_t count, const void *x, void *ws, size_t ws_bytes,
+                                     unit_stream_t stream) {
+  using namespace unit;
+  const char *what = "unit_conv_chain_u8_ws";
+  if (!layers || !x || count < 0) return fail(UNIT_E_ARG, "%s: null pointer or negative count", what);
+  ChainStep st[kMaxChain];
+  ChainPlan p;
+  const bool pinned = tuning_override("UNIT_AMD_CONV_VARIANT") > 0 || tuning_override("UNIT_AMD_CONV_PANEL") > 0 ||
+                      tuning_override("UNIT_AMD_CONV_SPLITK") > 0;
+  if (!ws || reinterpret_cast<uintptr_t>(ws) % 16 || reinterpret_cast<uintptr_t>(x) % 16 || pinned ||
+      !plan_chain(layers, count, x, st, &p) || ws_bytes < p.bytes)
+    return unit_conv_chain_u8(layers, count, x, stream);
+  if (int rc = check_device()) return rc;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  char *base = static_cast<char *>(ws);
+  ChainStep *steps = reinterpret_cast<ChainStep *>(base + p.steps_off);
+  for (int i = 0; i < count; i += kSetupSteps) {
+    ChainSetup a;
+    const int n = std::min(kSetupSteps, count - i);
+    memcpy(a.s, st + i, n * sizeof(ChainStep));
+    const int quads = i == 0 ? ceil_div(p.clear_words, 4) : 0;
+    hipLaunchKernelGGL(chain_setup, dim3(std::max(1, std::min(256, ceil_div(quads, 256)))), dim3(256), 0, s, a, steps + i, n,
+                       reinterpret_cast<v4i *>(base), quads);
+  }
+  const ChainArgs a{steps,        reinterpret_cast<int *>(base), count,        layers[0].desc.N,           p.per, p.groups,
+                    p.slot_pitch, p.flags0,                      p.flag_pitch, FastDiv::make(p.tickets)};
+  hipLaunchKernelGGL(chain_run, dim3(256 * kPerCu), dim3(kThreads), sizeof(ChainLds), s, a);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(UNIT_E_LAUNCH, "%s: launch: %s", what, hipGetErrorString(e));
+  for (int i = 0; i < count; ++i)
+    if (layers[i].variant)
+      snprintf(layers[i].variant, 96, "q8chain_x%d_y%d_g%d_d%d", 64 << st[i].wx_log, 64 << st[i].wy_log, 1 << st[i].kg_log, kDepth);
+  set_variant("q8chain_l%d_n%d_d%d", count, p.per, kDepth);
+  return UNIT_OK;
+}

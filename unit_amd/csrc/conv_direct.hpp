@@ -145,23 +145,19 @@ __device__ __forceinline__ void store_block(const typename ConvEpilogue<Op>::Par
   }
 }
 
-// Requantised output: one 32-channel x 32-pixel int32 block -> u8 (N, K/16, OH, OW, 16),
+// Requantised output: one 32-channel x 32-pixel int32 block -> u8,
 //   q = clamp(((acc + addend[c]) * scale + 2^(shift-1)) >> shift, 0, 255)
 // with the product and the shift in 64 bits.  A lane holds 16 channels of one pixel (4 h + 8 q + e);
 // after packing each quad into a dword the two 32-lane halves swap two dwords each, so that half h
-// holds the 16 bytes of plane c0 / 16 + h of its pixel: one 16-byte store per lane, 512 consecutive
-// bytes per plane, no LDS.
-template <class Op>
-__device__ __forceinline__ void store_block_q8(const typename ConvEpilogue<Op>::Params &p, const v16i &acc, const int *wsb,
-                                               int c0, int m0, int lane) {
-  const int l32 = lane & 31, half = lane >> 5;
+// holds the 16 bytes of plane c0 / 16 + h of its pixel, which is what this returns: no LDS.
+__device__ __forceinline__ v4i requant_row(const v16i &acc, const int *wsb, int scale, int shift, int half) {
   int d[4];
-  if (p.shift >= 33) {
+  if (shift >= 33) {
     // The rounding term 2^(shift-1) is a multiple of 2^32, so it and the shift act on the high
     // dword of the product alone: floor((hi * 2^32 + lo + R) / 2^shift) = (hi + R / 2^32) >> (shift - 32).
     // (The host doubles scale and increments shift while that keeps scale in int32 -- the same
     // rational number -- so practical shifts arrive here.)
-    const int rhi = 1 << (p.shift - 33), sh = p.shift - 32;
+    const int rhi = 1 << (shift - 33), sh = shift - 32;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       int t[4];
@@ -169,7 +165,7 @@ __device__ __forceinline__ void store_block_q8(const typename ConvEpilogue<Op>::
       for (int e = 0; e < 4; ++e) {
         int v = acc[4 * q + e];
         if (wsb) v += wsb[8 * q + 4 * half + e];
-        t[e] = __mulhi(v, p.scale) + rhi;
+        t[e] = __mulhi(v, scale) + rhi;
       }
       // v_ashr_pk_u8_i32: shift, saturate to 0..255 and pack two values into the low 16 bits (the
       // builtin's result is 16 bits wide; the upper half of the register is not zero, and the
@@ -179,7 +175,7 @@ __device__ __forceinline__ void store_block_q8(const typename ConvEpilogue<Op>::
       d[q] = (int)__builtin_amdgcn_perm(hi, lo, 0x05040100u);
     }
   } else {
-    const long long rnd = 1ll << (p.shift - 1);
+    const long long rnd = 1ll << (shift - 1);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       u32 packed = 0;
@@ -187,7 +183,7 @@ __device__ __forceinline__ void store_block_q8(const typename ConvEpilogue<Op>::
       for (int e = 0; e < 4; ++e) {
         int v = acc[4 * q + e];
         if (wsb) v += wsb[8 * q + 4 * half + e];
-        long long t = ((long long)v * p.scale + rnd) >> p.shift;
+        long long t = ((long long)v * scale + rnd) >> shift;
         t = t < 0 ? 0 : (t > 255 ? 255 : t);
         packed |= (u32)t << (8 * e);
       }
@@ -198,7 +194,15 @@ __device__ __forceinline__ void store_block_q8(const typename ConvEpilogue<Op>::
   // half 1 keeps d2, d3 (20-23, 28-31) and needs the partner's d2, d3 (16-19, 24-27)
   const int s0 = half ? d[0] : d[2], s1 = half ? d[1] : d[3];
   const int r0 = __shfl_xor(s0, 32), r1 = __shfl_xor(s1, 32);
-  const v4i row = half ? v4i{r0, d[2], r1, d[3]} : v4i{d[0], r0, d[1], r1};
+  return half ? v4i{r0, d[2], r1, d[3]} : v4i{d[0], r0, d[1], r1};
+}
+
+// The block -> u8 (N, K/16, OH, OW, 16): one 16-byte store per lane, 512 consecutive bytes per plane.
+template <class Op>
+__device__ __forceinline__ void store_block_q8(const typename ConvEpilogue<Op>::Params &p, const v16i &acc, const int *wsb,
+                                               int c0, int m0, int lane) {
+  const int l32 = lane & 31, half = lane >> 5;
+  const v4i row = requant_row(acc, wsb, p.scale, p.shift, half);
   const int m = m0 + l32, c = c0 + half * 16;
   if (c < p.K && m < p.npix) {
     int n, pix;
