@@ -161,6 +161,30 @@ def last_variant():
     return _lib.last_variant()
 
 
+# ------------------------------------------------------------------------------- native calls
+class _Calls:
+    """The operators' common case as native functions (csrc/calls.cpp): each returns the result, or None for a call that
+    it does not take, which then runs through the Python below.  Bound on first use to the library that ctypes loaded."""
+
+    _LIBRARY = ("unit_conv_out_hw", "unit_conv2d_nchwc_u8s8s32", "unit_conv2d_nchwc_u8s8s32_prepared", "unit_conv2d_nchwc_s8s8s32_fused",
+                "unit_conv2d_nchwc_s8s8s32_fused_prepared", "unit_conv2d_nchwc_u8s8u8_requant_prepared", "unit_conv3d_ncdhwc_s8s8s32",
+                "unit_conv2d_nchw16c_f16f32", "unit_conv2d_nchw16c_f16f32_prepared", "unit_conv2d_nchw_f16f32",
+                "unit_conv2d_nchw_f16f32_ws_bytes", "unit_dense_dotprod_u8s8s32", "unit_dense_u8s8s32", "unit_dense_u8s8s32_prepared",
+                "unit_gemm_f16", "unit_gemm_f16_prepared", "unit_gemm_f16_ws")
+
+    def __getattr__(self, name):  # the first use of each function
+        L = _lib.load()
+        from . import _calls
+        _calls.bind(tuple(ctypes.cast(getattr(L, f), ctypes.c_void_p).value for f in self._LIBRARY), PreparedConvWeight,
+                    PreparedDenseWeight, PreparedGemmB, torch.int8, torch.float16)
+        fn = getattr(_calls, name)
+        setattr(self, name, fn)
+        return fn
+
+
+_native = _Calls()
+
+
 # ------------------------------------------------------------------------------- prepared weights
 class PreparedConvWeight:
     """Convolution weights in the MFMA fragment order of the kernels (see prepare_conv2d_weight).
@@ -233,6 +257,10 @@ def conv2d_NCHWc_int8(data, kernel, stride, padding, dilation=1, out_dtype="int3
     As in TVM the channel block is taken from the tensor shapes; `layout` / `out_layout` are
     checked for form only (the reference's driver passes 'NCHW4c' for 16-channel blocks too).
     """
+    if out_dtype == "int32" and layout == "NCHW16c" and out_layout == "NCHW16c":
+        out = _native.conv_u8(data, kernel, stride, padding, dilation)
+        if out is not None:
+            return out
     data = _dev(data, "data", torch.uint8, 5)
     prepared = isinstance(kernel, PreparedConvWeight)
     if not prepared:
@@ -273,6 +301,10 @@ def conv2d_NCHWc_int8_fused(data, kernel, bias, scale, stride, padding, dilation
     (result.log:25) into the store: returns int32 (N, out_channels, OH, OW), out_channels
     (default K) being the channel count before the caller padded it up to a multiple of 16.
     """
+    if out_dtype == "int32" and layout == "NCHW16c" and out_layout == "NCHW16c" and out_channels is None:
+        out = _native.conv_fused(data, kernel, bias, scale, stride, padding, dilation)
+        if out is not None:
+            return out
     data = _dev(data, "data", torch.int8, 5)
     prepared = isinstance(kernel, PreparedConvWeight)
     if not prepared:
@@ -331,6 +363,9 @@ def conv2d_NCHWc_int8_requant(data, kernel, bias, scale, shift, stride, padding,
     (apps/cpu/relay/result.log:15-24); this is the integer requantisation that follows it in a
     quantised network.
     """
+    out = _native.conv_requant(data, kernel, bias, scale, shift, stride, padding, dilation)
+    if out is not None:
+        return out
     data = _dev(data, "data", torch.uint8, 5)
     if not isinstance(kernel, PreparedConvWeight):
         kernel = prepare_conv2d_weight(kernel)
@@ -372,6 +407,9 @@ def conv3d_NCDHWc_int8(data, kernel, stride=1):
     kernel int8  (K/16, C/cb, KD, KH, KW, cb/4, 16, 4)
     returns int32 (N, K/16, OD, OH, OW, 16)
     """
+    out = _native.conv3d(data, kernel, stride)
+    if out is not None:
+        return out
     data = _dev(data, "data", torch.int8, 6)
     kernel = _dev(kernel, "kernel", torch.int8, 8)
     _, ref, shape = _plan_3d(data.shape, kernel.shape, int(stride))
@@ -383,6 +421,10 @@ def conv3d_NCDHWc_int8(data, kernel, stride=1):
 def dense_dotprod(data, weight, bias=None, out_dtype="int32"):
     """u8 (M, K) x s8 packed (N/128, K/4, 128, 4) -> i32 (M, N) = data . W^T.
     A 2-D weight (N, K) is taken as the un-packed relay.nn.dense operand."""
+    if bias is None and out_dtype == "int32" and not isinstance(weight, PreparedDenseWeight):
+        out = _native.dense(data, weight)
+        if out is not None:
+            return out
     data = _dev(data, "data", torch.uint8, 2)
     weight = _dev(weight, "weight", torch.int8, (2, 4))
     if out_dtype != "int32":
@@ -427,6 +469,10 @@ def prepare_dense_weight(weight):
 
 def dense(data, weight, out_dtype="int32"):
     """relay.nn.dense(x u8 (M, K), w s8 (N, K)) -> i32 (M, N); `weight` may be a PreparedDenseWeight."""
+    if out_dtype == "int32":
+        out = _native.dense(data, weight) if not isinstance(weight, torch.Tensor) or weight.dim() == 2 else None
+        if out is not None:
+            return out
     if isinstance(weight, PreparedDenseWeight):
         data = _dev(data, "data", torch.uint8, 2)
         if out_dtype != "int32":
@@ -479,6 +525,10 @@ def gemm_fp16(a, b, out_dtype="float32", workspace=None):
     apps/gpu/gemm-pack.py:9,14-18 takes it (re-laid on every call: prepare it once instead).
     workspace (b (K, N) only): True, or a uint8 tensor of `gemm_fp16_workspace_bytes(M, N, K)` bytes: k-splits keep
     their partial tiles in it and are added in split order (run-to-run identical results, also for float16 output)."""
+    if out_dtype == "float32" or out_dtype == "float16":
+        out = _native.gemm(a, b, out_dtype == "float16", workspace)
+        if out is not None:
+            return out
     a = _dev(a, "a", torch.float16, 2)
     if out_dtype not in ("float32", "float16"):
         raise ValueError(f"out_dtype: expected 'float32' or 'float16', got {out_dtype!r}")
@@ -525,6 +575,9 @@ def conv2d_NCHW16c_OHWI16o(a, b, stride_h, stride_w, out_type="float32"):
     Returns float32 (N, K/16, OH, OW, 16)."""
     if out_type != "float32":
         raise ValueError(f"out_type: only 'float32' is supported, got {out_type!r}")
+    out = _native.conv_f16(a, b, stride_h, stride_w)
+    if out is not None:
+        return out
     a = _dev(a, "a", torch.float16, (4, 5))
     L = _lib.load()
     if isinstance(b, PreparedConvWeight):
