@@ -453,9 +453,40 @@ inline float large_tile_cost(int M, int N, int kb) {
   return 2.f + (float)((tiles + 255) / 256) * (3.f + (tiles <= 200 ? 18.7f : 24.9f) * kb / 2048) + (float)M * N * 4 / 6.4e6f;
 }
 
+// Stages of 128 bytes instead of 64 while there is at most one tile per CU.  A row of a stage is then a whole cache line
+// (with 64 bytes every line is asked for twice, half of it each time), and the waves meet at half as many barriers.  Their
+// rings leave room for one workgroup per CU (96 - 144 KiB), where those of 64-byte stages have up to three: past 256 tiles
+// that is worth more.  us on operands that change from call to call, 64 / 128 bytes: fp16 700 x 2304 x 3008 20.5 / 16.9,
+// 900 x 1664 x 1600 12.6 / 10.8, prepared 500 x 2048 x 2048 11.3 / 9.3, 1500 x 1536 x 1504 17.4 / 15.1; int8 packed 900 x
+// 1664 x 1600 11.4 / 9.9, 1500 x 1536 x 1504 14.7 / 11.8, row-major 700 x 2304 x 3008 16.0 / 13.3; geometric mean over the 84 of
+// 231 random products that it takes 1.11, lowest 0.98; fp16 1000 x 1516 x 1096, whose rows of b end inside lines, 10.5 / 10.5.
+// The other way: 512 tiles of 64 x 64 (2000 x 1024 x 512) 6.8 / 7.9, 640 bytes of reduction (702 x 1216 x 320) 4.3 / 4.5 and, on
+// 32 x 32 tiles, 1088 (93 x 2112 x 544) 3.75 / 3.88, b by
+// columns on 32 x 32 tiles, whose rows of b stay 64 bytes, 15 x 2560 x 5488 17.6 / 20.1.  int8 products of up to 64 rows and
+// 4096 columns keep the tiles that the tests name for them.
+template <class Op, int YM>
+bool group_wide_stages(const GroupGemm &p, const GroupPlan &plan) {
+  const GroupCost &g = kGroupCosts[plan.tile];
+  return plan.splits == 1 && p.kb >= (plan.tile < 2 ? 1536 : 960) && (long)ceil_div(p.M, g.bx) * ceil_div(p.N, g.by) <= 256 &&
+         !(Op::kInt && p.M <= 64 && p.N <= 4096) && !(YM == Y_COLS && plan.tile < 2);
+}
+
 template <class Op, int YM, int WS, bool OUT_F16>
 int run_group_plan(const char *what, const char *tag, const GroupGemm &p, const GroupPlan &plan, hipStream_t s) {
   using Wide = std::conditional_t<YM == Y_VNNI, GroupTile<2, 2, 2, 2, 1, 64, 4>, GroupTile<1, 2, 4, 2, 1, 64, 4>>;
+  if (group_wide_stages<Op, YM>(p, plan)) {
+    switch (plan.tile) {
+      case 0:
+      case 1:
+        if constexpr (YM != Y_COLS) return run_gemm_group<Op, GroupTile<1, 1, 1, 1, 4, 128, 3>, YM, WS, OUT_F16>(what, tag, p, 1, s);
+        break;
+      case 2: return run_gemm_group<Op, GroupTile<1, 1, 1, 2, 4, 128, 3>, YM, WS, OUT_F16>(what, tag, p, 1, s);
+      case 3: return run_gemm_group<Op, GroupTile<1, 1, 2, 2, 2, 128, 3>, YM, WS, OUT_F16>(what, tag, p, 1, s);
+      case 4: return run_gemm_group<Op, GroupTile<1, 2, 2, 2, 2, 128, 3>, YM, WS, OUT_F16>(what, tag, p, 1, s);
+      case 5: return run_gemm_group<Op, GroupTile<1, 2, 4, 2, 1, 128, 3>, YM, WS, OUT_F16>(what, tag, p, 1, s);
+      default: break;
+    }
+  }
   switch (plan.tile) {
     case 0: return run_gemm_group<Op, GroupTile<1, 1, 1, 1, 8, 64, 4>, YM, WS, OUT_F16>(what, tag, p, plan.splits, s);
     case 1: return run_gemm_group<Op, GroupTile<1, 1, 1, 1, 4, 64, 4>, YM, WS, OUT_F16>(what, tag, p, plan.splits, s);
