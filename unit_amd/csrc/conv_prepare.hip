@@ -31,6 +31,9 @@ int conv_planar_c4(const unit_conv_desc *d, const ConvGeom &g, int in_channels, 
                    int scale, void *out, int oc, hipStream_t s);  // conv_planar_c4.hip
 int conv_q8_prepared(const ConvPlan &plan, const unit_conv_desc *d, const ConvGeom &g, const void *data, const void *w,
                      const int *addend, const int *bias, int scale, int shift, void *out, hipStream_t s);  // conv_prepared_q8.hip
+bool patch_f16_takes(const unit_conv_desc *d, const ConvGeom &g);
+int conv_f16_patch(const unit_conv_desc *d, const ConvGeom &g, const void *a, const void *w, void *out,
+                       hipStream_t s);  // conv_patch_f16.hip
 int conv_f16_prepared(const ConvPlan &plan, const unit_conv_desc *d, const ConvGeom &g, const void *a, const void *w,
                       void *out, hipStream_t s);  // conv_prepared_f16.hip
 
@@ -355,6 +358,8 @@ extern "C" int unit_conv2d_nchw16c_f16f32_prepared(const unit_conv_desc *d, cons
   ConvGeom g;
   if (int rc = check_prepared_conv(what, d, 32, &g, a, prepared, out)) return rc;
   const int ntable = (int)(sizeof(kTunedF16Prepared) / sizeof(kTunedF16Prepared[0])) - 1;
+  if (tuning_override("UNIT_AMD_CONV_VARIANT") <= 0 && patch_f16_takes(d, g))
+    return conv_f16_patch(d, g, a, prepared, out, static_cast<hipStream_t>(stream));
   const ConvPlan p = plan_prepared(d, g, g.ntaps * 32, kTunedF16Prepared, ntable, false, true);
   if (kConvTiles[p.variant].lds) return conv_f16_prepared_lds(p, d, g, a, prepared, out, static_cast<hipStream_t>(stream));
   return conv_f16_prepared(p, d, g, a, prepared, out, static_cast<hipStream_t>(stream));
