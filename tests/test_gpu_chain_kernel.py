@@ -19,6 +19,10 @@ BLOCKS = [(64, (1, 1), 1, 0, None), (64, (3, 3), 1, 1, None), (256, (1, 1), 1, 0
 DEEP = [(256, (3, 3), 1, 1, None), (256, (3, 3), 1, 1, None), (1040, (1, 1), 1, 0, None), (96, (1, 1), 1, 0, None),
         (96, (3, 3), 2, 1, None), (96, (1, 1), 1, 0, None), (96, (1, 1), 1, 0, None), (96, (1, 1), 1, 0, 4),
         (96, (1, 1), 1, 0, 4), (96, (1, 1), 1, 0, 5), (96, (1, 1), 1, 0, None), (96, (1, 1), 1, 0, None)]
+# 3 x 3 windows over whole pairs of channel blocks per k-group: strides, uneven and no padding
+THREES = [(64, (3, 3), 2, (1, 0, 2, 1), None), (64, (3, 3), 1, 0, None), (128, (3, 3), 1, 1, None), (32, (3, 3), 3, 2, 1),
+          (128, (3, 3), 1, (2, 2, 0, 1), None), (64, (3, 3), 1, 1, None), (96, (3, 3), 2, 2, None), (32, (3, 3), 1, 2, None),
+          (256, (3, 3), 1, 2, None), (64, (3, 3), 2, 1, None), (32, (3, 3), 1, 1, None), (64, (3, 3), 1, 1, 4)]
 WIDE = [(512, (1, 1), 1, 0, None), (1024, (1, 1), 1, 0, None), (1008, (1, 1), 1, 0, 0)] + [(32, (1, 1), 1, 0, None)] * 10
 CASES = {
     "odd_blocks_uneven_groups": (ODD, 9, 48, 21, 17),
@@ -27,6 +31,8 @@ CASES = {
     "blocks_uneven_groups": (BLOCKS, 17, 64, 14, 13),
     "blocks_one_image": (BLOCKS, 1, 64, 28, 28),
     "wide": (WIDE, 8, 256, 23, 23),
+    "threes": (THREES, 12, 32, 27, 30),
+    "threes_one_image": (THREES, 1, 32, 30, 27),
     "deep": (DEEP, 3, 128, 9, 8),
     "deep_few_pixels": (DEEP, 64, 128, 3, 3),
 }

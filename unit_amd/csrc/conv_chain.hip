@@ -9,8 +9,8 @@
 //     the tile's results have reached the L2 (a message from one workgroup to another through the L2 takes 0.2 us; a
 //     kernel boundary 1.2 - 1.5 us and the caches);
 //   * the weights of a tile, which depend on no other tile, are under way while it waits.
-// Measured against the launches, us: ResNet-50 batch 1 213 / 237, 8 223 / 310, 16 252 / 361, 32 389 / 489, 128 1057 /
-// 1294; ResNet-18 95 / 100 at 4, 106 / 139 at 16, 133 / 168 at 32.
+// Measured against the launches, us: ResNet-50 batch 1 201 / 238, 8 212 / 311, 16 241 / 362, 32 380 / 474; ResNet-18
+// 81 / 94 at 1, 98 / 139 at 16, 119 / 169 at 32.
 //
 // Tiles are handed out by a ticket counter per XCD, in the order of the layers.  A workgroup that holds a ticket runs, and
 // everything its tile waits for has an earlier ticket, so the earliest unfinished tile never waits: the kernel ends
@@ -38,7 +38,7 @@ int conv_geom(const unit_conv_desc *d, int tapb, ConvGeom *g, const char *what);
 namespace {
 
 constexpr int kWaves = 4, kThreads = 64 * kWaves;
-constexpr int kPerCu = 2;         // workgroups per CU: 222 VGPRs (three of 168 with three k-steps in flight: 392 us at batch 32, 234 at 8)
+constexpr int kPerCu = 2;         // workgroups per CU: 235 VGPRs (three of 168 with three k-steps in flight: 392 us at batch 32, 234 at 8)
 constexpr int kDepth = 5;         // k-steps of fragments in flight per wave
 constexpr int kMaxXcd = 16, kMaxChain = 256;
 constexpr int kAgent = 16;        // sc1
@@ -225,6 +225,68 @@ __device__ __forceinline__ void chain_reduce(v16i (&acc)[2][2], __amdgpu_buffer_
   });
 }
 
+// MODE 3: 3 x 3 windows, padded or not, and a share of whole periods of nine k-steps (two channel blocks).  The taps of
+// a period are known here: an offset and a mask bit per lane and step, set up once, instead of a walk per step; and the
+// loads of the ring stand between the MFMAs, where a wave's other instructions cost nothing.  us with the walk of MODE 2 /
+// here: ResNet-50 batch 1 213 / 201, 16 252 / 241, 32 389 / 380; ResNet-18 106 / 98 at 16, 133 / 119 at 32.  Loads between the
+// MFMAs of the other modes give under 1 % at 1 x 1 windows and take 3 % at ResNet-18, batch 32.  A ring of six in a period of 18 spilled.
+__device__ __forceinline__ void chain_reduce_3x3(v16i (&acc)[2][2], __amdgpu_buffer_rsrc_t wbuf, const u32 (&wp)[2],
+                                                 __amdgpu_buffer_rsrc_t data, const u32 lane16, const int (&pixoff)[2],
+                                                 const u32 (&inside)[2], v4i (&xf)[kDepth][2], int half, int s0, int s1,
+                                                 int hw16, int w16) {
+  constexpr int D = 3, P = 9;
+  static_assert(P % D == 0 && D <= kDepth, "the ring's slots repeat with the period");
+  // offset of tap 2 s + half of a period; all ones, out of range, outside the image
+  u32 at[9][2];
+#pragma unroll
+  for (int s = 0; s < 9; ++s) {
+    const int e = 2 * s, o = 2 * s + 1;
+    const int oe = (e / 9) * hw16 + (e % 9 / 3) * w16 + (e % 9 % 3) * 16, oo = (o / 9) * hw16 + (o % 9 / 3) * w16 + (o % 9 % 3) * 16;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      at[s][j] = (u32)(pixoff[j] + (half ? oo : oe)) | ~(u32)__builtin_amdgcn_sbfe((int)inside[j], (u32)(half ? o % 9 : e % 9), 1u);
+  }
+  v4i yf[D][2];
+  int soff = 2 * (s0 / 9) * hw16;
+  u32 sw = (u32)s0 * 1024u;
+  auto load_d = [&](int s, int j) __attribute__((always_inline)) {
+    yf[s % D][j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(data, (int)at[s % 9][j], soff + s / 9 * (2 * hw16), kAgent));
+  };
+#pragma unroll
+  for (int s = 0; s < D; ++s) load_d(s, 0), load_d(s, 1);
+  __builtin_amdgcn_sched_barrier(0);
+  auto period = [&](auto last) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < P; ++s) {
+      const bool fetch = !decltype(last)::value || s + D < P;
+      v4i y[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) y[j][d] = yf[s % D][j][d] ^ (int)0x80808080;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          acc[i][j] = OpI8::mma(xf[s % D][i], y[j], acc[i][j]);
+          __builtin_amdgcn_sched_barrier(0);
+          if (fetch && i == 0) load_d(s + D, j);
+          if (fetch && j == 1)
+            xf[s % D][i] = __builtin_bit_cast(
+                v4i, __builtin_amdgcn_raw_buffer_load_b128(wbuf, (int)lane16, (int)(wp[i] + sw + (u32)(s + D) * 1024u), 0));
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+  };
+  for (int s = s0; s + P < s1; s += P) {
+    period(std::false_type{});
+    soff += 2 * hw16;
+    sw += P * 1024u;
+  }
+  period(std::true_type{});
+}
+
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kPerCu, kPerCu))) void chain_run(const ChainArgs a) {
   extern __shared__ __attribute__((aligned(16))) char lds_raw[];
   ChainLds &sh = *reinterpret_cast<ChainLds *>(lds_raw);
@@ -331,7 +393,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kPerCu
         const int oh = quot(pix, L.by_ow), ow = pix - __mul24(oh, (int)L.OW);
         const int ih0 = __mul24(oh, (int)L.sh) - L.pt, iw0 = __mul24(ow, (int)L.sw) - L.pl;
         pixoff[j] = n * L.img_bytes + (__mul24(ih0, W) + iw0) * 16;
-        if (L.mode == 2) {
+        if (L.mode >= 2) {
           const int KH = L.KH, KW = L.KW;
           const int ka = min(max(-iw0, 0), KW), kb = min(max(W - iw0, ka), KW);
           const int ra = min(max(-ih0, 0), KH), rb = min(max(H - ih0, ra), KH);
@@ -357,7 +419,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kPerCu
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
     const TapWalk tw{L.ntaps, L.KW, L.win, (W - L.KW) * 16, (H - L.KH) * W * 16, H * W * 16, W * 16, L.by_win, L.by_kw};
-    if (L.mode == 0)
+    if (L.mode == 3) {
+      if (s0 < s1) chain_reduce_3x3(acc, wbuf, wp, data, lane16, pixoff, inside, xf, half, s0, s1, H * W * 16, W * 16);
+    } else if (L.mode == 0)
       chain_reduce<0>(acc, wbuf, wp, data, lane16, pixoff, inside, xf, half, s0, s1, slast, tw);
     else if (L.mode == 1)
       chain_reduce<1>(acc, wbuf, wp, data, lane16, pixoff, inside, xf, half, s0, s1, slast, tw);
@@ -493,6 +557,7 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
     const int sets = 4 / kg;
     int wx = 1;
     while (wx < sets && d.K >= 128 * wx) wx *= 2;
+    if (d.KH == 3 && d.KW == 3 && s.ntaps % (18 * kg) == 0) s.mode = 3;
     const int wy = sets / wx;
     s.kg_log = (unsigned char)(kg >> 1), s.wx_log = (unsigned char)(wx >> 1), s.wy_log = (unsigned char)(wy >> 1);
     s.nct = ceil_div(d.K, 64 * wx);
