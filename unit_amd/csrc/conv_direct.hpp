@@ -13,7 +13,8 @@
 //   * fp16 data (N, C/16, H, W, 16): a pixel and tap are 32 bytes = one k-step; lanes 0-31 take
 //     channels 0-7, lanes 32-63 channels 8-15;
 //   * fp16 weights (K/16, C/16, KH, KW, 16 in, 16 out): out-channel o of a tap owns the halves at
-//     o*2 + i*32: eight 16-bit loads per lane, packed in pairs by the load instruction.
+//     o*2 + i*32, eight 16-bit loads per lane.  Instead a lane takes eight out-channels of one in-channel with a 16-byte
+//     load, and groups of eight lanes transpose their 8 x 8 halves in registers (transpose8) before the MFMA.
 //
 // A workgroup is KG waves that all compute the same (32 TX channels) x (32 TY pixels) tile, each
 // over its own share of the k-steps with a D-deep register prefetch ring; the partial tiles are
@@ -45,6 +46,35 @@
 #include "trace.hpp"
 
 namespace unit {
+
+// The lanes of an aligned group of eight hold rows of an 8 x 8 matrix of halves, lane = row: afterwards lane = column.
+// Lane bit 0 changes places with the half of a dword, bits 1 and 2 with the dword's number.  `sel` is transpose8_sel(lane).
+// Twenty VALU instructions per fragment in place of eight 16-bit loads: those kept the address unit busy for 32 clocks a
+// fragment, half as long again as all loads of prepared weights take together, and held the register of every half.  us before /
+// after: 912 -> 16, 5 x 5 on 8 x 11, batch 9 33.5 / 24.8; 1 x 1 864 -> 288 on 16 x 12, batch 2 6.4 / 4.8; 256 -> 256 on 16 x 16,
+// batch 32 16.9 / 14.4; with the planner's new lines geometric mean 1.18 over 160 random shapes and 1.17 over the table's.
+// Slower where the results' stores are all there is: 1 x 1 128 -> 512 on 56 x 56, batch 32, 40.0 / 41.4 - 42.9.
+__device__ __forceinline__ u32 transpose8_sel(int lane) { return lane & 1 ? 0x03020706u : 0x05040100u; }
+__device__ __forceinline__ v4i transpose8(v4i x, u32 sel, bool bit1) {
+  constexpr int kXor1 = 0xb1, kXor2 = 0x4e, kFrom4Up = 0x104, kFrom4Down = 0x114;  // quad_perm, row_shl:4, row_shr:4
+#pragma unroll
+  for (int d = 0; d < 4; ++d)
+    x[d] = (int)__builtin_amdgcn_perm((u32)__builtin_amdgcn_update_dpp(0, x[d], kXor1, 0xf, 0xf, true), (u32)x[d], sel);
+#pragma unroll
+  for (int d = 0; d < 4; d += 2) {
+    const int a = __builtin_amdgcn_update_dpp(0, x[d], kXor2, 0xf, 0xf, true);
+    const int b = __builtin_amdgcn_update_dpp(0, x[d + 1], kXor2, 0xf, 0xf, true);
+    x[d] = bit1 ? b : x[d];
+    x[d + 1] = bit1 ? x[d + 1] : a;
+  }
+  v4i y;
+#pragma unroll
+  for (int d = 0; d < 2; ++d) {
+    y[d] = __builtin_amdgcn_update_dpp(x[d], x[d + 2], kFrom4Down, 0xf, 0xa, false);  // lanes 4 - 7 of each eight
+    y[d + 2] = __builtin_amdgcn_update_dpp(x[d + 2], x[d], kFrom4Up, 0xf, 0x5, false);  // lanes 0 - 3
+  }
+  return y;
+}
 
 // PAD: the convolution has zero padding, so taps can fall outside the image and are masked per
 // lane; without it every tap of every valid pixel lies inside and the masking code is left out.
@@ -292,7 +322,7 @@ __global__ __launch_bounds__(S::NT) __attribute__((amdgpu_waves_per_eu(PREP && !
   for (int i = 0; i < TX; ++i) {
     int n = x0 + i * 32 + l32;
     n = n < ep.K ? n : ep.K - 1;
-    xoff[i] = (u32)(n >> 4) * (u32)(g.ntaps * WTAP) + (kInt ? (u32)(n & 15) * 4u : (u32)(n & 15) * 2u + (u32)half * 256u);
+    xoff[i] = (u32)(n >> 4) * (u32)(g.ntaps * WTAP) + (kInt ? (u32)(n & 15) * 4u : (u32)((lane & 7) + half * 8) * 32u + (u32)(lane & 8) * 2u);
     if constexpr (PREP) {  // blocks past the last one re-read it
       const int kb = min((x0 >> 5) + i, (ep.K - 1) >> 5);
       xoff[i] = ((u32)(kb * nsteps) * 64u + (u32)lane) * 16u;
@@ -316,6 +346,8 @@ __global__ __launch_bounds__(S::NT) __attribute__((amdgpu_waves_per_eu(PREP && !
     if constexpr (D > 6) f(std::integral_constant<int, 6>{});
     if constexpr (D > 7) f(std::integral_constant<int, 7>{});
   };
+
+  const u32 wsel = transpose8_sel(lane);  // fp16 weights in the reference's layout
 
   // prefetch ring: D k-steps of fragments in registers
   v4i xf[D][TX], yf[D][TY];
@@ -352,10 +384,7 @@ __global__ __launch_bounds__(S::NT) __attribute__((amdgpu_waves_per_eu(PREP && !
 #pragma unroll
         for (int d = 0; d < 4; ++d) xf[U][i][d] = *reinterpret_cast<const int *>(wgt + o + d * 64);
       } else {
-        v8h h;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) h[k] = *reinterpret_cast<const _Float16 *>(wgt + o + k * 32);
-        xf[U][i] = __builtin_bit_cast(v4i, h);
+        xf[U][i] = *reinterpret_cast<const v4i *>(wgt + o);  // rows of in-channels; consume() transposes
       }
     }
   };
@@ -528,9 +557,12 @@ __global__ __launch_bounds__(S::NT) __attribute__((amdgpu_waves_per_eu(PREP && !
         for (int d = 0; d < 4; ++d) wsx[i] = __builtin_amdgcn_sdot4(xf[U][i][d], 0x01010101, wsx[i], false);
     }
 #pragma unroll
-    for (int i = 0; i < TX; ++i)
+    for (int i = 0; i < TX; ++i) {
+      v4i x = xf[U][i];
+      if constexpr (!kInt && !PREP) x = transpose8(x, wsel, (lane & 2) != 0);
 #pragma unroll
-      for (int j = 0; j < TY; ++j) acc[i][j] = Op::mma(xf[U][i], y[j], acc[i][j]);
+      for (int j = 0; j < TY; ++j) acc[i][j] = Op::mma(x, y[j], acc[i][j]);
+    }
   };
 
   if (need_tab) __syncthreads();  // tap table (and the zeroed sums) visible

@@ -104,12 +104,33 @@ inline ConvPlan heuristic_plan(const unit_conv_desc *d, int npix, int kbytes, bo
     } else {  // the fp16 operator (a k-step is one tap of 16 channels), same source
       const int nsteps = kbytes / 32;
       const bool wide = K % 128 == 0;
-      // Weights in the reference's layout (staged_too): with a reduction of 32 steps or more and enough large tiles
-      // the staged kernels, which share both operands through LDS, beat the direct ones (batch 256: 3 x 3 256 -> 256
-      // on 14 x 14 in 69 against 122 us; measured gain 5 - 45 % from 98 tiles of 256 x 256 up, a loss below)
-      if (staged_too && nsteps >= 32) {
-        if (K % 256 == 0 && tiles(256, 256) >= 196) return ConvPlan{0, 1, 0};
-        if (wide && tiles(256, 256) >= 98) return ConvPlan{18, 1, 0};
+      // Weights in the reference's layout (staged_too), whose fragments cost the direct kernels twenty instructions of
+      // transposition each: a wave alone on its SIMD waits for them.  The lines lie where the waves of a tile size leave
+      // SIMDs without a second wave; us of the tiles for prepared weights / of these:
+      //   long reductions, from 196 tiles of 256 x 256 up: staged, both operands shared through LDS (at 192 46.4 / 42.0; 160,
+      //   3 x 3 192 -> 128 on 56 x 56, batch 14, the direct kernel takes 32.2 where staged tiles take 41.7);
+      //   up to one 64 x 128 tile per CU: four k-groups on them (64 -> 352, 5 x 5 on 36 x 38, batch 4, 22.6 / 11.6; 112 ->
+      //   368, 3 x 3 on 76 x 64 15.4 / 9.2; 432 -> 224, 3 x 3 on 74 x 61 29.1 / 20.3), with 9 - 24 k-steps and no more than
+      //   392 tiles of 64 x 64 rather on 64 x 32 (32 -> 608, 3 x 3 on 20 x 26, batch 4, 7.9 / 5.4);
+      //   then two k-groups, six deep, to three tiles per CU (144 -> 2048, 3 x 3 on 22 x 30, batch 2, 21.4 / 15.3; 208 -> 400, 3 x 3 on
+      //   36 x 57, batch 3, 25.5 / 19.0; 32 channels, half of the tile padding, 10.6 / 12.1: not these; 780 tiles 25.2 / 27.9);
+      //   up to 1568 tiles, where 128-channel tiles or staged ones ran, one wave per tile or, past 90 k-steps and with two of them per CU, 64 x 128 (512 ->
+      //   128, 1 x 1 on 28 x 28, batch 32, 14.5 / 9.8; 128 -> 1312, 5 x 5 on 14 x 20, batch 15, 38.2 / 35.4);
+      //   from 1568 tiles on four deep (64 -> 32, 3 x 3 on 65 x 83, batch 27, 19.9 / 16.9; 512 -> 608, 1 x 1 on 86 x 60, batch 3,
+      //   23.5 / 20.8).
+      if (staged_too) {
+        if (nsteps >= 32 && K % 256 == 0 && tiles(256, 256) >= 196) return ConvPlan{0, 1, 0};
+        if (t64 > 256 && nsteps > 8) {
+          if (t64 < 392 && nsteps <= 24) return ConvPlan{60, 1, 0};
+          if (tiles(64, 128) <= 256 && nsteps > 24) return ConvPlan{59, 1, 0};
+          if (t64 > 512 && t64 <= 768 && nsteps > 24 && K > 32) return ConvPlan{67, 1, 0};
+          if (t64 >= 784 && t64 < 1568) {
+            if (nsteps >= 90 && tiles(64, 128) <= 512) return ConvPlan{59, 1, 0};
+            if (nsteps > 36) return ConvPlan{68, 1, 0};
+            if (nsteps > 16) return ConvPlan{50, 1, 0};
+          }
+          if (t64 >= 1568 && (!wide || nsteps > 36)) return ConvPlan{50, 1, 0};
+        }
       }
       if (t64 < 196)
         v = 60;
