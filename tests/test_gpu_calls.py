@@ -124,3 +124,15 @@ def test_native_calls_leave_errors_to_the_python_operators(dev, monkeypatch):
             with pytest.raises((TypeError, ValueError)) as there:
                 fn()
         assert type(here.value) is type(there.value) and str(here.value) == str(there.value), name
+
+
+def test_wrapped_tensors_raise_as_in_the_python_operators(dev, monkeypatch):
+    """torch.vmap's tensors have no data pointer: an error on the host, before any launch."""
+    _, _, f16 = _operands(dev)
+    batch, b = f16((3, 4, 16)), f16((16, 8))
+    with pytest.raises(RuntimeError) as here:
+        torch.vmap(lambda a: U.gemm_fp16(a, b))(batch)
+    monkeypatch.setattr(ops, "_native", _Declines())
+    with pytest.raises(RuntimeError) as there:
+        torch.vmap(lambda a: U.gemm_fp16(a, b))(batch)
+    assert str(here.value) == str(there.value)

@@ -49,7 +49,10 @@ PyObject *n_buf, *n_K, *n_C, *n_KH, *n_KW, *n_cb, *n_dtype, *n_w, *n_wsum, *n_bt
 const at::Tensor *operand(PyObject *o, at::ScalarType type, int dim) {
   if (!THPVariable_CheckExact(o)) return nullptr;
   const at::Tensor &t = THPVariable_Unpack(o);
-  return t.is_cuda() && t.scalar_type() == type && t.dim() == dim && t.layout() == at::kStrided && t.is_contiguous() ? &t : nullptr;
+  // has_storage: the wrapped tensors of torch.func's transforms are torch.Tensors too, and have no data pointer
+  return t.is_cuda() && t.has_storage() && t.scalar_type() == type && t.dim() == dim && t.layout() == at::kStrided && t.is_contiguous()
+             ? &t
+             : nullptr;
 }
 
 bool number(PyObject *o, int32_t *v) {
@@ -124,13 +127,22 @@ at::Tensor result(const at::Tensor &like, at::IntArrayRef shape, at::ScalarType 
   return at::empty(shape, like.options().dtype(type));
 }
 
-template <class F>
-PyObject *finish(at::Tensor &&out, F &&call) {
+// other Python threads run while one is in scope, also out of which an exception leads
+struct WithoutGil {
+  PyThreadState *state = PyEval_SaveThread();
+  ~WithoutGil() { PyEval_RestoreThread(state); }
+};
+
+// call(stream, operands..., result), with data pointers for the tensors (taken first: that may throw)
+template <class F, class... T>
+PyObject *finish(at::Tensor &&out, F &&call, const T &...operands) {
   int rc;
-  void *const s = stream();
-  Py_BEGIN_ALLOW_THREADS;
-  rc = call(s);
-  Py_END_ALLOW_THREADS;
+  const auto run = [&](auto... p) {
+    void *const s = stream(), *const o = out.data_ptr();
+    WithoutGil others;
+    rc = call(s, p..., o);
+  };
+  run(operands.data_ptr()...);
   if (rc != UNIT_OK) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(out));
 }
@@ -175,7 +187,8 @@ bool bias_of(PyObject *o, int32_t k, const at::Tensor &data, const int32_t **p) 
   if (o == Py_None) return true;
   if (!THPVariable_CheckExact(o)) return false;
   const at::Tensor &b = THPVariable_Unpack(o);
-  if (b.scalar_type() != at::kInt || b.numel() != k || b.device() != data.device() || b.layout() != at::kStrided || !b.is_contiguous())
+  if (b.scalar_type() != at::kInt || b.numel() != k || b.device() != data.device() || b.layout() != at::kStrided || !b.has_storage() ||
+      !b.is_contiguous())
     return false;
   *p = static_cast<const int32_t *>(b.data_ptr());
   return true;
@@ -192,10 +205,9 @@ PyObject *conv_u8(PyObject *const *a, Py_ssize_t n) {
       !pair(a[4], &d.dh, &d.dw) || !out_hw(d, &oh, &ow))
     Py_RETURN_NONE;
   at::Tensor out = result(*x, {d.N, d.K / 16, oh, ow, 16}, at::kInt);
-  void *const o = out.data_ptr();
-  return finish(std::move(out), [&](void *s) {
-    return (prepared ? lib.conv_u8_prepared : lib.conv_u8)(&d, x->data_ptr(), w.data_ptr(), o, s);
-  });
+  return finish(std::move(out), [&](void *s, void *xp, void *wp, void *o) {
+    return (prepared ? lib.conv_u8_prepared : lib.conv_u8)(&d, xp, wp, o, s);
+  }, *x, w);
 }
 
 // (data, kernel, bias, scale, stride, padding, dilation)
@@ -210,10 +222,9 @@ PyObject *conv_fused(PyObject *const *a, Py_ssize_t n) {
       !pair(a[4], &d.sh, &d.sw) || !padding(a[5], &d) || !pair(a[6], &d.dh, &d.dw) || !out_hw(d, &oh, &ow))
     Py_RETURN_NONE;
   at::Tensor out = result(*x, {d.N, d.K / 16, oh, ow, 16}, at::kInt);
-  void *const o = out.data_ptr();
-  return finish(std::move(out), [&](void *s) {
-    return (prepared ? lib.fused_prepared : lib.fused)(&d, x->data_ptr(), w.data_ptr(), bias, scale, o, s);
-  });
+  return finish(std::move(out), [&](void *s, void *xp, void *wp, void *o) {
+    return (prepared ? lib.fused_prepared : lib.fused)(&d, xp, wp, bias, scale, o, s);
+  }, *x, w);
 }
 
 // (data, prepared kernel, bias, scale, shift, stride, padding, dilation)
@@ -229,8 +240,8 @@ PyObject *conv_requant(PyObject *const *a, Py_ssize_t n) {
       !out_hw(d, &oh, &ow))
     Py_RETURN_NONE;
   at::Tensor out = result(*x, {d.N, d.K / 16, oh, ow, 16}, at::kByte);
-  void *const o = out.data_ptr();
-  return finish(std::move(out), [&](void *s) { return lib.requant(&d, x->data_ptr(), w.data_ptr(), bias, scale, shift, o, s); });
+  return finish(std::move(out), [&](void *s, void *xp, void *wp, void *o) { return lib.requant(&d, xp, wp, bias, scale, shift, o, s); }, *x,
+                w);
 }
 
 // (data, kernel, stride)
@@ -247,8 +258,7 @@ PyObject *conv3d(PyObject *const *a, Py_ssize_t n) {
   if (d.KD > d.D || d.KH > d.H || d.KW > d.W) Py_RETURN_NONE;
   at::Tensor out = result(*x, {d.N, d.K / 16, (d.D - d.KD) / d.stride + 1, (d.H - d.KH) / d.stride + 1, (d.W - d.KW) / d.stride + 1, 16},
                           at::kInt);
-  void *const o = out.data_ptr();
-  return finish(std::move(out), [&](void *s) { return lib.conv3d(&d, x->data_ptr(), w->data_ptr(), o, s); });
+  return finish(std::move(out), [&](void *s, void *xp, void *wp, void *o) { return lib.conv3d(&d, xp, wp, o, s); }, *x, *w);
 }
 
 // (a, b, stride_h, stride_w): blocked a with blocked or prepared b, or both plain
@@ -268,17 +278,16 @@ PyObject *conv_f16(PyObject *const *a, Py_ssize_t n) {
     size_t need = 0;
     if (lib.conv_f16_plain_bytes(&d, &need) != UNIT_OK || need == 0) Py_RETURN_NONE;
     at::Tensor ws = result(*x, {(int64_t)need}, at::kByte), out = result(*x, {d.N, d.K / 16, oh, ow, 16}, at::kFloat);
-    void *const o = out.data_ptr();
-    return finish(std::move(out), [&](void *s) { return lib.conv_f16_plain(&d, x->data_ptr(), w->data_ptr(), o, ws.data_ptr(), need, s); });
+    return finish(std::move(out), [&](void *s, void *xp, void *wp, void *sp, void *o) { return lib.conv_f16_plain(&d, xp, wp, o, sp, need, s); },
+                  *x, *w, ws);
   }
   at::Tensor w;
   bool prepared;
   if (!conv_operands(a[0], a[1], at::kHalf, &d, &x, &w, &prepared) || !out_hw(d, &oh, &ow)) Py_RETURN_NONE;
   at::Tensor out = result(*x, {d.N, d.K / 16, oh, ow, 16}, at::kFloat);
-  void *const o = out.data_ptr();
-  return finish(std::move(out), [&](void *s) {
-    return (prepared ? lib.conv_f16_prepared : lib.conv_f16)(&d, x->data_ptr(), w.data_ptr(), o, s);
-  });
+  return finish(std::move(out), [&](void *s, void *xp, void *wp, void *o) {
+    return (prepared ? lib.conv_f16_prepared : lib.conv_f16)(&d, xp, wp, o, s);
+  }, *x, w);
 }
 
 // (data, weight): packed, row-major or prepared
@@ -294,22 +303,21 @@ PyObject *dense(PyObject *const *a, Py_ssize_t n) {
       Py_RETURN_NONE;
     const int32_t nn = (int32_t)w.size(0);
     at::Tensor out = result(*x, {m, nn}, at::kInt);
-    void *const o = out.data_ptr();
-    return finish(std::move(out), [&](void *s) { return lib.dense_prepared(x->data_ptr(), w.data_ptr(), sums.data_ptr<int>(), o, m, nn, k, s); });
+    return finish(std::move(out), [&](void *s, void *xp, void *wp, void *sp, void *o) {
+      return lib.dense_prepared(xp, wp, static_cast<int *>(sp), o, m, nn, k, s);
+    }, *x, w, sums);
   }
   if (const at::Tensor *w = operand(a[1], at::kChar, 4)) {
     if (w->size(2) != 128 || w->size(3) != 4 || w->size(1) * 4 != k || w->size(0) > INT_MAX / 128) Py_RETURN_NONE;
     const int32_t nn = (int32_t)w->size(0) * 128;
     at::Tensor out = result(*x, {m, nn}, at::kInt);
-    void *const o = out.data_ptr();
-    return finish(std::move(out), [&](void *s) { return lib.dense_packed(x->data_ptr(), w->data_ptr(), o, m, nn, k, s); });
+    return finish(std::move(out), [&](void *s, void *xp, void *wp, void *o) { return lib.dense_packed(xp, wp, o, m, nn, k, s); }, *x, *w);
   }
   const at::Tensor *w = operand(a[1], at::kChar, 2);
   if (!w || !small(*w) || w->size(1) != k) Py_RETURN_NONE;
   const int32_t nn = (int32_t)w->size(0);
   at::Tensor out = result(*x, {m, nn}, at::kInt);
-  void *const o = out.data_ptr();
-  return finish(std::move(out), [&](void *s) { return lib.dense(x->data_ptr(), w->data_ptr(), o, m, nn, k, s); });
+  return finish(std::move(out), [&](void *s, void *xp, void *wp, void *o) { return lib.dense(xp, wp, o, m, nn, k, s); }, *x, *w);
 }
 
 // (a, b, fp16 result?, workspace or None): b (K, N) or prepared
@@ -326,8 +334,7 @@ PyObject *gemm(PyObject *const *a, Py_ssize_t n) {
         bt.size(0) != nn || bt.size(1) != k)
       Py_RETURN_NONE;
     at::Tensor out = result(*x, {m, nn}, type);
-    void *const o = out.data_ptr();
-    return finish(std::move(out), [&](void *s) { return lib.gemm_prepared(x->data_ptr(), bt.data_ptr(), o, m, nn, k, half, s); });
+    return finish(std::move(out), [&](void *s, void *xp, void *bp, void *o) { return lib.gemm_prepared(xp, bp, o, m, nn, k, half, s); }, *x, bt);
   }
   const at::Tensor *b = operand(a[1], at::kHalf, 2);
   if (!b || !small(*b) || b->size(0) != k) Py_RETURN_NONE;
@@ -335,16 +342,16 @@ PyObject *gemm(PyObject *const *a, Py_ssize_t n) {
   if (a[3] != Py_None) {
     if (!THPVariable_CheckExact(a[3])) Py_RETURN_NONE;
     const at::Tensor &ws = THPVariable_Unpack(a[3]);
-    if (!ws.is_cuda() || ws.scalar_type() != at::kByte || ws.layout() != at::kStrided || !ws.is_contiguous()) Py_RETURN_NONE;
+    if (!ws.is_cuda() || !ws.has_storage() || ws.scalar_type() != at::kByte || ws.layout() != at::kStrided || !ws.is_contiguous())
+      Py_RETURN_NONE;
     at::Tensor out = result(*x, {m, nn}, type);
-    void *const o = out.data_ptr();
-    return finish(std::move(out), [&](void *s) {
-      return lib.gemm_ws(x->data_ptr(), b->data_ptr(), o, m, nn, k, half, ws.data_ptr(), (size_t)ws.numel(), s);
-    });
+    const size_t bytes = (size_t)ws.numel();
+    return finish(std::move(out), [&](void *s, void *xp, void *bp, void *sp, void *o) {
+      return lib.gemm_ws(xp, bp, o, m, nn, k, half, sp, bytes, s);
+    }, *x, *b, ws);
   }
   at::Tensor out = result(*x, {m, nn}, type);
-  void *const o = out.data_ptr();
-  return finish(std::move(out), [&](void *s) { return lib.gemm(x->data_ptr(), b->data_ptr(), o, m, nn, k, half, s); });
+  return finish(std::move(out), [&](void *s, void *xp, void *bp, void *o) { return lib.gemm(xp, bp, o, m, nn, k, half, s); }, *x, *b);
 }
 
 // (addresses in Library's order, the three prepared classes, torch.int8, torch.float16)
