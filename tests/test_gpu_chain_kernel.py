@@ -5,7 +5,8 @@ import pytest
 import torch
 
 from test_gpu_chain import _oracle_chain, _t, _to_chain
-from unit_amd import chain, rng
+from unit_amd import chain, ops, rng
+from unit_amd._lib import check
 
 pytestmark = pytest.mark.gpu
 
@@ -125,3 +126,22 @@ def test_chain_with_reused_buffers_runs_layer_by_layer(dev, oracle):
     c(_t(x, dev))
     assert np.array_equal(c.outputs[-1].cpu().numpy(), want[-1])
     assert not any(v.startswith("q8chain_") for v in c.variants)
+
+
+@pytest.mark.parametrize("offset", [0, 16, 64, 112])
+def test_workspace_at_any_16_bytes(dev, oracle, offset):
+    """The library aligns its own lines inside the workspace and stays within the size that it asked for."""
+    spec, n, c0, h, w = CASES["odd_blocks_uneven_groups"]
+    x, layers, want = _build(oracle, spec, n, c0, h, w)
+    c = chain.ConvChain(_to_chain(layers, dev), x.shape)
+    xd = _t(x, dev)
+    c(xd)
+    buf = torch.full((256 + c._ws_bytes + 256,), 0x5A, dtype=torch.uint8, device=dev)
+    assert buf.data_ptr() % 128 == 0
+    ws = buf[offset:offset + c._ws_bytes]
+    for o in c.outputs:
+        o.fill_(77)
+    check(c._L.unit_conv_chain_u8_ws(c._native, len(c._native), xd.data_ptr(), ws.data_ptr(), c._ws_bytes, ops._stream()))
+    torch.cuda.synchronize()
+    assert all(np.array_equal(o.cpu().numpy(), r) for o, r in zip(c.outputs, want))
+    assert (buf[:offset] == 0x5A).all() and (buf[offset + c._ws_bytes:] == 0x5A).all()

@@ -81,7 +81,8 @@ __device__ __forceinline__ ChainStep load_step(StepPtr p) {
 
 // The workspace: control words (zeroed by chain_setup), then the layers.  Words: groups claimed; a line per XCD with its
 // ticket counter; per XCD the groups it has claimed (+ 1), in its order; per group the tiles' flags.  No line of it is
-// written by two XCDs but the first.
+// written by two XCDs but the first, so it begins on a line wherever the caller's memory does (kWsAlign).
+constexpr int kWsAlign = 128;
 constexpr int kCtlGroups = 0, kCtlTickets = 32, kCtlSlots = kCtlTickets + 32 * kMaxXcd;
 
 struct ChainArgs {
@@ -605,7 +606,7 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
   p->flag_pitch = (p->tickets + 31) / 32 * 32;
   p->clear_words = p->flags0 + p->groups * p->flag_pitch;
   p->steps_off = ((size_t)p->clear_words * 4 + 255) / 256 * 256;
-  p->bytes = p->steps_off + (size_t)count * sizeof(ChainStep);
+  p->bytes = p->steps_off + (size_t)count * sizeof(ChainStep) + kWsAlign - 16;  // ws itself is at 16 bytes
   return true;
 }
 
@@ -635,7 +636,7 @@ extern "C" int unit_conv_chain_u8_ws(const unit_chain_layer *layers, int32_t cou
     return unit_conv_chain_u8(layers, count, x, stream);
   if (int rc = check_device()) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  char *base = static_cast<char *>(ws);
+  char *base = reinterpret_cast<char *>((reinterpret_cast<uintptr_t>(ws) + kWsAlign - 1) / kWsAlign * kWsAlign);
   ChainStep *steps = reinterpret_cast<ChainStep *>(base + p.steps_off);
   for (int i = 0; i < count; i += kSetupSteps) {
     ChainSetup a;
