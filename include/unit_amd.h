@@ -324,6 +324,13 @@ int unit_conv_chain_u8_ws_bytes(const unit_chain_layer *layers, int32_t count, s
 int unit_conv_chain_u8_ws(const unit_chain_layer *layers, int32_t count, const void *x, void *ws, size_t ws_bytes,
                           unit_stream_t stream);
 
+/* The same with a word for the outcome.  The kernel's tiles wait for each other, each wave a bounded number of polls
+ * (seconds); one that gives up ends the wait and writes 1 to *status (4 bytes of device memory or of pinned host memory,
+ * valid until the call has run on the stream, never cleared here): the run's results are then not valid.  status == NULL,
+ * and unit_conv_chain_u8_ws, take the workspace's first int32 instead, which a caller that looks at it clears before the call. */
+int unit_conv_chain_u8_status(const unit_chain_layer *layers, int32_t count, const void *x, void *ws, size_t ws_bytes,
+                              int32_t *status, unit_stream_t stream);
+
 /* ------------------------------------------------------------------ diagnostics */
 
 /* One v_mfma_i32_32x32x32_i8 / v_mfma_f32_32x32x16_f16 on a single wavefront, operands and

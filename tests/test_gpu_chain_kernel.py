@@ -6,7 +6,7 @@ import torch
 
 from test_gpu_chain import _oracle_chain, _t, _to_chain
 from unit_amd import chain, ops, rng
-from unit_amd._lib import check
+from unit_amd._lib import UnitError, check
 
 pytestmark = pytest.mark.gpu
 
@@ -145,3 +145,46 @@ def test_workspace_at_any_16_bytes(dev, oracle, offset):
     torch.cuda.synchronize()
     assert all(np.array_equal(o.cpu().numpy(), r) for o, r in zip(c.outputs, want))
     assert (buf[:offset] == 0x5A).all() and (buf[offset + c._ws_bytes:] == 0x5A).all()
+
+
+def test_a_run_that_gives_up_says_so(dev, oracle, monkeypatch):
+    """One poll per wave: waits end at once, every kernel still ends by itself, and the run is reported instead of passing for good."""
+    spec, n, c0, h, w = CASES["odd_blocks_uneven_groups"]
+    x, layers, want = _build(oracle, spec, n, c0, h, w)
+    c, other = chain.ConvChain(_to_chain(layers, dev), x.shape), chain.ConvChain(_to_chain(layers, dev), x.shape)
+    xd = _t(x, dev)
+    replay = c.graph(xd)
+    torch.cuda.synchronize()
+    c.check()
+    monkeypatch.setenv("UNIT_AMD_CHAIN_POLLS", "1")
+    c(xd)
+    torch.cuda.synchronize()
+    other.check()
+    with pytest.raises(UnitError, match="gave up"):
+        c.check()
+    c.check()  # said once
+    c(xd)
+    torch.cuda.synchronize()
+    with pytest.raises(UnitError, match="gave up"):
+        c(xd)
+    c(xd)
+    torch.cuda.synchronize()
+    with pytest.raises(UnitError, match="gave up"):
+        replay()
+    # without a word of the caller's: the workspace's first
+    ws = torch.zeros(c._ws_bytes, dtype=torch.uint8, device=dev)
+    check(c._L.unit_conv_chain_u8_ws(c._native, len(c._native), xd.data_ptr(), ws.data_ptr(), c._ws_bytes, ops._stream()))
+    torch.cuda.synchronize()
+    assert ws[:4].view(torch.int32).item() == 1
+    monkeypatch.delenv("UNIT_AMD_CHAIN_POLLS")
+    ws.zero_()
+    check(c._L.unit_conv_chain_u8_ws(c._native, len(c._native), xd.data_ptr(), ws.data_ptr(), c._ws_bytes, ops._stream()))
+    torch.cuda.synchronize()
+    assert ws[:4].view(torch.int32).item() == 0
+    for call in (lambda: c(xd), replay):
+        for o in c.outputs:
+            o.fill_(77)
+        call()
+        torch.cuda.synchronize()
+        c.check()
+        assert all(np.array_equal(o.cpu().numpy(), r) for o, r in zip(c.outputs, want))

@@ -50,6 +50,7 @@ SYMBOLS = (
     "unit_conv_chain_u8",
     "unit_conv_chain_u8_ws_bytes",
     "unit_conv_chain_u8_ws",
+    "unit_conv_chain_u8_status",
     "unit_mfma_tile_i8",
     "unit_mfma_tile_f16",
     "unit_mfma_peak",
@@ -130,6 +131,7 @@ def load():
     L.unit_conv_chain_u8.argtypes = [ctypes.POINTER(ChainLayerDesc), i32, vp, vp]
     L.unit_conv_chain_u8_ws_bytes.argtypes = [ctypes.POINTER(ChainLayerDesc), i32, ctypes.POINTER(ctypes.c_size_t)]
     L.unit_conv_chain_u8_ws.argtypes = [ctypes.POINTER(ChainLayerDesc), i32, vp, vp, ctypes.c_size_t, vp]
+    L.unit_conv_chain_u8_status.argtypes = [ctypes.POINTER(ChainLayerDesc), i32, vp, vp, ctypes.c_size_t, vp, vp]
     L.unit_mfma_tile_i8.argtypes = [vp, vp, vp, vp]
     L.unit_mfma_tile_f16.argtypes = [vp, vp, vp, vp]
     L.unit_mfma_peak.argtypes = [i32, i32, i32, vp, vp]

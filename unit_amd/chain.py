@@ -7,10 +7,12 @@ cpu-shapes.log:388-420.
 Every layer is the requantising convolution (ops.conv2d_NCHWc_int8_requant): u8 in, u8 out, so a layer's
 output is the next layer's input as it lies in memory.  The runner owns all activation buffers and
 prepared weights and issues nothing but kernel launches through the C ABI (a chain that pays for it as one
-persistent kernel, with a few KiB of the caching allocator's memory per run), and can therefore be captured into
-a HIP graph.
+persistent kernel, with a workspace of the caching allocator per run: 120 KB for the ResNet-50 below at batch 32), and can
+therefore be captured into a HIP graph.
 """
 import ctypes
+import itertools
+import threading
 from collections import namedtuple
 
 import torch
@@ -22,6 +24,27 @@ from ._lib import ChainLayerDesc, ConvDesc, check
 ChainLayer = namedtuple("ChainLayer", "weight bias scale shift stride padding source", defaults=(None,))
 
 
+class _StatusWords:
+    """A word of pinned host memory per chain, which the chain's kernel sets if it gives up (unit_conv_chain_u8_status).  The
+    memory lasts as long as the process, since a kernel may be under way when its chain goes; past 4096 chains words are shared."""
+
+    COUNT = 4096
+
+    def __init__(self):
+        self._lock, self._next, self._words = threading.Lock(), itertools.count(), None
+
+    def take(self):
+        with self._lock:
+            if self._words is None:
+                if torch.cuda.is_current_stream_capturing():  # no allocation of host memory here
+                    return None
+                self._words = torch.zeros(self.COUNT, dtype=torch.int32, pin_memory=True)
+            return ctypes.c_int32.from_address(self._words.data_ptr() + 4 * (next(self._next) % self.COUNT))
+
+
+_status_words = _StatusWords()
+
+
 class ConvChain:
     """layers: ChainLayer items with `weight` an int8 OIHW tensor (IC, OC multiples of 16) or a
     PreparedConvWeight, `bias` int32 (OC,) or None, integer `scale`, `shift` in 1..62, `stride`, `padding`.
@@ -29,7 +52,10 @@ class ConvChain:
 
     run(x) runs every layer on the current stream and returns the last layer's output buffer (owned by
     the chain and overwritten by the next run); outputs[i] is layer i's.  graph(x) captures run(x) once and
-    returns a callable that replays it (x's storage is the graph's input)."""
+    returns a callable that replays it (x's storage is the graph's input).
+
+    A chain that runs as one kernel waits on the device for its own tiles, within bounds.  If a run gave up, check() raises
+    UnitError once it has ended, and so do the next run and the next replay: what it left in outputs is not valid."""
 
     def __init__(self, layers, input_shape):
         if len(input_shape) != 5 or input_shape[4] != 16:
@@ -75,6 +101,7 @@ class ConvChain:
             raise ValueError("layers: empty chain")
         self.variants = [None] * len(self.outputs)
         self._native, self._bound = (), None
+        self._status = _status_words.take()
         self._bind()
 
     def _bind(self):
@@ -96,7 +123,14 @@ class ConvChain:
             check(self._L.unit_conv_chain_u8_ws_bytes(self._native, count, ctypes.byref(size)))
             self._bound, self._ws_bytes = bound, size.value
 
+    def check(self):
+        """Raises UnitError if a run that has ended gave up waiting (once: the chain may be run again)."""
+        if self._status is not None and self._status.value:
+            self._status.value = 0
+            raise _lib.UnitError("ConvChain: a run gave up waiting for its own tiles; its outputs are not valid")
+
     def run(self, x):
+        self.check()
         x = ops._dev(x, "x", torch.uint8, 5)
         if tuple(x.shape) != self.input_shape:
             raise ValueError(f"x: expected {self.input_shape}, got {tuple(x.shape)}")
@@ -107,8 +141,8 @@ class ConvChain:
                 self._native[i].variant = ctypes.addressof(self._names) + 96 * i
         # a run's own: runs of one chain on several streams share nothing but the activation buffers
         ws = torch.empty(self._ws_bytes, dtype=torch.uint8, device=x.device)
-        check(self._L.unit_conv_chain_u8_ws(self._native, len(self._native), x.data_ptr(), ws.data_ptr(), self._ws_bytes,
-                                            ops._stream()))
+        check(self._L.unit_conv_chain_u8_status(self._native, len(self._native), x.data_ptr(), ws.data_ptr(), self._ws_bytes,
+                                                None if self._status is None else ctypes.addressof(self._status), ops._stream()))
         for i in unnamed:
             self.variants[i] = self._names[96 * i:96 * i + 96].split(b"\0")[0].decode()
             self._native[i].variant = None
@@ -140,6 +174,7 @@ class ConvChain:
             self.run(x)
 
         def replay():
+            self.check()
             g.replay()
             return self.outputs[-1]
 

@@ -43,7 +43,8 @@ constexpr int kDepth = 5;         // k-steps of fragments in flight per wave
 constexpr int kMaxXcd = 16, kMaxChain = 256;
 constexpr int kAgent = 16;        // sc1
 // Polls a wave may spend in all before it stops waiting (seconds; a whole chain takes some thousand): every wave ends, also
-// after a fault in another one.
+// after a fault in another one.  A wave that stops waiting says so in the status word (ChainArgs): the run's results are then
+// not valid.  UNIT_AMD_CHAIN_POLLS sets another number (a test takes one).
 constexpr int kPolls = 1 << 24;
 
 // q = n / d for n * d < 2^31
@@ -82,7 +83,7 @@ __device__ __forceinline__ ChainStep load_step(StepPtr p) {
 // The workspace: control words (zeroed by chain_setup), then the layers.  Words: groups claimed; a line per XCD with its
 // ticket counter; per XCD the groups it has claimed (+ 1), in its order; per group the tiles' flags.  No line of it is
 // written by two XCDs but the first, so it begins on a line wherever the caller's memory does (kWsAlign).
-constexpr int kWsAlign = 128;
+constexpr int kWsAlign = 128, kWsHead = 16;  // kWsHead: the status word of callers without one of their own
 constexpr int kCtlGroups = 0, kCtlTickets = 32, kCtlSlots = kCtlTickets + 32 * kMaxXcd;
 
 struct ChainArgs {
@@ -91,6 +92,8 @@ struct ChainArgs {
   int count, images, per, groups;
   int slot_pitch, flags0, flag_pitch;
   FastDiv by_tickets;
+  int *status;  // the caller's, in device or pinned host memory: 1 once a wave has given up waiting, else as it was
+  int polls;
 };
 
 // The layers travel as kernel arguments (at most 4 KiB of them), so that a captured chain keeps the ones it was captured
@@ -111,6 +114,10 @@ struct alignas(16) ChainLds {
   int addend[kWaves][64];
   int ticket[2], group;
 };
+
+__device__ __forceinline__ void give_up(const ChainArgs &a) {
+  __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 __device__ __forceinline__ int load_l2(const int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
@@ -299,7 +306,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kPerCu
   int *const slots = a.ctl + kCtlSlots + xcd * a.slot_pitch;
   if (tid == 0) sh.ticket[0] = __hip_atomic_fetch_add(tickets, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
-  int turn = 0, q_now = -1, group = 0, l = 0, budget = kPolls;
+  int turn = 0, q_now = -1, group = 0, l = 0, budget = a.polls;
   for (;;) {
     const int ticket = __builtin_amdgcn_readfirstlane(sh.ticket[turn]);
     turn ^= 1;
@@ -314,7 +321,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kPerCu
           store_result<0>(result_buffer(slots), (u32)q * 4u, v);
         } else {
           while ((v = load_l2(slots + q)) == 0 && --budget > 0) __builtin_amdgcn_s_sleep(1);
-          if (v == 0) v = a.groups + 1;
+          if (v == 0) give_up(a), v = a.groups + 1;
         }
         sh.group = v - 1;
       }
@@ -410,6 +417,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kPerCu
       for (int b = fa + 64; b < fb; b += 64) {
         while (!__all(load_l2(wanted + (u32)min(b + lane, fb - 1)) != 0) && --budget > 0) __builtin_amdgcn_s_sleep(1);
       }
+      if (budget <= 0) give_up(a);
     }
 
     v16i acc[2][2];
@@ -606,7 +614,7 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
   p->flag_pitch = (p->tickets + 31) / 32 * 32;
   p->clear_words = p->flags0 + p->groups * p->flag_pitch;
   p->steps_off = ((size_t)p->clear_words * 4 + 255) / 256 * 256;
-  p->bytes = p->steps_off + (size_t)count * sizeof(ChainStep) + kWsAlign - 16;  // ws itself is at 16 bytes
+  p->bytes = p->steps_off + (size_t)count * sizeof(ChainStep) + kWsAlign;  // ws itself is at 16 bytes, and its head in front
   return true;
 }
 
@@ -624,9 +632,15 @@ extern "C" int unit_conv_chain_u8_ws_bytes(const unit_chain_layer *layers, int32
 
 extern "C" int unit_conv_chain_u8_ws(const unit_chain_layer *layers, int32_t count, const void *x, void *ws, size_t ws_bytes,
                                      unit_stream_t stream) {
+  return unit_conv_chain_u8_status(layers, count, x, ws, ws_bytes, nullptr, stream);
+}
+
+extern "C" int unit_conv_chain_u8_status(const unit_chain_layer *layers, int32_t count, const void *x, void *ws, size_t ws_bytes,
+                                         int32_t *status, unit_stream_t stream) {
   using namespace unit;
   const char *what = "unit_conv_chain_u8_ws";
   if (!layers || !x || count < 0) return fail(UNIT_E_ARG, "%s: null pointer or negative count", what);
+  if (reinterpret_cast<uintptr_t>(status) % 4) return fail(UNIT_E_ARG, "%s: status must be 4-byte aligned", what);
   ChainStep st[kMaxChain];
   ChainPlan p;
   const bool pinned = tuning_override("UNIT_AMD_CONV_VARIANT") > 0 || tuning_override("UNIT_AMD_CONV_PANEL") > 0 ||
@@ -636,7 +650,7 @@ extern "C" int unit_conv_chain_u8_ws(const unit_chain_layer *layers, int32_t cou
     return unit_conv_chain_u8(layers, count, x, stream);
   if (int rc = check_device()) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  char *base = reinterpret_cast<char *>((reinterpret_cast<uintptr_t>(ws) + kWsAlign - 1) / kWsAlign * kWsAlign);
+  char *base = reinterpret_cast<char *>((reinterpret_cast<uintptr_t>(ws) + kWsHead + kWsAlign - 1) / kWsAlign * kWsAlign);
   ChainStep *steps = reinterpret_cast<ChainStep *>(base + p.steps_off);
   for (int i = 0; i < count; i += kSetupSteps) {
     ChainSetup a;
@@ -647,7 +661,8 @@ extern "C" int unit_conv_chain_u8_ws(const unit_chain_layer *layers, int32_t cou
                        reinterpret_cast<v4i *>(base), quads);
   }
   const ChainArgs a{steps,        reinterpret_cast<int *>(base), count,        layers[0].desc.N,           p.per, p.groups,
-                    p.slot_pitch, p.flags0,                      p.flag_pitch, FastDiv::make(p.tickets)};
+                    p.slot_pitch, p.flags0,                      p.flag_pitch, FastDiv::make(p.tickets),    status ? status : static_cast<int *>(ws),
+                    tuning_override("UNIT_AMD_CHAIN_POLLS") > 0 ? tuning_override("UNIT_AMD_CHAIN_POLLS") : kPolls};
   hipLaunchKernelGGL(chain_run, dim3(256 * kPerCu), dim3(kThreads), sizeof(ChainLds), s, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(UNIT_E_LAUNCH, "%s: launch: %s", what, hipGetErrorString(e));
