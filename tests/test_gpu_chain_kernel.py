@@ -188,3 +188,20 @@ def test_a_run_that_gives_up_says_so(dev, oracle, monkeypatch):
         torch.cuda.synchronize()
         c.check()
         assert all(np.array_equal(o.cpu().numpy(), r) for o, r in zip(c.outputs, want))
+
+
+def test_short_chain_takes_no_workspace(dev, oracle):
+    """Two layers run launch by launch, with nothing of the kernel's in the way: no workspace, no plan on every run."""
+    x, layers, want = _build(oracle, ODD[:2], 2, 48, 21, 17)
+    c = chain.ConvChain(_to_chain(layers, dev), x.shape)
+    called = []
+
+    class Noted:
+        def __getattr__(self, name):
+            called.append(name)
+            return getattr(lib, name)
+
+    lib, c._L = c._L, Noted()
+    c(_t(x, dev))
+    assert called == ["unit_conv_chain_u8"]
+    assert all(np.array_equal(o.cpu().numpy(), r) for o, r in zip(c.outputs, want))

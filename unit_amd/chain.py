@@ -139,10 +139,13 @@ class ConvChain:
         for i in unnamed:
             if not self._native[i].variant:
                 self._native[i].variant = ctypes.addressof(self._names) + 96 * i
-        # a run's own: runs of one chain on several streams share nothing but the activation buffers
-        ws = torch.empty(self._ws_bytes, dtype=torch.uint8, device=x.device)
-        check(self._L.unit_conv_chain_u8_status(self._native, len(self._native), x.data_ptr(), ws.data_ptr(), self._ws_bytes,
-                                                None if self._status is None else ctypes.addressof(self._status), ops._stream()))
+        if self._ws_bytes:
+            # a run's own: runs of one chain on several streams share nothing but the activation buffers
+            ws = torch.empty(self._ws_bytes, dtype=torch.uint8, device=x.device)
+            check(self._L.unit_conv_chain_u8_status(self._native, len(self._native), x.data_ptr(), ws.data_ptr(), self._ws_bytes,
+                                                    None if self._status is None else ctypes.addressof(self._status), ops._stream()))
+        else:  # no workspace to allocate and no plan to make: two launches are 8.7 us, those cost 0.8
+            check(self._L.unit_conv_chain_u8(self._native, len(self._native), x.data_ptr(), ops._stream()))
         for i in unnamed:
             self.variants[i] = self._names[96 * i:96 * i + 96].split(b"\0")[0].decode()
             self._native[i].variant = None
