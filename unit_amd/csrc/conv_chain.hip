@@ -510,7 +510,7 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
   p->per = per;
   p->groups = (N + per - 1) / per;
   long first = 0;
-  double here = 7, launches = 0;  // us, below
+  double here = 5.5, launches = 0.9;  // us, below
   Range outs[kMaxChain];
   for (int i = 0; i < count; ++i) {
     const unit_chain_layer &l = layers[i];
@@ -549,8 +549,6 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
     const bool masked = d.pt || d.pl || d.pb || d.pr;
     s.mode = masked ? 2 : (s.win == 1 && s.ntaps % 2 == 0 ? 0 : 1);
     s.flat = !masked && d.KH == 1 && d.KW == 1 && d.sh == 1 && d.sw == 1;
-    const double gmac = 1e-9 * s.ohw * d.K * s.ntaps * 16;  // of an image
-    here += 2.5 + gmac * per / 0.1, launches += 3.9 + gmac * N / 0.65;
     const long npix = (long)per * s.ohw;
     if (npix * s.ohw > 0x7fffffffl) return false;
     // k-groups: a tile costs 2.6 us beside its reduction (decode, first loads, requantisation, stores, flag), 0.4 more with
@@ -573,6 +571,11 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
     s.by_nct = small_div(s.nct);
     const long npt = (npix + 64 * wy - 1) / (64 * wy);
     if (npt * s.nct * s.nct > 0x7fffffffl) return false;
+    const double gmac = 1e-9 * s.ohw * d.K * s.ntaps * 16, mb = 1e-6 * ((double)g.img_bytes + (double)s.ohw * d.K);  // of an image
+    const double rounds = npt * s.nct / 64.0, ksteps = ceil_div(s.nsteps, kg);
+    here += 1.45 + (kg > 1 ? 0.15 : 0.0) + 0.8 * std::max(1.0, rounds) +
+            (s.mode == 1 || s.mode == 2 ? 0.3 : 0.21) * ksteps * std::max(0.5, rounds) + 1.28 * mb * per;
+    launches += 3.6 + 1.15 * gmac * N + 0.176 * mb * N + 0.019 * std::min(s.nsteps, 80);
     s.first = (int)first;
     first += npt * s.nct;
     s.next = (int)first;
@@ -586,12 +589,16 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
         break;
       }
   }
-  // Short chains, and few images through large layers, stay launches: the kernel costs 7 us before its first tile, 2.5 us a
-  // layer and 10 us per GMAC of an XCD's group, a launch 3.9 us and 1.5 us per GMAC of the batch.  us here / as launches:
-  // 3 x 3 64 -> 64 on 56 x 56, batch 1, 2 layers 13.7 / 7.9, 12 layers 48.9 / 48.0; batch 8, 3 layers 17.6 / 20.1, 8 layers
-  // 36.9 / 53.6; 1 x 1 256 -> 256 on 14 x 14, batch 1, 2 layers 10.0 / 7.5, 8 layers 24.3 / 30.3; seven 3 x 3 layers of 128 to 512
-  // channels from 56 x 56 on, batch 1 54.8 / 34.6, 8 56.4 / 57.3, 128 398 / 432.
-  if (here > 0.95 * launches) return false;
+  // Short chains, few images through large layers and activations that outgrow an XCD's 4 MB of L2 stay launches.  The
+  // kernel costs 5.5 us before its first tile; a layer 1.5 us, and 0.8 us for each round of an XCD's 64 workgroups, 0.2 (0.3 with
+  // the tap walk) per k-step of it and 1.3 per MB that the group reads and writes; a launch 3.6 us, 1.2 per GMAC and 0.18 per MB
+  // of the batch.  Fitted to 300 random chains and 32 of ResNets, both ways each: errors of 7 % and 6 % (root mean square); of
+  // the 225 it gives to the kernel 7 lose there, up to 10 %, and without the bytes and the rounds chains of wide images at 14 - 54
+  // images lost 10 - 22 %.  us here / as launches: 3 x 3 64 -> 64 on 56 x 56, batch 8, 3 layers 17.6 / 20.1; 1 x 1 256 -> 256 on
+  // 14 x 14, batch 1, 8 layers 24.3 / 30.3; ResNet-18 batch 1 82 / 88, 32 118 / 157; ResNet-50 batch 1 197 / 219, 128 1026 / 1216;
+  // the other way 14 layers from 51 x 51, batch 14 245 / 201, 10 layers from 50 x 50, batch 52 197 / 167, 9 layers of 224 channels
+  // on 20 x 20, batch 2 42.9 / 38.0.
+  if (here > 0.975 * launches) return false;
   // The layers no longer run one after the other: none may write what another one reads or writes, but for a source's
   // whole result.
   std::sort(outs, outs + count, [](const Range &u, const Range &v) { return u.a < v.a; });
