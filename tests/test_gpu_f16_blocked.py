@@ -19,6 +19,17 @@ SHAPES = [
     (7, 80, 37, 41, 352, 3, 1, "x64_y64_g1_d6"),     # 45 k-steps
     (6, 80, 46, 66, 400, 3, 1, "x64_y64_g1_d4"),     # more than 1568 tiles
     (2, 48, 31, 33, 272, 5, 2, None),
+    (12, 80, 62, 50, 32, 3, 1, "x32_y64_g4_d6n"),     # 32 channels, 45 k-steps
+    (8, 48, 70, 66, 16, 3, 1, "x32_y64_g4_d6n"),     # 16 channels, 27 k-steps
+    (13, 80, 26, 22, 1264, 3, 2, "x64_y64_g2_d6n"),  # 500 tiles, 260 of 64 x 128
+    (11, 96, 16, 15, 1904, 3, 1, "x64_y64_g1_d6n"),  # 960 tiles, 54 k-steps: below the next line
+    (13, 96, 16, 15, 1904, 3, 1, "x64_y64_g1_d6hn"), # 1110 tiles, 54 k-steps: eight loads per fragment
+    (14, 96, 17, 15, 1744, 3, 1, "x64_y64_g1_d6hn"), # 1204 tiles, half a tile of channels at the end
+    (20, 96, 40, 33, 144, 3, 1, "x64_y64_g1_d6hn"),
+    (45, 64, 18, 17, 912, 1, 1, "x64_y64_g1_d3w4n"), # 3240 tiles, four k-steps
+    (9, 32, 70, 70, 688, 1, 1, "x64_y64_g1_d6n"),    # 7590 tiles, two k-steps
+    (12, 32, 80, 60, 1648, 3, 2, "x64_y64_g1_d4n"),  # 5538 tiles, 18 k-steps
+    (12, 32, 80, 112, 1648, 3, 2, "x64_y64_g1_d3n"), # 10478 tiles
 ]
 
 

@@ -53,7 +53,7 @@ namespace unit {
 // fragment, half as long again as all loads of prepared weights take together, and held the register of every half.  us before /
 // after: 912 -> 16, 5 x 5 on 8 x 11, batch 9 33.5 / 24.8; 1 x 1 864 -> 288 on 16 x 12, batch 2 6.4 / 4.8; 256 -> 256 on 16 x 16,
 // batch 32 16.9 / 14.4; with the planner's new lines geometric mean 1.18 over 160 random shapes and 1.17 over the table's.
-// Slower where the results' stores are all there is: 1 x 1 128 -> 512 on 56 x 56, batch 32, 40.0 / 41.4 - 42.9.
+// Slower for long reductions with barely more than one wave per SIMD (heuristic_plan): those keep the eight loads.
 __device__ __forceinline__ u32 transpose8_sel(int lane) { return lane & 1 ? 0x03020706u : 0x05040100u; }
 __device__ __forceinline__ v4i transpose8(v4i x, u32 sel, bool bit1) {
   constexpr int kXor1 = 0xb1, kXor2 = 0x4e, kFrom4Up = 0x104, kFrom4Down = 0x114;  // quad_perm, row_shl:4, row_shr:4
@@ -79,8 +79,10 @@ __device__ __forceinline__ v4i transpose8(v4i x, u32 sel, bool bit1) {
 // PAD: the convolution has zero padding, so taps can fall outside the image and are masked per
 // lane; without it every tap of every valid pixel lies inside and the masking code is left out.
 // D_ = ring depth, + 16 when the kernel is to be built for four waves per SIMD.
-template <int TX_, int TY_, int KG_, int D_, bool PAD_ = true>
+// HALVES: fp16 weights in the reference's layout come as eight 16-bit loads per fragment and need no transposition.
+template <int TX_, int TY_, int KG_, int D_, bool PAD_ = true, bool HALVES_ = false>
 struct DirectShape {
+  static constexpr bool HALVES = HALVES_;
   static constexpr int TX = TX_, TY = TY_, KG = KG_, D = D_ % 16;
   static constexpr bool PAD = PAD_;
   static constexpr int BX = TX * 32, BY = TY * 32;
@@ -322,7 +324,9 @@ __global__ __launch_bounds__(S::NT) __attribute__((amdgpu_waves_per_eu(PREP && !
   for (int i = 0; i < TX; ++i) {
     int n = x0 + i * 32 + l32;
     n = n < ep.K ? n : ep.K - 1;
-    xoff[i] = (u32)(n >> 4) * (u32)(g.ntaps * WTAP) + (kInt ? (u32)(n & 15) * 4u : (u32)((lane & 7) + half * 8) * 32u + (u32)(lane & 8) * 2u);
+    xoff[i] = (u32)(n >> 4) * (u32)(g.ntaps * WTAP) + (kInt ? (u32)(n & 15) * 4u
+                                                       : S::HALVES ? (u32)(n & 15) * 2u + (u32)half * 256u
+                                                                   : (u32)((lane & 7) + half * 8) * 32u + (u32)(lane & 8) * 2u);
     if constexpr (PREP) {  // blocks past the last one re-read it
       const int kb = min((x0 >> 5) + i, (ep.K - 1) >> 5);
       xoff[i] = ((u32)(kb * nsteps) * 64u + (u32)lane) * 16u;
@@ -383,6 +387,11 @@ __global__ __launch_bounds__(S::NT) __attribute__((amdgpu_waves_per_eu(PREP && !
       } else if constexpr (kInt) {
 #pragma unroll
         for (int d = 0; d < 4; ++d) xf[U][i][d] = *reinterpret_cast<const int *>(wgt + o + d * 64);
+      } else if constexpr (S::HALVES) {
+        v8h h;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) h[k] = *reinterpret_cast<const _Float16 *>(wgt + o + k * 32);
+        xf[U][i] = __builtin_bit_cast(v4i, h);
       } else {
         xf[U][i] = *reinterpret_cast<const v4i *>(wgt + o);  // rows of in-channels; consume() transposes
       }
@@ -559,7 +568,7 @@ __global__ __launch_bounds__(S::NT) __attribute__((amdgpu_waves_per_eu(PREP && !
 #pragma unroll
     for (int i = 0; i < TX; ++i) {
       v4i x = xf[U][i];
-      if constexpr (!kInt && !PREP) x = transpose8(x, wsel, (lane & 2) != 0);
+      if constexpr (!kInt && !PREP && !S::HALVES) x = transpose8(x, wsel, (lane & 2) != 0);
 #pragma unroll
       for (int j = 0; j < TY; ++j) acc[i][j] = Op::mma(x, y[j], acc[i][j]);
     }

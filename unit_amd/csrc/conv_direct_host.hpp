@@ -24,8 +24,8 @@ int run_direct(const char *what, const char *tag, const unit_conv_desc *d, const
   const int gx = ceil_div(d->K, S::BX), gy = ceil_div(g.npix, S::BY);
   const int panel = plan.panel > 0 && plan.panel < gx ? plan.panel : 0;
   const GridMap gm = GridMap::make(gx, gy, panel ? panel : gx, 1);
-  set_variant("%s_x%d_y%d_g%d_d%d%s%s%s_s1", tag, S::BX, S::BY, S::KG, S::D,
-              S::kFourWaves ? "w4" : "", S::PAD ? "" : "n", Panel{panel});
+  set_variant("%s_x%d_y%d_g%d_d%d%s%s%s%s_s1", tag, S::BX, S::BY, S::KG, S::D,
+              S::kFourWaves ? "w4" : "", S::HALVES ? "h" : "", S::PAD ? "" : "n", Panel{panel});
   hipLaunchKernelGGL(kern, dim3(gm.total), dim3(S::NT), lds, s, static_cast<const char *>(data),
                      static_cast<const char *>(w), ep, g, gm UNIT_TRACE(, trace_buffer()));
   hipError_t e = hipGetLastError();

@@ -37,6 +37,7 @@ struct ConvPlan {
   // a small panel gives each XCD a slice of the weights and all pixels: the better choice is the
   // one that pulls fewer bytes into the 8 L2s, which start cold at every kernel.
   int panel;
+  bool halves = false;  // variant 68 of the fp16 operator on blocked weights: DirectShape's HALVES
 };
 
 struct TunedConv {
@@ -117,18 +118,38 @@ inline ConvPlan heuristic_plan(const unit_conv_desc *d, int npix, int kbytes, bo
       //   up to 1568 tiles, where 128-channel tiles or staged ones ran, one wave per tile or, past 90 k-steps and with two of them per CU, 64 x 128 (512 ->
       //   128, 1 x 1 on 28 x 28, batch 32, 14.5 / 9.8; 128 -> 1312, 5 x 5 on 14 x 20, batch 15, 38.2 / 35.4);
       //   from 1568 tiles on four deep (64 -> 32, 3 x 3 on 65 x 83, batch 27, 19.9 / 16.9; 512 -> 608, 1 x 1 on 86 x 60, batch 3,
-      //   23.5 / 20.8).
+      //   23.5 / 20.8), but from 10000 tiles and up to 18 k-steps three (32 -> 1648, 3 x 3 stride 2 on 80 x 112, batch 12, four deep
+      //   64.3, three 60.7, six 61.1; 16 -> 1328, 3 x 3 on 80 x 111, batch 5 48.9 and 45.7).
+      // Where these tiles are slower than with eight 16-bit loads per fragment, us then / these tiles / now:
+      //   up to 32 channels, half of a 64-channel tile padding: 32 x 64 tiles of four groups (144 -> 32, 3 x 3 on 105 x 66, batch 5
+      //   16.7 / 18.4 / 9.9; 496 -> 16, 5 x 5 on 30 x 41, batch 37 141 / 151 / 60; 512 -> 32 on 74 x 97, batch 11 71.7 / 77.3 / 41.6);
+      //   few tiles, but more than 256 of 64 x 128: two groups there too (160 -> 1264, 3 x 3 stride 2 on 26 x 22, batch 13 18.3 /
+      //   20.0 / 16.8);
+      //   1025 to 1280 tiles, hardly more than one wave per SIMD, and 48 steps or more: the eight loads (128 -> 1904, 3 x 3 on
+      //   16 x 15, batch 13 22.5 / 23.8; 448 -> 112, 3 x 3 on 55 x 54, batch 12 62.4 / 66.1; 40 - 45 steps 0.98 - 1.01 of them, 1287
+      //   tiles 0.96);
+      //   9 - 16 k-steps on 784 to 1568 tiles: one wave per tile there too (256 -> 1792 on 12 x 8, batch 24 9.5 / 9.8 / 7.8);
+      //   up to 8 k-steps the stores decide: three deep at four waves per SIMD below 4000 tiles (64 -> 912 on 18 x 17, batch 45 12.0 /
+      //   12.7 / 12.0; 80 -> 1520 on 20 x 16, batch 26 12.8 / 13.2 / 12.2; on 25 others 0.76 - 0.98 of then), six deep from 7000
+      //   tiles and up to 4 steps (16 -> 240 on 99 x 112, batch 17 32.2 / 34.4 / 32.9; 64 -> 1088 on 81 x 112, batch 3 24.3 / 25.4 /
+      //   24.1).  Left: 128 -> 1040 on 34 x 50, batch 6 11.8 / 12.3 / 12.1.
       if (staged_too) {
         if (nsteps >= 32 && K % 256 == 0 && tiles(256, 256) >= 196) return ConvPlan{0, 1, 0};
+        if (nsteps <= 8 && t64 >= 1568) {
+          if (t64 < 4000 && nsteps < 8) return ConvPlan{71, 1, 0};
+          if (t64 >= 7000 && nsteps <= 4) return ConvPlan{68, 1, 0};
+        }
         if (t64 > 256 && nsteps > 8) {
           if (t64 < 392 && nsteps <= 24) return ConvPlan{60, 1, 0};
           if (tiles(64, 128) <= 256 && nsteps > 24) return ConvPlan{59, 1, 0};
-          if (t64 > 512 && t64 <= 768 && nsteps > 24 && K > 32) return ConvPlan{67, 1, 0};
+          if (K <= 32 && nsteps > 24 && t64 < 1568) return ConvPlan{61, 1, 0};
+          if (t64 >= 392 && t64 <= 768 && nsteps > 24) return ConvPlan{67, 1, 0};
+          if (t64 > 1024 && t64 <= 1280 && nsteps >= 48) return ConvPlan{68, 1, 0, true};
           if (t64 >= 784 && t64 < 1568) {
             if (nsteps >= 90 && tiles(64, 128) <= 512) return ConvPlan{59, 1, 0};
-            if (nsteps > 36) return ConvPlan{68, 1, 0};
-            if (nsteps > 16) return ConvPlan{50, 1, 0};
+            return ConvPlan{nsteps > 36 ? 68 : 50, 1, 0};
           }
+          if (t64 >= 10000 && nsteps <= 18) return ConvPlan{65, 1, 0};
           if (t64 >= 1568 && (!wide || nsteps > 36)) return ConvPlan{50, 1, 0};
         }
       }
@@ -193,7 +214,7 @@ inline ConvPlan plan_conv(const unit_conv_desc *d, int npix, int kbytes, const T
     if (t.kg * (scratch + tile) + (long)(kbytes / 32) * 8 > kMaxLds) p = ConvPlan{68, 1, p.panel};
   }
   const int ov = tuning_override("UNIT_AMD_CONV_VARIANT"), os = tuning_override("UNIT_AMD_CONV_SPLITK");
-  if (ov > 0 && ov <= kNumConvTiles) p.variant = ov - 1;
+  if (ov > 0 && ov <= kNumConvTiles) p.variant = ov - 1, p.halves = false;
   if (os > 0) p.splits = os;
   const int op = tuning_override("UNIT_AMD_CONV_PANEL");
   if (op > 0) p.panel = op;
@@ -201,7 +222,7 @@ inline ConvPlan plan_conv(const unit_conv_desc *d, int npix, int kbytes, const T
   // the LDS-shared variants exist for prepared weights with 16-channel blocks only: elsewhere their ids run the heuristic's choice
   if (kConvTiles[p.variant].lds && !lds_ok) {
     const ConvPlan h = heuristic_plan(d, npix, kbytes, allow_split, direct_ok, staged_too);
-    p.variant = h.variant;
+    p.variant = h.variant, p.halves = h.halves;
     if (!allow_split) p.splits = 1;
   }
   return p;
