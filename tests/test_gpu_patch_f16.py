@@ -40,3 +40,28 @@ def test_infinities_stay_in_their_windows(dev):
     bad = torch.isinf(out).nonzero()
     assert len(bad) == 9 * 256 and set(map(tuple, bad[:, [0, 2, 3]].tolist())) == {(5, h, v) for h in (1, 2, 3) for v in (7, 8, 9)}
     assert torch.equal(out[~torch.isinf(out)], torch.full_like(out[~torch.isinf(out)], 2304.0))
+
+
+# N, C, H, W, K where other kernels are faster: a measured choice of the table, 128-channel tiles that fill the chip, a second round
+# that few channel blocks do not pay for, one round of short reductions
+OTHERS = [(256, 512, 9, 9, 512, "f16lds_"), (20, 336, 25, 33, 512, "f16prep_x128_y64_"), (9, 288, 18, 20, 1456, "f16prep_x64_y64_"),
+          (102, 144, 16, 21, 48, "f16prep_x64_y64_"), (6, 832, 49, 73, 96, "f16prep_x64_y64_")]
+
+
+@pytest.mark.parametrize("N,C,H,W,K,name", OTHERS)
+def test_shapes_that_stay_with_other_kernels(dev, N, C, H, W, K, name):
+    w = U.prepare_conv2d_weight(torch.ones((K // 16, C // 16, 3, 3, 16, 16), device=dev, dtype=torch.float16))
+    out = U.conv2d_NCHW16c_OHWI16o(torch.ones((N, C // 16, H, W, 16), device=dev, dtype=torch.float16), w, 1, 1)
+    assert U.last_variant().startswith(name), U.last_variant()
+    assert (out == 9.0 * C).all()
+
+
+@pytest.mark.parametrize("pin", ["UNIT_AMD_CONV_VARIANT", "UNIT_AMD_CONV_PANEL", "UNIT_AMD_CONV_SPLITK"])
+def test_pinned_plans_reach_the_other_kernels(dev, monkeypatch, pin):
+    N, C, H, W, K, _ = SHAPES[0]
+    w = U.prepare_conv2d_weight(torch.ones((K // 16, C // 16, 3, 3, 16, 16), device=dev, dtype=torch.float16))
+    x = torch.ones((N, C // 16, H, W, 16), device=dev, dtype=torch.float16)
+    monkeypatch.setenv(pin, "60" if pin.endswith("VARIANT") else "1")
+    out = U.conv2d_NCHW16c_OHWI16o(x, w, 1, 1)
+    assert "patch" not in U.last_variant(), U.last_variant()
+    assert (out == 9.0 * C).all()

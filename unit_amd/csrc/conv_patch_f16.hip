@@ -239,17 +239,29 @@ int run_patch(const unit_conv_desc *d, const ConvGeom &g, const void *a, const v
 
 }  // namespace
 
-// Where it pays: us here 5.9 + 0.37 per channel block while there is at most one tile per CU, else 4.6 + 0.45 per channel
-// block for each round of 256 tiles (a workgroup's start and its 128 KB of output meet nobody's arithmetic), as direct tiles
-// 3.2 + 2.7 per GMAC.  Measured, direct / here: 220 tiles of 33 channel blocks 32.3 / 22.1, 188 of 21 19.2 / 14.8, 396 of 52
-// 66.7 / 50.7, 915 of 23 62.9 / 60.2; the other way 792 of 26 59.4 / 65.6, 374 of 14 17.2 / 23.1, 1770 of 9 47.4 / 63.2, 104 of
-// 32 14.3 / 15.0, 100 of 16 8.2 / 9.9.
+// Where it pays: us here / on the direct kernels' tiles, by the kernel that heuristic_plan would take.  A round of 256 tiles costs
+// 4.6 us and, per channel block (the wave with the most of them counts), half a microsecond, half as much in the first and in
+// the last round, by how full that one is (a workgroup's start and its 128 KB of output meet nobody's arithmetic); weights 0.2 us
+// per MB.  Direct tiles: few of 64 x 64 3.2 us + 2.7 per GMAC; one wave per tile 3 us and, per channel block, 0.78 with up to two of
+// them per CU, 0.84 with three, 1.22 with four, else 0.32 for each; 128-channel tiles of four groups 4.6 + 0.53, and past 1568
+// tiles of 64 x 64 128-channel tiles of one wave are not beaten.  Fitted to 843 random shapes timed both ways: of the 597 it takes
+// 5 lose, up to 8 % (geometric mean 0.72); a rule on arithmetic alone lost up to 33 %.  220 tiles of 33 channel blocks 22.1 / 32.3,
+// 188 of 21 14.8 / 19.2; the other way 104 of 32 15.0 / 14.3, 212 of 9 12.8 / 10.4, 483 of 18 29.4 / 24.1, 896 of 21, 128-channel
+// tiles, 55.2 / 41.6.
 bool patch_f16_takes(const unit_conv_desc *d, const ConvGeom &g) {
   const int cc = d->C / 16;
   if (d->sh != 1 || d->sw != 1 || d->KH != 3 || d->KW != 3 || cc < kGroups || patch_pixels(g) > 64 * 8) return false;
-  const long tiles = (long)ceil_div(d->K, kBX) * ceil_div(g.npix, kBY), rounds = (tiles + 255) / 256;
-  const double direct = 3.2 + 2.7e-9 * g.npix * d->K * cc * 144;
-  return rounds == 1 ? 5.9 + 0.37 * cc < 0.97 * direct : rounds * (4.6 + 0.45 * cc) < 0.92 * direct;
+  const long tiles = (long)ceil_div(d->K, kBX) * ceil_div(g.npix, kBY), t64 = (long)ceil_div(d->K, 64) * ceil_div(g.npix, 64);
+  if (t64 < 392) return 5.9 + 0.37 * cc < 0.97 * (3.2 + 2.7e-9 * g.npix * d->K * cc * 144);
+  const bool wide = d->K % 128 == 0;
+  if (wide && t64 >= 1568) return false;
+  const long rounds = (tiles + 255) / 256, waves = (t64 + 255) / 256;
+  const double last = tiles / 256.0 - (rounds - 1);
+  const double here = 1 + 4.6 * rounds + (ceil_div(cc, kGroups) * kGroups - 1.5) * (0.5 * rounds - 0.3 + 0.26 * last) +
+                      0.2e-6 * d->K * cc * 288;
+  const double block = waves <= 2 ? 0.78 : waves == 3 ? 0.84 : waves == 4 ? 1.22 : 0.32 * waves;
+  const double direct = wide && waves <= 2 ? 4.6 + 0.53 * cc : 3 + block * cc;
+  return here < 0.96 * direct;
 }
 
 int conv_f16_patch(const unit_conv_desc *d, const ConvGeom &g, const void *a, const void *w, void *out, hipStream_t s) {

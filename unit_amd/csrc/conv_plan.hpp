@@ -190,22 +190,26 @@ inline ConvPlan heuristic_plan(const unit_conv_desc *d, int npix, int kbytes, bo
   return ConvPlan{v, splits, 0};
 }
 
-inline ConvPlan plan_conv(const unit_conv_desc *d, int npix, int kbytes, const TunedConv *table, int ntable,
-                          bool allow_split, bool direct_ok, bool staged_too = false, bool lds_ok = false) {
-  ConvPlan p = heuristic_plan(d, npix, kbytes, allow_split, direct_ok, staged_too);
+// The measured choice for this shape, or null.
+inline const TunedConv *tuned_row(const unit_conv_desc *d, int npix, const TunedConv *table, int ntable, bool direct_ok, bool lds_ok) {
   // UNIT_AMD_CONV_NOTABLE=1: heuristic only (the tuner measures it as the baseline)
-  if (tuning_override("UNIT_AMD_CONV_NOTABLE") > 0) ntable = 0;
+  if (tuning_override("UNIT_AMD_CONV_NOTABLE") > 0) return nullptr;
   for (int i = 0; i < ntable; ++i) {
     const TunedConv &e = table[i];
     // the tables were tuned on square strides without dilation; a direct choice needs a window the direct
     // kernels can run, otherwise the heuristic's (staged) choice stands
     if (e.npix == npix && e.K == d->K && e.C == d->C && e.KH == d->KH && e.KW == d->KW && e.sh == d->sh &&
         d->sw == d->sh && d->dh == 1 && d->dw == 1 && (direct_ok || !kConvTiles[e.variant].direct) &&
-        (lds_ok || !kConvTiles[e.variant].lds)) {
-      p = ConvPlan{e.variant, e.splits, e.panel};
-      break;
-    }
+        (lds_ok || !kConvTiles[e.variant].lds))
+      return &e;
   }
+  return nullptr;
+}
+
+inline ConvPlan plan_conv(const unit_conv_desc *d, int npix, int kbytes, const TunedConv *table, int ntable,
+                          bool allow_split, bool direct_ok, bool staged_too = false, bool lds_ok = false) {
+  ConvPlan p = heuristic_plan(d, npix, kbytes, allow_split, direct_ok, staged_too);
+  if (const TunedConv *e = tuned_row(d, npix, table, ntable, direct_ok, lds_ok)) p = ConvPlan{e->variant, e->splits, e->panel};
   // A direct variant whose k-groups park one float tile each can outgrow the LDS on very deep reductions (the tap
   // table follows the tiles): the one-wave six-deep kernel of the same family always fits.
   if (!allow_split && kConvTiles[p.variant].direct && kConvTiles[p.variant].kg > 1) {

@@ -358,7 +358,10 @@ extern "C" int unit_conv2d_nchw16c_f16f32_prepared(const unit_conv_desc *d, cons
   ConvGeom g;
   if (int rc = check_prepared_conv(what, d, 32, &g, a, prepared, out)) return rc;
   const int ntable = (int)(sizeof(kTunedF16Prepared) / sizeof(kTunedF16Prepared[0])) - 1;
-  if (tuning_override("UNIT_AMD_CONV_VARIANT") <= 0 && patch_f16_takes(d, g))
+  // measured choices and pinned ones first: the patch kernel is no variant that a table row could name
+  const bool pinned = tuning_override("UNIT_AMD_CONV_VARIANT") > 0 || tuning_override("UNIT_AMD_CONV_PANEL") > 0 ||
+                      tuning_override("UNIT_AMD_CONV_SPLITK") > 0;
+  if (!pinned && !tuned_row(d, g.npix, kTunedF16Prepared, ntable, true, true) && patch_f16_takes(d, g))
     return conv_f16_patch(d, g, a, prepared, out, static_cast<hipStream_t>(stream));
   const ConvPlan p = plan_prepared(d, g, g.ntaps * 32, kTunedF16Prepared, ntable, false, true);
   if (kConvTiles[p.variant].lds) return conv_f16_prepared_lds(p, d, g, a, prepared, out, static_cast<hipStream_t>(stream));
