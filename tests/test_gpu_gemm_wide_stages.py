@@ -17,7 +17,9 @@ def _ints(g, lo, hi, shape, dtype, dev):
 F16 = [(70, 260, 808, None, "x32_y32_k128_w1x1_g4_r3"), (129, 1028, 1000, None, "x32_y32_k128_w1x1_g4_r3"),
        (700, 700, 712, "x32_y64_k128_w1x2_g4_r3", "x32_y64_k128_w1x2_g4_r3"),
        (900, 900, 520, "x64_y64_k128_w2x2_g2_r3", "x64_y64_k128_w2x2_g2_r3"),
-       (1000, 1516, 1096, "x64_y128_k128_w2x2_g2_r3", "x64_y128_k128_w2x2_g2_r3"),
+       (1000, 1516, 1096, None, "x64_y128_k128_w2x2_g2_r3"),  # rows of b end inside lines: from 3 KiB of reduction on
+       (1000, 1536, 1096, "x64_y128_k128_w2x2_g2_r3", "x64_y128_k128_w2x2_g2_r3"),
+       (800, 1500, 1536, "x64_y128_k128_w2x2_g2_r3", "x64_y128_k128_w2x2_g2_r3"),
        (900, 1660, 1608, "x64_y128_k128_w2x2_g2_r3", "x64_y128_k128_w2x2_g2_r3"),
        (1500, 1508, 1496, "x128_y128_k128_w4x2_g1_r3", "x128_y128_k128_w4x2_g1_r3")]
 # M, N, K (bytes), tile with row-major, prepared and packed weights

@@ -459,16 +459,18 @@ inline float large_tile_cost(int M, int N, int kb) {
 // that is worth more.  us on operands that change from call to call, 64 / 128 bytes: fp16 700 x 2304 x 3008 20.5 / 16.9,
 // 900 x 1664 x 1600 12.6 / 10.8, prepared 500 x 2048 x 2048 11.3 / 9.3, 1500 x 1536 x 1504 17.4 / 15.1; int8 packed 900 x
 // 1664 x 1600 11.4 / 9.9, 1500 x 1536 x 1504 14.7 / 11.8, row-major 700 x 2304 x 3008 16.0 / 13.3; geometric mean over the 84 of
-// 231 random products that it takes 1.11, lowest 0.98; fp16 1000 x 1516 x 1096, whose rows of b end inside lines, 10.5 / 10.5.
+// 231 random products that it takes 1.11, lowest 0.98.
 // The other way: 512 tiles of 64 x 64 (2000 x 1024 x 512) 6.8 / 7.9, 640 bytes of reduction (702 x 1216 x 320) 4.3 / 4.5 and, on
-// 32 x 32 tiles, 1088 (93 x 2112 x 544) 3.75 / 3.88, b by
-// columns on 32 x 32 tiles, whose rows of b stay 64 bytes, 15 x 2560 x 5488 17.6 / 20.1.  int8 products of up to 64 rows and
-// 4096 columns keep the tiles that the tests name for them.
+// 32 x 32 tiles, 1088 (93 x 2112 x 544) 3.75 / 3.88, b by columns on 32 x 32 tiles, whose rows of b stay 64 bytes, 15 x 2560 x 5488
+// 17.6 / 20.1.  b by columns whose rows end inside lines, on 64 x 128 tiles, up to 3 KiB of reduction: 1000 x 1516 x 1096 10.34 /
+// 10.41 (fp32 result 10.7 / 11.0), 966 x 1804 x 856 9.6 / 10.0, 822 x 2280 x 1016 10.4 / 10.7, others down to 0.93; from 3 KiB on
+// 0.91 - 1.01.  int8 products of up to 64 rows and 4096 columns keep the tiles that the tests name for them.
 template <class Op, int YM>
 bool group_wide_stages(const GroupGemm &p, const GroupPlan &plan) {
   const GroupCost &g = kGroupCosts[plan.tile];
   return plan.splits == 1 && p.kb >= (plan.tile < 2 ? 1536 : 960) && (long)ceil_div(p.M, g.bx) * ceil_div(p.N, g.by) <= 256 &&
-         !(Op::kInt && p.M <= 64 && p.N <= 4096) && !(YM == Y_COLS && plan.tile < 2);
+         !(Op::kInt && p.M <= 64 && p.N <= 4096) &&
+         !(YM == Y_COLS && (plan.tile < 2 || (plan.tile == 4 && p.kb < 3072 && p.ldy % 128)));
 }
 
 template <class Op, int YM, int WS, bool OUT_F16>
