@@ -15,9 +15,10 @@ F16 = [(1, 8, 8, "x32_y32_k64_w1x1_g4"), (33, 12, 24, "x32_y32"), (37, 36, 200, 
        (700, 700, 712, "x32_y64"), (300, 3004, 296, "x64_y64"), (1000, 1516, 1096, "x64_y128"),
        (1500, 1508, 1496, "x128_y128"), (2180, 2052, 2056, "x128_y128"), (3840, 2044, 2056, "x256_y128"), (129, 8192, 40, "")]
 # M, N, K; the tile with row-major or prepared weights, and with packed ones (None: N is no multiple of 128)
-G4, G8 = "x32_y32_k64_w1x1_g4", "x32_y32_k64_w1x1_g8"
-I8 = [(1, 4, 16, G4, None), (33, 36, 80, G4, None), (1, 256, 480, G8, G8), (50, 260, 1040, G4, None), (37, 128, 4112, G4, G4),
-      (64, 4096, 4096, G8, G8), (700, 704, 720, "x32_y64", None), (128, 3072, 784, "x32_y64", "x32_y64"),
+G4, G8, G4W = "x32_y32_k64_w1x1_g4", "x32_y32_k64_w1x1_g8", "x32_y32_k128_w1x1_g4"
+I8 = [(1, 4, 16, G4, None), (33, 36, 80, G4, None), (1, 256, 480, G8, G8), (50, 260, 1040, G4, None), (37, 128, 4112, G4, G4W),
+      (64, 4096, 2064, "x32_y32_k64", "x32_y32_k64"), (64, 4096, 3056, "x32_y32_k64", "x32_y32_k64"), (64, 4096, 4096, G4W, G4W),
+      (700, 704, 720, "x32_y64", None), (128, 3072, 784, "x32_y64", "x32_y64"),
       (129, 8192, 48, "x64_y64", "x64_y64"), (300, 3072, 304, "x64_y64", "x64_y64"), (1467, 1108, 976, "x64_y128", None),
       (1000, 1536, 1104, "x64_y128", "x64_y128"), (1500, 1536, 1552, "x128_y128", "x128_y128"),
       (2180, 2176, 2064, "x128_y128", "x128_y128"), (1175, 4864, 1632, "x256_y128", "x256_y128"),

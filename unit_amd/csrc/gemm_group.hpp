@@ -464,12 +464,14 @@ inline float large_tile_cost(int M, int N, int kb) {
 // 32 x 32 tiles, 1088 (93 x 2112 x 544) 3.75 / 3.88, b by columns on 32 x 32 tiles, whose rows of b stay 64 bytes, 15 x 2560 x 5488
 // 17.6 / 20.1.  b by columns whose rows end inside lines, on 64 x 128 tiles, up to 3 KiB of reduction: 1000 x 1516 x 1096 10.34 /
 // 10.41 (fp32 result 10.7 / 11.0), 966 x 1804 x 856 9.6 / 10.0, 822 x 2280 x 1016 10.4 / 10.7, others down to 0.93; from 3 KiB on
-// 0.91 - 1.01.  int8 products of up to 64 rows and 4096 columns keep the tiles that the tests name for them.
+// 0.91 - 1.01.  int8 products of up to 64 rows and 4096 columns, where a launch's latency is most of it, up to 3 KiB:
+// 64 x 4096 x 1536 prepared 5.0 / 5.4, 1 x 4096 x 2048 4.8 / 5.2, packed 23 x 2944 x 2240 5.0 / 5.3; from there on 64 x 4096 x 4096
+// row-major 7.8 / 6.3, packed 7.1 / 6.5, 1 x 4096 x 4096 6.2 / 6.0, 57 x 3712 x 8112 prepared 15.9 / 12.6 (64 x 8192 x 1536 6.0 / 4.9).
 template <class Op, int YM>
 bool group_wide_stages(const GroupGemm &p, const GroupPlan &plan) {
   const GroupCost &g = kGroupCosts[plan.tile];
-  return plan.splits == 1 && p.kb >= (plan.tile < 2 ? 1536 : 960) && (long)ceil_div(p.M, g.bx) * ceil_div(p.N, g.by) <= 256 &&
-         !(Op::kInt && p.M <= 64 && p.N <= 4096) &&
+  const int least = plan.tile >= 2 ? 960 : Op::kInt && p.M <= 64 && p.N <= 4096 ? 3072 : 1536;
+  return plan.splits == 1 && p.kb >= least && (long)ceil_div(p.M, g.bx) * ceil_div(p.N, g.by) <= 256 &&
          !(YM == Y_COLS && (plan.tile < 2 || (plan.tile == 4 && p.kb < 3072 && p.ldy % 128)));
 }
 
