@@ -22,10 +22,13 @@ F16 = [(70, 260, 808, None, "x32_y32_k128_w1x1_g4_r3"), (129, 1028, 1000, None, 
        (800, 1500, 1536, "x64_y128_k128_w2x2_g2_r3", "x64_y128_k128_w2x2_g2_r3"),
        (900, 1660, 1608, "x64_y128_k128_w2x2_g2_r3", "x64_y128_k128_w2x2_g2_r3"),
        (1500, 1508, 1496, "x128_y128_k128_w4x2_g1_r3", "x128_y128_k128_w4x2_g1_r3")]
-# M, N, K (bytes), tile with row-major, prepared and packed weights
-I8 = [(65, 512, 1552, "x32_y32_k128_w1x1_g4_r3"), (128, 768, 3024, "x32_y32_k128_w1x1_g4_r3"),
-      (330, 1280, 2608, "x32_y64_k128_w1x2_g4_r3"), (1000, 1024, 1008, "x64_y64_k128_w2x2_g2_r3"),
-      (900, 1664, 1616, "x64_y128_k128_w2x2_g2_r3"), (1501, 1536, 1552, "x128_y128_k128_w4x2_g1_r3")]
+# M, N, K (bytes), tile with row-major and prepared weights (None: shared between workgroups, 64-byte stages), and with packed ones
+I8 = [(65, 512, 1552, None, "x32_y32_k128_w1x1_g4_r3"), (128, 768, 3024, None, "x32_y32_k128_w1x1_g4_r3"),
+      (64, 1536, 3088, "x32_y32_k128_w1x1_g4_r3", "x32_y32_k128_w1x1_g4_r3"),
+      (330, 1280, 2608, "x32_y64_k128_w1x2_g4_r3", "x32_y64_k128_w1x2_g4_r3"),
+      (1000, 1024, 1008, "x64_y64_k128_w2x2_g2_r3", "x64_y64_k128_w2x2_g2_r3"),
+      (900, 1664, 1616, "x64_y128_k128_w2x2_g2_r3", "x64_y128_k128_w2x2_g2_r3"),
+      (1501, 1536, 1552, "x128_y128_k128_w4x2_g1_r3", "x128_y128_k128_w4x2_g1_r3")]
 
 
 @pytest.mark.parametrize("M,N,K,by_columns,prepared", F16)
@@ -39,17 +42,15 @@ def test_fp16(dev, M, N, K, by_columns, prepared):
         assert torch.equal(U.gemm_fp16(a, operand).double(), ref), U.last_variant()
 
 
-@pytest.mark.parametrize("M,N,K,tile", I8)
-def test_int8(dev, M, N, K, tile):
+@pytest.mark.parametrize("M,N,K,rows,packed", I8)
+def test_int8(dev, M, N, K, rows, packed):
     g = np.random.RandomState(M + N + K)
     a, w = _ints(g, 0, 256, (M, K), torch.uint8, dev), _ints(g, -128, 128, (N, K), torch.int8, dev)
     ref = (a.double() @ w.double().t()).to(torch.int32)
-    taken = 0
-    for call in (lambda: U.dense(a, w), lambda: U.dense(a, U.prepare_dense_weight(w)),
-                 lambda: U.dense_dotprod(a, U.prepack_dense_weight(w))):
+    for call, tile in ((lambda: U.dense(a, w), rows), (lambda: U.dense(a, U.prepare_dense_weight(w)), rows),
+                       (lambda: U.dense_dotprod(a, U.prepack_dense_weight(w)), packed)):
         assert torch.equal(call(), ref), U.last_variant()
-        taken += tile in U.last_variant()
-    assert taken, U.last_variant()
+        assert (tile or "_k64_") in U.last_variant(), U.last_variant()
 
 
 def test_fp16_infinity_past_a_row(dev):
