@@ -1,5 +1,5 @@
-"""The native operator calls (csrc/calls.cpp) built for CPU tensors, without a GPU: what they do with tensors that have no data
-pointer.  The library behind them refuses the call (no device), which is what an ordinary operand gets here."""
+"""The native operator calls (csrc/calls.cpp) without a GPU: built for CPU tensors, what they do with tensors that have no data
+pointer; and the package without them, or without the library."""
 import os
 import subprocess
 import sys
@@ -7,6 +7,9 @@ import sysconfig
 
 import pytest
 import torch
+
+import unit_amd
+from unit_amd import _lib, ops
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -94,3 +97,30 @@ def test_tensors_without_storage_are_declined(module):
     """vmap's wrapped tensors are torch.Tensors of the right type and shape; asking one for its data throws."""
     r = subprocess.run([sys.executable, "-c", PROGRAM, str(module), ROOT], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and r.stdout.strip() == "declined", (r.returncode, r.stdout, r.stderr[-2000:])
+
+
+def test_without_the_module_the_python_operators_take_the_call(monkeypatch):
+    monkeypatch.delattr(unit_amd, "_calls", raising=False)
+    monkeypatch.setitem(sys.modules, "unit_amd._calls", None)
+    monkeypatch.setattr(ops, "_native", ops._Calls())
+    a = torch.zeros((4, 16), dtype=torch.float16)
+    with pytest.warns(RuntimeWarning, match="make -C"), pytest.raises(ValueError, match="must live on the GPU"):
+        ops.gemm_fp16(a, a)
+    with pytest.raises(ValueError, match="must live on the GPU"):  # said once
+        ops.dense(a.to(torch.uint8), a.to(torch.int8))
+
+
+def test_without_the_library_arguments_are_checked_first(monkeypatch):
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "LIB_PATH", os.path.join(ROOT, "no such library"))
+    monkeypatch.setattr(ops, "_native", ops._Calls())
+    with pytest.raises(TypeError, match="expected a torch.Tensor"):
+        ops.gemm_fp16([1.0], None)
+    with pytest.raises(_lib.UnitError, match="make -C"):
+        _lib.load()
+
+
+def test_make_without_torch_builds_the_library_alone():
+    make = ["make", "-n", "-C", os.path.join(ROOT, "unit_amd", "csrc"), "-W", "calls.cpp", "all"]
+    assert "_calls.so" in subprocess.run(make, capture_output=True, text=True, check=True).stdout
+    assert "_calls.so" not in subprocess.run(make + ["TORCH="], capture_output=True, text=True, check=True).stdout

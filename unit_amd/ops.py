@@ -11,7 +11,9 @@ Reference call sites:
   gemm_fp16                apps/gpu/gemm.py:8-20
 """
 import ctypes
+import os
 import re
+import warnings
 from functools import lru_cache
 
 import torch
@@ -164,7 +166,10 @@ def last_variant():
 # ------------------------------------------------------------------------------- native calls
 class _Calls:
     """The operators' common case as native functions (csrc/calls.cpp): each returns the result, or None for a call that
-    it does not take, which then runs through the Python below.  Bound on first use to the library that ctypes loaded."""
+    it does not take, which then runs through the Python below.  Bound on first use to the library that ctypes loaded.  The
+    module is built against the installed torch (csrc/Makefile); where there is none that fits, the Python takes every call."""
+
+    _NAMES = ("conv_u8", "conv_fused", "conv_requant", "conv3d", "conv_f16", "dense", "gemm")
 
     _LIBRARY = ("unit_conv_out_hw", "unit_conv2d_nchwc_u8s8s32", "unit_conv2d_nchwc_u8s8s32_prepared", "unit_conv2d_nchwc_s8s8s32_fused",
                 "unit_conv2d_nchwc_s8s8s32_fused_prepared", "unit_conv2d_nchwc_u8s8u8_requant_prepared", "unit_conv3d_ncdhwc_s8s8s32",
@@ -173,13 +178,30 @@ class _Calls:
                 "unit_gemm_f16", "unit_gemm_f16_prepared", "unit_gemm_f16_ws")
 
     def __getattr__(self, name):  # the first use of each function
-        L = _lib.load()
-        from . import _calls
-        _calls.bind(tuple(ctypes.cast(getattr(L, f), ctypes.c_void_p).value for f in self._LIBRARY), PreparedConvWeight,
-                    PreparedDenseWeight, PreparedGemmB, torch.int8, torch.float16)
-        fn = getattr(_calls, name)
+        if name not in self._NAMES:
+            raise AttributeError(name)
+        try:
+            L = _lib.load()
+        except _lib.UnitError:  # not built: said by the Python operator, after its checks
+            return _declined
+        try:
+            from . import _calls
+            _calls.bind(tuple(ctypes.cast(getattr(L, f), ctypes.c_void_p).value for f in self._LIBRARY), PreparedConvWeight,
+                        PreparedDenseWeight, PreparedGemmB, torch.int8, torch.float16)
+            fn = getattr(_calls, name)
+        except (ImportError, AttributeError, ValueError) as e:
+            fn = _declined
+            if "_said" not in self.__dict__:
+                self._said = True
+                warnings.warn(f"unit_amd: the native operator calls do not fit this torch or are not built ({e}); every call goes "
+                              f"through Python, about 2 us slower. Build them with `make -C {os.path.dirname(__file__)}/csrc`.",
+                              RuntimeWarning, stacklevel=3)
         setattr(self, name, fn)
         return fn
+
+
+def _declined(*args):
+    return None
 
 
 _native = _Calls()
