@@ -316,10 +316,10 @@ typedef struct unit_chain_layer {
 } unit_chain_layer;
 int unit_conv_chain_u8(const unit_chain_layer *layers, int32_t count, const void *x, unit_stream_t stream);
 
-/* The same with a workspace of unit_conv_chain_u8_ws_bytes(layers, count) bytes (16-byte aligned, of any contents, the
- * call's alone until it has run on the stream): the layers then run inside one persistent kernel.  A count of 0 bytes
- * says that the chain has no such form; it then runs as unit_conv_chain_u8 does, as it also does with ws == NULL, with
- * too small a workspace or with a kernel variant pinned. */
+/* From version 108 on.  The same with a workspace of unit_conv_chain_u8_ws_bytes(layers, count) bytes (16-byte aligned,
+ * of any contents, the call's alone until it has run on the stream): the layers then run inside one persistent kernel.  A
+ * count of 0 bytes says that the chain has no such form; it then runs as unit_conv_chain_u8 does, as it also does with
+ * ws == NULL, with too small a workspace or with a kernel variant pinned. */
 int unit_conv_chain_u8_ws_bytes(const unit_chain_layer *layers, int32_t count, size_t *bytes);
 int unit_conv_chain_u8_ws(const unit_chain_layer *layers, int32_t count, const void *x, void *ws, size_t ws_bytes,
                           unit_stream_t stream);
