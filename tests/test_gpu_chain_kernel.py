@@ -113,6 +113,32 @@ def test_chain_kernel_replay_and_two_streams(dev, oracle):
     assert all(np.array_equal(o.cpu().numpy(), r) for o, r in zip(c.outputs, want))
 
 
+def test_chains_on_two_streams(dev, oracle):
+    """Two chains of the same layers on different inputs, run after run on two streams at once: neither sees the other's tickets,
+    flags or results."""
+    spec, n, c0, h, w = CASES["odd_blocks_uneven_groups"]
+    x, layers, want = _build(oracle, spec, n, c0, h, w)
+    inputs = [x, rng.uniform_u8(x.shape, 99)]
+    wants = [want, _oracle_chain(oracle, layers, inputs[1])]
+    assert not np.array_equal(wants[0][-1], wants[1][-1])
+    chains = [chain.ConvChain(_to_chain(layers, dev), x.shape) for _ in inputs]
+    xs = [_t(a, dev) for a in inputs]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    kept = [[], []]
+    torch.cuda.synchronize()
+    for _ in range(6):
+        for k in (0, 1):
+            with torch.cuda.stream(streams[k]):
+                chains[k](xs[k])
+                kept[k].append([o.clone() for o in chains[k].outputs])  # every run's, not the last one's only
+    torch.cuda.synchronize()
+    for k in (0, 1):
+        chains[k].check()
+        for outs in kept[k]:
+            assert all(np.array_equal(o.cpu().numpy(), r) for o, r in zip(outs, wants[k]))
+    assert all(v.startswith("q8chain_") for c in chains for v in c.variants)
+
+
 def test_chain_with_reused_buffers_runs_layer_by_layer(dev, oracle):
     spec = [(32, (3, 3), 1, 1, None)] * 12
     x, layers, want = _build(oracle, spec, 9, 32, 9, 9)
