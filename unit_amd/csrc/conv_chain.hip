@@ -43,7 +43,7 @@ constexpr int kDepth = 5;         // k-steps of fragments in flight per wave
 constexpr int kMaxXcd = 16, kMaxChain = 256;
 constexpr int kAgent = 16;        // sc1
 // Polls a wave may spend in all before it stops waiting (seconds; a whole chain takes some thousand): every wave ends, also
-// after a fault in another one.  A wave that stops waiting says so in the status word (ChainArgs): the run's results are then
+// after a fault in another one.  A wave that stops waiting says so in the status word: the run's results are then
 // not valid.  UNIT_AMD_CHAIN_POLLS sets another number (a test takes one).
 constexpr int kPolls = 1 << 24;
 
@@ -87,13 +87,11 @@ constexpr int kWsAlign = 128, kWsHead = 16;  // kWsHead: the status word of call
 constexpr int kCtlGroups = 0, kCtlTickets = 32, kCtlSlots = kCtlTickets + 32 * kMaxXcd;
 
 struct ChainArgs {
-  const ChainStep *steps;
+  const ChainStep *steps;  // the first layer's; the entry in front of it holds the status word's address (give_up)
   int *ctl;
-  int count, images, per, groups;
+  int polls, images, per, groups;
   int slot_pitch, flags0, flag_pitch;
   FastDiv by_tickets;
-  int *status;  // the caller's, in device or pinned host memory: 1 once a wave has given up waiting, else as it was
-  int polls;
 };
 
 // The layers travel as kernel arguments (at most 4 KiB of them), so that a captured chain keeps the ones it was captured
@@ -115,8 +113,11 @@ struct alignas(16) ChainLds {
   int ticket[2], group;
 };
 
+// The caller's status word, in device or pinned host memory: 1 once a wave has given up waiting, else as it was.  Its address
+// travels as one more step: as a kernel argument it cost registers, and a run 2 us.
 __device__ __forceinline__ void give_up(const ChainArgs &a) {
-  __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  int *const status = reinterpret_cast<int *>(a.steps[-1].out);
+  __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __device__ __forceinline__ int load_l2(const int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -321,7 +322,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kPerCu
           store_result<0>(result_buffer(slots), (u32)q * 4u, v);
         } else {
           while ((v = load_l2(slots + q)) == 0 && --budget > 0) __builtin_amdgcn_s_sleep(1);
-          if (v == 0) give_up(a), v = a.groups + 1;
+          if (v == 0) v = a.groups + 1;
         }
         sh.group = v - 1;
       }
@@ -417,7 +418,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kPerCu
       for (int b = fa + 64; b < fb; b += 64) {
         while (!__all(load_l2(wanted + (u32)min(b + lane, fb - 1)) != 0) && --budget > 0) __builtin_amdgcn_s_sleep(1);
       }
-      if (budget <= 0) give_up(a);
     }
 
     v16i acc[2][2];
@@ -489,6 +489,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kPerCu
     __syncthreads();
     if (tid == 0) store_result<0>(result_buffer(flags), (u32)idx * 4u, 1);
   }
+  if (budget <= 0) give_up(a);  // here and not at the waits: a store there cost every run 2 - 10 us
 }
 
 struct ChainPlan {
@@ -621,7 +622,7 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
   p->flag_pitch = (p->tickets + 31) / 32 * 32;
   p->clear_words = p->flags0 + p->groups * p->flag_pitch;
   p->steps_off = ((size_t)p->clear_words * 4 + 255) / 256 * 256;
-  p->bytes = p->steps_off + (size_t)count * sizeof(ChainStep) + kWsAlign;  // ws itself is at 16 bytes, and its head in front
+  p->bytes = p->steps_off + (size_t)(count + 1) * sizeof(ChainStep) + kWsAlign;  // ws itself is at 16 bytes, and its head in front
   return true;
 }
 
@@ -659,17 +660,21 @@ extern "C" int unit_conv_chain_u8_status(const unit_chain_layer *layers, int32_t
   hipStream_t s = static_cast<hipStream_t>(stream);
   char *base = reinterpret_cast<char *>((reinterpret_cast<uintptr_t>(ws) + kWsHead + kWsAlign - 1) / kWsAlign * kWsAlign);
   ChainStep *steps = reinterpret_cast<ChainStep *>(base + p.steps_off);
-  for (int i = 0; i < count; i += kSetupSteps) {
+  for (int i = 0; i <= count; i += kSetupSteps) {  // the status word's entry, then the layers
     ChainSetup a;
-    const int n = std::min(kSetupSteps, count - i);
-    memcpy(a.s, st + i, n * sizeof(ChainStep));
+    const int n = std::min(kSetupSteps, count + 1 - i), head = i == 0;
+    if (head) {
+      memset(a.s, 0, sizeof(ChainStep));
+      a.s[0].out = reinterpret_cast<char *>(status ? status : static_cast<int32_t *>(ws));
+    }
+    memcpy(a.s + head, st + i - !head, (n - head) * sizeof(ChainStep));
     const int quads = i == 0 ? ceil_div(p.clear_words, 4) : 0;
     hipLaunchKernelGGL(chain_setup, dim3(std::max(1, std::min(256, ceil_div(quads, 256)))), dim3(256), 0, s, a, steps + i, n,
                        reinterpret_cast<v4i *>(base), quads);
   }
-  const ChainArgs a{steps,        reinterpret_cast<int *>(base), count,        layers[0].desc.N,           p.per, p.groups,
-                    p.slot_pitch, p.flags0,                      p.flag_pitch, FastDiv::make(p.tickets),    status ? status : static_cast<int *>(ws),
-                    tuning_override("UNIT_AMD_CHAIN_POLLS") > 0 ? tuning_override("UNIT_AMD_CHAIN_POLLS") : kPolls};
+  const int polls = tuning_override("UNIT_AMD_CHAIN_POLLS");
+  const ChainArgs a{steps + 1, reinterpret_cast<int *>(base), polls > 0 ? polls : kPolls, layers[0].desc.N, p.per, p.groups,
+                    p.slot_pitch, p.flags0, p.flag_pitch, FastDiv::make(p.tickets)};
   hipLaunchKernelGGL(chain_run, dim3(256 * kPerCu), dim3(kThreads), sizeof(ChainLds), s, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(UNIT_E_LAUNCH, "%s: launch: %s", what, hipGetErrorString(e));
