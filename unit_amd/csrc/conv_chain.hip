@@ -2,15 +2,17 @@
 //
 // What bounds a chain of launches: a layer of a residual network at batch 32 is 6.5 - 14 us of which the launch gap, the
 // argument fetch, the decode, the first loads from cold L2s and the last write-back are 4 - 5 us, fifty-two times over
-// (ResNet-50 behind its stem: 489 us; at batch 1, where nothing else is left, 237 us).  Here
+// (ResNet-50 behind its stem: 491 us; at batch 1, where nothing else is left, 219 us).  Here
 //   * the images are dealt to the XCDs in groups (batch / 8 each), and an XCD takes its group through all layers: what a
 //     layer writes, the next one reads from the same L2, with no write-back and no cold cache in between;
 //   * a layer's tile waits for the tiles of its source layer that it reads, not for the layer: a flag per tile, set when
 //     the tile's results have reached the L2 (a message from one workgroup to another through the L2 takes 0.2 us; a
 //     kernel boundary 1.2 - 1.5 us and the caches);
 //   * the weights of a tile, which depend on no other tile, are under way while it waits.
-// Measured against the launches, us: ResNet-50 batch 1 201 / 238, 8 212 / 311, 16 241 / 362, 32 380 / 474; ResNet-18
-// 81 / 94 at 1, 98 / 139 at 16, 119 / 169 at 32.
+// Measured against the launches, us a pass among others, its setup included: ResNet-50 batch 32 on inputs and buffers that
+// change 381 / 491; on two inputs in turn 195 / 219 at batch 1, 212 / 282 at 8, 243 / 331 at 16, 377 / 447 at 32; ResNet-18
+// 84 / 88 at 1, 99 / 126 at 16, 120 / 156 at 32.  At batch 32 the matrix pipes are busy 15 % of the time and a CU takes in 19
+// bytes of operands per clock: what is left is the latency of fifty-two layers.
 //
 // Tiles are handed out by a ticket counter per XCD, in the order of the layers.  A workgroup that holds a ticket runs, and
 // everything its tile waits for has an earlier ticket, so the earliest unfinished tile never waits: the kernel ends
