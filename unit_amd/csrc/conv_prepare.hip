@@ -358,10 +358,13 @@ extern "C" int unit_conv2d_nchw16c_f16f32_prepared(const unit_conv_desc *d, cons
   ConvGeom g;
   if (int rc = check_prepared_conv(what, d, 32, &g, a, prepared, out)) return rc;
   const int ntable = (int)(sizeof(kTunedF16Prepared) / sizeof(kTunedF16Prepared[0])) - 1;
-  // measured choices and pinned ones first: the patch kernel is no variant that a table row could name
-  const bool pinned = tuning_override("UNIT_AMD_CONV_VARIANT") > 0 || tuning_override("UNIT_AMD_CONV_PANEL") > 0 ||
-                      tuning_override("UNIT_AMD_CONV_SPLITK") > 0;
-  if (!pinned && !tuned_row(d, g.npix, kTunedF16Prepared, ntable, true, true) && patch_f16_takes(d, g))
+  // the rule's arithmetic first: most calls need nothing else.  Measured choices and pinned ones stand above it (the patch
+  // kernel is no variant that a table row could name)
+  const auto pinned = [] {
+    return tuning_override("UNIT_AMD_CONV_VARIANT") > 0 || tuning_override("UNIT_AMD_CONV_PANEL") > 0 ||
+           tuning_override("UNIT_AMD_CONV_SPLITK") > 0;
+  };
+  if (patch_f16_takes(d, g) && !pinned() && !tuned_row(d, g.npix, kTunedF16Prepared, ntable, true, true))
     return conv_f16_patch(d, g, a, prepared, out, static_cast<hipStream_t>(stream));
   const ConvPlan p = plan_prepared(d, g, g.ntaps * 32, kTunedF16Prepared, ntable, false, true);
   if (kConvTiles[p.variant].lds) return conv_f16_prepared_lds(p, d, g, a, prepared, out, static_cast<hipStream_t>(stream));
