@@ -30,6 +30,8 @@ SHAPES = [
     (9, 32, 70, 70, 688, 1, 1, "x64_y64_g1_d6n"),    # 7590 tiles, two k-steps
     (12, 32, 80, 60, 1648, 3, 2, "x64_y64_g1_d4n"),  # 5538 tiles, 18 k-steps
     (12, 32, 80, 112, 1648, 3, 2, "x64_y64_g1_d3n"), # 10478 tiles
+    (16, 512, 7, 7, 2048, 1, 1, "x64_y128_g4_d3n_r4"),  # table rows
+    (256, 1024, 14, 14, 512, 1, 2, "x128_y64_g1_d3n"),
 ]
 
 
