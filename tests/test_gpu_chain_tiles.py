@@ -1,0 +1,52 @@
+"""The chain kernel's wave tiles (64 x 64, 64 x 32, 32 x 32 channels x pixels) with every k-group count and tap walk, channels and pixels
+that end inside a tile, a last group of fewer images; bit-exact against the oracle's operators chained the same way."""
+import numpy as np
+import pytest
+
+from test_gpu_chain import _oracle_chain, _t, _to_chain
+from test_gpu_chain_kernel import _build
+from unit_amd import chain, rng
+
+pytestmark = pytest.mark.gpu
+
+# (oc, (kh, kw), stride, padding, source or None for the layer before), images, channels, rows, columns
+CASES = {
+    "large": ([(64, (3, 3), 1, 1, None), (80, (1, 1), 1, 0, None), (272, (1, 1), 1, 0, None), (64, (3, 3), 1, 0, None),
+               (208, (3, 3), 1, 1, 0), (64, (2, 3), 1, (1, 1, 0, 1), 0), (336, (1, 1), 1, 0, 0), (48, (5, 5), 1, 2, 0),
+               (96, (1, 1), 1, 0, 6), (128, (3, 3), 1, 1, 0), (16, (1, 1), 1, 0, None)], 11, 64, 41, 37),
+    "half": ([(128, (3, 3), 1, 1, None), (144, (1, 1), 1, 0, None), (128, (3, 2), 1, 0, 0), (112, (3, 3), 1, 1, 0),
+              (304, (1, 1), 1, 0, 0), (176, (1, 1), 2, 0, 0), (96, (1, 3), 1, (0, 1, 0, 1), 0), (144, (3, 3), 2, 1, 0),
+              (128, (1, 1), 1, 0, 0), (560, (1, 1), 1, 0, 0), (64, (1, 1), 1, 0, 9)], 7, 128, 28, 27),
+}
+
+
+@pytest.mark.parametrize("name", CASES)
+def test_tiles_bit_exact(dev, oracle, name):
+    spec, n, c0, h, w = CASES[name]
+    x, layers, want = _build(oracle, spec, n, c0, h, w)
+    c = chain.ConvChain(_to_chain(layers, dev), x.shape)
+    for o in c.outputs:
+        o.fill_(77)
+    c(_t(x, dev))
+    for i, (got, ref) in enumerate(zip(c.outputs, want)):
+        assert np.array_equal(got.cpu().numpy(), ref), f"layer {i} ({c.variants[i]})"
+    depths = {"large": {"d5", "d6", "d9"}, "half": {"d6", "d9"}}[name]  # k-steps in flight: 64 x 64, 64 x 32, 32 x 32
+    assert {v.split("_")[4] for v in c.variants} == depths, c.variants
+
+
+@pytest.mark.parametrize("hw", [7, 30])
+def test_scales_too_wide_to_double(dev, oracle, hw):
+    """Scales from 2^30 on leave the shift below 33: the 64-bit form of the requantisation, on whole blocks and on quarters."""
+    x = rng.uniform_u8((3, 4, hw, hw, 16), 5)
+    layers = []
+    for i, (oc, k) in enumerate([(64, 1), (64, 3), (32, 1), (256, 3), (512, 1), (64, 1), (64, 3), (64, 1), (64, 1), (64, 1), (64, 1)]):
+        ic = layers[-1][0].shape[0] if layers else 64
+        wt = (rng.uniform_s8((oc, ic, k, k), 30 + i) % 3 - 1).astype(np.int8)
+        layers.append((wt, None, (1 << 30) + 12345 * i, 32 - i % 3, 1, k // 2, i - 1))
+    want = _oracle_chain(oracle, layers, x)
+    c = chain.ConvChain(_to_chain(layers, dev), x.shape)
+    c(_t(x, dev))
+    for i, (got, ref) in enumerate(zip(c.outputs, want)):
+        assert np.array_equal(got.cpu().numpy(), ref), f"layer {i} ({c.variants[i]})"
+    assert all(v.startswith("q8chain_") for v in c.variants), c.variants
+    assert 0.01 < (want[-1] > 0).mean() and len(np.unique(want[-1])) > 16

@@ -10,9 +10,10 @@
 //     kernel boundary 1.2 - 1.5 us and the caches);
 //   * the weights of a tile, which depend on no other tile, are under way while it waits.
 // Measured against the launches, us a pass among others, its setup included: ResNet-50 batch 32 on inputs and buffers that
-// change 381 / 491; on two inputs in turn 195 / 219 at batch 1, 212 / 282 at 8, 243 / 331 at 16, 377 / 447 at 32; ResNet-18
-// 84 / 88 at 1, 99 / 126 at 16, 120 / 156 at 32.  At batch 32 the matrix pipes are busy 15 % of the time and a CU takes in 19
-// bytes of operands per clock: what is left is the latency of fifty-two layers.
+// change 361 / 491; on two inputs in turn 151 / 219 at batch 1, 173 / 282 at 8, 244 / 331 at 16; ResNet-18 65 / 88 at 1, 82 / 126 at
+// 16, 110 / 156 at 32.  At batch 32 the matrix pipes are busy 16 % of the time and a CU takes in 20 bytes of operands per clock:
+// what is left is the latency of fifty-two layers, 3 us each at batch 1 (0.6 - 0.8 decode, 0.3 until the flag is seen, 0.8 - 1.4
+// loads and reduction, 0.5 k-group sum, requantisation and stores, 0.2 their acknowledgement, 0.2 flag).
 //
 // Tiles are handed out by a ticket counter per XCD, in the order of the layers.  A workgroup that holds a ticket runs, and
 // everything its tile waits for has an earlier ticket, so the earliest unfinished tile never waits: the kernel ends
@@ -25,8 +26,9 @@
 // for the ResNet-50 above).  Stores and flags are plain: they stay in the L2 (an sc1 store goes to memory, and a load
 // after it with it).
 //
-// The tile: four waves of 64 channels x 64 pixels each, operands straight into registers as in conv_direct.hpp, either
-// side by side (over channels first, then pixels) or in two or four k-groups that share a tile.
+// The tile: four waves of 64 channels x 64 pixels, 64 x 32 or 32 x 32 each, operands straight into registers as in conv_direct.hpp,
+// either side by side (over channels first, then pixels) or in two or four k-groups that share a tile.  With 64 x 64 alone the
+// layers behind the second stage of a ResNet keep 8 - 26 of an XCD's 64 workgroups busy at an image per XCD, for up to 5 us each.
 #include "conv_direct.hpp"
 #include "conv_prepare.hpp"
 #include "host.hpp"
@@ -40,8 +42,12 @@ int conv_geom(const unit_conv_desc *d, int tapb, ConvGeom *g, const char *what);
 namespace {
 
 constexpr int kWaves = 4, kThreads = 64 * kWaves;
-constexpr int kPerCu = 2;         // workgroups per CU: 235 VGPRs (three of 168 with three k-steps in flight: 392 us at batch 32, 234 at 8)
-constexpr int kDepth = 5;         // k-steps of fragments in flight per wave
+constexpr int kPerCu = 2;                 // workgroups per CU: 246 VGPRs (three of 168 with three k-steps in flight: 392 us at batch 32, 234 at 8)
+// A wave's tile is TX x TY blocks of 32 channels x 32 pixels: 2 x 2, 2 x 1 or 1 x 1.  k-steps of fragments in flight per wave: few
+// blocks are few MFMAs per step, so more steps to cover a load's latency (nine for one block, a period of chain_reduce_3x3; nine for
+// two blocks spilled).  A wave whose share of a 1 x 1 layer is short loads no more than kShort steps.
+template <int TX, int TY> constexpr int kRing = TX * TY == 4 ? 5 : TX == 1 ? 9 : 6;
+template <int TX, int TY> constexpr int kShort = TX * TY == 4 ? 2 : 4;
 constexpr int kMaxXcd = 16, kMaxChain = 256;
 constexpr int kAgent = 16;        // sc1
 // Polls a wave may spend in all before it stops waiting (seconds; a whole chain takes some thousand): every wave ends, also
@@ -69,7 +75,7 @@ struct alignas(128) ChainStep {
   unsigned char shift, win, mode;  // KH * KW; chain_reduce's MODE
   unsigned char flat;              // 1 x 1 at stride 1: output pixels are input pixels
   unsigned char reads, src_shift;  // the source is a layer of the chain, its pixel tiles are 1 << src_shift
-  unsigned char kg_log, wx_log, wy_log, unused;
+  unsigned char kg_log, wx_log, wy_log, tile;  // tile: log2 of a wave's channels and, in the upper half, of its pixels
 };
 static_assert(sizeof(ChainStep) == 128, "ChainStep");
 using StepPtr = const __attribute__((address_space(4))) ChainStep *;
@@ -110,7 +116,7 @@ __global__ __launch_bounds__(256) void chain_setup(const ChainSetup a, ChainStep
 }
 
 struct alignas(16) ChainLds {
-  v4i part[kWaves][3][4][64];  // [wave][block, its own left out][quad][lane]: partial blocks for their owners
+  v4i part[kWaves][16][64];  // [wave][quad of its blocks][lane]: partial sums for their owners
   int addend[kWaves][64];
   int ticket[2], group;
 };
@@ -134,20 +140,18 @@ struct TapWalk {
   u32 by_win, by_kw;
 };
 
-template <int MODE>
-__device__ __forceinline__ void chain_reduce(v16i (&acc)[2][2], __amdgpu_buffer_rsrc_t wbuf, const u32 (&wp)[2], __amdgpu_buffer_rsrc_t data, const u32 lane16,
-                                             int (&pixoff)[2], const u32 (&inside)[2], v4i (&xf)[kDepth][2], int half, int s0, int s1,
+template <class F, int... U>
+__device__ __forceinline__ void for_each_slot(F f, std::integer_sequence<int, U...>) {
+  (f(std::integral_constant<int, U>{}), ...);
+}
+
+// TX x TY blocks, D k-steps in flight; ONCE: the wave's share is at most D steps
+template <int MODE, int TX, int TY, int D, bool ONCE>
+__device__ __forceinline__ void chain_reduce(v16i (&acc)[TX][TY], __amdgpu_buffer_rsrc_t wbuf, const u32 (&wp)[TX], __amdgpu_buffer_rsrc_t data, const u32 lane16,
+                                             int (&pixoff)[TY], const u32 (&inside)[TY], v4i (&xf)[kRing<TX, TY>][TX], int half, int s0, int s1,
                                              int slast, const TapWalk &tw) {
-  constexpr int D = kDepth;
-  v4i yf[D][2];
-  auto for_slots = [&](auto f) __attribute__((always_inline)) {
-    f(std::integral_constant<int, 0>{});
-    f(std::integral_constant<int, 1>{});
-    f(std::integral_constant<int, 2>{});
-    if constexpr (D > 3) f(std::integral_constant<int, 3>{});
-    if constexpr (D > 4) f(std::integral_constant<int, 4>{});
-    if constexpr (D > 5) f(std::integral_constant<int, 5>{});
-  };
+  v4i yf[D][TY];
+  auto for_slots = [&](auto f) __attribute__((always_inline)) { for_each_slot(f, std::make_integer_sequence<int, D>{}); };
   // The state of the running tap; it advances by a k-step per fetch and stops at the wave's last one.  Uniform and
   // without branches, so that the loads keep one order on all paths.
   int sf = s0;
@@ -160,13 +164,14 @@ __device__ __forceinline__ void chain_reduce(v16i (&acc)[2][2], __amdgpu_buffer_
     off = ci * tw.hw16 + kh * tw.w16 + kw * 16;
   } else {
     off = 2 * s0 * tw.hw16;
-    if (half) pixoff[0] += tw.hw16, pixoff[1] += tw.hw16;
+#pragma unroll
+    for (int j = 0; j < TY; ++j) pixoff[j] += half ? tw.hw16 : 0;
   }
   auto fetch_d = [&](auto slot) __attribute__((always_inline)) {
     constexpr int U = decltype(slot)::value;
     if constexpr (MODE == 0) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < TY; ++j)
         yf[U][j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(data, pixoff[j], off, kAgent));
       const bool more = sf < slast;
       sf += more;
@@ -186,7 +191,7 @@ __device__ __forceinline__ void chain_reduce(v16i (&acc)[2][2], __amdgpu_buffer_
       const bool odd = 2 * sf + 1 < tw.ntaps;
       const int o = half ? (odd ? o2 : off) : off, ps = half ? (odd ? p2 : 31) : pos;
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < TY; ++j) {
         u32 v = (u32)(pixoff[j] + o);
         if constexpr (MODE == 2) v |= ~(u32)__builtin_amdgcn_sbfe((int)inside[j], (u32)ps, 1u);
         yf[U][j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(data, (int)v, 0, kAgent));
@@ -199,15 +204,15 @@ __device__ __forceinline__ void chain_reduce(v16i (&acc)[2][2], __amdgpu_buffer_
   };
   auto consume = [&](auto slot) __attribute__((always_inline)) {
     constexpr int U = decltype(slot)::value;
-    v4i y[2];
+    v4i y[TY];
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < TY; ++j)
 #pragma unroll
       for (int d = 0; d < 4; ++d) y[j][d] = yf[U][j][d] ^ (int)0x80808080;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < TX; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = OpI8::mma(xf[U][i], y[j], acc[i][j]);
+      for (int j = 0; j < TY; ++j) acc[i][j] = OpI8::mma(xf[U][i], y[j], acc[i][j]);
   };
   for_slots([&](auto u) __attribute__((always_inline)) { fetch_d(u); });
   __builtin_amdgcn_sched_barrier(0);
@@ -219,16 +224,18 @@ __device__ __forceinline__ void chain_reduce(v16i (&acc)[2][2], __amdgpu_buffer_
       __builtin_amdgcn_sched_barrier(0);
       constexpr int U = decltype(u)::value;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) xf[U][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wbuf, (int)lane16, (int)(wp[i] + sw), 0));
+      for (int i = 0; i < TX; ++i) xf[U][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wbuf, (int)lane16, (int)(wp[i] + sw), 0));
       sw = min(sw + 1024u, swlast);
       fetch_d(u);
       __builtin_amdgcn_sched_barrier(0);
     });
   };
   int s = s0;
-  if (s + D < s1) {
-    round();
-    for (s += D; s + D < s1; s += D) round();
+  if constexpr (!ONCE) {
+    if (s + D < s1) {
+      round();
+      for (s += D; s + D < s1; s += D) round();
+    }
   }
   for_slots([&](auto u) __attribute__((always_inline)) {
     if (s + decltype(u)::value < s1) consume(u);
@@ -241,48 +248,52 @@ __device__ __forceinline__ void chain_reduce(v16i (&acc)[2][2], __amdgpu_buffer_
 // loads of the ring stand between the MFMAs, where a wave's other instructions cost nothing.  us with the walk of MODE 2 /
 // here: ResNet-50 batch 1 213 / 201, 16 252 / 241, 32 389 / 380; ResNet-18 106 / 98 at 16, 133 / 119 at 32.  Loads between the
 // MFMAs of the other modes give under 1 % at 1 x 1 windows and take 3 % at ResNet-18, batch 32.  A ring of six in a period of 18 spilled.
-__device__ __forceinline__ void chain_reduce_3x3(v16i (&acc)[2][2], __amdgpu_buffer_rsrc_t wbuf, const u32 (&wp)[2],
-                                                 __amdgpu_buffer_rsrc_t data, const u32 lane16, const int (&pixoff)[2],
-                                                 const u32 (&inside)[2], v4i (&xf)[kDepth][2], int half, int s0, int s1,
+template <int TX, int TY> constexpr int kRing3 = TX * TY != 1 ? 3 : 9;
+template <int TX, int TY>
+__device__ __forceinline__ void chain_reduce_3x3(v16i (&acc)[TX][TY], __amdgpu_buffer_rsrc_t wbuf, const u32 (&wp)[TX],
+                                                 __amdgpu_buffer_rsrc_t data, const u32 lane16, const int (&pixoff)[TY],
+                                                 const u32 (&inside)[TY], v4i (&xf)[kRing<TX, TY>][TX], int half, int s0, int s1,
                                                  int hw16, int w16) {
-  constexpr int D = 3, P = 9;
-  static_assert(P % D == 0 && D <= kDepth, "the ring's slots repeat with the period");
+  constexpr int D = kRing3<TX, TY>, P = 9;
+  static_assert(P % D == 0 && D <= kRing<TX, TY>, "the ring's slots repeat with the period");
   // offset of tap 2 s + half of a period; all ones, out of range, outside the image
-  u32 at[9][2];
+  u32 at[9][TY];
 #pragma unroll
   for (int s = 0; s < 9; ++s) {
     const int e = 2 * s, o = 2 * s + 1;
     const int oe = (e / 9) * hw16 + (e % 9 / 3) * w16 + (e % 9 % 3) * 16, oo = (o / 9) * hw16 + (o % 9 / 3) * w16 + (o % 9 % 3) * 16;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < TY; ++j)
       at[s][j] = (u32)(pixoff[j] + (half ? oo : oe)) | ~(u32)__builtin_amdgcn_sbfe((int)inside[j], (u32)(half ? o % 9 : e % 9), 1u);
   }
-  v4i yf[D][2];
+  v4i yf[D][TY];
   int soff = 2 * (s0 / 9) * hw16;
   u32 sw = (u32)s0 * 1024u;
   auto load_d = [&](int s, int j) __attribute__((always_inline)) {
     yf[s % D][j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(data, (int)at[s % 9][j], soff + s / 9 * (2 * hw16), kAgent));
   };
 #pragma unroll
-  for (int s = 0; s < D; ++s) load_d(s, 0), load_d(s, 1);
+  for (int s = 0; s < D; ++s)
+#pragma unroll
+    for (int j = 0; j < TY; ++j) load_d(s, j);
   __builtin_amdgcn_sched_barrier(0);
   auto period = [&](auto last) __attribute__((always_inline)) {
 #pragma unroll
     for (int s = 0; s < P; ++s) {
       const bool fetch = !decltype(last)::value || s + D < P;
-      v4i y[2];
+      v4i y[TY];
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < TY; ++j)
 #pragma unroll
         for (int d = 0; d < 4; ++d) y[j][d] = yf[s % D][j][d] ^ (int)0x80808080;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i < TX; ++i) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < TY; ++j) {
           acc[i][j] = OpI8::mma(xf[s % D][i], y[j], acc[i][j]);
           __builtin_amdgcn_sched_barrier(0);
           if (fetch && i == 0) load_d(s + D, j);
-          if (fetch && j == 1)
+          if (fetch && j == TY - 1)
             xf[s % D][i] = __builtin_bit_cast(
                 v4i, __builtin_amdgcn_raw_buffer_load_b128(wbuf, (int)lane16, (int)(wp[i] + sw + (u32)(s + D) * 1024u), 0));
           __builtin_amdgcn_sched_barrier(0);
@@ -296,6 +307,23 @@ __device__ __forceinline__ void chain_reduce_3x3(v16i (&acc)[2][2], __amdgpu_buf
     sw += P * 1024u;
   }
   period(std::true_type{});
+}
+
+// requant_row's arithmetic for four channels, the addend already in them
+__device__ __forceinline__ int requant_quad(const v4i &v, int scale, int shift) {
+  if (shift >= 33) {
+    const int rhi = 1 << (shift - 33), sh = shift - 32;
+    const u32 lo = (unsigned short)__builtin_amdgcn_ashr_pk_u8_i32(__mulhi(v[0], scale) + rhi, __mulhi(v[1], scale) + rhi, sh);
+    const u32 hi = (unsigned short)__builtin_amdgcn_ashr_pk_u8_i32(__mulhi(v[2], scale) + rhi, __mulhi(v[3], scale) + rhi, sh);
+    return (int)__builtin_amdgcn_perm(hi, lo, 0x05040100u);
+  }
+  u32 packed = 0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const long long t = ((long long)v[e] * scale + (1ll << (shift - 1))) >> shift;
+    packed |= (u32)(t < 0 ? 0 : (t > 255 ? 255 : t)) << (8 * e);
+  }
+  return (int)packed;
 }
 
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kPerCu, kPerCu))) void chain_run(const ChainArgs a) {
@@ -340,14 +368,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kPerCu
     const int local = idx - L.first;
     const int pt = quot(local, L.by_nct), ct = local - pt * nct;
     const int image0 = group * a.per, npix = min(a.per, a.images - image0) * ohw;
-    const int m0 = pt << (6 + L.wy_log), me = min(m0 + (64 << L.wy_log), npix) - 1;
+    const int tx = L.tile & 15, ty = L.tile >> 4, m0 = pt << (ty + L.wy_log), me = min(m0 + (1 << (ty + L.wy_log)), npix) - 1;
     if (m0 > me) {  // the last group may hold fewer images
       if (tid == 0) sh.ticket[turn] = __hip_atomic_fetch_add(tickets, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __syncthreads();
       continue;
     }
     const int set = wave >> kl, kidx = wave & ((1 << kl) - 1);
-    const int x0 = ((ct << wl) + (set & ((1 << wl) - 1))) * 64, y0 = m0 + (set >> wl) * 64;
+    const int x0 = ((ct << wl) + (set & ((1 << wl) - 1))) << tx, y0 = m0 + ((set >> wl) << ty);
     const bool idle = x0 >= K || y0 >= npix;
     const int s0 = idle ? 0 : (nsteps * kidx) >> kl, s1 = idle ? 0 : (nsteps * (kidx + 1)) >> kl;
     const int slast = max(s1 - 1, s0);
@@ -369,124 +397,177 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kPerCu
     const int flag = load_l2(wanted + (u32)min(fa + lane, max(fb - 1, 0)));
     __builtin_amdgcn_sched_barrier(0);
 
-    // weights: the ring's fragments depend on the tile alone
-    const u32 lane16 = (u32)lane * 16u;
-    const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc((void *)L.w, 0, -1, 0x00020000);
-    const int kblocks = (K + 31) >> 5;
-    u32 wp[2];  // byte offsets of the two 32-channel blocks; blocks past the last one re-read it
-#pragma unroll
-    for (int i = 0; i < 2; ++i) wp[i] = (u32)(min((x0 >> 5) + i, kblocks - 1) * nsteps) * 1024u;
-    v4i xf[kDepth][2];
-#pragma unroll
-    for (int u = 0; u < kDepth; ++u)
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        xf[u][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wbuf, (int)lane16, (int)(wp[i] + (u32)min(s0 + u, slast) * 1024u), 0));
-    const u32 cc = (u32)min(x0 + lane, K - 1) * 4u;
-    const int add0 = __builtin_amdgcn_raw_buffer_load_b32(wbuf, (int)cc, kblocks * nsteps * 1024, 0);
-    const int add1 = L.bias ? ((Global<int>)L.bias)[cc >> 2] : 0;
-    __builtin_amdgcn_sched_barrier(0);
-
-    const __amdgpu_buffer_rsrc_t data = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)(L.data + (size_t)image0 * (size_t)(u32)L.img_bytes), 0, min(a.per, a.images - image0) * L.img_bytes, 0x00020000);
-    int pixoff[2];
-    u32 inside[2], dst[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int m = y0 + j * 32 + l32;
-      const int mm = m < npix ? m : 0;
-      const int n = quot(mm, L.by_ohw), pix = mm - n * ohw;
-      dst[j] = ((u32)(n * (K >> 4) * ohw) + (u32)pix) * 16u;
-      inside[j] = 0;
-      if (L.flat) {
-        pixoff[j] = n * L.img_bytes + pix * 16;
-      } else {
-        const int oh = quot(pix, L.by_ow), ow = pix - __mul24(oh, (int)L.OW);
-        const int ih0 = __mul24(oh, (int)L.sh) - L.pt, iw0 = __mul24(ow, (int)L.sw) - L.pl;
-        pixoff[j] = n * L.img_bytes + (__mul24(ih0, W) + iw0) * 16;
-        if (L.mode >= 2) {
-          const int KH = L.KH, KW = L.KW;
-          const int ka = min(max(-iw0, 0), KW), kb = min(max(W - iw0, ka), KW);
-          const int ra = min(max(-ih0, 0), KH), rb = min(max(H - ih0, ra), KH);
-          const u32 rows = L.row_ones & ((1u << __mul24(rb, KW)) - (1u << __mul24(ra, KW)));
-          inside[j] = m < npix ? ((1u << kb) - (1u << ka)) * rows : 0u;
-        }
-      }
-    }
-    if (L.reads) {
-      if (!__all(flag != 0)) {
-        while (!__all(load_l2(wanted + (u32)min(fa + lane, fb - 1)) != 0) && --budget > 0) __builtin_amdgcn_s_sleep(1);
-      }
-      for (int b = fa + 64; b < fb; b += 64) {
-        while (!__all(load_l2(wanted + (u32)min(b + lane, fb - 1)) != 0) && --budget > 0) __builtin_amdgcn_s_sleep(1);
-      }
-    }
-
-    v16i acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
-    const TapWalk tw{L.ntaps, L.KW, L.win, (W - L.KW) * 16, (H - L.KH) * W * 16, H * W * 16, W * 16, L.by_win, L.by_kw};
-    if (L.mode == 3) {
-      if (s0 < s1) chain_reduce_3x3(acc, wbuf, wp, data, lane16, pixoff, inside, xf, half, s0, s1, H * W * 16, W * 16);
-    } else if (L.mode == 0)
-      chain_reduce<0>(acc, wbuf, wp, data, lane16, pixoff, inside, xf, half, s0, s1, slast, tw);
-    else if (L.mode == 1)
-      chain_reduce<1>(acc, wbuf, wp, data, lane16, pixoff, inside, xf, half, s0, s1, slast, tw);
-    else
-      chain_reduce<2>(acc, wbuf, wp, data, lane16, pixoff, inside, xf, half, s0, s1, slast, tw);
     int next = 0;
-    if (tid == 0) next = __hip_atomic_fetch_add(tickets, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    auto tile = [&](auto tx_, auto ty_) __attribute__((always_inline)) {
+      constexpr int TX = decltype(tx_)::value, TY = decltype(ty_)::value;
+      // weights: the ring's fragments depend on the tile alone
+      const u32 lane16 = (u32)lane * 16u;
+      const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc((void *)L.w, 0, -1, 0x00020000);
+      const int kblocks = (K + 31) >> 5;
+      u32 wp[TX];  // byte offsets of the 32-channel blocks; blocks past the last one re-read it
+#pragma unroll
+      for (int i = 0; i < TX; ++i) wp[i] = (u32)(min((x0 >> 5) + i, kblocks - 1) * nsteps) * 1024u;
+      v4i xf[kRing<TX, TY>][TX];
+      auto load_w = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < TX; ++i)
+          xf[u][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wbuf, (int)lane16, (int)(wp[i] + (u32)min(s0 + u, slast) * 1024u), 0));
+      };
+#pragma unroll
+      for (int u = 0; u < kShort<TX, TY>; ++u) load_w(u);
+      const bool is_short = s1 - s0 <= kShort<TX, TY> && L.mode == 0;
+      if (!is_short) {
+#pragma unroll
+        for (int u = kShort<TX, TY>; u < kRing<TX, TY>; ++u) load_w(u);
+      }
+      const u32 cc = (u32)min(x0 + lane, K - 1) * 4u;
+      const int add0 = __builtin_amdgcn_raw_buffer_load_b32(wbuf, (int)cc, kblocks * nsteps * 1024, 0);
+      const int add1 = L.bias ? ((Global<int>)L.bias)[cc >> 2] : 0;
+      __builtin_amdgcn_sched_barrier(0);
 
-    sh.addend[wave][lane] = add0 + add1;
-    const __amdgpu_buffer_rsrc_t obuf = result_buffer(L.out + (size_t)image0 * (size_t)(u32)(K * ohw));
-    auto store = [&](int i, int j, const v16i &v) __attribute__((always_inline)) {
-      const v4i row = requant_row(v, &sh.addend[wave][i * 32], L.scale, L.shift, half);
-      const int c = x0 + i * 32 + half * 16;
-      if (c < K && y0 + j * 32 + l32 < npix) store_result<0>(obuf, dst[j] + (u32)((c >> 4) * ohw) * 16u, row);
-    };
-    // KG k-groups: each parks the blocks that others own and adds up its own
-    auto finish = [&](auto kg_) __attribute__((always_inline)) {
-      constexpr int KG = decltype(kg_)::value, OWN = 4 / KG;
+      const __amdgpu_buffer_rsrc_t data = __builtin_amdgcn_make_buffer_rsrc(
+          (void *)(L.data + (size_t)image0 * (size_t)(u32)L.img_bytes), 0, min(a.per, a.images - image0) * L.img_bytes, 0x00020000);
+      int pixoff[TY];
+      u32 inside[TY], dst[TY];
 #pragma unroll
-      for (int b = 0; b < 4; ++b)
-        if (b / OWN != kidx) {
-#pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4)
-            sh.part[wave][KG == 2 ? b & 1 : b - (b > kidx)][q4][lane] =
-                v4i{acc[b >> 1][b & 1][4 * q4], acc[b >> 1][b & 1][4 * q4 + 1], acc[b >> 1][b & 1][4 * q4 + 2],
-                    acc[b >> 1][b & 1][4 * q4 + 3]};
+      for (int j = 0; j < TY; ++j) {
+        const int m = y0 + j * 32 + l32;
+        const int mm = m < npix ? m : 0;
+        const int n = quot(mm, L.by_ohw), pix = mm - n * ohw;
+        dst[j] = ((u32)(n * (K >> 4) * ohw) + (u32)pix) * 16u;
+        inside[j] = 0;
+        if (L.flat) {
+          pixoff[j] = n * L.img_bytes + pix * 16;
+        } else {
+          const int oh = quot(pix, L.by_ow), ow = pix - __mul24(oh, (int)L.OW);
+          const int ih0 = __mul24(oh, (int)L.sh) - L.pt, iw0 = __mul24(ow, (int)L.sw) - L.pl;
+          pixoff[j] = n * L.img_bytes + (__mul24(ih0, W) + iw0) * 16;
+          if (L.mode >= 2) {
+            const int KH = L.KH, KW = L.KW;
+            const int ka = min(max(-iw0, 0), KW), kb = min(max(W - iw0, ka), KW);
+            const int ra = min(max(-ih0, 0), KH), rb = min(max(H - ih0, ra), KH);
+            const u32 rows = L.row_ones & ((1u << __mul24(rb, KW)) - (1u << __mul24(ra, KW)));
+            inside[j] = m < npix ? ((1u << kb) - (1u << ka)) * rows : 0u;
+          }
         }
-      __syncthreads();
+      }
+      if (L.reads) {
+        if (!__all(flag != 0)) {
+#ifdef PREF
+          if (s1 - s0 > kRing<TX, TY>) {
+            int got = 0;
+            for (u32 o = (u32)(s0 + kRing<TX, TY>) * 1024u; o < (u32)s1 * 1024u; o += 8192u) {
 #pragma unroll
-      for (int b = 0; b < 4; ++b)
-        if (b / OWN == kidx) {
-          v16i v = acc[b >> 1][b & 1];
+              for (int i = 0; i < TX; ++i) got ^= __builtin_amdgcn_raw_buffer_load_b32(wbuf, (int)min(lane16 * 8u + o, (u32)slast * 1024u), (int)wp[i], 0);
+            }
+            asm volatile("" ::"v"(got));
+          }
+#endif
+          while (!__all(load_l2(wanted + (u32)min(fa + lane, fb - 1)) != 0) && --budget > 0) __builtin_amdgcn_s_sleep(1);
+        }
+        for (int b = fa + 64; b < fb; b += 64) {
+          while (!__all(load_l2(wanted + (u32)min(b + lane, fb - 1)) != 0) && --budget > 0) __builtin_amdgcn_s_sleep(1);
+        }
+      }
+
+      v16i acc[TX][TY];
 #pragma unroll
-          for (int o = 1; o < KG; ++o) {
-            const int other = (kidx + o) & (KG - 1);
+      for (int i = 0; i < TX; ++i)
 #pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4) {
-              const v4i x = sh.part[set * KG + other][KG == 2 ? b & 1 : b - (b > other)][q4][lane];
+        for (int j = 0; j < TY; ++j)
 #pragma unroll
-              for (int e = 0; e < 4; ++e) v[4 * q4 + e] += x[e];
+          for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+      const TapWalk tw{L.ntaps, L.KW, L.win, (W - L.KW) * 16, (H - L.KH) * W * 16, H * W * 16, W * 16, L.by_win, L.by_kw};
+      if (L.mode == 3) {
+        if (s0 < s1) chain_reduce_3x3<TX, TY>(acc, wbuf, wp, data, lane16, pixoff, inside, xf, half, s0, s1, H * W * 16, W * 16);
+      } else if (is_short)
+        chain_reduce<0, TX, TY, kShort<TX, TY>, true>(acc, wbuf, wp, data, lane16, pixoff, inside, xf, half, s0, s1, slast, tw);
+      else if (L.mode == 0)
+        chain_reduce<0, TX, TY, kRing<TX, TY>, false>(acc, wbuf, wp, data, lane16, pixoff, inside, xf, half, s0, s1, slast, tw);
+      else if (L.mode == 1)
+        chain_reduce<1, TX, TY, kRing<TX, TY>, false>(acc, wbuf, wp, data, lane16, pixoff, inside, xf, half, s0, s1, slast, tw);
+      else
+        chain_reduce<2, TX, TY, kRing<TX, TY>, false>(acc, wbuf, wp, data, lane16, pixoff, inside, xf, half, s0, s1, slast, tw);
+      // Taken no earlier: a workgroup that still waits would tie a later tile to itself (a tile earlier: 151 -> 161 us at batch 1)
+      sh.addend[wave][lane] = add0 + add1;
+      __builtin_amdgcn_sched_barrier(0);
+      if (tid == 0) {
+        // divergent as far as the compiler knows: of a uniform address it makes a wave-wide sum, and waits for it on the spot, 0.3 us
+        // a tile (batch 1 164 / 154 us, batch 32 376 / 366)
+        auto *at = (__attribute__((address_space(1))) int *)tickets;
+        asm("" : "+v"(at));
+        next = __hip_atomic_fetch_add(at, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      const __amdgpu_buffer_rsrc_t obuf = result_buffer(L.out + (size_t)image0 * (size_t)(u32)(K * ohw));
+      auto store = [&](int i, int j, const v16i &v) __attribute__((always_inline)) {
+        const v4i row = requant_row(v, &sh.addend[wave][i * 32], L.scale, L.shift, half);
+        const int c = x0 + i * 32 + half * 16;
+        if (c < K && y0 + j * 32 + l32 < npix) store_result<0>(obuf, dst[j] + (u32)((c >> 4) * ohw) * 16u, row);
+      };
+      // KG k-groups: each parks the quads (four channels of a lane's pixel) that others own and adds up its own
+      auto finish = [&](auto kg_) __attribute__((always_inline)) {
+        constexpr int KG = decltype(kg_)::value, QUADS = 4 * TX * TY, OWN = QUADS / KG;
+        auto quad = [&](int q) __attribute__((always_inline)) {
+          const v16i &v = acc[q / 4 / TY][q / 4 % TY];
+          return v4i{v[4 * (q & 3)], v[4 * (q & 3) + 1], v[4 * (q & 3) + 2], v[4 * (q & 3) + 3]};
+        };
+        auto sum = [&](int q) __attribute__((always_inline)) {
+          v4i v = quad(q);
+#pragma unroll
+          for (int o = 1; o < KG; ++o) v += sh.part[set * KG + ((kidx + o) & (KG - 1))][q][lane];
+          return v;
+        };
+#pragma unroll
+        for (int o = 0; o < KG; ++o)
+          if (o != kidx) {
+#pragma unroll
+            for (int q = o * OWN; q < (o + 1) * OWN; ++q) sh.part[wave][q][lane] = quad(q);
+          }
+        __syncthreads();
+#pragma unroll
+        for (int o = 0; o < KG; ++o)
+          if (o == kidx) {
+            if constexpr (OWN % 4 == 0) {
+#pragma unroll
+              for (int b = o * OWN / 4; b < (o + 1) * OWN / 4; ++b) {
+                v16i v;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                  const v4i x = sum(4 * b + q);
+#pragma unroll
+                  for (int e = 0; e < 4; ++e) v[4 * q + e] = x[e];
+                }
+                store(b / TY, b % TY, v);
+              }
+            } else {
+#pragma unroll
+              for (int q = o * OWN; q < (o + 1) * OWN; ++q) {
+                const int i = q / 4 / TY, j = q / 4 % TY, c = x0 + i * 32 + (q >> 1 & 1) * 16;
+                const v4i v = sum(q) + *reinterpret_cast<const v4i *>(&sh.addend[wave][i * 32 + 8 * (q & 3) + 4 * half]);
+                if (c < K && y0 + j * 32 + l32 < npix)
+                  store_result<0>(obuf, dst[j] + (u32)((c >> 4) * ohw) * 16u + (u32)((q & 1) * 8 + half * 4), requant_quad(v, L.scale, L.shift));
+              }
             }
           }
-          store(b >> 1, b & 1, v);
-        }
-    };
-    if (kl == 2) {
-      finish(std::integral_constant<int, 4>{});
-    } else if (kl == 1) {
-      finish(std::integral_constant<int, 2>{});
-    } else {
+      };
+      if (kl == 2) {
+        finish(std::integral_constant<int, 4>{});
+      } else if (kl == 1) {
+        finish(std::integral_constant<int, 2>{});
+      } else {
 #pragma unroll
-      for (int b = 0; b < 4; ++b) store(b >> 1, b & 1, acc[b >> 1][b & 1]);
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // results are in this XCD's L2
+        for (int b = 0; b < TX * TY; ++b) store(b / TY, b % TY, acc[b / TY][b % TY]);
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // results are in this XCD's L2
+    };
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
+    if (ty == 6)
+      tile(Two{}, Two{});
+    else if (tx == 6)
+      tile(Two{}, One{});
+    else
+      tile(One{}, One{});
     if (tid == 0) sh.ticket[turn] = next;
     __syncthreads();
     if (tid == 0) store_result<0>(result_buffer(flags), (u32)idx * 4u, 1);
@@ -554,41 +635,52 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
     s.flat = !masked && d.KH == 1 && d.KW == 1 && d.sh == 1 && d.sw == 1;
     const long npix = (long)per * s.ohw;
     if (npix * s.ohw > 0x7fffffffl) return false;
-    // k-groups: a tile costs 2.6 us beside its reduction (decode, first loads, requantisation, stores, flag), 0.4 more with
-    // k-groups, and 0.25 us per k-step of a wave; an XCD runs 64 at a time
-    const long wt = (long)ceil_div(d.K, 64) * ((npix + 63) / 64);
-    int kg = 1;
+    // Tile and k-groups: a tile of 64 x 64 costs 2.6 us beside its reduction (decode, first loads, requantisation, stores, flag), 0.4
+    // more with k-groups, and 0.25 us per k-step of a wave; an XCD runs 64 at a time.  Smaller tiles move more operand bytes per
+    // result, so they only pay where the large ones leave workgroups idle: the rounds say where.  us with 64 x 64 alone / with 32 x 32 /
+    // and 64 x 32: ResNet-50 batch 1 203 / 164 / 151, 8 232 / 187 / 173, 16 275 / 258 / 244, 32 377 / 376 / 361; ResNet-18 1 83 / 67 / 65, 32
+    // 118 / 117 / 110.  Steps of 0.12 - 0.18 and fixed parts 0.2 lower or higher: within 2 %; 0.1 for 32 x 32 costs 4 % at 16 images.
+    const auto split = [&](int cx, int cy, double fixed, double shared, double step, double &best) {
+      const long wt = (long)ceil_div(d.K, cx) * ((npix + cy - 1) / cy);
+      int kg = 0;
+      for (int k = 1; k <= 4 && k <= s.nsteps; k *= 2) {
+        const double rounds = std::max(1.0, (double)wt * k / 4 / 64);
+        const double t = rounds * (fixed + (k > 1 ? shared : 0.0) + step * ceil_div(s.nsteps, k));
+        if (t < best) best = t, kg = k;
+      }
+      return kg;
+    };
     double best = 1e30;
-    for (int k = 1; k <= 4 && k <= s.nsteps; k *= 2) {
-      const double rounds = std::max(1.0, (double)wt * k / 4 / 64);
-      const double t = rounds * (2.6 + (k > 1 ? 0.4 : 0.0) + 0.25 * ceil_div(s.nsteps, k));
-      if (t < best) best = t, kg = k;
-    }
+    int kg = split(64, 64, 2.6, 0.4, 0.25, best), sx = 64, sy = 64;
+    const int kg64 = kg;
+    if (const int k = split(64, 32, 2.2, 0.2, 0.2, best)) kg = k, sy = 32;
+    if (const int k = split(32, 32, 2.0, 0.2, 0.15, best)) kg = k, sx = sy = 32;
     const int sets = 4 / kg;
     int wx = 1;
-    while (wx < sets && d.K >= 128 * wx) wx *= 2;
+    while (wx < sets && d.K >= 2 * sx * wx) wx *= 2;
     if (d.KH == 3 && d.KW == 3 && s.ntaps % (18 * kg) == 0) s.mode = 3;
     const int wy = sets / wx;
     s.kg_log = (unsigned char)(kg >> 1), s.wx_log = (unsigned char)(wx >> 1), s.wy_log = (unsigned char)(wy >> 1);
-    s.nct = ceil_div(d.K, 64 * wx);
+    s.tile = (unsigned char)((sx == 64 ? 6 : 5) | (sy == 64 ? 6 : 5) << 4);
+    s.nct = ceil_div(d.K, sx * wx);
     s.by_nct = small_div(s.nct);
-    const long npt = (npix + 64 * wy - 1) / (64 * wy);
+    const long npt = (npix + sy * wy - 1) / (sy * wy);
     if (npt * s.nct * s.nct > 0x7fffffffl) return false;
     const double gmac = 1e-9 * s.ohw * d.K * s.ntaps * 16, mb = 1e-6 * ((double)g.img_bytes + (double)s.ohw * d.K);  // of an image
-    const double rounds = npt * s.nct / 64.0, ksteps = ceil_div(s.nsteps, kg);
-    here += 1.45 + (kg > 1 ? 0.15 : 0.0) + 0.8 * std::max(1.0, rounds) +
+    const double rounds = (double)ceil_div(d.K, 64) * ((npix + 63) / 64) * kg64 / 256, ksteps = ceil_div(s.nsteps, kg64);
+    here += 1.45 + (kg64 > 1 ? 0.15 : 0.0) + 0.8 * std::max(1.0, rounds) +
             (s.mode == 1 || s.mode == 2 ? 0.3 : 0.21) * ksteps * std::max(0.5, rounds) + 1.28 * mb * per;
     launches += 3.6 + 1.15 * gmac * N + 0.176 * mb * N + 0.019 * std::min(s.nsteps, 80);
     s.first = (int)first;
     first += npt * s.nct;
     s.next = (int)first;
     if (first * (p->groups + 2) + 4096 > 0x7fffffffl) return false;
-    s.reads = 0, s.src_first = 0, s.src_nct = 0, s.src_shift = 0, s.unused = 0;
+    s.reads = 0, s.src_first = 0, s.src_nct = 0, s.src_shift = 0;
     for (int j = i - 1; j >= 0; --j)
       if (layers[j].out == s.data) {
         if (layers[j].desc.K != d.C || st[j].OW != d.W || st[j].ohw != d.H * d.W) return false;
         s.reads = 1;
-        s.src_first = st[j].first, s.src_nct = st[j].nct, s.src_shift = (unsigned char)(6 + st[j].wy_log);
+        s.src_first = st[j].first, s.src_nct = st[j].nct, s.src_shift = (unsigned char)((st[j].tile >> 4) + st[j].wy_log);
         break;
       }
   }
@@ -682,7 +774,8 @@ extern "C" int unit_conv_chain_u8_status(const unit_chain_layer *layers, int32_t
   if (e != hipSuccess) return fail(UNIT_E_LAUNCH, "%s: launch: %s", what, hipGetErrorString(e));
   for (int i = 0; i < count; ++i)
     if (layers[i].variant)
-      snprintf(layers[i].variant, 96, "q8chain_x%d_y%d_g%d_d%d", 64 << st[i].wx_log, 64 << st[i].wy_log, 1 << st[i].kg_log, kDepth);
-  set_variant("q8chain_l%d_n%d_d%d", count, p.per, kDepth);
+      snprintf(layers[i].variant, 96, "q8chain_x%d_y%d_g%d_d%d", 1 << ((st[i].tile & 15) + st[i].wx_log),
+               1 << ((st[i].tile >> 4) + st[i].wy_log), 1 << st[i].kg_log, st[i].tile >> 4 == 6 ? kRing<2, 2> : (st[i].tile & 15) == 6 ? kRing<2, 1> : kRing<1, 1>);
+  set_variant("q8chain_l%d_n%d_d%d", count, p.per, kRing<2, 2>);
   return UNIT_OK;
 }
