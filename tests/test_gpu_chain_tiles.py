@@ -50,3 +50,20 @@ def test_scales_too_wide_to_double(dev, oracle, hw):
         assert np.array_equal(got.cpu().numpy(), ref), f"layer {i} ({c.variants[i]})"
     assert all(v.startswith("q8chain_") for v in c.variants), c.variants
     assert 0.01 < (want[-1] > 0).mean() and len(np.unique(want[-1])) > 16
+
+
+# 3 x 3 windows over a patch of pixels in LDS: rows of a patch that end on a load of 64 pixels or one past it (32 + 2 W + 2 and
+# 64 + 2 W + 2 pixels), images of a row or a column, tiles over many images, the largest patch that fits and the first that does not
+@pytest.mark.parametrize("n,c,h,w", [(1, 128, 14, 14), (2, 128, 9, 15), (9, 128, 1, 5), (3, 128, 6, 1), (33, 128, 7, 7), (17, 64, 31, 30), (24, 128, 30, 30),
+                                     (24, 128, 29, 31), (1, 128, 20, 47), (5, 512, 7, 7), (8, 512, 5, 20), (16, 512, 5, 31), (3, 96, 17, 12)])
+def test_patches_bit_exact(dev, oracle, n, c, h, w):
+    spec = [(c, (3, 3), 1, 1, None)] * (3 if c >= 512 else 10) + [(32, (1, 1), 1, 0, None)] * (8 if c >= 512 else 1)
+    x, layers, want = _build(oracle, spec, n, c, h, w)
+    ch = chain.ConvChain(_to_chain(layers, dev), x.shape)
+    for _ in range(2):
+        for o in ch.outputs:
+            o.fill_(77)
+        ch(_t(x, dev))
+        for i, (got, ref) in enumerate(zip(ch.outputs, want)):
+            assert np.array_equal(got.cpu().numpy(), ref), f"layer {i} ({ch.variants[i]})"
+    assert all(v.startswith("q8chain_") for v in ch.variants), ch.variants

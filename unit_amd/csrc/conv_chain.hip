@@ -10,8 +10,8 @@
 //     kernel boundary 1.2 - 1.5 us and the caches);
 //   * the weights of a tile, which depend on no other tile, are under way while it waits.
 // Measured against the launches, us a pass among others, its setup included: ResNet-50 batch 32 on inputs and buffers that
-// change 361 / 491; on two inputs in turn 151 / 219 at batch 1, 173 / 282 at 8, 244 / 331 at 16; ResNet-18 65 / 88 at 1, 82 / 126 at
-// 16, 110 / 156 at 32.  At batch 32 the matrix pipes are busy 16 % of the time and a CU takes in 20 bytes of operands per clock:
+// change 350 / 491; on two inputs in turn 151 / 219 at batch 1, 171 / 282 at 8, 237 / 331 at 16; ResNet-18 62 / 88 at 1, 79 / 126 at
+// 16, 106 / 156 at 32.  At batch 32 the matrix pipes are busy 16 % of the time and a CU takes in 20 bytes of operands per clock:
 // what is left is the latency of fifty-two layers, 3 us each at batch 1 (0.6 - 0.8 decode, 0.3 until the flag is seen, 0.8 - 1.4
 // loads and reduction, 0.5 k-group sum, requantisation and stores, 0.2 their acknowledgement, 0.2 flag).
 //
@@ -47,6 +47,7 @@ constexpr int kPerCu = 2;                 // workgroups per CU: 246 VGPRs (three
 // blocks are few MFMAs per step, so more steps to cover a load's latency (nine for one block, a period of chain_reduce_3x3; nine for
 // two blocks spilled).  A wave whose share of a 1 x 1 layer is short loads no more than kShort steps.
 template <int TX, int TY> constexpr int kRing = TX * TY == 4 ? 5 : TX == 1 ? 9 : 6;
+template <int TX, int TY> constexpr int kMaxRing = TX * TY == 4 ? 5 : 9;  // with chain_reduce_patch's, which needs no pixels in registers
 template <int TX, int TY> constexpr int kShort = TX * TY == 4 ? 2 : 4;
 constexpr int kMaxXcd = 16, kMaxChain = 256;
 constexpr int kAgent = 16;        // sc1
@@ -72,7 +73,7 @@ struct alignas(128) ChainStep {
   u32 row_ones;                              // ConvGeom
   unsigned short H, W, OW;
   unsigned char pt, pl, KH, KW, sh, sw;
-  unsigned char shift, win, mode;  // KH * KW; chain_reduce's MODE
+  unsigned char shift, win, mode;  // KH * KW; MODE of the reduction
   unsigned char flat;              // 1 x 1 at stride 1: output pixels are input pixels
   unsigned char reads, src_shift;  // the source is a layer of the chain, its pixel tiles are 1 << src_shift
   unsigned char kg_log, wx_log, wy_log, tile;  // tile: log2 of a wave's channels and, in the upper half, of its pixels
@@ -116,7 +117,7 @@ __global__ __launch_bounds__(256) void chain_setup(const ChainSetup a, ChainStep
 }
 
 struct alignas(16) ChainLds {
-  v4i part[kWaves][16][64];  // [wave][quad of its blocks][lane]: partial sums for their owners
+  v4i part[kWaves][16][64];  // [wave][quad of its blocks][lane]: partial sums for their owners; before them, a wave's pixels
   int addend[kWaves][64];
   int ticket[2], group;
 };
@@ -148,7 +149,7 @@ __device__ __forceinline__ void for_each_slot(F f, std::integer_sequence<int, U.
 // TX x TY blocks, D k-steps in flight; ONCE: the wave's share is at most D steps
 template <int MODE, int TX, int TY, int D, bool ONCE>
 __device__ __forceinline__ void chain_reduce(v16i (&acc)[TX][TY], __amdgpu_buffer_rsrc_t wbuf, const u32 (&wp)[TX], __amdgpu_buffer_rsrc_t data, const u32 lane16,
-                                             int (&pixoff)[TY], const u32 (&inside)[TY], v4i (&xf)[kRing<TX, TY>][TX], int half, int s0, int s1,
+                                             int (&pixoff)[TY], const u32 (&inside)[TY], v4i (&xf)[kMaxRing<TX, TY>][TX], int half, int s0, int s1,
                                              int slast, const TapWalk &tw) {
   v4i yf[D][TY];
   auto for_slots = [&](auto f) __attribute__((always_inline)) { for_each_slot(f, std::make_integer_sequence<int, D>{}); };
@@ -252,7 +253,7 @@ template <int TX, int TY> constexpr int kRing3 = TX * TY != 1 ? 3 : 9;
 template <int TX, int TY>
 __device__ __forceinline__ void chain_reduce_3x3(v16i (&acc)[TX][TY], __amdgpu_buffer_rsrc_t wbuf, const u32 (&wp)[TX],
                                                  __amdgpu_buffer_rsrc_t data, const u32 lane16, const int (&pixoff)[TY],
-                                                 const u32 (&inside)[TY], v4i (&xf)[kRing<TX, TY>][TX], int half, int s0, int s1,
+                                                 const u32 (&inside)[TY], v4i (&xf)[kMaxRing<TX, TY>][TX], int half, int s0, int s1,
                                                  int hw16, int w16) {
   constexpr int D = kRing3<TX, TY>, P = 9;
   static_assert(P % D == 0 && D <= kRing<TX, TY>, "the ring's slots repeat with the period");
@@ -324,6 +325,71 @@ __device__ __forceinline__ int requant_quad(const v4i &v, int scale, int shift) 
     packed |= (u32)(t < 0 ? 0 : (t > 255 ? 255 : t)) << (8 * e);
   }
   return (int)packed;
+}
+
+// MODE 4: 3 x 3 windows at stride 1 whose output is as large as their input, and a share of whole periods: the pixels under a
+// wave's windows are a run of 32 TY + 2 W + 2 pixels per channel block, delivered once into the wave's own part of LDS instead of
+// up to nine times into registers: a 64 x 64 tile on 14 x 14 takes 8 KiB of pixels, not 36.  Raw buffer loads: what lies
+// outside the group arrives as zeros, and so does the last pixel of a block's rows, which stands for padding.  us with MODE 3 /
+// here: ResNet-50 batch 1 152 / 150, 16 244 / 237, 32 362 / 350; ResNet-18 64 / 62, 82 / 79, 109 - 113 / 102 - 110 (machine to machine).  Weights nine steps ahead for
+// 64 x 64 tiles spill (batch 32 369); staged through registers, exclusive-ors done there, 357.
+template <int TX, int TY> constexpr int kRingPatch = TX * TY == 4 ? 3 : 9;
+__host__ __device__ constexpr int patch_rows(int pixels, int w) { return (pixels + 2 * w + 2) / 64 + 1; }  // of 64 pixels, 1 KiB
+template <int TX, int TY>
+__device__ __forceinline__ void chain_reduce_patch(v16i (&acc)[TX][TY], __amdgpu_buffer_rsrc_t wbuf, const u32 (&wp)[TX], const u32 lane16,
+                                                   const char *patch, const u32 (&inside)[TY], v4i (&xf)[kMaxRing<TX, TY>][TX], int half,
+                                                   int s0, int s1, int rows, int w16) {
+  constexpr int P = 9, D = kRingPatch<TX, TY>, Y = 3;
+  static_assert(P % D == 0 && P % Y == 0 && D <= kMaxRing<TX, TY>, "the rings' slots repeat with the period");
+  const u32 l16 = lane16 & 511u, padding = (u32)(rows * 1024 - 16);
+  u32 at[P][TY];  // tap 2 s + half of a period
+#pragma unroll
+  for (int s = 0; s < P; ++s) {
+    const int e = 2 * s, o = 2 * s + 1;
+    const u32 oe = (u32)((e / 9) * rows * 1024 + (e % 9 / 3) * w16 + (e % 9 % 3) * 16);
+    const u32 oo = (u32)((o / 9) * rows * 1024 + (o % 9 / 3) * w16 + (o % 9 % 3) * 16);
+#pragma unroll
+    for (int j = 0; j < TY; ++j)
+      at[s][j] = inside[j] >> (half ? o % 9 : e % 9) & 1u ? l16 + (u32)(j * 512) + (half ? oo : oe) : padding;
+  }
+  v4i yf[Y][TY];
+  auto load_d = [&](int s, int j) __attribute__((always_inline)) {
+    yf[s % Y][j] = *reinterpret_cast<const v4i *>(patch + at[s % P][j] + (u32)(s / P * 2 * rows * 1024));
+  };
+#pragma unroll
+  for (int s = 0; s < Y; ++s)
+#pragma unroll
+    for (int j = 0; j < TY; ++j) load_d(s, j);
+  u32 sw = (u32)(s0 + D) * 1024u;
+  auto period = [&](auto last) __attribute__((always_inline)) {
+    constexpr bool kLast = decltype(last)::value;
+#pragma unroll
+    for (int s = 0; s < P; ++s) {
+      v4i y[TY];
+#pragma unroll
+      for (int j = 0; j < TY; ++j)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) y[j][d] = yf[s % Y][j][d] ^ (int)0x80808080;
+#pragma unroll
+      for (int i = 0; i < TX; ++i) {
+#pragma unroll
+        for (int j = 0; j < TY; ++j) {
+          acc[i][j] = OpI8::mma(xf[s % D][i], y[j], acc[i][j]);
+          __builtin_amdgcn_sched_barrier(0);
+          if (i == 0 && (!kLast || s + Y < P)) load_d(s + Y, j);
+          if (j == TY - 1 && (!kLast || s + D < P))
+            xf[s % D][i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wbuf, (int)lane16, (int)(wp[i] + sw + (u32)s * 1024u), 0));
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+  };
+  for (int s = s0; s + P < s1; s += P) {
+    period(std::false_type{});
+    patch += 2 * rows * 1024;
+    sw += P * 1024u;
+  }
+  period(std::true_type{});
 }
 
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kPerCu, kPerCu))) void chain_run(const ChainArgs a) {
@@ -407,7 +473,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kPerCu
       u32 wp[TX];  // byte offsets of the 32-channel blocks; blocks past the last one re-read it
 #pragma unroll
       for (int i = 0; i < TX; ++i) wp[i] = (u32)(min((x0 >> 5) + i, kblocks - 1) * nsteps) * 1024u;
-      v4i xf[kRing<TX, TY>][TX];
+      v4i xf[kMaxRing<TX, TY>][TX];
       auto load_w = [&](int u) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < TX; ++i)
@@ -419,6 +485,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kPerCu
       if (!is_short) {
 #pragma unroll
         for (int u = kShort<TX, TY>; u < kRing<TX, TY>; ++u) load_w(u);
+        if (kRing<TX, TY> < kRingPatch<TX, TY> && L.mode == 4) {
+#pragma unroll
+          for (int u = kRing<TX, TY>; u < kRingPatch<TX, TY>; ++u) load_w(u);
+        }
       }
       const u32 cc = (u32)min(x0 + lane, K - 1) * 4u;
       const int add0 = __builtin_amdgcn_raw_buffer_load_b32(wbuf, (int)cc, kblocks * nsteps * 1024, 0);
@@ -478,7 +548,21 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kPerCu
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
       const TapWalk tw{L.ntaps, L.KW, L.win, (W - L.KW) * 16, (H - L.KH) * W * 16, H * W * 16, W * 16, L.by_win, L.by_kw};
-      if (L.mode == 3) {
+      if (L.mode == 4) {
+        if (s0 < s1) {
+          const int rows = patch_rows(32 * TY, W), cb0 = 2 * (s0 / 9), cb1 = 2 * (s1 / 9);
+          char *const patch = reinterpret_cast<char *>(sh.part[wave]);
+          for (int k = 0; k < rows; ++k) {
+            const int p = k * 64 + lane, m = y0 - W - 1 + p;
+            const int n = quot(max(m, 0), L.by_ohw);
+            const u32 from = m >= 0 && m < npix && p < rows * 64 - 1 ? (u32)(n * L.img_bytes + (m - n * ohw) * 16) : ~0u;
+            for (int cb = cb0; cb < cb1; ++cb)
+              __builtin_amdgcn_raw_ptr_buffer_load_lds(data, (__attribute__((address_space(3))) void *)(patch + ((cb - cb0) * rows + k) * 1024), 16, (int)from, cb * ohw * 16, 0, kAgent);
+          }
+          __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+          chain_reduce_patch<TX, TY>(acc, wbuf, wp, lane16, patch, inside, xf, half, s0, s1, rows, W * 16);
+        }
+      } else if (L.mode == 3) {
         if (s0 < s1) chain_reduce_3x3<TX, TY>(acc, wbuf, wp, data, lane16, pixoff, inside, xf, half, s0, s1, H * W * 16, W * 16);
       } else if (is_short)
         chain_reduce<0, TX, TY, kShort<TX, TY>, true>(acc, wbuf, wp, data, lane16, pixoff, inside, xf, half, s0, s1, slast, tw);
@@ -658,7 +742,11 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
     const int sets = 4 / kg;
     int wx = 1;
     while (wx < sets && d.K >= 2 * sx * wx) wx *= 2;
-    if (d.KH == 3 && d.KW == 3 && s.ntaps % (18 * kg) == 0) s.mode = 3;
+    if (d.KH == 3 && d.KW == 3 && s.ntaps % (18 * kg) == 0) {
+      const bool same = d.sh == 1 && d.sw == 1 && d.pt == 1 && d.pl == 1 && g.OH == d.H && g.OW == d.W;
+      // a wave's part of LDS is 16 KiB
+      s.mode = same && d.C / 16 / kg * patch_rows(sy, d.W) <= (int)sizeof(ChainLds::part) / kWaves / 1024 ? 4 : 3;
+    }
     const int wy = sets / wx;
     s.kg_log = (unsigned char)(kg >> 1), s.wx_log = (unsigned char)(wx >> 1), s.wy_log = (unsigned char)(wy >> 1);
     s.tile = (unsigned char)((sx == 64 ? 6 : 5) | (sy == 64 ? 6 : 5) << 4);
