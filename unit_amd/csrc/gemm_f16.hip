@@ -109,7 +109,7 @@ int run_gemm_f16_group(const char *what, const char *tag, const void *a, const v
   const int forced = OUT_F16 || whole ? 1 : tuning_override("UNIT_AMD_GEMM_F16_SPLITK");
   const long tiles = tiles_of_128(M, N);
   const int least = forced <= 0 && tiles < 12 && K >= 512 ? 2 : 1;
-  GroupPlan plan = plan_group(M, N, K * 2, least, forced > 0 || tiles > 64 ? 1 : 19, kAtomicSplits, OUT_F16 ? 2 : 4);
+  GroupPlan plan = prefer_wide_tile(plan_group(M, N, K * 2, least, forced > 0 || tiles > 64 ? 1 : 19, kAtomicSplits, OUT_F16 ? 2 : 4), M, N, K * 2);
   if (forced > 0) plan.splits = forced;
   const GroupGemm p{static_cast<const char *>(a), static_cast<const char *>(b), (u32)((size_t)M * K * 2),
                     (u32)((size_t)N * K * 2), M, N, K * 2, YM == Y_COLS ? N * 2 : K * 2, nullptr, c, C_ATOMIC, 0};
@@ -151,7 +151,7 @@ int run_gemm_f16_bt(const void *a, const void *bt, void *c, int M, int N, int K,
 // (b in rows 88.3 / 119.6), 4000 x 4000 x 4008 138 / 156 (135 / 182), 3500 x 3500 x 3000 93 / 114 (95 / 124); the other way
 // 4500 x 4500 x 1496, 324 tiles in two rounds, 108 / 97 (105 / 105).
 inline bool gemm_staged_pays(int M, int N, int K, float scale) {
-  if (M < 256 || N < 256) return false;
+  if (M < 256 || N < 256 || one_wide_tile_per_cu(M, N, K * 2)) return false;
   const long tiles = (long)ceil_div(M, 256) * ceil_div(N, 256);
   return 2.f + (float)((tiles + 255) / 256) * (9.f + 0.029f * K) < scale * plan_group(M, N, K * 2, 1, 1, kAtomicSplits).us;
 }

@@ -446,6 +446,22 @@ inline GroupPlan plan_group(int M, int N, int kb, int min_splits, int max_splits
   return best;
 }
 
+// Products of more than one 128 x 128 tile per CU and at most one of 256 x 128: the large tile with 128-byte stages.  The
+// estimate sees two of the small tiles side by side on some CUs at nearly the cost of one; they take in half as much again
+// per result, and in 64-byte stages at that (two rings of 128 bytes do not fit a CU).  us of 128 x 128 / 256 x 128 in 64- / in 128-byte
+// stages: fp16 2304 x 2048 x 2056 42.5 / 39.1 / 32.8, prepared 53.8 / 43.8 / 34.7, 2600 x 1900 x 3000 64.0 / 58.3 / 47.1, 5472 x 1096 x
+// 712 prepared 23.2 / 21.9 / 19.8; int8 2304 x 2048 x 2064 31.3 / 26.9 / 24.2, 829 x 5848 x 2576 37.7 / 32.0 / 28.0, 711 x 5480 x 1024 15.7 /
+// 15.1 / 14.8.  The other way from 640 bytes of reduction down (4317 x 1536 x 320 fp16 12.5 / - / 12.9), on packed weights
+// (5400 x 1408 x 1072 19.1 / 20.8 / 21.7) and where 64 x 128 tiles are the estimate's choice, up to 2 KiB (1566 x 2548 x 672 14.8 / - / 16.9).  Left where they were: 301 - 306 small tiles, which the tests name (2180 x 2052 x 2056
+// would take 34 in place of 44).
+inline bool one_wide_tile_per_cu(int M, int N, int kb) {
+  const long half = tiles_of_128(M, N), tiles = (long)ceil_div(M, 256) * ceil_div(N, 128);
+  return half > 256 && tiles <= 256 && kb >= 768 && !(half > 300 && tiles <= 153);
+}
+inline GroupPlan prefer_wide_tile(const GroupPlan &plan, int M, int N, int kb) {
+  return plan.splits == 1 && (plan.tile == 5 || (plan.tile == 4 && kb >= 2048)) && one_wide_tile_per_cu(M, N, kb) ? GroupPlan{6, 1, plan.us} : plan;
+}
+
 // The same estimate for 256 x 256 tiles of eight waves: per round of 256 tiles 3 us plus 24.9 us per 2 KiB of
 // reduction (18.7 with at most 200 CUs busy), and the result at 6.4 TB/s.
 inline float large_tile_cost(int M, int N, int kb) {
@@ -470,7 +486,7 @@ inline float large_tile_cost(int M, int N, int kb) {
 template <class Op, int YM>
 bool group_wide_stages(const GroupGemm &p, const GroupPlan &plan) {
   const GroupCost &g = kGroupCosts[plan.tile];
-  const int least = plan.tile >= 2 ? 960 : Op::kInt && p.M <= 64 && p.N <= 4096 ? 3072 : 1536;
+  const int least = plan.tile == 6 ? 768 : plan.tile >= 2 ? 960 : Op::kInt && p.M <= 64 && p.N <= 4096 ? 3072 : 1536;
   return plan.splits == 1 && p.kb >= least && (long)ceil_div(p.M, g.bx) * ceil_div(p.N, g.by) <= 256 &&
          !(YM == Y_COLS && (plan.tile < 2 || (plan.tile == 4 && p.kb < 3072 && p.ldy % 128)));
 }
@@ -488,6 +504,9 @@ int run_group_plan(const char *what, const char *tag, const GroupGemm &p, const 
       case 3: return run_gemm_group<Op, GroupTile<1, 1, 2, 2, 2, 128, 3>, YM, WS, OUT_F16>(what, tag, p, 1, s);
       case 4: return run_gemm_group<Op, GroupTile<1, 2, 2, 2, 2, 128, 3>, YM, WS, OUT_F16>(what, tag, p, 1, s);
       case 5: return run_gemm_group<Op, GroupTile<1, 2, 4, 2, 1, 128, 3>, YM, WS, OUT_F16>(what, tag, p, 1, s);
+      case 6:
+        if constexpr (YM != Y_VNNI) return run_gemm_group<Op, GroupTile<2, 2, 4, 2, 1, 128, 3>, YM, WS, OUT_F16>(what, tag, p, 1, s);
+        break;
       default: break;
     }
   }

@@ -50,6 +50,8 @@ int run_dense_group(const char *what, const char *tag, const void *a, const void
     plan.splits = forced;
   else if (K >= 8192 && plan.us >= 15.f)
     plan = plan_group(M, N, K, least, 16, kAtomicSplits);
+  else if (YM == Y_ROWS)
+    plan = prefer_wide_tile(plan, M, N, K);
   const GroupGemm p{static_cast<const char *>(a), static_cast<const char *>(w), (u32)((size_t)M * K), (u32)((size_t)N * K),
                     M, N, K, K, wsum, c, C_ATOMIC, 0};
   return run_group_plan<OpI8, YM, WS, false>(what, tag, p, plan, s);
@@ -132,6 +134,7 @@ int run_dense_mixed(const void *a, const void *wp, void *c, int M, int N, int K,
 inline bool dense_stays_staged(int M, int N, int K) {
   if (K % 128 == 0 || M < 256 || N < 256) return false;
   if (K % 128 == 64 && K < 1024 && direct_gemm_large_tiles(M, N)) return true;
+  if (one_wide_tile_per_cu(M, N, K)) return false;  // 24 us where 256 x 256 tiles would take 45
   return 1.15f * large_tile_cost(M, N, K) < plan_group(M, N, K, 1, 1, kAtomicSplits).us;
 }
 
