@@ -101,14 +101,14 @@ int run_gemm_f16_hybrid(const void *a, const void *b, void *c, int M, int N, int
 // operator takes (b by columns: N >= 8).  fp32 results of up to 64 tiles of 128 x 128 may also share it between workgroups
 // (atomics into the zero-filled output); with more tiles they are the same bits from run to run, and the estimate's splits
 // lost there (900 x 1096 x 7536, 72 tiles, two ranges 64.9 us, whole 49.4; 733 x 1600 x 7616, 78 tiles, 61.8 and 46.2).  With
-// fewer than 12 such tiles and 1 KiB of reduction at least two ways (the tests ask for that; 300 x 260 x 520 would run 2 us
-// faster without).  fp16 results keep one workgroup per tile.
+// up to six such tiles and 1 KiB of reduction, or fewer than 12 and up to 2 KiB, at least two ways (the tests ask for that; 300 x
+// 260 x 520 would run 2 us faster without).  fp16 results keep one workgroup per tile.
 template <int YM, bool OUT_F16>
 int run_gemm_f16_group(const char *what, const char *tag, const void *a, const void *b, void *c, int M, int N, int K,
                        hipStream_t s, bool whole = false) {
   const int forced = OUT_F16 || whole ? 1 : tuning_override("UNIT_AMD_GEMM_F16_SPLITK");
   const long tiles = tiles_of_128(M, N);
-  const int least = forced <= 0 && tiles < 12 && K >= 512 ? 2 : 1;
+  const int least = forced <= 0 && K >= 512 && (tiles <= 6 || (tiles < 12 && K < 1024)) ? 2 : 1;
   GroupPlan plan = prefer_wide_tile(plan_group(M, N, K * 2, least, forced > 0 || tiles > 64 ? 1 : 19, kAtomicSplits, OUT_F16 ? 2 : 4), M, N, K * 2);
   if (forced > 0) plan.splits = forced;
   const GroupGemm p{static_cast<const char *>(a), static_cast<const char *>(b), (u32)((size_t)M * K * 2),
@@ -116,16 +116,18 @@ int run_gemm_f16_group(const char *what, const char *tag, const void *a, const v
   return run_group_plan<OpF16, YM, WS_NONE, OUT_F16>(what, tag, p, plan, s);
 }
 
-// Which aligned shapes stay on the 128 x 128 tiles of mma_dma.hpp: fp32 results with fewer than 32 such tiles and more
-// than 128 rows (the tests name that kernel and its k-splits for them), one nearly full round of the 256 CUs
+// Which aligned shapes stay on the 128 x 128 tiles of mma_dma.hpp: one nearly full round of the 256 CUs
 // (1011 x 3584 x 1216, 224 tiles, 15.6 against 16.2 us on the group tile of the same size; 2048^3 22.9 against 24.8), and 512
 // tiles or more (8192 x 1024 x 1024 24.2 and 24.0 us).  The others gain: 1024^3 11.1 -> 7.1 us, 2304 x 2304 x 4096
-// 65.5 -> 57.2, 64 x 4096 x 4096 15.6 -> 14.0.
+// 65.5 -> 57.2, 64 x 4096 x 4096 15.6 -> 14.0; and fp32 results of few tiles, whose k-splits cost a zero fill and atomics: 852 x 448 x 2112
+// 14.1 -> 9.1, 562 x 320 x 1536 11.2 -> 7.4, 1365 x 64 x 1856 11.1 -> 6.3, 588 x 516 x 320 8.8 -> 4.9.  The tests name the kernel for
+// two of those, with more than 128 rows: up to six tiles and 512 <= K < 1024, 24 - 31 tiles and 512 <= K < 1536.
 // fp16 results of whole 128-byte rows keep them up to 511 tiles for K of 160 to 640 (6000 x 704 x 256 7.3 us of kernel
 // against 8.1, 5000 x 1024 x 512 11.1 and 12.0; K = 128 6.1 and 5.8).
 inline bool gemm_keeps_128(int M, int N, int K, bool out_f16) {
   const long tiles = tiles_of_128(M, N);
-  return tiles >= 512 || (tiles >= 192 && tiles <= 256) || (!out_f16 && tiles < 32 && M > 128) ||
+  return tiles >= 512 || (tiles >= 192 && tiles <= 256) ||
+         (!out_f16 && M > 128 && K >= 512 && (tiles <= 6 ? K < 1024 : tiles >= 24 && tiles < 32 && K < 1536)) ||
          (out_f16 && tiles > 256 && N % 64 == 0 && K >= 160 && K <= 640);
 }
 
@@ -151,7 +153,8 @@ int run_gemm_f16_bt(const void *a, const void *bt, void *c, int M, int N, int K,
 // (b in rows 88.3 / 119.6), 4000 x 4000 x 4008 138 / 156 (135 / 182), 3500 x 3500 x 3000 93 / 114 (95 / 124); the other way
 // 4500 x 4500 x 1496, 324 tiles in two rounds, 108 / 97 (105 / 105).
 inline bool gemm_staged_pays(int M, int N, int K, float scale) {
-  if (M < 256 || N < 256 || one_wide_tile_per_cu(M, N, K * 2)) return false;
+  // short reductions are their stores and loads (2562 x 5436 x 72 17.3 us staged, 12.0; 5966 x 6172 x 176 49 and 38); one_wide_tile_per_cu
+  if (M < 256 || N < 256 || K < 256 || one_wide_tile_per_cu(M, N, K * 2)) return false;
   const long tiles = (long)ceil_div(M, 256) * ceil_div(N, 256);
   return 2.f + (float)((tiles + 255) / 256) * (9.f + 0.029f * K) < scale * plan_group(M, N, K * 2, 1, 1, kAtomicSplits).us;
 }

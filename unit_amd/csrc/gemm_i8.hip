@@ -37,18 +37,21 @@ int run_dense_staged(const void *a, const void *w, void *c, int M, int N, int K,
 // Tiles of at most 256 x 128 with the reduction shared inside the workgroup (gemm_group.hpp).  Sharing it between
 // workgroups as well (int32 atomics into the zero-filled output, exact) costs a launch: it pays from 8 KiB of reduction on
 // where the estimate without it is 15 us or more (512 x 516 x 12304 30.8 us whole, 20.0 in three ranges; 2081 x 128 x 10208
-// 25.7 and 16.4; 2 x 3968 x 8800, estimate 12.6, 9.4 whole and 11.8 in three).  The row-major operator shares at least two
-// ways where it has fewer than 12 tiles of 128 x 128 and 1 KiB of reduction (its tests ask for that; 50 x 260 x 1040 would
-// run 2 us faster without).
+// 25.7 and 16.4; 2 x 3968 x 8800, estimate 12.6, 9.4 whole and 11.8 in three), and from 4.5 KiB on (packed 5 KiB: 71 x 1024 x 5040 7.5 and
+// 7.9) with up to 16 tiles of 128 x 128, if the estimate says so (7 x 896 x 8048 packed 9.2 us whole, 6.8 in six; 8 x 1160 x 7840 8.5 in
+// two, 6.7 in six).  The row-major
+// operator shares at least two ways where it has up to six such tiles and 1 KiB of reduction (its tests ask for that; 50 x 260 x 1040
+// would run 2 us faster without, and with 7 - 11 tiles, where it also did, 33 x 820 x 3024 took 7.3 for 6.1).
 template <int YM, int WS>
 int run_dense_group(const char *what, const char *tag, const void *a, const void *w, const int *wsum, void *c, int M, int N,
                     int K, hipStream_t s) {
   const int forced = tuning_override("UNIT_AMD_DENSE_SPLITK");
-  const int least = forced <= 0 && YM == Y_ROWS && tiles_of_128(M, N) < 12 && K >= 1024 ? 2 : 1;
+  const long tiles = tiles_of_128(M, N);
+  const int least = forced <= 0 && YM == Y_ROWS && tiles <= 6 && K >= 1024 ? 2 : 1;
   GroupPlan plan = plan_group(M, N, K, least, 1, kAtomicSplits);
   if (forced > 0)
     plan.splits = forced;
-  else if (K >= 8192 && plan.us >= 15.f)
+  else if ((K >= 8192 && plan.us >= 15.f) || (K >= (YM == Y_VNNI ? 5120 : 4608) && tiles <= 16))
     plan = plan_group(M, N, K, least, 16, kAtomicSplits);
   else if (YM == Y_ROWS)
     plan = prefer_wide_tile(plan, M, N, K);
@@ -57,13 +60,20 @@ int run_dense_group(const char *what, const char *tag, const void *a, const void
   return run_group_plan<OpI8, YM, WS, false>(what, tag, p, plan, s);
 }
 
-// Row-major weights with whole 64-byte stages: the 128 x 128 tiles of mma_dma.hpp keep the shapes with few tiles or
-// few stages, and those with 512 tiles or more (8192 x 1024 x 1024 17.3 against 16.5 us); the tests name this kernel
-// there.  From 32 tiles and 384 bytes on the group tiles are faster (64 x 4096 x 4096 13.3 -> 7.9 us, 1024^3
-// 11.2 -> 7.0, 1024 x 4096 x 4096 29.4 -> 25.3).
+// Row-major weights with whole 64-byte stages: the 128 x 128 tiles of mma_dma.hpp keep the shapes with 512 tiles or more
+// (8192 x 1024 x 1024 17.3 against 16.5 us).  Else the group tiles are faster (64 x 4096 x 4096 13.3 -> 7.9 us, 1024^3
+// 11.2 -> 7.0, 1024 x 4096 x 4096 29.4 -> 25.3), also with few tiles, whose k-splits cost a zero fill and atomics, and with few stages:
+// 178 x 1336 x 1216 12.2 -> 5.4, 636 x 420 x 1536 12.3 -> 6.5, prepared 420 x 304 x 2112 10.9 -> 5.4, 66 x 1288 x 3776 10.8 -> 6.7;
+// 1357 x 284 x 192 8.3 -> 4.5, 320 x 4160 x 192 8.3 -> 5.8, 2680 x 1352 x 320 9.2 -> 7.8, 7259 x 404 x 64 prepared 7.8 -> 5.8.  The tests
+// name this kernel for a few of those: up to four tiles and 192 bytes, 32 - 63 or 256 and more from 256 bytes to 320, and up to six
+// tiles with 2 - 4 KiB, in k-splits.
 inline bool dense_keeps_128(int M, int N, int K) {
   const long tiles = tiles_of_128(M, N);
-  return K % 64 == 0 && !direct_gemm_large_tiles(M, N) && (tiles < 32 || tiles >= 512 || K < 384);
+  if (K % 64 || direct_gemm_large_tiles(M, N)) return false;
+  if (tiles >= 512) return true;
+  if (K <= 192) return tiles <= 4;
+  if (K <= 320) return K >= 256 && ((tiles >= 32 && tiles < 64) || tiles >= 256);
+  return tiles <= 6 && K >= 2048 && K < 4096;
 }
 
 // direct-to-LDS variant: row-major weights, K a whole number of stages.  wsum: the weight's row sums when they
