@@ -57,3 +57,17 @@ LAUNCHES = {
 @pytest.mark.parametrize("name", LAUNCHES)
 def test_chains_that_lose_in_the_kernel_stay_launches(name):
     assert _workspace(*LAUNCHES[name]) == 0
+
+
+# The estimate with the tiles taken, where 64 x 64 alone (and k-groups that leave whole periods or not) said launches
+KERNEL = {
+    "six images of 8 x 8, 19.9 / 27.2": ([(48, 3, 1, None)] * 3 + [(192, 3, 1, None)] * 3, 6, 48, 8, 8),
+    "narrow layers, 23.1 / 29.9": ([(16, 3, 1, None), (80, 3, 1, None), (96, 3, 1, None), (16, 3, 1, None), (16, 1, 1, None),
+                                    (48, 3, 1, None), (96, 3, 1, None)], 6, 272, 7, 7),
+    "24 images, 40.1 / 49.9": ([(32, 3, 1, None)] * 4 + [(336, 3, 1, None), (304, 3, 1, None)], 24, 32, 28, 21),
+}
+
+
+@pytest.mark.parametrize("name", KERNEL)
+def test_chains_that_win_with_small_tiles_take_the_kernel(name):
+    assert _workspace(*KERNEL[name]) > 0

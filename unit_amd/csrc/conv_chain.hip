@@ -42,7 +42,7 @@ int conv_geom(const unit_conv_desc *d, int tapb, ConvGeom *g, const char *what);
 namespace {
 
 constexpr int kWaves = 4, kThreads = 64 * kWaves;
-constexpr int kPerCu = 2;                 // workgroups per CU: 246 VGPRs (three of 168 with three k-steps in flight: 392 us at batch 32, 234 at 8)
+constexpr int kPerCu = 2;                 // workgroups per CU: 256 VGPRs (three of 168 with three k-steps in flight: 392 us at batch 32, 234 at 8)
 // A wave's tile is TX x TY blocks of 32 channels x 32 pixels: 2 x 2, 2 x 1 or 1 x 1.  k-steps of fragments in flight per wave: few
 // blocks are few MFMAs per step, so more steps to cover a load's latency (nine for one block, a period of chain_reduce_3x3; nine for
 // two blocks spilled).  A wave whose share of a 1 x 1 layer is short loads no more than kShort steps.
@@ -678,7 +678,7 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
   p->per = per;
   p->groups = (N + per - 1) / per;
   long first = 0;
-  double here = 5.5, launches = 0.9;  // us, below
+  double here = 5.35, here64 = 5.5, launches = 0.9;  // us, below
   Range outs[kMaxChain];
   for (int i = 0; i < count; ++i) {
     const unit_chain_layer &l = layers[i];
@@ -715,39 +715,45 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
     s.row_ones = g.row_ones;
     s.KH = (unsigned char)d.KH, s.KW = (unsigned char)d.KW, s.sh = (unsigned char)d.sh, s.sw = (unsigned char)d.sw;
     const bool masked = d.pt || d.pl || d.pb || d.pr;
-    s.mode = masked ? 2 : (s.win == 1 && s.ntaps % 2 == 0 ? 0 : 1);
     s.flat = !masked && d.KH == 1 && d.KW == 1 && d.sh == 1 && d.sw == 1;
     const long npix = (long)per * s.ohw;
     if (npix * s.ohw > 0x7fffffffl) return false;
-    // Tile and k-groups: a tile of 64 x 64 costs 2.6 us beside its reduction (decode, first loads, requantisation, stores, flag), 0.4
-    // more with k-groups, and 0.25 us per k-step of a wave; an XCD runs 64 at a time.  Smaller tiles move more operand bytes per
-    // result, so they only pay where the large ones leave workgroups idle: the rounds say where.  us with 64 x 64 alone / with 32 x 32 /
-    // and 64 x 32: ResNet-50 batch 1 203 / 164 / 151, 8 232 / 187 / 173, 16 275 / 258 / 244, 32 377 / 376 / 361; ResNet-18 1 83 / 67 / 65, 32
-    // 118 / 117 / 110.  Steps of 0.12 - 0.18 and fixed parts 0.2 lower or higher: within 2 %; 0.1 for 32 x 32 costs 4 % at 16 images.
-    const auto split = [&](int cx, int cy, double fixed, double shared, double step, double &best) {
-      const long wt = (long)ceil_div(d.K, cx) * ((npix + cy - 1) / cy);
-      int kg = 0;
-      for (int k = 1; k <= 4 && k <= s.nsteps; k *= 2) {
-        const double rounds = std::max(1.0, (double)wt * k / 4 / 64);
-        const double t = rounds * (fixed + (k > 1 ? shared : 0.0) + step * ceil_div(s.nsteps, k));
-        if (t < best) best = t, kg = k;
-      }
-      return kg;
-    };
-    double best = 1e30;
-    int kg = split(64, 64, 2.6, 0.4, 0.25, best), sx = 64, sy = 64;
-    const int kg64 = kg;
-    if (const int k = split(64, 32, 2.2, 0.2, 0.2, best)) kg = k, sy = 32;
-    if (const int k = split(32, 32, 2.0, 0.2, 0.15, best)) kg = k, sx = sy = 32;
-    const int sets = 4 / kg;
-    int wx = 1;
-    while (wx < sets && d.K >= 2 * sx * wx) wx *= 2;
-    if (d.KH == 3 && d.KW == 3 && s.ntaps % (18 * kg) == 0) {
-      const bool same = d.sh == 1 && d.sw == 1 && d.pt == 1 && d.pl == 1 && g.OH == d.H && g.OW == d.W;
+    // Tile and k-groups.  A layer costs the decode, first loads, requantisation, stores and flag of its tiles (2.1 - 2.5 us, 0.1 more
+    // with k-groups, 1.9 for each further round of an XCD's 64 workgroups) and a price per k-step of a wave: by tile and walk, less while
+    // workgroups are idle, since the others then have the loads to themselves.  Smaller tiles move more operand bytes per result and
+    // pay where large ones leave workgroups idle; k-groups that leave whole periods of nine k-steps keep the cheap walk (3 x 3, 64
+    // channels, 28 x 28, batch 4: four groups of 5 k-steps that walk 3.8 us a layer, two of 9 2.7).  Fitted to 1400 chains of two
+    // alternating layers, each with all nine combinations: the choice is within 1.9 % of the best one (geometric mean), within 4.5 %
+    // for layers under 4 us.  us with 64 x 64 alone / now: ResNet-50 batch 1 203 / 149, 8 232 / 171, 16 275 / 236, 32 377 / 350;
+    // ResNet-18 1 83 / 62, 32 118 / 107.  Prices for 1 x 1 layers 0.05 lower: ResNet-50 at 12 images and more 3 - 10 % slower.
+    const bool same = d.sh == 1 && d.sw == 1 && d.pt == 1 && d.pl == 1 && g.OH == d.H && g.OW == d.W;
+    const auto mode_of = [&](int cy, int k) {
+      if (d.KH != 3 || d.KW != 3 || s.ntaps % (18 * k)) return masked ? 2 : s.win == 1 && s.ntaps % 2 == 0 ? 0 : 1;
       // a wave's part of LDS is 16 KiB
-      s.mode = same && d.C / 16 / kg * patch_rows(sy, d.W) <= (int)sizeof(ChainLds::part) / kWaves / 1024 ? 4 : 3;
-    }
-    const int wy = sets / wx;
+      return same && d.C / 16 / k * patch_rows(cy, d.W) <= (int)sizeof(ChainLds::part) / kWaves / 1024 ? 4 : 3;
+    };
+    int kg = 1, sx = 64, sy = 64, wx = 1;
+    double tiles_us = 1e30, steps_us = 0;
+    const auto rounds_of = [&](int cx, int cy, int k, int &x) {  // x: a workgroup's waves side by side along the channels
+      x = 1;
+      while (x < 4 / k && d.K >= 2 * cx * x) x *= 2;
+      const int cols = cx * x, rows = cy * (4 / k / x);
+      return (double)ceil_div(d.K, cols) * ((npix + rows - 1) / rows) / 64;
+    };
+    const auto offer = [&](int cx, int cy, double first, const double (&step)[5]) {
+      for (int k = 1; k <= 4 && k <= s.nsteps; k *= 2) {
+        int x;
+        const double rounds = rounds_of(cx, cy, k, x);
+        const double t = first + (k > 1 ? 0.1 : 0.0) + 1.9 * std::max(0.0, rounds - 1);
+        const double u = step[mode_of(cy, k)] * ceil_div(s.nsteps, k) * std::max(rounds, 0.5 + 0.5 * std::min(1.0, rounds));
+        if (t + u < tiles_us + steps_us) tiles_us = t, steps_us = u, kg = k, sx = cx, sy = cy, wx = x;
+      }
+    };
+    offer(64, 64, 2.5, {0.27, 0.32, 0.32, 0.26, 0.24});
+    offer(64, 32, 2.15, {0.2, 0.26, 0.26, 0.19, 0.15});
+    offer(32, 32, 2.1, {0.15, 0.21, 0.21, 0.12, 0.09});
+    s.mode = mode_of(sy, kg);
+    const int wy = 4 / kg / wx;
     s.kg_log = (unsigned char)(kg >> 1), s.wx_log = (unsigned char)(wx >> 1), s.wy_log = (unsigned char)(wy >> 1);
     s.tile = (unsigned char)((sx == 64 ? 6 : 5) | (sy == 64 ? 6 : 5) << 4);
     s.nct = ceil_div(d.K, sx * wx);
@@ -755,9 +761,18 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
     const long npt = (npix + sy * wy - 1) / (sy * wy);
     if (npt * s.nct * s.nct > 0x7fffffffl) return false;
     const double gmac = 1e-9 * s.ohw * d.K * s.ntaps * 16, mb = 1e-6 * ((double)g.img_bytes + (double)s.ohw * d.K);  // of an image
-    const double rounds = (double)ceil_div(d.K, 64) * ((npix + 63) / 64) * kg64 / 256, ksteps = ceil_div(s.nsteps, kg64);
-    here += 1.45 + (kg64 > 1 ? 0.15 : 0.0) + 0.8 * std::max(1.0, rounds) +
-            (s.mode == 1 || s.mode == 2 ? 0.3 : 0.21) * ksteps * std::max(0.5, rounds) + 1.28 * mb * per;
+    here += 0.78 * tiles_us + 1.06 * steps_us + 0.9 * mb * per;
+    int k64 = 1, x64;
+    double best = 1e30;
+    for (int k = 1; k <= 4 && k <= s.nsteps; k *= 2) {
+      const double t = std::max(1.0, (double)ceil_div(d.K, 64) * ((npix + 63) / 64) * k / 256) *
+                       (2.6 + (k > 1 ? 0.4 : 0.0) + 0.25 * ceil_div(s.nsteps, k));
+      if (t < best) best = t, k64 = k;
+    }
+    const double rounds = rounds_of(64, 64, k64, x64);
+    const int m64 = mode_of(64, k64);
+    here64 += 1.45 + (k64 > 1 ? 0.15 : 0.0) + 0.8 * std::max(1.0, rounds) +
+              (m64 == 1 || m64 == 2 ? 0.3 : 0.21) * ceil_div(s.nsteps, k64) * std::max(0.5, rounds) + 1.28 * mb * per;
     launches += 3.6 + 1.15 * gmac * N + 0.176 * mb * N + 0.019 * std::min(s.nsteps, 80);
     s.first = (int)first;
     first += npt * s.nct;
@@ -772,16 +787,16 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
         break;
       }
   }
-  // Short chains, few images through large layers and activations that outgrow an XCD's 4 MB of L2 stay launches.  The
-  // kernel costs 5.5 us before its first tile; a layer 1.5 us, and 0.8 us for each round of an XCD's 64 workgroups, 0.2 (0.3 with
-  // the tap walk) per k-step of it and 1.3 per MB that the group reads and writes; a launch 3.6 us, 1.2 per GMAC and 0.18 per MB
-  // of the batch.  Fitted to 300 random chains and 32 of ResNets, both ways each: errors of 7 % and 6 % (root mean square); of
-  // the 225 it gives to the kernel 7 lose there, up to 10 %, and without the bytes and the rounds chains of wide images at 14 - 54
-  // images lost 10 - 22 %.  us here / as launches: 3 x 3 64 -> 64 on 56 x 56, batch 8, 3 layers 17.6 / 20.1; 1 x 1 256 -> 256 on
-  // 14 x 14, batch 1, 8 layers 24.3 / 30.3; ResNet-18 batch 1 82 / 88, 32 118 / 157; ResNet-50 batch 1 197 / 219, 128 1026 / 1216;
-  // the other way 14 layers from 51 x 51, batch 14 245 / 201, 10 layers from 50 x 50, batch 52 197 / 167, 9 layers of 224 channels
-  // on 20 x 20, batch 2 42.9 / 38.0.
-  if (here > 0.975 * launches) return false;
+  // Short chains, few images through large layers and activations that outgrow an XCD's 4 MB of L2 stay launches.  The kernel
+  // costs 5.4 us before its first tile, then the layers as estimated above and 0.9 us per MB that the group reads and writes; a launch
+  // 3.6 us, 1.2 per GMAC and 0.18 per MB of the batch.  here64 is the estimate for 64 x 64 tiles alone (a layer 1.5 us, 0.8 for each
+  // round of an XCD's 64 workgroups, 0.2, with the tap walk 0.3, per k-step of it), which the tiles taken are not slower than.  Both have
+  // errors of 6 - 7 % (root mean square) that differ, and either one is taken at its word: over 500 random chains of 3 to 48 layers
+  // timed both ways, here64 alone ends 2.4 % from always the faster way, `here` alone 1.2 %, either 0.8 %; of the 413 given to
+  // the kernel two lose more than 3 % there, both of 3 layers.  us here / as launches: 3 x 3 64 -> 64 on 56 x 56, batch 8, 3 layers
+  // 17.6 / 20.1; 1 x 1 256 -> 256 on 14 x 14, batch 1, 8 layers 24.3 / 30.3; the other way, with 64 x 64 tiles, 14 layers from
+  // 51 x 51, batch 14 245 / 201, 10 layers from 50 x 50, batch 52 197 / 167, 9 layers of 224 channels on 20 x 20, batch 2 42.9 / 38.0.
+  if (here64 > 0.975 * launches && here > 0.93 * launches) return false;
   // The layers no longer run one after the other: none may write what another one reads or writes, but for a source's
   // whole result.
   std::sort(outs, outs + count, [](const Range &u, const Range &v) { return u.a < v.a; });
