@@ -7,7 +7,7 @@ cpu-shapes.log:388-420.
 Every layer is the requantising convolution (ops.conv2d_NCHWc_int8_requant): u8 in, u8 out, so a layer's
 output is the next layer's input as it lies in memory.  The runner owns all activation buffers and
 prepared weights and issues nothing but kernel launches through the C ABI (a chain that pays for it as one
-persistent kernel, with a workspace of the caching allocator per run: 120 KB for the ResNet-50 below at batch 32), and can
+persistent kernel, with a workspace of the caching allocator per run: 125 KB for the ResNet-50 below at batch 32), and can
 therefore be captured into a HIP graph.
 """
 import ctypes

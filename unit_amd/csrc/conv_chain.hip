@@ -11,7 +11,7 @@
 //   * the weights of a tile, which depend on no other tile, are under way while it waits.
 // Measured against the launches, us a pass among others, its setup included: ResNet-50 batch 32 on inputs and buffers that
 // change 350 / 491; on two inputs in turn 151 / 219 at batch 1, 171 / 282 at 8, 237 / 331 at 16; ResNet-18 62 / 88 at 1, 79 / 126 at
-// 16, 106 / 156 at 32.  At batch 32 the matrix pipes are busy 16 % of the time and a CU takes in 20 bytes of operands per clock:
+// 16, 107 / 156 at 32.  At batch 32 the matrix pipes are busy 16 % of the time and a CU takes in 20 bytes of operands per clock:
 // what is left is the latency of fifty-two layers, 3 us each at batch 1 (0.6 - 0.8 decode, 0.3 until the flag is seen, 0.8 - 1.4
 // loads and reduction, 0.5 k-group sum, requantisation and stores, 0.2 their acknowledgement, 0.2 flag).
 //
@@ -331,8 +331,9 @@ __device__ __forceinline__ int requant_quad(const v4i &v, int scale, int shift) 
 // wave's windows are a run of 32 TY + 2 W + 2 pixels per channel block, delivered once into the wave's own part of LDS instead of
 // up to nine times into registers: a 64 x 64 tile on 14 x 14 takes 8 KiB of pixels, not 36.  Raw buffer loads: what lies
 // outside the group arrives as zeros, and so does the last pixel of a block's rows, which stands for padding.  us with MODE 3 /
-// here: ResNet-50 batch 1 152 / 150, 16 244 / 237, 32 362 / 350; ResNet-18 64 / 62, 82 / 79, 109 - 113 / 102 - 110 (machine to machine).  Weights nine steps ahead for
-// 64 x 64 tiles spill (batch 32 369); staged through registers, exclusive-ors done there, 357.
+// here: ResNet-50 batch 1 152 / 150, 16 244 / 237, 32 362 / 350; ResNet-18 64 / 62, 82 / 79, 109 - 113 / 102 - 110 (machine to
+// machine).  Weights nine steps ahead for 64 x 64 tiles spill (batch 32 369), and so do whole steps unrolled (146 registers);
+// staged through registers, exclusive-ors done there, 357.
 template <int TX, int TY> constexpr int kRingPatch = TX * TY == 4 ? 3 : 9;
 __host__ __device__ constexpr int patch_rows(int pixels, int w) { return (pixels + 2 * w + 2) / 64 + 1; }  // of 64 pixels, 1 KiB
 template <int TX, int TY>

@@ -452,8 +452,8 @@ inline GroupPlan plan_group(int M, int N, int kb, int min_splits, int max_splits
 // stages: fp16 2304 x 2048 x 2056 42.5 / 39.1 / 32.8, prepared 53.8 / 43.8 / 34.7, 2600 x 1900 x 3000 64.0 / 58.3 / 47.1, 5472 x 1096 x
 // 712 prepared 23.2 / 21.9 / 19.8; int8 2304 x 2048 x 2064 31.3 / 26.9 / 24.2, 829 x 5848 x 2576 37.7 / 32.0 / 28.0, 711 x 5480 x 1024 15.7 /
 // 15.1 / 14.8.  The other way from 640 bytes of reduction down (4317 x 1536 x 320 fp16 12.5 / - / 12.9), on packed weights
-// (5400 x 1408 x 1072 19.1 / 20.8 / 21.7) and where 64 x 128 tiles are the estimate's choice, up to 2 KiB (1566 x 2548 x 672 14.8 / - / 16.9).  Left where they were: 301 - 306 small tiles, which the tests name (2180 x 2052 x 2056
-// would take 34 in place of 44).
+// (5400 x 1408 x 1072 19.1 / 20.8 / 21.7) and where 64 x 128 tiles are the estimate's choice, up to 2 KiB (1566 x 2548 x 672 14.8 / - /
+// 16.9).  Left where they were: 301 - 306 small tiles, which the tests name (2180 x 2052 x 2056 would take 34 in place of 44).
 inline bool one_wide_tile_per_cu(int M, int N, int kb) {
   const long half = tiles_of_128(M, N), tiles = (long)ceil_div(M, 256) * ceil_div(N, 128);
   return half > 256 && tiles <= 256 && kb >= 768 && !(half > 300 && tiles <= 153);
