@@ -523,19 +523,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kPerCu
         }
       }
       if (L.reads) {
-        if (!__all(flag != 0)) {
-#ifdef PREF
-          if (s1 - s0 > kRing<TX, TY>) {
-            int got = 0;
-            for (u32 o = (u32)(s0 + kRing<TX, TY>) * 1024u; o < (u32)s1 * 1024u; o += 8192u) {
-#pragma unroll
-              for (int i = 0; i < TX; ++i) got ^= __builtin_amdgcn_raw_buffer_load_b32(wbuf, (int)min(lane16 * 8u + o, (u32)slast * 1024u), (int)wp[i], 0);
-            }
-            asm volatile("" ::"v"(got));
-          }
-#endif
+        if (!__all(flag != 0))
           while (!__all(load_l2(wanted + (u32)min(fa + lane, fb - 1)) != 0) && --budget > 0) __builtin_amdgcn_s_sleep(1);
-        }
         for (int b = fa + 64; b < fb; b += 64) {
           while (!__all(load_l2(wanted + (u32)min(b + lane, fb - 1)) != 0) && --budget > 0) __builtin_amdgcn_s_sleep(1);
         }
