@@ -37,7 +37,7 @@
 
 namespace unit {
 
-int conv_geom(const unit_conv_desc *d, int tapb, ConvGeom *g, const char *what);  // abi.hip
+int conv_sizes(const unit_conv_desc *d, int tapb, ConvGeom *g, const char *what);  // abi.hip
 
 namespace {
 
@@ -56,8 +56,8 @@ constexpr int kAgent = 16;        // sc1
 // not valid.  UNIT_AMD_CHAIN_POLLS sets another number (a test takes one).
 constexpr int kPolls = 1 << 24;
 
-// q = n / d for n * d < 2^31
-inline u32 small_div(int d) { return (u32)(0x80000000ull / (unsigned)d) + (d != 1); }
+// q = n / d for n * d < 2^31 (a double's quotient is exact enough: 2^31 / d is at least 1 / d below the next whole number)
+inline u32 small_div(int d) { return (u32)(2147483648.0 / d) + (d != 1); }
 __device__ __forceinline__ int quot(int n, u32 mul) { return (int)__umulhi((u32)n << 1, mul); }
 
 // A layer as the kernel reads it.  Sizes are those of a group of images.
@@ -658,6 +658,54 @@ struct Range {
   const char *a, *b;
 };
 
+// Every run makes its plan again, so sizes of tiles and k-groups, powers of two, stand here as their logarithms (shifts, no
+// divisions), and what few chains need (estimate64) is worked out for those: ResNet-50 5.8 us of host time, 10.6 without either.
+inline long ceil_shift(long n, int log) { return (n + (1l << log) - 1) >> log; }
+
+// the reduction (MODE) of a layer in 1 << klog k-groups: all of them at once, one for each tile height of 32 and 64 pixels
+struct Modes {
+  unsigned char of[2][3];
+  Modes(const unit_conv_desc &d, const ChainStep &s) {
+    const int ntaps = s.ntaps, W = d.W;
+    const int plain = d.pt || d.pl || d.pb || d.pr ? 2 : d.KH * d.KW == 1 && ntaps % 2 == 0 ? 0 : 1;
+    const int periods = d.KH == 3 && d.KW == 3 && ntaps % 18 == 0 ? ntaps / 18 : 0;  // of nine k-steps
+    const bool same = d.sh == 1 && d.sw == 1 && d.pt == 1 && d.pl == 1 && s.OW == W && s.ohw == d.H * W;
+    for (int y = 0; y < 2; ++y)
+      for (int k = 0; k < 3; ++k) {
+        // a wave's part of LDS is 16 KiB
+        const bool fits = same && (d.C >> (4 + k)) * patch_rows(32 << y, W) <= (int)sizeof(ChainLds::part) / kWaves / 1024;
+        of[y][k] = (unsigned char)(!periods || periods & ((1 << k) - 1) ? plain : fits ? 4 : 3);
+      }
+  }
+};
+
+// rounds of an XCD's 64 workgroups; x: log2 of a workgroup's waves side by side along the channels
+inline double rounds_of(int K, long npix, int xlog, int ylog, int klog, int &x) {
+  x = std::max(0, std::min(2 - klog, 31 - __builtin_clz((u32)K) - xlog));
+  return (double)(ceil_shift(K, xlog + x) * ceil_shift(npix, ylog + 2 - klog - x)) * 0.015625;
+}
+
+// us of all layers on 64 x 64 tiles alone
+inline double estimate64(const unit_chain_layer *layers, const ChainStep *st, int count, int per) {
+  double here = 5.5;
+  for (int i = 0; i < count; ++i) {
+    const ChainStep &s = st[i];
+    const long npix = (long)per * s.ohw;
+    int kg = 0, x;
+    double best = 1e30;
+    const double tiles = (double)(ceil_shift(s.K, 6) * ceil_shift(npix, 6));
+    for (int k = 0; k <= 2 && 1 << k <= s.nsteps; ++k) {
+      const double t = std::max(1.0, tiles * (1 << k) * 0.00390625) * (2.6 + (k ? 0.4 : 0.0) + 0.25 * ceil_shift(s.nsteps, k));
+      if (t < best) best = t, kg = k;
+    }
+    const double rounds = rounds_of(s.K, npix, 6, 6, kg, x), mb = 1e-6 * ((double)(u32)s.img_bytes + (double)s.ohw * s.K);
+    const int mode = Modes(layers[i].desc, s).of[1][kg];
+    here += 1.45 + (kg ? 0.15 : 0.0) + 0.8 * std::max(1.0, rounds) +
+            (mode == 1 || mode == 2 ? 0.3 : 0.21) * ceil_shift(s.nsteps, kg) * std::max(0.5, rounds) + 1.28 * mb * per;
+  }
+  return here;
+}
+
 // false: the layers run one launch each
 bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainStep *st, ChainPlan *p) {
   if (count < 2 || count > kMaxChain) return false;
@@ -668,7 +716,7 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
   p->per = per;
   p->groups = (N + per - 1) / per;
   long first = 0;
-  double here = 5.35, here64 = 5.5, launches = 0.9;  // us, below
+  double here = 5.35, launches = 0.9;  // us, below
   Range outs[kMaxChain];
   for (int i = 0; i < count; ++i) {
     const unit_chain_layer &l = layers[i];
@@ -676,7 +724,7 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
     if (!l.prepared || !l.out || l.shift < 1 || l.shift > 62 || check_aligned("chain", {l.data, l.prepared, l.out})) return false;
     if (d.N != N || d.cb != 16 || d.dh != 1 || d.dw != 1 || d.C <= 0 || d.K <= 0 || d.KH <= 0 || d.KW <= 0) return false;
     ConvGeom g;
-    if (conv_geom(&d, 16, &g, "chain") != UNIT_OK) return false;
+    if (conv_sizes(&d, 16, &g, "chain") != UNIT_OK) return false;
     if (d.KH * d.KW > 31 || d.sh > 255 || d.sw > 255 || d.pt > 255 || d.pl > 255) return false;
     const long out_bytes = (long)g.npix * d.K;
     if (out_bytes > 0x7fffffffl) return false;
@@ -686,10 +734,10 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
     s.w = static_cast<const char *>(l.prepared);
     s.out = static_cast<char *>(l.out);
     s.bias = l.bias;
-    int scale = l.scale, shift = l.shift;
-    while (shift < 33 && scale >= -(1 << 30) && scale < (1 << 30)) scale *= 2, ++shift;
-    s.scale = scale;
-    s.shift = (unsigned char)shift;
+    // doubled up to a shift of 33, while there is room for the sign
+    const int up = std::max(0, std::min(33 - l.shift, l.scale ? __builtin_clrsb(l.scale) : 32));
+    s.scale = (int)((unsigned long long)(u32)l.scale << up);
+    s.shift = (unsigned char)(l.shift + up);
     s.K = d.K;
     s.ntaps = g.ntaps;
     s.nsteps = (g.ntaps + 1) / 2;
@@ -716,53 +764,32 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
     // alternating layers, each with all nine combinations: the choice is within 1.9 % of the best one (geometric mean), within 4.5 %
     // for layers under 4 us.  us with 64 x 64 alone / now: ResNet-50 batch 1 203 / 149, 8 232 / 171, 16 275 / 236, 32 377 / 350;
     // ResNet-18 1 83 / 62, 32 118 / 107.  Prices for 1 x 1 layers 0.05 lower: ResNet-50 at 12 images and more 3 - 10 % slower.
-    const bool same = d.sh == 1 && d.sw == 1 && d.pt == 1 && d.pl == 1 && g.OH == d.H && g.OW == d.W;
-    const auto mode_of = [&](int cy, int k) {
-      if (d.KH != 3 || d.KW != 3 || s.ntaps % (18 * k)) return masked ? 2 : s.win == 1 && s.ntaps % 2 == 0 ? 0 : 1;
-      // a wave's part of LDS is 16 KiB
-      return same && d.C / 16 / k * patch_rows(cy, d.W) <= (int)sizeof(ChainLds::part) / kWaves / 1024 ? 4 : 3;
-    };
-    int kg = 1, sx = 64, sy = 64, wx = 1;
+    const Modes modes(d, s);
+    const int K = d.K, nsteps = s.nsteps;
+    int kg = 0, sx = 6, sy = 6, wx = 0;
     double tiles_us = 1e30, steps_us = 0;
-    const auto rounds_of = [&](int cx, int cy, int k, int &x) {  // x: a workgroup's waves side by side along the channels
-      x = 1;
-      while (x < 4 / k && d.K >= 2 * cx * x) x *= 2;
-      const int cols = cx * x, rows = cy * (4 / k / x);
-      return (double)ceil_div(d.K, cols) * ((npix + rows - 1) / rows) / 64;
-    };
-    const auto offer = [&](int cx, int cy, double first, const double (&step)[5]) {
-      for (int k = 1; k <= 4 && k <= s.nsteps; k *= 2) {
+    const auto offer = [&](int xlog, int ylog, double first, const double (&step)[5]) {
+      for (int k = 0; k <= 2 && 1 << k <= nsteps; ++k) {
         int x;
-        const double rounds = rounds_of(cx, cy, k, x);
-        const double t = first + (k > 1 ? 0.1 : 0.0) + 1.9 * std::max(0.0, rounds - 1);
-        const double u = step[mode_of(cy, k)] * ceil_div(s.nsteps, k) * std::max(rounds, 0.5 + 0.5 * std::min(1.0, rounds));
-        if (t + u < tiles_us + steps_us) tiles_us = t, steps_us = u, kg = k, sx = cx, sy = cy, wx = x;
+        const double rounds = rounds_of(K, npix, xlog, ylog, k, x);
+        const double t = first + (k ? 0.1 : 0.0) + 1.9 * std::max(0.0, rounds - 1);
+        const double u = step[modes.of[ylog - 5][k]] * ceil_shift(nsteps, k) * std::max(rounds, 0.5 + 0.5 * std::min(1.0, rounds));
+        if (t + u < tiles_us + steps_us) tiles_us = t, steps_us = u, kg = k, sx = xlog, sy = ylog, wx = x;
       }
     };
-    offer(64, 64, 2.5, {0.27, 0.32, 0.32, 0.26, 0.24});
-    offer(64, 32, 2.15, {0.2, 0.26, 0.26, 0.19, 0.15});
-    offer(32, 32, 2.1, {0.15, 0.21, 0.21, 0.12, 0.09});
-    s.mode = mode_of(sy, kg);
-    const int wy = 4 / kg / wx;
-    s.kg_log = (unsigned char)(kg >> 1), s.wx_log = (unsigned char)(wx >> 1), s.wy_log = (unsigned char)(wy >> 1);
-    s.tile = (unsigned char)((sx == 64 ? 6 : 5) | (sy == 64 ? 6 : 5) << 4);
-    s.nct = ceil_div(d.K, sx * wx);
+    offer(6, 6, 2.5, {0.27, 0.32, 0.32, 0.26, 0.24});
+    offer(6, 5, 2.15, {0.2, 0.26, 0.26, 0.19, 0.15});
+    offer(5, 5, 2.1, {0.15, 0.21, 0.21, 0.12, 0.09});
+    s.mode = modes.of[sy - 5][kg];
+    const int wy = 2 - kg - wx, cols = sx + wx, rows = sy + wy;
+    s.kg_log = (unsigned char)kg, s.wx_log = (unsigned char)wx, s.wy_log = (unsigned char)wy;
+    s.tile = (unsigned char)(sx | sy << 4);
+    s.nct = (int)ceil_shift(K, cols);
     s.by_nct = small_div(s.nct);
-    const long npt = (npix + sy * wy - 1) / (sy * wy);
+    const long npt = ceil_shift(npix, rows);
     if (npt * s.nct * s.nct > 0x7fffffffl) return false;
     const double gmac = 1e-9 * s.ohw * d.K * s.ntaps * 16, mb = 1e-6 * ((double)g.img_bytes + (double)s.ohw * d.K);  // of an image
     here += 0.78 * tiles_us + 1.06 * steps_us + 0.9 * mb * per;
-    int k64 = 1, x64;
-    double best = 1e30;
-    for (int k = 1; k <= 4 && k <= s.nsteps; k *= 2) {
-      const double t = std::max(1.0, (double)ceil_div(d.K, 64) * ((npix + 63) / 64) * k / 256) *
-                       (2.6 + (k > 1 ? 0.4 : 0.0) + 0.25 * ceil_div(s.nsteps, k));
-      if (t < best) best = t, k64 = k;
-    }
-    const double rounds = rounds_of(64, 64, k64, x64);
-    const int m64 = mode_of(64, k64);
-    here64 += 1.45 + (k64 > 1 ? 0.15 : 0.0) + 0.8 * std::max(1.0, rounds) +
-              (m64 == 1 || m64 == 2 ? 0.3 : 0.21) * ceil_div(s.nsteps, k64) * std::max(0.5, rounds) + 1.28 * mb * per;
     launches += 3.6 + 1.15 * gmac * N + 0.176 * mb * N + 0.019 * std::min(s.nsteps, 80);
     s.first = (int)first;
     first += npt * s.nct;
@@ -779,14 +806,14 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
   }
   // Short chains, few images through large layers and activations that outgrow an XCD's 4 MB of L2 stay launches.  The kernel
   // costs 5.4 us before its first tile, then the layers as estimated above and 0.9 us per MB that the group reads and writes; a launch
-  // 3.6 us, 1.2 per GMAC and 0.18 per MB of the batch.  here64 is the estimate for 64 x 64 tiles alone (a layer 1.5 us, 0.8 for each
+  // 3.6 us, 1.2 per GMAC and 0.18 per MB of the batch.  estimate64 is the one for 64 x 64 tiles alone (a layer 1.5 us, 0.8 for each
   // round of an XCD's 64 workgroups, 0.2, with the tap walk 0.3, per k-step of it), which the tiles taken are not slower than.  Both have
   // errors of 6 - 7 % (root mean square) that differ, and either one is taken at its word: over 500 random chains of 3 to 48 layers
-  // timed both ways, here64 alone ends 2.4 % from always the faster way, `here` alone 1.2 %, either 0.8 %; of the 413 given to
+  // timed both ways, estimate64 alone ends 2.4 % from always the faster way, `here` alone 1.2 %, either 0.8 %; of the 413 given to
   // the kernel two lose more than 3 % there, both of 3 layers.  us here / as launches: 3 x 3 64 -> 64 on 56 x 56, batch 8, 3 layers
   // 17.6 / 20.1; 1 x 1 256 -> 256 on 14 x 14, batch 1, 8 layers 24.3 / 30.3; the other way, with 64 x 64 tiles, 14 layers from
   // 51 x 51, batch 14 245 / 201, 10 layers from 50 x 50, batch 52 197 / 167, 9 layers of 224 channels on 20 x 20, batch 2 42.9 / 38.0.
-  if (here64 > 0.975 * launches && here > 0.93 * launches) return false;
+  if (here > 0.93 * launches && estimate64(layers, st, count, per) > 0.975 * launches) return false;
   // The layers no longer run one after the other: none may write what another one reads or writes, but for a source's
   // whole result.
   std::sort(outs, outs + count, [](const Range &u, const Range &v) { return u.a < v.a; });
