@@ -871,6 +871,12 @@ extern "C" int unit_conv_chain_u8_status(const unit_chain_layer *layers, int32_t
       !plan_chain(layers, count, x, st, &p) || ws_bytes < p.bytes)
     return unit_conv_chain_u8(layers, count, x, stream);
   if (int rc = check_device()) return rc;
+  static thread_local bool allowed = false;  // the opt-in for > 64 KiB of dynamic LDS is sticky per kernel
+  if (!allowed) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(chain_run), hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds);
+    if (e != hipSuccess) return fail(UNIT_E_LAUNCH, "%s: hipFuncSetAttribute: %s", what, hipGetErrorString(e));
+    allowed = true;
+  }
   hipStream_t s = static_cast<hipStream_t>(stream);
   char *base = reinterpret_cast<char *>((reinterpret_cast<uintptr_t>(ws) + kWsHead + kWsAlign - 1) / kWsAlign * kWsAlign);
   ChainStep *steps = reinterpret_cast<ChainStep *>(base + p.steps_off);
