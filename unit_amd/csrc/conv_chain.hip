@@ -654,6 +654,14 @@ struct ChainPlan {
   size_t steps_off, bytes;
 };
 
+struct Rings {  // k-steps in flight
+  int of_walk, of_short, of_3x3, of_patch;
+};
+template <int TX, int TY>
+constexpr Rings rings() {
+  return {kRing<TX, TY>, kShort<TX, TY>, kRing3<TX, TY>, kRingPatch<TX, TY>};
+}
+
 struct Range {
   const char *a, *b;
 };
@@ -898,10 +906,16 @@ extern "C" int unit_conv_chain_u8_status(const unit_chain_layer *layers, int32_t
   hipLaunchKernelGGL(chain_run, dim3(256 * kPerCu), dim3(kThreads), sizeof(ChainLds), s, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(UNIT_E_LAUNCH, "%s: launch: %s", what, hipGetErrorString(e));
+  // the workgroup's tile, its k-groups, the k-steps in flight of the general walk (5, 6, 9: wave tiles of 64 x 64, 64 x 32, 32 x 32),
+  // the layer's own walk (MODE) and the k-steps of weights in flight in that
   for (int i = 0; i < count; ++i)
-    if (layers[i].variant)
-      snprintf(layers[i].variant, 96, "q8chain_x%d_y%d_g%d_d%d", 1 << ((st[i].tile & 15) + st[i].wx_log),
-               1 << ((st[i].tile >> 4) + st[i].wy_log), 1 << st[i].kg_log, st[i].tile >> 4 == 6 ? kRing<2, 2> : (st[i].tile & 15) == 6 ? kRing<2, 1> : kRing<1, 1>);
+    if (layers[i].variant) {
+      const ChainStep &t = st[i];
+      const Rings r = t.tile >> 4 == 6 ? rings<2, 2>() : (t.tile & 15) == 6 ? rings<2, 1>() : rings<1, 1>();
+      const bool is_short = t.mode == 0 && ceil_shift(t.nsteps, t.kg_log) <= r.of_short;
+      snprintf(layers[i].variant, 96, "q8chain_x%d_y%d_g%d_d%d_m%d_r%d", 1 << ((t.tile & 15) + t.wx_log), 1 << ((t.tile >> 4) + t.wy_log),
+               1 << t.kg_log, r.of_walk, t.mode, is_short ? r.of_short : t.mode == 4 ? r.of_patch : t.mode == 3 ? r.of_3x3 : r.of_walk);
+    }
   set_variant("q8chain_l%d_n%d_d%d", count, p.per, kRing<2, 2>);
   return UNIT_OK;
 }
