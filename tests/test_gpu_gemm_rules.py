@@ -30,6 +30,18 @@ def test_fp16(dev, M, N, K, tile):
         assert torch.equal(U.gemm_fp16(a, operand, "float16"), ref.half()), U.last_variant()
 
 
+# M, N, K, whether fp32 results share the reduction between workgroups, with b by columns and prepared
+@pytest.mark.parametrize("M,N,K,columns,prepared", [(1082, 100, 2456, True, False), (535, 236, 3080, True, False), (121, 1196, 2304, True, False),
+                                                    (121, 1196, 2296, False, False), (1461, 60, 2456, False, False)])
+def test_fp16_splits(dev, M, N, K, columns, prepared):
+    g = np.random.RandomState(M + N + K)
+    a, b = _ints(g, -3, 4, (M, K), torch.float16, dev), _ints(g, -2, 3, (K, N), torch.float16, dev)
+    ref = a.double() @ b.double()
+    for operand, shared in ((b, columns), (U.prepare_gemm_b(b), prepared)):
+        assert torch.equal(U.gemm_fp16(a, operand).double(), ref), U.last_variant()
+        assert U.last_variant().endswith("_s1") != shared, U.last_variant()
+
+
 # M, N, K, the tile with row-major and prepared weights
 @pytest.mark.parametrize("M,N,K,tile", [(2304, 2048, 784, WIDE), (2305, 2044, 1040, WIDE), (2304, 2048, 752, "_k64_"), (4090, 2048, 1040, WIDE),
                                         (4097, 2048, 784, "x128_y128"), (178, 1336, 1216, "x32_y32"), (636, 420, 1536, "x32_y64"),

@@ -102,13 +102,16 @@ int run_gemm_f16_hybrid(const void *a, const void *b, void *c, int M, int N, int
 // (atomics into the zero-filled output); with more tiles they are the same bits from run to run, and the estimate's splits
 // lost there (900 x 1096 x 7536, 72 tiles, two ranges 64.9 us, whole 49.4; 733 x 1600 x 7616, 78 tiles, 61.8 and 46.2).  With
 // up to six such tiles and 1 KiB of reduction, or fewer than 12 and up to 2 KiB, at least two ways (the tests ask for that; 300 x
-// 260 x 520 would run 2 us faster without).  fp16 results keep one workgroup per tile.
+// 260 x 520 would run 2 us faster without).  b by columns also with fewer than 12 tiles and 4.5 KiB or more, where the estimate's
+// whole tiles take up to a quarter longer (1082 x 100 x 2456 11.9 us, in three ranges 9.4; 535 x 236 x 3080 14.0 and 11.1; 22 products
+// of 2456 and 3080 1.04 in the mean, lowest 0.94; at 4 KiB 535 x 236 x 2056 10.7 and 9.8, 978 x 72 x 2056 7.1 and 8.0).
+// fp16 results keep one workgroup per tile.
 template <int YM, bool OUT_F16>
 int run_gemm_f16_group(const char *what, const char *tag, const void *a, const void *b, void *c, int M, int N, int K,
                        hipStream_t s, bool whole = false) {
   const int forced = OUT_F16 || whole ? 1 : tuning_override("UNIT_AMD_GEMM_F16_SPLITK");
   const long tiles = tiles_of_128(M, N);
-  const int least = forced <= 0 && K >= 512 && (tiles <= 6 || (tiles < 12 && K < 1024)) ? 2 : 1;
+  const int least = forced <= 0 && K >= 512 && (tiles <= 6 || (tiles < 12 && (K < 1024 || (YM == Y_COLS && K >= 2304)))) ? 2 : 1;
   GroupPlan plan = prefer_wide_tile(plan_group(M, N, K * 2, least, forced > 0 || tiles > 64 ? 1 : 19, kAtomicSplits, OUT_F16 ? 2 : 4), M, N, K * 2);
   if (forced > 0) plan.splits = forced;
   const GroupGemm p{static_cast<const char *>(a), static_cast<const char *>(b), (u32)((size_t)M * K * 2),
