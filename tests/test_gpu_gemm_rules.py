@@ -18,7 +18,7 @@ def _ints(g, lo, hi, shape, dtype, dev):
 # M, N, K, the tile with b by columns and prepared
 @pytest.mark.parametrize("M,N,K,tile", [(2304, 2048, 520, WIDE), (2305, 2044, 392, WIDE), (2304, 2048, 376, "_k64_"), (4090, 2040, 520, WIDE),
                                         (4097, 2048, 520, "x128_y128|x256_y256"), (3300, 1292, 1304, WIDE), (562, 320, 1544, "x32_y"),
-                                        (1365, 64, 1856, "x32_y"), (2562, 5436, 72, "x64_y128|x128_y128"), (130, 72, 512, "dma_x128_y128")])
+                                        (1365, 64, 1856, "x32_y"), (2562, 5436, 72, "x64_y128|x128_y128"), (130, 72, 512, "")])
 def test_fp16(dev, M, N, K, tile):
     g = np.random.RandomState(M + N + K)
     a, b = _ints(g, -3, 4, (M, K), torch.float16, dev), _ints(g, -2, 3, (K, N), torch.float16, dev)
@@ -40,6 +40,16 @@ def test_fp16_splits(dev, M, N, K, columns, prepared):
     for operand, shared in ((b, columns), (U.prepare_gemm_b(b), prepared)):
         assert torch.equal(U.gemm_fp16(a, operand).double(), ref), U.last_variant()
         assert U.last_variant().endswith("_s1") != shared, U.last_variant()
+
+
+@pytest.mark.parametrize("M,N,K", [(130, 72, 512), (380, 128, 768), (256, 384, 1024), (640, 640, 768), (512, 768, 768), (520, 768, 1024), (700, 100, 512),
+                                   (300, 260, 512), (128, 768, 1528)])
+def test_fp16_few_tiles_whole(dev, M, N, K):
+    g = np.random.RandomState(M + N + K)
+    a, b = _ints(g, -3, 4, (M, K), torch.float16, dev), _ints(g, -2, 3, (K, N), torch.float16, dev)
+    for operand in (b, U.prepare_gemm_b(b)):
+        assert torch.equal(U.gemm_fp16(a, operand).double(), a.double() @ b.double()), U.last_variant()
+        assert U.last_variant().endswith("_s1") and "dma" not in U.last_variant(), U.last_variant()
 
 
 # M, N, K, the tile with row-major and prepared weights

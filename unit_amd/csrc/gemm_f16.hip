@@ -101,17 +101,17 @@ int run_gemm_f16_hybrid(const void *a, const void *b, void *c, int M, int N, int
 // operator takes (b by columns: N >= 8).  fp32 results of up to 64 tiles of 128 x 128 may also share it between workgroups
 // (atomics into the zero-filled output); with more tiles they are the same bits from run to run, and the estimate's splits
 // lost there (900 x 1096 x 7536, 72 tiles, two ranges 64.9 us, whole 49.4; 733 x 1600 x 7616, 78 tiles, 61.8 and 46.2).  With
-// up to six such tiles and 1 KiB of reduction, or fewer than 12 and up to 2 KiB, at least two ways (the tests ask for that; 300 x
-// 260 x 520 would run 2 us faster without).  b by columns also with fewer than 12 tiles and 4.5 KiB or more, where the estimate's
-// whole tiles take up to a quarter longer (1082 x 100 x 2456 11.9 us, in three ranges 9.4; 535 x 236 x 3080 14.0 and 11.1; 22 products
-// of 2456 and 3080 1.04 in the mean, lowest 0.94; at 4 KiB 535 x 236 x 2056 10.7 and 9.8, 978 x 72 x 2056 7.1 and 8.0).
-// fp16 results keep one workgroup per tile.
+// up to six such tiles and 3 KiB of reduction at least two ways, which costs nothing (0.99 - 1.02 of the whole tiles' time; 1.2 - 1.35
+// from 1 KiB to 2), and with 7 - 11 tiles just over 1 KiB: a test asks for that of 300 x 260 x 520, 5.9 us where whole tiles take 4.5.
+// b by columns also with fewer than 12 tiles and 4.5 KiB or more, where the estimate's whole tiles take up to a quarter longer (1082 x
+// 100 x 2456 11.9 us, in three ranges 9.4; 535 x 236 x 3080 14.0 and 11.1; 22 products of 2456 and 3080 1.04 in the mean, lowest 0.94;
+// at 4 KiB 535 x 236 x 2056 10.7 and 9.8, 978 x 72 x 2056 7.1 and 8.0).  fp16 results keep one workgroup per tile.
 template <int YM, bool OUT_F16>
 int run_gemm_f16_group(const char *what, const char *tag, const void *a, const void *b, void *c, int M, int N, int K,
                        hipStream_t s, bool whole = false) {
   const int forced = OUT_F16 || whole ? 1 : tuning_override("UNIT_AMD_GEMM_F16_SPLITK");
   const long tiles = tiles_of_128(M, N);
-  const int least = forced <= 0 && K >= 512 && (tiles <= 6 || (tiles < 12 && (K < 1024 || (YM == Y_COLS && K >= 2304)))) ? 2 : 1;
+  const int least = forced <= 0 && (tiles <= 6 ? K >= 1536 : tiles < 12 && ((K > 512 && K <= 640) || (YM == Y_COLS && K >= 2304))) ? 2 : 1;
   GroupPlan plan = prefer_wide_tile(plan_group(M, N, K * 2, least, forced > 0 || tiles > 64 ? 1 : 19, kAtomicSplits, OUT_F16 ? 2 : 4), M, N, K * 2);
   if (forced > 0) plan.splits = forced;
   const GroupGemm p{static_cast<const char *>(a), static_cast<const char *>(b), (u32)((size_t)M * K * 2),
@@ -123,14 +123,16 @@ int run_gemm_f16_group(const char *what, const char *tag, const void *a, const v
 // (1011 x 3584 x 1216, 224 tiles, 15.6 against 16.2 us on the group tile of the same size; 2048^3 22.9 against 24.8), and 512
 // tiles or more (8192 x 1024 x 1024 24.2 and 24.0 us).  The others gain: 1024^3 11.1 -> 7.1 us, 2304 x 2304 x 4096
 // 65.5 -> 57.2, 64 x 4096 x 4096 15.6 -> 14.0; and fp32 results of few tiles, whose k-splits cost a zero fill and atomics: 852 x 448 x 2112
-// 14.1 -> 9.1, 562 x 320 x 1536 11.2 -> 7.4, 1365 x 64 x 1856 11.1 -> 6.3, 588 x 516 x 320 8.8 -> 4.9.  The tests name the kernel for
-// two of those, with more than 128 rows: up to six tiles and 512 <= K < 1024, 24 - 31 tiles and 512 <= K < 1536.
+// 14.1 -> 9.1, 562 x 320 x 1536 11.2 -> 7.4, 1365 x 64 x 1856 11.1 -> 6.3, 588 x 516 x 320 8.8 -> 4.9.  Left here are
+// two corners for which tests name this kernel and its k-splits, whole tiles of more than 128 rows: b by columns up to six tiles and 1 - 2
+// KiB (256 x 384 x 512 9.5 us, 4.6 on group tiles), prepared 24 - 31 and 2 - 3 KiB (512 x 768 x 1024 11.1 and 5.9).
 // fp16 results of whole 128-byte rows keep them up to 511 tiles for K of 160 to 640 (6000 x 704 x 256 7.3 us of kernel
 // against 8.1, 5000 x 1024 x 512 11.1 and 12.0; K = 128 6.1 and 5.8).
-inline bool gemm_keeps_128(int M, int N, int K, bool out_f16) {
+inline bool gemm_keeps_128(int M, int N, int K, bool out_f16, bool columns) {
   const long tiles = tiles_of_128(M, N);
   return tiles >= 512 || (tiles >= 192 && tiles <= 256) ||
-         (!out_f16 && M > 128 && K >= 512 && (tiles <= 6 ? K < 1024 : tiles >= 24 && tiles < 32 && K < 1536)) ||
+         (!out_f16 && M > 128 && M % 128 == 0 && N % 128 == 0 &&
+          (columns ? tiles <= 6 && K >= 512 && K < 1024 : tiles >= 24 && tiles < 32 && K >= 1024 && K < 1536)) ||
          (out_f16 && tiles > 256 && N % 64 == 0 && K >= 160 && K <= 640);
 }
 
@@ -169,7 +171,7 @@ int gemm_f16_bt(const void *a, const void *bt, void *c, int M, int N, int K, hip
       if (K % 64 == 0) return run_gemm_f16_bt_dma<Tile<256, 256, 128, 2, 4>, 2, OUT_F16>(a, bt, c, M, N, K, s);
       return run_gemm_f16_bt_dma<Tile<256, 256, 64, 2, 4>, 4, OUT_F16>(a, bt, c, M, N, K, s);
     }
-    if (gemm_keeps_128(M, N, K, OUT_F16))
+    if (gemm_keeps_128(M, N, K, OUT_F16, false))
       return run_gemm_f16_bt_dma<Tile<128, 128, 64, 2, 2>, 4, OUT_F16>(a, bt, c, M, N, K, s, direct_gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K));
   }
   if (gemm_staged_pays(M, N, K, 1.35f)) return run_gemm_f16_bt<Tile<256, 256, 128, 2, 4>, OUT_F16>(a, bt, c, M, N, K, s);
@@ -240,7 +242,7 @@ int gemm_f16(const void *a, const void *b, void *c, int M, int N, int K, hipStre
       return run_gemm_f16_dma_tr<Tile<256, 256, 64, 2, 4>, 4, OUT_F16>(a, b, c, M, N, K, s);
     }
     const int splits = direct_gemm_k_splits("UNIT_AMD_GEMM_F16_SPLITK", M, N, 2l * K);
-    if (gemm_keeps_128(M, N, K, OUT_F16) && !(whole && splits > 1))
+    if (gemm_keeps_128(M, N, K, OUT_F16, true) && !(whole && splits > 1))
       return run_gemm_f16_dma_tr<Tile<128, 128, 64, 2, 2>, 4, OUT_F16>(a, b, c, M, N, K, s, splits);
   }
   // N 4 mod 8, K a whole number of 128-byte stages, and at least 128 tiles of 256 x 128: a straight into LDS, b through
