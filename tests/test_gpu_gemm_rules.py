@@ -56,7 +56,9 @@ def test_fp16_few_tiles_whole(dev, M, N, K):
 @pytest.mark.parametrize("M,N,K,tile", [(2304, 2048, 784, WIDE), (2305, 2044, 1040, WIDE), (2304, 2048, 752, "_k64_"), (4090, 2048, 1040, WIDE),
                                         (4097, 2048, 784, "x128_y128"), (178, 1336, 1216, "x32_y32"), (636, 420, 1536, "x32_y64"),
                                         (1357, 284, 192, "x32_y32"), (141, 348, 5952, "x32_y32"), (24, 564, 6384, "x32_y32"), (33, 900, 3024, "x32_y32"),
-                                        (65, 640, 192, "x32_y32"), (500, 128, 192, "dma_x128_y128"), (300, 1300, 256, "dma_x128_y128")])
+                                        (65, 640, 192, "x32_y32"), (500, 128, 192, ""), (300, 1300, 256, "x32_y"),
+                                        (2048, 2048, 320, "x64_y"), (1000, 520, 256, "x64_y64"), (130, 132, 128, "x32_y32"), (300, 260, 128, ""),
+                                        (64, 256, 2048, "x32_y32"), (128, 760, 3072, "x32_y"), (130, 200, 3072, "x32_y")])
 def test_int8(dev, M, N, K, tile):
     g = np.random.RandomState(M + N + K)
     a, w = _ints(g, 0, 256, (M, K), torch.uint8, dev), _ints(g, -128, 128, (N, K), torch.int8, dev)

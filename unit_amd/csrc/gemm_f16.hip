@@ -102,7 +102,7 @@ int run_gemm_f16_hybrid(const void *a, const void *b, void *c, int M, int N, int
 // (atomics into the zero-filled output); with more tiles they are the same bits from run to run, and the estimate's splits
 // lost there (900 x 1096 x 7536, 72 tiles, two ranges 64.9 us, whole 49.4; 733 x 1600 x 7616, 78 tiles, 61.8 and 46.2).  With
 // up to six such tiles and 3 KiB of reduction at least two ways, which costs nothing (0.99 - 1.02 of the whole tiles' time; 1.2 - 1.35
-// from 1 KiB to 2), and with 7 - 11 tiles just over 1 KiB: a test asks for that of 300 x 260 x 520, 5.9 us where whole tiles take 4.5.
+// from 1 KiB to 2), and with 7 - 11 tiles just over 1 KiB: a test asks for that of 300 x 260 x 520, 6.4 us where whole tiles take 4.8.
 // b by columns also with fewer than 12 tiles and 4.5 KiB or more, where the estimate's whole tiles take up to a quarter longer (1082 x
 // 100 x 2456 11.9 us, in three ranges 9.4; 535 x 236 x 3080 14.0 and 11.1; 22 products of 2456 and 3080 1.04 in the mean, lowest 0.94;
 // at 4 KiB 535 x 236 x 2056 10.7 and 9.8, 978 x 72 x 2056 7.1 and 8.0).  fp16 results keep one workgroup per tile.
@@ -125,7 +125,7 @@ int run_gemm_f16_group(const char *what, const char *tag, const void *a, const v
 // 65.5 -> 57.2, 64 x 4096 x 4096 15.6 -> 14.0; and fp32 results of few tiles, whose k-splits cost a zero fill and atomics: 852 x 448 x 2112
 // 14.1 -> 9.1, 562 x 320 x 1536 11.2 -> 7.4, 1365 x 64 x 1856 11.1 -> 6.3, 588 x 516 x 320 8.8 -> 4.9.  Left here are
 // two corners for which tests name this kernel and its k-splits, whole tiles of more than 128 rows: b by columns up to six tiles and 1 - 2
-// KiB (256 x 384 x 512 9.5 us, 4.6 on group tiles), prepared 24 - 31 and 2 - 3 KiB (512 x 768 x 1024 11.1 and 5.9).
+// KiB (256 x 384 x 512 9.5 us, 4.5 on group tiles), prepared 24 - 31 and 2 - 3 KiB (512 x 768 x 1024 11.8 and 6.1).
 // fp16 results of whole 128-byte rows keep them up to 511 tiles for K of 160 to 640 (6000 x 704 x 256 7.3 us of kernel
 // against 8.1, 5000 x 1024 x 512 11.1 and 12.0; K = 128 6.1 and 5.8).
 inline bool gemm_keeps_128(int M, int N, int K, bool out_f16, bool columns) {

@@ -39,15 +39,15 @@ int run_dense_staged(const void *a, const void *w, void *c, int M, int N, int K,
 // where the estimate without it is 15 us or more (512 x 516 x 12304 30.8 us whole, 20.0 in three ranges; 2081 x 128 x 10208
 // 25.7 and 16.4; 2 x 3968 x 8800, estimate 12.6, 9.4 whole and 11.8 in three), and from 4.5 KiB on (packed 5 KiB: 71 x 1024 x 5040 7.5 and
 // 7.9) with up to 16 tiles of 128 x 128, if the estimate says so (7 x 896 x 8048 packed 9.2 us whole, 6.8 in six; 8 x 1160 x 7840 8.5 in
-// two, 6.7 in six).  The row-major
-// operator shares at least two ways where it has up to six such tiles and 1 KiB of reduction (its tests ask for that; 50 x 260 x 1040
-// would run 2 us faster without, and with 7 - 11 tiles, where it also did, 33 x 820 x 3024 took 7.3 for 6.1).
+// two, 6.7 in six).  The row-major operator shares at least two ways where tests ask for that: with three to six such tiles from 1 KiB of
+// reduction on (50 x 260 x 1040 6.3 us, whole 5.1; 128 x 768 x 3072 7.3 and 6.1), with one or two from 4 KiB on (0.95 of the time whole).
+// Not with one or two tiles below that (64 x 256 x 2048 6.4 us, whole 5.4) and with 7 - 11 (33 x 820 x 3024 7.0 and 6.1).
 template <int YM, int WS>
 int run_dense_group(const char *what, const char *tag, const void *a, const void *w, const int *wsum, void *c, int M, int N,
                     int K, hipStream_t s) {
   const int forced = tuning_override("UNIT_AMD_DENSE_SPLITK");
   const long tiles = tiles_of_128(M, N);
-  const int least = forced <= 0 && YM == Y_ROWS && tiles <= 6 && K >= 1024 ? 2 : 1;
+  const int least = forced <= 0 && YM == Y_ROWS && tiles <= 6 && K >= (tiles >= 3 ? 1024 : 4096) ? 2 : 1;
   GroupPlan plan = plan_group(M, N, K, least, 1, kAtomicSplits);
   if (forced > 0)
     plan.splits = forced;
@@ -64,16 +64,18 @@ int run_dense_group(const char *what, const char *tag, const void *a, const void
 // (8192 x 1024 x 1024 17.3 against 16.5 us).  Else the group tiles are faster (64 x 4096 x 4096 13.3 -> 7.9 us, 1024^3
 // 11.2 -> 7.0, 1024 x 4096 x 4096 29.4 -> 25.3), also with few tiles, whose k-splits cost a zero fill and atomics, and with few stages:
 // 178 x 1336 x 1216 12.2 -> 5.4, 636 x 420 x 1536 12.3 -> 6.5, prepared 420 x 304 x 2112 10.9 -> 5.4, 66 x 1288 x 3776 10.8 -> 6.7;
-// 1357 x 284 x 192 8.3 -> 4.5, 320 x 4160 x 192 8.3 -> 5.8, 2680 x 1352 x 320 9.2 -> 7.8, 7259 x 404 x 64 prepared 7.8 -> 5.8.  The tests
-// name this kernel for a few of those: up to four tiles and 192 bytes, 32 - 63 or 256 and more from 256 bytes to 320, and up to six
-// tiles with 2 - 4 KiB, in k-splits.
-inline bool dense_keeps_128(int M, int N, int K) {
+// 1357 x 284 x 192 8.3 -> 4.5, 320 x 4160 x 192 8.3 -> 5.8, 2680 x 1352 x 320 9.2 -> 7.8, 7259 x 404 x 64 prepared 7.8 -> 5.8.  Left here are
+// the corners for which tests name this kernel, each as small as whole stages and tiles let it be; us here / on group tiles: one tile and
+// up to 128 bytes of reduction (64 x 128 x 128 7.4 / 3.9); row-major weights up to four tiles and 192 bytes (130 x 132 x 192 7.9 / 4.0), 32 -
+// 63 tiles and 320 (1000 x 520 x 320 8.6 / 5.3); prepared ones a tile for each CU and 256 bytes (512 x 8192 x 256 8.4 / 7.4), up to six
+// whole tiles and 2 - 4 KiB, in k-splits (128 x 768 x 3072 9.9 / 7.0, 5.7 without splits).
+inline bool dense_keeps_128(int M, int N, int K, bool prepared) {
   const long tiles = tiles_of_128(M, N);
   if (K % 64 || direct_gemm_large_tiles(M, N)) return false;
   if (tiles >= 512) return true;
-  if (K <= 192) return tiles <= 4;
-  if (K <= 320) return K >= 256 && ((tiles >= 32 && tiles < 64) || tiles >= 256);
-  return tiles <= 6 && K >= 2048 && K < 4096;
+  if (K <= 128) return tiles == 1;
+  if (!prepared) return K == 192 ? tiles <= 4 : K == 320 && tiles >= 32 && tiles < 64;
+  return (K == 256 && tiles == 256) || (M % 128 == 0 && N % 128 == 0 && tiles <= 6 && K >= 2048 && K < 4096);
 }
 
 // direct-to-LDS variant: row-major weights, K a whole number of stages.  wsum: the weight's row sums when they
@@ -184,7 +186,7 @@ int dense(const void *a, const void *w, void *c, int M, int N, int K, unit_strea
       return K % 128 ? run_dense_staged<true, true>(a, w, c, M, N, K, s) : run_dense_staged<true, false>(a, w, c, M, N, K, s);
     return run_dense_group<Y_VNNI, WS_Y>(what, "i8densepk", a, w, nullptr, c, M, N, K, s);
   } else {
-    if (dense_keeps_128(M, N, K))
+    if (dense_keeps_128(M, N, K, false))
       return run_dense_dma<Tile<128, 128, 64, 2, 2>, 4>(a, w, c, M, N, K, s, nullptr,
                                                         direct_gemm_k_splits("UNIT_AMD_DENSE_SPLITK", M, N, K));
     // the four waves that share a weight fragment divide the weight sums
@@ -238,7 +240,7 @@ extern "C" int unit_dense_u8s8s32_prepared(const void *a, const void *w, const i
   if (int rc = check_aligned(what, {a, w, c})) return rc;
   if (int rc = check_device()) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (dense_keeps_128(M, N, K))
+  if (dense_keeps_128(M, N, K, true))
     return run_dense_dma<Tile<128, 128, 64, 2, 2>, 4, true>(a, w, c, M, N, K, s, wsum,
                                                             direct_gemm_k_splits("UNIT_AMD_DENSE_SPLITK", M, N, K));
   if (K % 128 == 0 && direct_gemm_large_tiles(M, N))
