@@ -17,8 +17,8 @@ def _ints(g, lo, hi, shape, dtype, dev):
 
 # M, N, K, the tile with b by columns and prepared
 @pytest.mark.parametrize("M,N,K,tile", [(2304, 2048, 520, WIDE), (2305, 2044, 392, WIDE), (2304, 2048, 376, "_k64_"), (4090, 2040, 520, WIDE),
-                                        (4097, 2048, 520, "x128_y128|x256_y256"), (3300, 1292, 1304, WIDE), (562, 320, 1544, "x32_y"),
-                                        (1365, 64, 1856, "x32_y"), (2562, 5436, 72, "x64_y128|x128_y128"), (130, 72, 512, "")])
+                                        (4097, 2048, 520, "x128_y128|x256_y256"), (3300, 1292, 1304, WIDE), (2048, 2432, 1032, WIDE), (2180, 2052, 1016, WIDE),
+                                        (562, 320, 1544, "x32_y"), (1365, 64, 1856, "x32_y"), (2562, 5436, 72, "x64_y128|x128_y128"), (130, 72, 512, "")])
 def test_fp16(dev, M, N, K, tile):
     g = np.random.RandomState(M + N + K)
     a, b = _ints(g, -3, 4, (M, K), torch.float16, dev), _ints(g, -2, 3, (K, N), torch.float16, dev)
@@ -54,7 +54,7 @@ def test_fp16_few_tiles_whole(dev, M, N, K):
 
 # M, N, K, the tile with row-major and prepared weights
 @pytest.mark.parametrize("M,N,K,tile", [(2304, 2048, 784, WIDE), (2305, 2044, 1040, WIDE), (2304, 2048, 752, "_k64_"), (4090, 2048, 1040, WIDE),
-                                        (4097, 2048, 784, "x128_y128"), (178, 1336, 1216, "x32_y32"), (636, 420, 1536, "x32_y64"),
+                                        (2048, 2432, 2064, WIDE), (2180, 2176, 1040, WIDE), (4097, 2048, 784, "x128_y128"), (178, 1336, 1216, "x32_y32"), (636, 420, 1536, "x32_y64"),
                                         (1357, 284, 192, "x32_y32"), (141, 348, 5952, "x32_y32"), (24, 564, 6384, "x32_y32"), (33, 900, 3024, "x32_y32"),
                                         (65, 640, 192, "x32_y32"), (500, 128, 192, ""), (300, 1300, 256, "x32_y"),
                                         (2048, 2048, 320, "x64_y"), (1000, 520, 256, "x64_y64"), (130, 132, 128, "x32_y32"), (300, 260, 128, ""),

@@ -453,10 +453,12 @@ inline GroupPlan plan_group(int M, int N, int kb, int min_splits, int max_splits
 // 712 prepared 23.2 / 21.9 / 19.8; int8 2304 x 2048 x 2064 31.3 / 26.9 / 24.2, 829 x 5848 x 2576 37.7 / 32.0 / 28.0, 711 x 5480 x 1024 15.7 /
 // 15.1 / 14.8.  The other way from 640 bytes of reduction down (4317 x 1536 x 320 fp16 12.5 / - / 12.9), on packed weights
 // (5400 x 1408 x 1072 19.1 / 20.8 / 21.7) and where 64 x 128 tiles are the estimate's choice, up to 2 KiB (1566 x 2548 x 672 14.8 / - /
-// 16.9).  Left where they were: 301 - 306 small tiles, which the tests name (2180 x 2052 x 2056 would take 34 in place of 44).
+// 16.9).  Left where they were: 301 - 306
+// small tiles of a result whose last row of large ones is cut off, from 2 KiB on, for which tests name the small ones (2180 x 2052 x 2056
+// fp16 43.2 us, 33.0 on the large ones; int8 2180 x 2176 x 2064 31.4 and 24.1).
 inline bool one_wide_tile_per_cu(int M, int N, int kb) {
   const long half = tiles_of_128(M, N), tiles = (long)ceil_div(M, 256) * ceil_div(N, 128);
-  return half > 256 && tiles <= 256 && kb >= 768 && !(half > 300 && tiles <= 153);
+  return half > 256 && tiles <= 256 && kb >= 768 && !(half > 300 && tiles <= 153 && M % 256 && kb >= 2048);
 }
 inline GroupPlan prefer_wide_tile(const GroupPlan &plan, int M, int N, int kb) {
   return plan.splits == 1 && (plan.tile == 5 || (plan.tile == 4 && kb >= 2048)) && one_wide_tile_per_cu(M, N, kb) ? GroupPlan{6, 1, plan.us} : plan;
