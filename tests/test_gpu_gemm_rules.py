@@ -76,6 +76,18 @@ def test_packed_splits(dev, M, N, K, shared):
     assert shared or U.last_variant().endswith("_s1"), U.last_variant()
 
 
+@pytest.mark.parametrize("splits,tile", [(1, WIDE), (2, "x128_y128_k64_"), (3, "x128_y128_k64_")])
+def test_pinned_splits_keep_the_estimate_s_tile(dev, monkeypatch, splits, tile):
+    """The wide tile is for whole reductions: a pinned count of ranges takes the tile that it was measured with."""
+    monkeypatch.setenv("UNIT_AMD_GEMM_F16_SPLITK", str(splits))
+    M, N, K = 2304, 2048, 1048
+    g = np.random.RandomState(splits)
+    a, b = _ints(g, -3, 4, (M, K), torch.float16, dev), _ints(g, -2, 3, (K, N), torch.float16, dev)
+    for operand in (b, U.prepare_gemm_b(b)):
+        assert torch.equal(U.gemm_fp16(a, operand).double(), a.double() @ b.double()), U.last_variant()
+        assert tile in U.last_variant() and U.last_variant().endswith(f"_s{splits}"), U.last_variant()
+
+
 def test_infinity_past_a_row_on_wide_tiles(dev):
     """0 x inf would be NaN: what lies behind a row's end must not reach the sums, in stages of 128 bytes too."""
     M, N, K = 2305, 2044, 392

@@ -112,8 +112,9 @@ int run_gemm_f16_group(const char *what, const char *tag, const void *a, const v
   const int forced = OUT_F16 || whole ? 1 : tuning_override("UNIT_AMD_GEMM_F16_SPLITK");
   const long tiles = tiles_of_128(M, N);
   const int least = forced <= 0 && (tiles <= 6 ? K >= 1536 : tiles < 12 && ((K > 512 && K <= 640) || (YM == Y_COLS && K >= 2304))) ? 2 : 1;
-  GroupPlan plan = prefer_wide_tile(plan_group(M, N, K * 2, least, forced > 0 || tiles > 64 ? 1 : 19, kAtomicSplits, OUT_F16 ? 2 : 4), M, N, K * 2);
+  GroupPlan plan = plan_group(M, N, K * 2, least, forced > 0 || tiles > 64 ? 1 : 19, kAtomicSplits, OUT_F16 ? 2 : 4);
   if (forced > 0) plan.splits = forced;
+  plan = prefer_wide_tile(plan, M, N, K * 2);
   const GroupGemm p{static_cast<const char *>(a), static_cast<const char *>(b), (u32)((size_t)M * K * 2),
                     (u32)((size_t)N * K * 2), M, N, K * 2, YM == Y_COLS ? N * 2 : K * 2, nullptr, c, C_ATOMIC, 0};
   return run_group_plan<OpF16, YM, WS_NONE, OUT_F16>(what, tag, p, plan, s);
