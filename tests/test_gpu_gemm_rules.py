@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import unit_amd as U
+from unit_amd._lib import check, load
 
 pytestmark = pytest.mark.gpu
 
@@ -68,12 +69,16 @@ def test_int8(dev, M, N, K, tile):
         assert tile in U.last_variant(), U.last_variant()
 
 
-@pytest.mark.parametrize("M,N,K,shared", [(7, 896, 5120, True), (7, 896, 5104, False), (130, 1024, 6000, True), (130, 1152, 6000, False)])
+# both sides of 5 KiB of reduction and of 16 tiles of 128 x 128
+@pytest.mark.parametrize("M,N,K,shared", [(7, 896, 5120, True), (7, 896, 5104, False), (30, 2048, 6400, True), (30, 2176, 6400, False)])
 def test_packed_splits(dev, M, N, K, shared):
+    """The result starts as garbage: the ranges add into what their launch has cleared."""
     g = np.random.RandomState(M + N + K)
     a, w = _ints(g, 0, 256, (M, K), torch.uint8, dev), _ints(g, -128, 128, (N, K), torch.int8, dev)
-    assert torch.equal(U.dense_dotprod(a, U.prepack_dense_weight(w)), (a.double() @ w.double().t()).to(torch.int32))
-    assert shared or U.last_variant().endswith("_s1"), U.last_variant()
+    wp, out = U.prepack_dense_weight(w), torch.full((M, N), 0x5a5a5a5a, dtype=torch.int32, device=dev)
+    check(load().unit_dense_dotprod_u8s8s32(a.data_ptr(), wp.data_ptr(), out.data_ptr(), M, N, K, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(out, (a.double() @ w.double().t()).to(torch.int32)), U.last_variant()
+    assert (int(U.last_variant().rsplit("_s", 1)[1]) > 1) == shared, U.last_variant()
 
 
 @pytest.mark.parametrize("splits,tile", [(1, WIDE), (2, "x128_y128_k64_"), (3, "x128_y128_k64_")])
