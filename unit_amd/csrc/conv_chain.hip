@@ -769,9 +769,14 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
     // workgroups are idle, since the others then have the loads to themselves.  Smaller tiles move more operand bytes per result and
     // pay where large ones leave workgroups idle; k-groups that leave whole periods of nine k-steps keep the cheap walk (3 x 3, 64
     // channels, 28 x 28, batch 4: four groups of 5 k-steps that walk 3.8 us a layer, two of 9 2.7).  Fitted to 1400 chains of two
-    // alternating layers, each with all nine combinations: the choice is within 1.9 % of the best one (geometric mean), within 4.5 %
-    // for layers under 4 us.  us with 64 x 64 alone / now: ResNet-50 batch 1 203 / 149, 8 232 / 171, 16 275 / 236, 32 377 / 350;
-    // ResNet-18 1 83 / 62, 32 118 / 107.  Prices for 1 x 1 layers 0.05 lower: ResNet-50 at 12 images and more 3 - 10 % slower.
+    // alternating layers, each with all nine combinations, but for 1 x 1 layers on 32 x 32 tiles: 0.10 by the fit, with which ResNet-50 at
+    // 12 images and more is 3 - 10 % slower (what its layers have that those chains lack is not in these prices).  The choice is 2.0 %
+    // from the best one (geometric mean).  us with 64 x 64 alone / now: ResNet-50 batch 1 203 / 151, 8 232 / 171, 16 275 / 237,
+    // 32 377 / 350; ResNet-18 1 83 / 62, 32 118 / 110; 1309 random chains 1.23 in the mean, seven of them 3 - 9 % slower, and 59 of
+    // the 1400: mostly tiles of few k-steps that occupy every workgroup (1 x 1 128 -> 128 on 32 x 32, two images, 16 layers 42.5 / 47.2; 3 x 3
+    // 112 -> 112 on 32 x 32, eight images, six layers 40.3 / 44.7), one with weights beyond the L2 (3 x 3 256 - 2048 on 14 x 14, eight
+    // images, 276 / 372).  0.5 us more from half a round to a full one, refitted: random chains 1.01, ResNet-50 at up to eight images 3 -
+    // 4 % slower; 0.2 us, not for 1 x 1 layers: 78 of 1200 random chains gain more than 3 %, five lose up to 9.  Neither is taken.
     const Modes modes(d, s);
     const int K = d.K, nsteps = s.nsteps;
     int kg = 0, sx = 6, sy = 6, wx = 0;
@@ -815,8 +820,9 @@ bool plan_chain(const unit_chain_layer *layers, int count, const void *x, ChainS
   // Short chains, few images through large layers and activations that outgrow an XCD's 4 MB of L2 stay launches.  The kernel
   // costs 5.4 us before its first tile, then the layers as estimated above and 0.9 us per MB that the group reads and writes; a launch
   // 3.6 us, 1.2 per GMAC and 0.18 per MB of the batch.  estimate64 is the one for 64 x 64 tiles alone (a layer 1.5 us, 0.8 for each
-  // round of an XCD's 64 workgroups, 0.2, with the tap walk 0.3, per k-step of it), which the tiles taken are not slower than.  Both have
-  // errors of 6 - 7 % (root mean square) that differ, and either one is taken at its word: over 500 random chains of 3 to 48 layers
+  // round of an XCD's 64 workgroups, 0.2, with the tap walk 0.3, per k-step of it); the tiles taken are 1.23 times as fast in the mean, but
+  // no chain is sure to be (above).  Both have errors of 6 - 7 % (root mean square) that differ, and either one is taken at its word, for
+  // what that measured: over 500 random chains of 3 to 48 layers
   // timed both ways, estimate64 alone ends 2.4 % from always the faster way, `here` alone 1.2 %, either 0.8 %; of the 413 given to
   // the kernel two lose more than 3 % there, both of 3 layers.  us here / as launches: 3 x 3 64 -> 64 on 56 x 56, batch 8, 3 layers
   // 17.6 / 20.1; 1 x 1 256 -> 256 on 14 x 14, batch 1, 8 layers 24.3 / 30.3; the other way, with 64 x 64 tiles, 14 layers from

@@ -249,6 +249,8 @@ int gemm_f16(const void *a, const void *b, void *c, int M, int N, int K, hipStre
   // N 4 mod 8, K a whole number of 128-byte stages, and at least 128 tiles of 256 x 128: a straight into LDS, b through
   // the transposing register loader.  256 x 256 tiles of eight waves, or 256 x 128 tiles of four when those need fewer
   // rounds of 256 workgroups for their cost (about 0.55 of a 256 x 256 tile).
+  // The 128-byte stages of one_wide_tile_per_cu are faster where they apply (2304 x 2044 x 1024 19.0 us, here 22.8; 4090 x 2044 x 512
+  // 19.4 and 20.2); a test names this kernel for such a product (2048 x 2052 x 512 13.5 and 15.6).
   if (N % 8 && M >= 256 && N >= 128 && K % 64 == 0 && K >= 128) {
     const long tiles_big = (long)ceil_div(M, 256) * ceil_div(N, 256), tiles_half = (long)ceil_div(M, 256) * ceil_div(N, 128);
     const long rounds_big = ceil_div((int)tiles_big, 256), rounds_half = ceil_div((int)tiles_half, 256);
